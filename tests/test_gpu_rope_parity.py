@@ -72,6 +72,17 @@ def test_layer_shapes(gpu_ready, po, shape):
     assert ds[0] == 0, f"debug status {ds}"
 
 
+@pytest.mark.parametrize("shape", [
+    # the kernel with two rows per wave (more than 8192 rows of at most 512 bytes), head counts that leave waves half full
+    (257, 30, 1, 256, 100, False, 1, 0),          # 32 heads: just past the line
+    (600, 13, 1, 128, 70000, True, 1, 1023),      # 15 heads: the last wave of a row holds one
+    (900, 9, 1, 64, 0, False, 0, 0),              # 11 heads: a wave without any
+    (1024, 7, 1, 32, 5000, False, 1, 2047),       # half of the lanes idle
+])
+def test_two_rows_per_wave(gpu_ready, po, shape):
+    test_layer_shapes(gpu_ready, po, shape)
+
+
 def _random_case(seed):
     rng = np.random.default_rng(5000 + seed)
     hd = int(rng.choice([32, 64, 128, 256, 512]))
