@@ -45,6 +45,7 @@ struct AttnParams {
   uint32_t part_half;    // split partials are normalised f16 rows instead of unnormalised fp32 ones
   uint32_t touch_ahead;  // head_dim 512: touch key/value tiles into the L2 some tiles before they are loaded
   uint32_t lo_explicit;  // lo_nc was given by the caller (not the window rule)
+  uint32_t cus;          // compute units of the device
   uint32_t sees_masked;  // causal rows also see the canvas keys behind the causal rows
   float scale_log2;      // softmax_scale * log2(e)
 };
@@ -103,6 +104,21 @@ __device__ __forceinline__ AttnParams resolve_step(const AttnParams& in) {
   p.tile_first = lo_all / (uint32_t)kBlockN;
   p.tile_end = max(p.tile_first, (p.t_all + (uint32_t)kBlockN - 1u) / (uint32_t)kBlockN);
   return p;
+}
+
+// Division of n < 2^31 by a divisor the host knows: q = (mulhi(n, mul) + n) >> shift (the round-up method: mul =
+// floor(2^32 (2^shift - d) / d) + 1 with shift = ceil(log2 d)).  Three scalar instructions where a run-time division is
+// two dozen on the vector unit.
+struct FastDiv {
+  uint32_t mul, shift;
+};
+inline FastDiv make_fast_div(uint32_t d) {
+  uint32_t shift = 0;
+  while ((1ull << shift) < d) ++shift;
+  return FastDiv{(uint32_t)((((1ull << shift) - d) << 32) / d + 1u), shift};
+}
+__host__ __device__ __forceinline__ uint32_t fast_div(uint32_t n, FastDiv d) {
+  return ((uint32_t)(((uint64_t)n * d.mul) >> 32) + n) >> d.shift;
 }
 
 struct RowBounds {

@@ -49,25 +49,28 @@ std::mutex g_dev_mu;
 
 // Which caches this thread's calls streamed lately, to tell whether a call's key/value rows can still be in the
 // memory-side cache (256 MB on MI355X): a cache is taken to be cold when other caches of more than 200 MiB in total
-// were streamed since its last use, or on its first use when it is large.  Decides only which instance of the
-// head_dim 512 kernel runs (the one that touches tiles into the L2 ahead of their loads: same bits, other timing);
-// under graph capture the decision recorded is the one made at capture.
+// were streamed since its last use, or on its first use when it is large (head_dim 512, where touching rows that were
+// cached after all costs 3 %) or of any size (below, where it costs nothing that can be measured).  Decides only whether
+// the kernels touch keys and values into the L2 ahead of their loads: same bits, other timing; under graph capture the
+// decision recorded is the one made at capture.  64 entries: a loop over a model's layers (30 caches) has to find each of
+// them again.
 struct CacheMemo {
   const void* region = nullptr;
   uint64_t streamed_at_last_use = 0;
 };
-thread_local CacheMemo g_memo[16];
+constexpr int kMemoEntries = 64;
+thread_local CacheMemo g_memo[kMemoEntries];
 thread_local uint64_t g_streamed = 0;
 
-bool cache_is_cold(const void* region, uint64_t bytes) {
+bool cache_is_cold(const void* region, uint64_t bytes, bool large_only) {
   int idx = -1, oldest = 0;
-  for (int i = 0; i < 16; ++i) {
+  for (int i = 0; i < kMemoEntries; ++i) {
     if (g_memo[i].region == region) idx = i;
     if (g_memo[i].streamed_at_last_use < g_memo[oldest].streamed_at_last_use) oldest = i;
   }
   bool cold;
   if (idx < 0) {
-    cold = bytes >= (32ull << 20);
+    cold = !large_only || bytes >= (32ull << 20);
     idx = oldest;
     g_memo[idx].region = region;
   } else {
@@ -128,6 +131,7 @@ struct Plan {
   uint32_t group = 0, rows_total = 0, n_mtiles = 0, rows_pad = 0;
   uint32_t t_all = 0, lo_nc = 0, extra_lo = 0, win_m1 = 0xffffffffu;
   uint32_t clip_lo = 0, clip_hi = 0;   // keys that count: [clip_lo, clip_hi); the whole range unless a partial is asked for
+  uint32_t cus = 256;
   uint32_t tile_first = 0, tile_end = 0, tiles_per_split = 0, n_splits = 1;
   uint32_t e_dtype = DG_BF16;   // element type the kernels compute in (bf16 or f16)
   bool convert_q = false, gather_kv = false, q_is_bf16 = false;
@@ -140,6 +144,7 @@ struct Plan {
 
 int make_plan(const dg_attn_desc* d, int cus, Plan* pl, const uint32_t* key_range = nullptr) {
   if (!d) return DG_ERR_NULL;
+  pl->cus = (uint32_t)cus;
   const uint32_t hd = d->head_dim;
   if (d->canvas == 0 || d->canvas > 65536 || d->n_q_heads == 0 || d->n_kv_heads == 0) return DG_ERR_SHAPE;
   if (d->n_q_heads % d->n_kv_heads != 0 || d->n_q_heads > 65535) return DG_ERR_SHAPE;
@@ -435,6 +440,7 @@ int fill_params(const dg_attn_desc* d, const Plan& pl, const void* q, const void
   p.out_dtype = d->out_dtype;
   p.out_trunc = (d->flags & DG_ATTN_F_OUT_TRUNCATE) ? 1u : 0u;
   p.part_half = pl.part_half ? 1u : 0u;
+  p.cus = pl.cus;
   p.lo_explicit = (d->flags & DG_ATTN_F_T_LO_EXPLICIT) ? 1u : 0u;
   p.sees_masked = (d->flags & DG_ATTN_F_CAUSAL_SEES_MASKED) ? 1u : 0u;
   // key/value rows this call streams: more than the 256 MiB memory-side cache holds cannot have
@@ -442,7 +448,7 @@ int fill_params(const dg_attn_desc* d, const Plan& pl, const void* q, const void
   const uint64_t kv_streamed = 2ull * d->n_kv_heads * (uint64_t)(pl.tile_end - pl.tile_first) * dg::kBlockN * d->head_dim * 2ull;
   // ... and a cache that other large caches were streamed after since its last use has been displaced
   // (cache_is_cold); DG_ATTN_F_KV_CACHED says the caller knows better
-  const bool cold = cache_is_cold(region, kv_streamed) && hd == 512;   // (every call counts towards what was streamed)
+  const bool cold = cache_is_cold(region, kv_streamed, hd == 512);
   p.touch_ahead = ((d->flags & DG_ATTN_F_KV_FROM_HBM) || kv_streamed > (256ull << 20) ||
                    (cold && !(d->flags & DG_ATTN_F_KV_CACHED))) ? 1u : 0u;
   p.scale_log2 = pl.scale * dg::kLog2e;

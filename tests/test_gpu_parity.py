@@ -4,6 +4,8 @@ max_abs 1e-2 / 2e-2, cosine >= 0.9999) on its own fixtures; max-abs <= 2e-2, mea
 on bf16 outputs and per-row LSE within 1e-3 relative on the benchmark configurations."""
 import ctypes as C
 
+from dataclasses import replace
+
 import numpy as np
 import pytest
 
@@ -275,6 +277,26 @@ def test_one_launch_kernel_against_the_general_one(gpu_ready, po, hd, hq, hkv, c
     assert np.max(np.abs(one[1][ok] - gen[1][ok]), initial=0.0) <= 2 * LSE_ABS      # each within 2^-8 of the exact value
     again = run_workload(po, w, out_f32=True)
     assert np.array_equal(one[0].view(np.uint32), again[0].view(np.uint32)) and np.array_equal(one[1].view(np.uint32), again[1].view(np.uint32))
+
+
+@pytest.mark.parametrize("hd,hq,hkv,canvas,kv_len,causal_rows,window,sees_masked,flags", [
+    (256, 16, 8, 513, 1500, 513, 1024, False, 0),        # just past one round of 32-row workgroups; last row tile of two rows
+    (256, 16, 8, 1000, 40, 1000, 0, False, capi.DG_ATTN_F_KV_FROM_HBM),   # no window: row tiles of 2 .. 33 key tiles
+    (256, 16, 8, 600, 3001, 300, 1024, True, 0),         # mixed rows, causal ones with a second key range
+    (128, 8, 8, 1033, 77, 0, 300, False, capi.DG_ATTN_F_KV_FROM_HBM), (64, 16, 8, 520, 5, 260, 0, False, 0),
+    (32, 12, 4, 700, 900, 700, 100, False, 0),           # group of 3
+])
+def test_one_launch_kernel_with_64_rows_per_workgroup(gpu_ready, po, hd, hq, hkv, canvas, kv_len, causal_rows, window, sees_masked,
+                                                      flags):
+    """More than 256 workgroups of 32 rows: the one-launch kernel takes 64 rows per workgroup.  Every row tile's edges
+    (ragged last tile, key ranges that start and end inside a key tile) against the oracle, for both storages."""
+    w = W.Workload("ws64", canvas, hq, hkv, hd, kv_len, causal_rows=causal_rows, window=window, seed=hd + canvas,
+                   sees_masked=sees_masked)
+    assert capi.resolved_splits(w.desc()) == 1 and capi.workspace_bytes(w.desc()) == 0
+    toks = np.unique(np.concatenate([np.arange(0, canvas, 37), np.arange(canvas - 3, canvas), [causal_rows - 1, causal_rows]]))
+    toks = toks[(toks >= 0) & (toks < canvas)].astype(np.uint32)
+    check_tolerances(*run_workload(po, w, flags=flags, toks=toks))
+    check_tolerances(*run_workload(po, replace(w, kv_f16=True), flags=flags, toks=toks, out_f32=True))
 
 
 # ------------------------------------------------------------------ size-independent properties at full size
