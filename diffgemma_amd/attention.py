@@ -169,11 +169,18 @@ def make_desc(canvas: int, n_q_heads: int, n_kv_heads: int, head_dim: int, kv_le
 # device plumbing (torch = memory + streams only)
 # ---------------------------------------------------------------------------------------
 
+_torch_module = None
+
+
 def _torch():
-    import torch
-    if not torch.cuda.is_available():
-        raise RuntimeError("no HIP device: the attention path runs only on a gfx950 GPU")
-    return torch
+    """torch, once it has been seen to have a device (asking again on every launch costs half a microsecond)."""
+    global _torch_module
+    if _torch_module is None:
+        import torch
+        if not torch.cuda.is_available():
+            raise RuntimeError("no HIP device: the attention path runs only on a gfx950 GPU")
+        _torch_module = torch
+    return _torch_module
 
 
 def to_device_bits(bits: np.ndarray):
@@ -183,7 +190,10 @@ def to_device_bits(bits: np.ndarray):
 
 
 def stream_handle() -> int:
-    return _torch().cuda.current_stream().cuda_stream
+    """torch's current stream as a hipStream_t.  The raw handle, not a Stream object around it: a layer step asks twice, and
+    the object takes as long to make as a kernel launch (3.8 us against 0.3)."""
+    torch = _torch()
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def forward(desc: capi.AttnDesc, q, kv, out, lse=None, workspace=None) -> None:

@@ -100,8 +100,8 @@ def snapshot_bytes(arr, kv_len: int) -> int:
 
 
 def _stream() -> int:
-    import torch
-    return torch.cuda.current_stream().cuda_stream
+    from .attention import stream_handle
+    return stream_handle()
 
 
 def gather_kv_prefix(buf, arr, kv_len: int):
