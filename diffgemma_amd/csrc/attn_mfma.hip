@@ -85,9 +85,6 @@ __device__ __forceinline__ uint32_t opaque(uint32_t v) {
   return v;
 }
 
-// the value brought into the finite range of f16 (NaN stays NaN)
-__device__ __forceinline__ float sat_f16(float x) { return __builtin_amdgcn_fmed3f(x, -65504.f, 65504.f); }
-
 // acc + lo + hi of a packed pair, in one dot-product instruction
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
@@ -102,9 +99,14 @@ __device__ __forceinline__ float add_pair(uint32_t pk, float acc) {
   }
 }
 
+struct MfmaArgs {
+  AttnParams p;
+  FastDiv div_mtiles, div_splits, div_group;
+};
+
 template <int D, bool F16, bool TOUCH>
-__global__ void __launch_bounds__(256) attn_mfma_kernel(const AttnParams p_in) {
-  const AttnParams p = resolve_step(p_in);
+__global__ void __launch_bounds__(256) attn_mfma_kernel(const MfmaArgs args) {
+  const AttnParams p = resolve_step(args.p);
   using L = Lay<D>;
   constexpr int NSTEP = D / 16, NDB = D / 32;
   // P.V work split: DSPLIT groups of d-blocks x RSPLIT groups of row-blocks = 4 waves
@@ -151,13 +153,8 @@ __global__ void __launch_bounds__(256) attn_mfma_kernel(const AttnParams p_in) {
   const uint32_t wg = blockIdx.x;
   const uint32_t unit = (wg & 7u) * per_xcd + (wg >> 3);
   if (unit >= n_units) return;
-  // (the divisions by run-time values are done by the vector unit; readfirstlane tells the
-  // compiler the results are the same in every lane, so everything derived from them stays in
-  // scalar registers)
-  const uint32_t stream = __builtin_amdgcn_readfirstlane(unit / p.n_mtiles);
-  const uint32_t mt = __builtin_amdgcn_readfirstlane(unit % p.n_mtiles);
-  const uint32_t kvh = __builtin_amdgcn_readfirstlane(stream / p.n_splits);
-  const uint32_t split = __builtin_amdgcn_readfirstlane(stream % p.n_splits);
+  const uint32_t stream = fast_div(unit, args.div_mtiles), mt = unit - stream * p.n_mtiles;
+  const uint32_t kvh = fast_div(stream, args.div_splits), split = stream - kvh * p.n_splits;
 
   const uint32_t lane = threadIdx.x & 63u;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -168,8 +165,8 @@ __global__ void __launch_bounds__(256) attn_mfma_kernel(const AttnParams p_in) {
   const uint32_t row0 = mt * kBlockM;
   const uint32_t r = row0 + wave * 32u + l32;
   const bool row_ok = r < p.rows_total;
-  const uint32_t tok = row_ok ? r / p.group : 0u;
-  const uint32_t qh = kvh * p.group + (row_ok ? r % p.group : 0u);
+  const uint32_t tok = row_ok ? fast_div(r, args.div_group) : 0u;
+  const uint32_t qh = kvh * p.group + (row_ok ? r - tok * p.group : 0u);
   RowBounds rb = row_bounds(p, tok);
   if (!row_ok) {
     rb.lo = 0;
@@ -181,7 +178,7 @@ __global__ void __launch_bounds__(256) attn_mfma_kernel(const AttnParams p_in) {
   uint32_t lo_min, lo_max, hi_min, hi_max;
   {
     const uint32_t last_row = min(row0 + kBlockM, p.rows_total) - 1u;
-    const uint32_t tok_a = row0 / p.group, tok_b = last_row / p.group;
+    const uint32_t tok_a = fast_div(row0, args.div_group), tok_b = fast_div(last_row, args.div_group);
     const RowBounds ba = row_bounds(p, tok_a), bb = row_bounds(p, tok_b);
     lo_min = min(ba.lo, bb.lo);
     lo_max = max(ba.lo, bb.lo);
@@ -245,56 +242,100 @@ __global__ void __launch_bounds__(256) attn_mfma_kernel(const AttnParams p_in) {
     }
   }
 
+  // ---- how tiles are loaded.  Loads for a tile past the last one are not branched around: they fetch the last tile again
+  // into a buffer nobody reads any more (or whose scores nobody uses). ----
+  lds_char* const k0 = (lds_char*)(smem + OFF_K0);
+  lds_char* const k1 = (lds_char*)(smem + OFF_K1);
+  lds_char* const v0 = (lds_char*)(smem + OFF_V0);
+  lds_char* const v1 = (lds_char*)(smem + OFF_V1);
+  const uint32_t t_last = (te - 1u) * kBlockN;
+  // (in the loop only tiles behind the workgroup's first one are loaded)
+  auto k_load = [&](uint32_t t0, lds_char* buf, uint32_t ln) {
+    return make_tile_load<D, false, false>(kbase, kstride_b, min(t0, t_last), 0u, p.t_all, p.ring_mask, buf, wave, ln);
+  };
+  auto v_load = [&](uint32_t t0, lds_char* buf, uint32_t ln) {
+    return make_tile_load<D, true, false>(vbase, vstride_b, min(t0, t_last), 0u, p.t_all, p.ring_mask, buf, wave, ln);
+  };
+  auto k_load_first = [&](lds_char* buf) {
+    return make_tile_load<D, false, true>(kbase, kstride_b, tb * kBlockN, lo_min, p.t_all, p.ring_mask, buf, wave, lane);
+  };
+  auto v_load_first = [&](lds_char* buf) {
+    return make_tile_load<D, true, true>(vbase, vstride_b, tb * kBlockN, lo_min, p.t_all, p.ring_mask, buf, wave, lane);
+  };
+
   // ---- Q fragments: B operand of S^T = K.Q^T, lane = row, 8 consecutive d per step ----
   // The operand layout gives a lane 16 bytes of its own row per step, so loading the fragments
   // straight from memory touches 32 bytes of 32 different cache lines per instruction, and the
   // four waves' 128 KiB pass through the compute unit's first-level cache several times over
   // (measured: 4.7 us until the rows had landed, 3.0 us this way).  Instead each wave brings its
-  // 32 rows into LDS as whole rows, in the layout of a K tile (the tile buffers are not in use
-  // yet), and reads the fragments from there the way it reads K fragments.
+  // 32 rows into LDS as whole pieces of rows and reads the fragments from there the way it reads K fragments.
+  // (Rows past the last one repeat it: finite values, and the rows are masked everywhere.)
   u32x4 qf[NSTEP];
   {
-    static_assert(4 * L::K_BYTES <= LDS_BYTES, "the four waves' query rows are staged in the tile buffers");
-    lds_char* const qb = (lds_char*)smem + wave * L::K_BYTES;
-    // byte offset of this lane's row (rows past the last one repeat it: finite values, and the
-    // rows are masked everywhere); below 4 GiB, which the host checks
-    const uint32_t rq = min(r, p.rows_total - 1u);
-    const uint32_t q_row_off = ((rq / p.group * p.hq) + kvh * p.group + rq % p.group) * (uint32_t)(2 * D);
+    const char* const q_base = (const char*)p.q + (size_t)kvh * p.group * (2 * D);
+    // byte offset of a stacked row; below 4 GiB, which the host checks
+    auto q_row_off = [&](uint32_t row) -> uint32_t {
+      const uint32_t rq = min(row, p.rows_total - 1u);
+      return (rq + fast_div(rq, args.div_group) * (p.hq - p.group)) * (uint32_t)(2 * D);
+    };
+    auto q_to_frag = [&](u32x4 raw, u32x4& f) {
+      if (F16 && p.q_is_bf16) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          f[e] = pack2<true>(__uint_as_float(raw[e] << 16), __uint_as_float(raw[e] & 0xffff0000u));
+      } else {
+        f = raw;
+      }
+    };
     if constexpr (L::PAD) {
-      // one instruction = one row
-      static_for<0, 32>([&](auto i_c) {
-        constexpr int i = decltype(i_c)::value;
-        const uint32_t off = __builtin_amdgcn_readlane(q_row_off, i);
-        lds_dma_16<i * L::K_STRIDE>((const char*)p.q + off, lane * 16u, (uint32_t)(size_t)qb);
-      });
+      // In two halves of head_dim, through the V tiles' LDS: the first K tiles can then be on their way at the same time
+      // (256 rows over 1033 keys: 33.9 -> 31.2 us with the divisions by reciprocals and the rolled loops; this part is run
+      // once, from code fetched cold at about 10 cycles an instruction, so its length counts as much as its waits).
+      // One instruction = half of rows i and i + 16, 16 bytes apart from the next pair.  A wave reads what it loaded
+      // itself, so there is no barrier between the halves.
+      constexpr uint32_t PAIR = 1024 + 16;
+      static_assert(4 * 16 * PAIR <= 2 * L::V_BYTES, "the V tiles hold half of the query rows");
+      lds_char* const qb = v0 + wave * (16u * PAIR);
+      auto load_half = [&](uint32_t half) {
+        const uint32_t rq = r - l32 + (lane >> 5) * 16u;
+#pragma unroll 1
+        for (uint32_t i = 0; i < 16u; ++i)
+          lds_dma_16<0>(q_base, q_row_off(rq + i) + half * (uint32_t)D + l32 * 16u, (uint32_t)(size_t)qb + i * PAIR);
+      };
+      lds_char* const ql = qb + i16 * PAIR + h16 * (uint32_t)D + g2 * 16u;
+      load_half(0u);
+      if (ntile > 0) {
+        issue_tile<D, false>(k_load_first(k0), wave, lane);
+        issue_tile<D, false>(k_load((tb + 1) * kBlockN, k1, lane), wave, lane);
+        wait_vmem_but<2 * L::NLD>();
+      } else {
+        wait_vmem_all();
+      }
+#pragma unroll
+      for (int st = 0; st < NSTEP / 2; ++st) q_to_frag(*(lds_u32x4*)(ql + 32 * st), qf[st]);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (read before the second half lands there)
+      load_half(1u);
+      wait_vmem_all();
+#pragma unroll
+      for (int st = 0; st < NSTEP / 2; ++st) q_to_frag(*(lds_u32x4*)(ql + 32 * st), qf[NSTEP / 2 + st]);
     } else {
+      // in the layout of a K tile, through the tile buffers
+      static_assert(4 * L::K_BYTES <= LDS_BYTES, "the four waves' query rows are staged in the tile buffers");
+      lds_char* const qb = (lds_char*)smem + wave * L::K_BYTES;
       // one instruction = 64 chunks of 16 bytes = 64 / CPR rows, swizzled like a K tile
       static_for<0, L::NBLK>([&](auto b_c) {
         constexpr int blk = decltype(b_c)::value;
         const uint32_t pch = blk * 64 + lane;
         const uint32_t rl = pch / L::CPR, pc = pch % L::CPR;
-        const uint32_t c = pc ^ L::swz_k(rl);
-        const uint32_t off = __shfl(q_row_off, (int)rl, 64) + c * 16u;
-        lds_dma_16<blk * 1024>((const char*)p.q, off, (uint32_t)(size_t)qb);
+        lds_dma_16<blk * 1024>(q_base, q_row_off(row0 + wave * 32u + rl) + (pc ^ L::swz_k(rl)) * 16u, (uint32_t)(size_t)qb);
       });
-    }
-    wait_vmem_all();
-    const uint32_t q_lane_off = l32 * L::K_STRIDE + (L::PAD ? g2 * 16u : 0u);
-    const uint32_t q_swz = L::swz_k(l32);
+      wait_vmem_all();
+      const uint32_t q_lane_off = l32 * L::K_STRIDE, q_swz = L::swz_k(l32);
 #pragma unroll
-    for (int s = 0; s < NSTEP; ++s) {
-      u32x4 raw;
-      if constexpr (L::PAD) raw = *(lds_u32x4*)(qb + q_lane_off + 32 * s);
-      else raw = *(lds_u32x4*)(qb + q_lane_off + ((((uint32_t)(2 * s) + g2) ^ q_swz) << 4));
-      if (F16 && p.q_is_bf16) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          qf[s][e] = pack2<true>(__uint_as_float(raw[e] << 16), __uint_as_float(raw[e] & 0xffff0000u));
-      } else {
-        qf[s] = raw;
-      }
+      for (int st = 0; st < NSTEP; ++st) q_to_frag(*(lds_u32x4*)(qb + q_lane_off + ((((uint32_t)(2 * st) + g2) ^ q_swz) << 4)), qf[st]);
     }
-    // every wave has its fragments before the first tiles overwrite the rows
+    // every wave has its fragments before the next tiles overwrite the rows (head_dim 512: and everybody's first K tiles
+    // have landed)
     __syncthreads();
   }
 
@@ -352,27 +393,6 @@ __global__ void __launch_bounds__(256) attn_mfma_kernel(const AttnParams p_in) {
   };
 
   if (ntile > 0) {
-    lds_char* const k0 = (lds_char*)(smem + OFF_K0);
-    lds_char* const k1 = (lds_char*)(smem + OFF_K1);
-    lds_char* const v0 = (lds_char*)(smem + OFF_V0);
-    lds_char* const v1 = (lds_char*)(smem + OFF_V1);
-    // Loads for a tile past the last one are not branched around: they fetch the last tile
-    // again into a buffer nobody reads any more (or whose scores nobody uses).
-    const uint32_t t_last = (te - 1u) * kBlockN;
-    // (in the loop only tiles behind the workgroup's first one are loaded)
-    auto k_load = [&](uint32_t t0, lds_char* buf, uint32_t ln) {
-      return make_tile_load<D, false, false>(kbase, kstride_b, min(t0, t_last), 0u, p.t_all, p.ring_mask, buf, wave, ln);
-    };
-    auto v_load = [&](uint32_t t0, lds_char* buf, uint32_t ln) {
-      return make_tile_load<D, true, false>(vbase, vstride_b, min(t0, t_last), 0u, p.t_all, p.ring_mask, buf, wave, ln);
-    };
-    auto k_load_first = [&](lds_char* buf) {
-      return make_tile_load<D, false, true>(kbase, kstride_b, tb * kBlockN, lo_min, p.t_all, p.ring_mask, buf, wave, lane);
-    };
-    auto v_load_first = [&](lds_char* buf) {
-      return make_tile_load<D, true, true>(vbase, vstride_b, tb * kBlockN, lo_min, p.t_all, p.ring_mask, buf, wave, lane);
-    };
-
     // ---- softmax of one tile, cut into NCH pieces ----
     // The pieces of tile jj run between the score MFMAs of tile jj+1: one wave per SIMD issues
     // in order, so vector work only overlaps the matrix pipe if it sits between MFMAs in
@@ -494,11 +514,15 @@ __global__ void __launch_bounds__(256) attn_mfma_kernel(const AttnParams p_in) {
     using ISPLIT = std::integral_constant<int, NSPLIT>;
     using IQK = std::integral_constant<int, NQK>;
 
-    issue_tile<D, false>(k_load_first(k0), wave, lane);
-    issue_tile<D, false>(k_load((tb + 1) * kBlockN, k1, lane), wave, lane);
-    issue_tile<D, true>(v_load_first(v0), wave, lane);
-    wait_vmem_all();
-    __syncthreads();
+    if constexpr (L::PAD) {
+      issue_tile<D, true>(v_load_first(v0), wave, lane);   // (waited for in front of the first tile's P.V)
+    } else {
+      issue_tile<D, false>(k_load_first(k0), wave, lane);
+      issue_tile<D, false>(k_load((tb + 1) * kBlockN, k1, lane), wave, lane);
+      issue_tile<D, true>(v_load_first(v0), wave, lane);
+      wait_vmem_all();
+      __syncthreads();
+    }
     // s_a: scores of the tile whose softmax is due; s_b: scores being accumulated for the next.
     // s_b is copied into s_a during each tile's P.V by copy_scores_part(), not by an assignment:
     // the compiler would merge the two and place its own copy right behind (or before) the last
@@ -648,6 +672,7 @@ __global__ void __launch_bounds__(256) attn_mfma_kernel(const AttnParams p_in) {
   }
 
   // ---- epilogue ----
+  if (p.part_half) f16_saturate();
   // row owners publish (m, l) of their rows; d owners normalise and store their slice of O
   const float l_tot = sum_across_halves(l_part + l_part2);
   const float m_pub = m_ref + kPOff<F16>;   // the exponent the sums are relative to
@@ -685,9 +710,7 @@ __global__ void __launch_bounds__(256) attn_mfma_kernel(const AttnParams p_in) {
 #pragma unroll
         for (int q4 = 0; q4 < 4; ++q4) {
           const f32x4 x = acc_read4<D == 512>(a, 4 * q4);
-          u32x2 h2;
-          h2[0] = pack2<true>(sat_f16(x[0] * inv), sat_f16(x[1] * inv));
-          h2[1] = pack2<true>(sat_f16(x[2] * inv), sat_f16(x[3] * inv));
+          const u32x2 h2 = {mul_pack_f16(x[0], x[1], inv), mul_pack_f16(x[2], x[3], inv)};
           *(__attribute__((address_space(3))) u32x2*)(stg + l32 * STG_ROW + (32 * i + 8 * q4 + 4 * g2) * 2) = h2;
         }
       }
@@ -731,7 +754,7 @@ __global__ void __launch_bounds__(256) attn_mfma_kernel(const AttnParams p_in) {
     if (rr >= p.rows_total) continue;
     const float l_row = sml[(rbk * 32u + l32) * 2u + 1u];
     const float inv = l_row > 0.f ? 1.f / l_row : 0.f;
-    const uint32_t tok_o = rr / p.group, qh_o = kvh * p.group + rr % p.group;
+    const uint32_t tok_o = fast_div(rr, args.div_group), qh_o = kvh * p.group + rr - tok_o * p.group;
 #pragma unroll
     for (int i = 0; i < NDBW; ++i) {
       const size_t idx0 = ((size_t)tok_o * p.hq + qh_o) * D + 32u * (dgrp * NDBW + i) + 4u * g2;
@@ -765,15 +788,19 @@ __global__ void __launch_bounds__(256) attn_mfma_kernel(const AttnParams p_in) {
 
 template <int D, bool F16>
 hipError_t launch_one(const AttnParams& p, hipStream_t s) {
-  const uint32_t nstream = p.hkv * p.n_splits;
-  const uint32_t grid = ((nstream * p.n_mtiles + 7u) / 8u) * 8u;
+  MfmaArgs a;
+  a.p = p;
+  a.div_mtiles = make_fast_div(p.n_mtiles);
+  a.div_splits = make_fast_div(p.n_splits);
+  a.div_group = make_fast_div(p.group);
+  const uint32_t grid = ((p.hkv * p.n_splits * p.n_mtiles + 7u) / 8u) * 8u;
   if constexpr (D == 512) {
     if (p.touch_ahead) {
-      hipLaunchKernelGGL((attn_mfma_kernel<D, F16, true>), dim3(grid), dim3(256), 0, s, p);
+      hipLaunchKernelGGL((attn_mfma_kernel<D, F16, true>), dim3(grid), dim3(256), 0, s, a);
       return hipGetLastError();
     }
   }
-  hipLaunchKernelGGL((attn_mfma_kernel<D, F16, false>), dim3(grid), dim3(256), 0, s, p);
+  hipLaunchKernelGGL((attn_mfma_kernel<D, F16, false>), dim3(grid), dim3(256), 0, s, a);
   return hipGetLastError();
 }
 

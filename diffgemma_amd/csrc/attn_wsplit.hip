@@ -69,14 +69,6 @@ __device__ __forceinline__ float ws_add_pair(uint32_t pk, float acc) {
   }
 }
 
-// all but the N most recent vector memory operations of the wave (N up to 63: vmcnt is bits 3:0 and 15:14)
-template <int N>
-__device__ __forceinline__ void ws_wait_vmem_but() {
-  static_assert(N >= 0 && N < 64, "six bits of vmcnt");
-  __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
-  asm volatile("" ::: "memory");
-}
-
 // A 32-key tile in LDS.  One direct-to-LDS instruction brings a KiB = RPK = 512 / D whole rows, and instruction i brings
 // rows i, i + NBLK, i + 2 NBLK, ...: the lanes' offset from the tile's first row is then the same for every instruction
 // of the tile, which only moves a scalar address by one row.  The KiB blocks are padded apart (K by 16 bytes, V by 64),
@@ -492,7 +484,7 @@ __global__ void __launch_bounds__(256) attn_wsplit_kernel(const WsArgs args) {
     if (more) issue_k(tile + 1u);
     static_for<0, MR>([&](auto m_c) { softmax(m_c, tmax[decltype(m_c)::value]); });
     // V(jj) has landed (the loads of K(jj+1), issued after it, may still be on their way)
-    if (more) ws_wait_vmem_but<NBLK>();
+    if (more) wait_vmem_but<NBLK>();
     else wait_vmem_all();
     pv();
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the V buffer is free for the next tile's loads

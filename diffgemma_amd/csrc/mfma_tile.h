@@ -120,6 +120,17 @@ __device__ __forceinline__ uint32_t pack2(float a, float b) {
     return __builtin_bit_cast(uint32_t, v);
   }
 }
+// (a c, b c) as a packed pair of halves, one instruction each and one rounding; f16_saturate() first, for products beyond
+// the range
+__device__ __forceinline__ uint32_t mul_pack_f16(float a, float b, float c) {
+  uint32_t d;
+  asm("v_fma_mixlo_f16 %0, %1, %2, 0" : "=v"(d) : "v"(a), "v"(c));
+  asm("v_fma_mixhi_f16 %0, %1, %2, 0" : "+v"(d) : "v"(b), "v"(c));
+  return d;
+}
+// From here on the wave's f16 results saturate to +-65504 instead of overflowing (FP16_OVFL; an infinite operand still
+// gives an infinity).
+__device__ __forceinline__ void f16_saturate() { asm volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 23, 1), 1" ::: "memory"); }
 template <bool F16>
 __device__ __forceinline__ float unpack_lo(uint32_t u) {
   if constexpr (F16) return (float)__builtin_bit_cast(_Float16, (uint16_t)(u & 0xffffu));
@@ -142,8 +153,8 @@ __device__ __forceinline__ void wait_vmem_all() {
 // all but the N most recent vector memory operations of the wave (they complete in order)
 template <int N>
 __device__ __forceinline__ void wait_vmem_but() {
-  static_assert(N >= 0 && N < 16, "low four bits of vmcnt");
-  __builtin_amdgcn_s_waitcnt(0x0F70 | N);
+  static_assert(N >= 0 && N < 64, "six bits of vmcnt");
+  __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
   asm volatile("" ::: "memory");
 }
 
