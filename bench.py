@@ -293,7 +293,7 @@ TOPK_SHAPES = {   # canvas, Hq, Hkv, hd, kv_len, causal_rows: global layers of t
 
 def bench_topk(args):
     """Top-k sparse attention of a global layer with the production k rule: one step = one
-    dg_attn_topk_forward (score kernel + select kernel per block of canvas rows)."""
+    dg_attn_topk_forward (thresholds and lists, then selection, per pass over canvas rows)."""
     import torch
     from diffgemma_amd import attention as A, attention_topk as T, capi, rounding as R, workloads as W
     from oracle import pyoracle as po
@@ -336,22 +336,21 @@ def bench_topk(args):
     select_ms /= args.steps
     ms = (t1 - t0) * 1e3 / args.steps
 
-    # algorithmic work: the score kernel multiplies every visible (row, key) pair once (2 * hd flop);
-    # the select kernel reads every visible fp32 score once, gathers the kept V rows and writes the row
+    # algorithmic work: every visible (row, key) pair is multiplied once (2 * hd flop) where the thresholds and lists are made;
+    # the selection gathers the kept V rows and writes the row
     kept = float(sum(min(max((-(-(kv_len + t + 1) // 256) * 256 if t < cr else w.t_all) // 128, 64), 512)
                      for t in range(canvas)))
     qk_flops = 2.0 * hd * nq * pairs
-    # (the gathered V rows of a block of canvas rows come from at most the whole V plane: what is
-    # gathered beyond that is cache traffic, reported separately)
+    # (the gathered V rows come from at most the whole V plane: what is gathered beyond that is cache traffic,
+    # reported separately)
     gathered = kept * nq * hd * 2
-    row_blocks = -(-canvas // max(1, (T.workspace_bytes(d, k_cfg) // (nq * 4 * (-(-w.t_all // 32) * 32)))))
-    sel_bytes = 4.0 * nq * pairs + min(gathered, row_blocks * float(w.t_all * nkv * hd * 2)) + canvas * nq * hd * 2
-    score_bytes = 4.0 * nq * pairs + w.t_all * nkv * hd * 2 + canvas * nq * hd * 2
+    sel_bytes = min(gathered, float(w.t_all * nkv * hd * 2)) + canvas * nq * hd * 2
+    score_bytes = w.t_all * nkv * hd * 2 + canvas * nq * hd * 2
     dominant_is_select = select_ms >= scores_ms
     roof = ({"bound": "hbm", "achieved": sel_bytes / (select_ms * 1e-3) / 1e9, "peak": PEAK_HBM_GBS, "unit": "GB/s",
-             "kernel": "topk_select_kernel", "kernel_ms": select_ms} if dominant_is_select else
+             "kernel": "topk_list_select_kernel", "kernel_ms": select_ms} if dominant_is_select else
             {"bound": "mfma", "achieved": qk_flops / (scores_ms * 1e-3) / 1e12, "peak": PEAK_BF16_TFLOPS,
-             "unit": "TFLOP/s", "kernel": "topk_scores_kernel", "kernel_ms": scores_ms})
+             "unit": "TFLOP/s", "kernel": "topk_filter_kernel (with the sampled scores and thresholds)", "kernel_ms": scores_ms})
     roof["frac"] = roof["achieved"] / roof["peak"]
     roof["traffic"] = None
     res = {"metric": f"top-k sparse attention of a global layer ({canvas}-row canvas @ {kv_len} prefix, k = t/128): "
@@ -360,14 +359,12 @@ def bench_topk(args):
            "ms_per_step": ms, "higher_is_better": True, "scaling": "weak", "vs_baseline": None, "dtype": "bf16",
            "data": "synthetic",
            "config": {"workload": args.workload, "canvas": canvas, "kv_prefix": kv_len, "n_q_heads": nq, "n_kv_heads": nkv,
-                      "head_dim": hd, "causal_rows": cr, "k_cfg": list(k_cfg), "row_blocks": n_blocks,
-                      "score_plane_bytes": T.workspace_bytes(d, k_cfg)},
-           "kernels": {"topk_scores_kernel": {"ms": scores_ms, "tflops": qk_flops / (scores_ms * 1e-3) / 1e12,
+                      "head_dim": hd, "causal_rows": cr, "k_cfg": list(k_cfg), "workspace_bytes": T.workspace_bytes(d, k_cfg)},
+           "kernels": {"topk_filter_kernel": {"ms": scores_ms, "tflops": qk_flops / (scores_ms * 1e-3) / 1e12,
                                               "frac_mfma_peak": qk_flops / (scores_ms * 1e-3) / 1e12 / PEAK_BF16_TFLOPS,
-                                              "written_gbs": 4.0 * nq * pairs / (scores_ms * 1e-3) / 1e9,
                                               "algorithmic_bytes": score_bytes},
-                       "topk_select_kernel": {"ms": select_ms, "gbs": sel_bytes / (select_ms * 1e-3) / 1e9,
-                                              "algorithmic_bytes": sel_bytes, "gathered_v_bytes": gathered}},
+                       "topk_list_select_kernel": {"ms": select_ms, "gbs": sel_bytes / (select_ms * 1e-3) / 1e9,
+                                                   "algorithmic_bytes": sel_bytes, "gathered_v_bytes": gathered}},
            "roofline": roof, "check": check}
     if not args.no_cpu_baseline:
         threads = min(po.max_threads(), 16)

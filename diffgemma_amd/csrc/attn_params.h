@@ -62,7 +62,23 @@ struct TopkParams {
   uint32_t tile_first, tile_end;
   uint32_t k_cfg[4];     // (fixed k | chunk grid, divisor, k_min, k_max)
   float scale;
+  // Filtered path (launch_topk_filter): n_mtiles counts 256-row tiles there.
+  uint32_t sample_stride;   // every sample_stride-th key has its scores in the sample plane
+  uint32_t sample_n, sample_pad;
+  float* sample_plane;   // [hq][ntok][sample_pad]
+  float* tau;            // [hkv][n_mtiles * 256]: a row's threshold
+  uint32_t* cand_n;      // [hkv][n_mtiles][n_splits][4 waves][kTopkSegs]: entries in a segment
+  void* cand;            // the same index space, kTopkSegAlloc entries of 8 bytes each
+  uint32_t* fail_rows;   // [canvas][hq]: rows the filtered path has left over (null: every row takes the general path)
+  uint32_t* fail_block;  // rows left over per block of canvas rows (general path: of this block)
+  uint32_t fail_block_tok;   // canvas rows per block
 };
+// A segment holds the candidates that one lane finds for one query row: half of the row's in a key-range split.  The spare
+// places behind the limit take what one more key tile may bring before the count is looked at.
+constexpr uint32_t kTopkSegs = 128;         // per wave of the filter kernel and split: two blocks of 32 rows, two lanes per row
+constexpr uint32_t kTopkSegCap = 80, kTopkSegAlloc = kTopkSegCap + 16;
+constexpr uint32_t kTopkFilterRows = 256;   // stacked rows per workgroup of the filter kernel
+constexpr uint32_t kTopkSampleMax = 8192;   // most sampled keys per row
 
 // Merging attention states of key-range partials (dg_attn_merge).  A state holds, per row
 // (row = canvas row * n_q_heads + query head), m and l in two planes of `rows` floats and then, from
@@ -204,6 +220,10 @@ hipError_t launch_kv_gather(const void* src, uint32_t src_dtype, void* dst, uint
                             uint32_t t_all, uint32_t head_dim, int64_t tok_stride, int64_t head_stride,
                             uint32_t ring_mask, hipStream_t s);
 
+// The filtered path over rows [tok0, tok0 + ntok): thresholds and lists (`sample`: the same rows over the sampled keys),
+// then selection out of the lists.
+hipError_t launch_topk_filter(const TopkParams& tp, const TopkParams& sample, uint32_t kv_dtype, hipStream_t s);
+hipError_t launch_topk_list_select(const TopkParams& tp, uint32_t k_most, uint32_t kv_dtype, hipStream_t s);
 hipError_t launch_topk_scores(const TopkParams& tp, uint32_t head_dim, uint32_t kv_dtype, hipStream_t s);
 hipError_t launch_topk_select(const TopkParams& tp, uint32_t head_dim, uint32_t kv_dtype, hipStream_t s);
 

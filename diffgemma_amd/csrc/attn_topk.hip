@@ -18,6 +18,7 @@
 //                       V rows are gathered with one 16-byte load per lane and row (hd 512).
 // The host walks the canvas in row blocks sized so that the score plane stays within the
 // memory-side cache.
+// Long rows at head_dim 512 take another way ("filtered path" below), without the plane.
 #include "attn_params.h"
 #include "mfma_tile.h"
 
@@ -48,6 +49,7 @@ __device__ __forceinline__ void wait_loads_then_barrier() {
 template <int D, bool F16>
 __global__ void __launch_bounds__(256) topk_scores_kernel(const TopkParams tp) {
   const AttnParams& p = tp.a;
+  if (tp.fail_block != nullptr && *tp.fail_block == 0u) return;   // no row of this block was left over
   using L = Lay<D>;
   constexpr int NSTEP = D / 16;
   constexpr int NLD = L::NLD;
@@ -258,6 +260,19 @@ __device__ __forceinline__ uint32_t visible_count(const RowBounds& b, uint32_t t
   return len_a + (t_all - b.extra);
 }
 
+// keys kept for a row (attention_topk.metal:160-182)
+__device__ __forceinline__ uint32_t row_k(const TopkParams& tp, uint32_t tok, uint32_t n_valid) {
+  uint32_t k_req;
+  if (tp.k_cfg[1] != 0u) {
+    const uint32_t gran = max(tp.k_cfg[0], 1u);
+    const uint32_t t_equiv = tok < tp.a.causal_rows ? ((n_valid + gran - 1u) / gran) * gran : n_valid;
+    k_req = min(max(t_equiv / tp.k_cfg[1], tp.k_cfg[2]), tp.k_cfg[3]);
+  } else {
+    k_req = max(tp.k_cfg[0], 1u);
+  }
+  return min(min(k_req, n_valid), (uint32_t)kTopkMaxK);
+}
+
 struct SelectShared {
   uint32_t hist[kMaxBins];
   uint32_t tot[256];
@@ -351,20 +366,12 @@ __global__ void __launch_bounds__(256) topk_select_kernel(const TopkParams tp) {
   const uint32_t lane = tid & 63u, wave = tid >> 6;
   const uint32_t tok_l = blockIdx.x, qh = blockIdx.y;
   const uint32_t tok = tp.tok0 + tok_l;
+  if (tp.fail_rows != nullptr && tp.fail_rows[(size_t)tok * p.hq + qh] == 0u) return;   // done by the filtered path
   const uint32_t kvh = qh / p.group;
   const RowBounds rb = row_bounds(p, tok);
   const uint32_t n_valid = visible_count(rb, p.t_all);
 
-  // keys kept for this row (attention_topk.metal:160-182)
-  uint32_t k_req;
-  if (tp.k_cfg[1] != 0u) {
-    const uint32_t gran = max(tp.k_cfg[0], 1u);
-    const uint32_t t_equiv = tok < p.causal_rows ? ((n_valid + gran - 1u) / gran) * gran : n_valid;
-    k_req = min(max(t_equiv / tp.k_cfg[1], tp.k_cfg[2]), tp.k_cfg[3]);
-  } else {
-    k_req = max(tp.k_cfg[0], 1u);
-  }
-  const uint32_t k = min(min(k_req, n_valid), (uint32_t)kTopkMaxK);
+  const uint32_t k = row_k(tp, tok, n_valid);
 
   const size_t out_off = ((size_t)tok * p.hq + qh) * D;
   if (k == 0u) {   // a row that sees no key stores zeros, like the dense path
@@ -712,6 +719,541 @@ __global__ void __launch_bounds__(256) topk_select_kernel(const TopkParams tp) {
   }
 }
 
+// ---------------------------------------------------------------------------------------------
+// filtered path: long rows at head_dim 512 without a score plane
+// ---------------------------------------------------------------------------------------------
+//
+// A call of the general path writes every score (541 MB for 256 rows over 33k keys) and reads it back to keep one key
+// in 128.  Here a row's threshold tau is guessed first, from the scores of every 17th key; the score kernel then
+// stores only scores at or above tau, as (score, position) entries in lists, and the select kernel works on a list of
+// two to four times k entries that one wave holds in registers.  Whatever tau is, the result is exact: a row whose
+// list holds fewer than k entries, or more than fit, is marked, and the general path redoes the marked rows (its
+// launches end at once where no row of the block is marked, 1.5 us each).
+// 256 rows x 16 heads over 33024 keys, layer step: 646 -> 283 us.  Launches: sampled scores 24 us (was: scores and plane, 4 x 55),
+// thresholds 16, filter 141 (0.98 PFLOP/s; the products alone, with their LDS reads and nothing else, 101), selection 99
+// (was 4 x 94; 70 of the 99 are the gathered V rows, 1.08 GB through the L2s).
+
+// scores through an ordinary-register accumulator, query fragment in accumulation registers (256 of them hold the 64
+// query rows of a wave; a comparison cannot read that file)
+template <bool F16, bool FIRST>
+__device__ __forceinline__ void mfma_filter(f32x16& s, const u32x4& k, const u32x4& q) {
+  if constexpr (FIRST) {
+    if constexpr (F16) asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, 0" : "=&v"(s) : "v"(k), "a"(q));
+    else asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(s) : "v"(k), "a"(q));
+  } else {
+    if constexpr (F16) asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+v"(s) : "v"(k), "a"(q));
+    else asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(s) : "v"(k), "a"(q));
+  }
+}
+// the last product of both row blocks and the wait states a non-MFMA read of the scores needs, in one statement
+template <bool F16>
+__device__ __forceinline__ void mfma_filter_last(f32x16& s0, f32x16& s1, const u32x4& k, const u32x4& q0, const u32x4& q1) {
+  if constexpr (F16)
+    asm volatile("v_mfma_f32_32x32x16_f16 %0, %2, %3, %0\n\tv_mfma_f32_32x32x16_f16 %1, %2, %4, %1\n\ts_nop 11"
+                 : "+v"(s0), "+v"(s1) : "v"(k), "a"(q0), "a"(q1));
+  else
+    asm volatile("v_mfma_f32_32x32x16_bf16 %0, %2, %3, %0\n\tv_mfma_f32_32x32x16_bf16 %1, %2, %4, %1\n\ts_nop 11"
+                 : "+v"(s0), "+v"(s1) : "v"(k), "a"(q0), "a"(q1));
+}
+// Four stores of the filter kernel, each by the lanes in its mask and by lane 0.
+__device__ __forceinline__ void store4_masked(const uint64_t (&m)[4], const uint32_t (&at)[4], u32x2 e0, u32x2 e1, u32x2 e2,
+                                              u32x2 e3, char* base) {
+  asm volatile(
+      "s_or_b64 exec, %0, 1\n\tglobal_store_dwordx2 %4, %8, %12\n\t"
+      "s_or_b64 exec, %1, 1\n\tglobal_store_dwordx2 %5, %9, %12\n\t"
+      "s_or_b64 exec, %2, 1\n\tglobal_store_dwordx2 %6, %10, %12\n\t"
+      "s_or_b64 exec, %3, 1\n\tglobal_store_dwordx2 %7, %11, %12\n\t"
+      "s_mov_b64 exec, -1" ::"s"(m[0]), "s"(m[1]), "s"(m[2]), "s"(m[3]), "v"(at[0]), "v"(at[1]), "v"(at[2]), "v"(at[3]),
+      "v"(e0), "v"(e1), "v"(e2), "v"(e3), "s"(base)
+      : "memory", "scc");
+}
+
+__device__ __forceinline__ uint32_t wave_max(uint32_t x) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) x = max(x, (uint32_t)__shfl_xor((int)x, off, 64));
+  return (uint32_t)__builtin_amdgcn_readfirstlane((int)x);
+}
+__device__ __forceinline__ float wave_sum(float x) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
+  return x;
+}
+__device__ __forceinline__ uint32_t rank_in(uint64_t mask) {   // set bits below this lane
+  return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+}
+// LDS written by this wave is read by it next (a wave's LDS operations complete in order; this holds the compiler)
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// Threshold of a row, one wave each: with `mean` = the number of sampled keys expected among the k largest, tau is about the
+// (mean + 5 sqrt(mean) + 3)-th largest sampled score, so that the k largest lie above it but for a five-sigma accident.
+// Any value near will do, so the bisection stops at the first key that leaves a count in a small range.
+template <int NV>
+__global__ void __launch_bounds__(256) topk_tau_kernel(const TopkParams tp) {
+  const AttnParams& p = tp.a;
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t rid = __builtin_amdgcn_readfirstlane(blockIdx.x * 4u + (threadIdx.x >> 6));
+  if (rid >= tp.ntok * p.hq) return;
+  const uint32_t rows = tp.ntok * p.group;
+  const uint32_t kvh = rid / rows, rr = rid % rows;
+  const uint32_t tok_l = rr / p.group, qh = kvh * p.group + rr % p.group;
+  const uint32_t tok = tp.tok0 + tok_l;
+  if (qh == 0u && tok_l % tp.fail_block_tok == 0u && lane == 0u) tp.fail_block[tok_l / tp.fail_block_tok] = 0u;
+  const RowBounds rb = row_bounds(p, tok);
+  const uint32_t k = row_k(tp, tok, visible_count(rb, p.t_all));
+  const float* srow = tp.sample_plane + ((size_t)qh * tp.ntok + tok_l) * tp.sample_pad;
+  uint32_t key[NV], top = 0u;
+#pragma unroll
+  for (int u = 0; u < NV; ++u) key[u] = __float_as_uint(srow[min(64u * u + lane, tp.sample_n - 1u)]);   // (all in flight)
+#pragma unroll
+  for (int u = 0; u < NV; ++u) {
+    const uint32_t i = 64u * u + lane;
+    const bool in = i < tp.sample_n && key_visible(rb, i * tp.sample_stride, p.t_all);
+    key[u] = in ? score_key(__uint_as_float(key[u])) : 0u;
+  }
+#pragma unroll
+  for (int u = 0; u < NV; ++u) top = max(top, key[u]);
+  const float mean = (float)k / (float)tp.sample_stride;
+  const uint32_t want = (uint32_t)(mean + 5.f * __builtin_sqrtf(mean) + 3.f);
+  // a lower end first, from the lanes' largest keys alone: the want-th largest of those 64 has at least `want` above it
+  // (one comparison a step instead of NV; `want` is below 64 at 512 keys kept)
+  uint32_t lo = ~wave_max(~top), hi = wave_max(top) + 1u;      // count(>= lo) >= want, count(>= hi) < want
+  for (uint32_t h = hi; h - lo > 1u;) {
+    const uint32_t mid = lo + ((h - lo) >> 1);
+    const uint32_t c = (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(top >= mid));
+    if (c >= want) lo = mid;
+    else h = mid;
+    if (c == want) break;
+  }
+  while (hi - lo > 1u) {
+    const uint32_t mid = lo + ((hi - lo) >> 1);
+    uint32_t c = 0u;
+#pragma unroll
+    for (int u = 0; u < NV; ++u) c += (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(key[u] >= mid));
+    if (c >= want) lo = mid;
+    else hi = mid;
+    if (c >= want && c <= want + 2u) break;
+  }
+  // (lo = 0, a row with fewer sampled keys than wanted, is the image of NaN: nothing passes, and the row is left over)
+  if (lane == 0u) tp.tau[(size_t)kvh * tp.n_mtiles * kTopkFilterRows + rr] = key_score(lo);
+}
+
+// Scores against thresholds.  256 stacked rows per workgroup, 64 per wave: with 32 (topk_scores_kernel) the four waves
+// together read the K tile from LDS as fast as the LDS can give it (128 bytes a cycle) and the matrix cores wait.
+// Splits take every n_splits-th key tile, so that keys that score high side by side spread over the segments.
+template <bool F16>
+__global__ void __launch_bounds__(256) topk_filter_kernel(const TopkParams tp) {
+  constexpr int D = 512;
+  const AttnParams& p = tp.a;
+  using L = Lay<D>;
+  constexpr int NSTEP = D / 16;
+  constexpr int NLD = L::NLD;
+  constexpr int PF = 3, NB = PF + 1;   // K tiles in flight ahead of the one being multiplied
+  __shared__ __attribute__((aligned(1024))) char smem[NB * L::K_BYTES];
+
+  const uint32_t n_units = p.hkv * tp.n_splits * tp.n_mtiles;
+  const uint32_t per_xcd = (n_units + 7u) >> 3;
+  const uint32_t unit = (blockIdx.x & 7u) * per_xcd + (blockIdx.x >> 3);
+  if (unit >= n_units) return;
+  // row tiles of one (KV head, split) next to each other: they read the same keys through one L2
+  const uint32_t mt = __builtin_amdgcn_readfirstlane(unit % tp.n_mtiles);
+  const uint32_t kvh = __builtin_amdgcn_readfirstlane(unit / tp.n_mtiles / tp.n_splits);
+  const uint32_t split = __builtin_amdgcn_readfirstlane(unit / tp.n_mtiles % tp.n_splits);
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t g2 = lane >> 5, l32 = lane & 31u;
+  const uint32_t rows_total = tp.ntok * p.group;
+  const uint32_t row0 = mt * kTopkFilterRows + wave * 64u;
+  const uint32_t n_tiles_all = (p.t_all + kBlockN - 1u) / kBlockN;
+  const uint32_t n_tiles = split < n_tiles_all ? (n_tiles_all - split + tp.n_splits - 1u) / tp.n_splits : 0u;
+  const uint32_t seg = (((kvh * tp.n_mtiles + mt) * tp.n_splits + split) * 4u + wave) * kTopkSegs;   // this wave's first segment
+  if (n_tiles == 0u) {
+    tp.cand_n[seg + lane] = tp.cand_n[seg + 64u + lane] = 0u;
+    return;
+  }
+
+  const char* kbase = (const char*)p.k + (int64_t)kvh * p.k_head_stride * 2;
+  const int64_t kstride_b = p.k_tok_stride * 2;
+  const uint32_t k_lane_off = l32 * L::K_STRIDE + g2 * 16u;
+  auto tile_t0 = [&](uint32_t i) { return (split + min(i, n_tiles - 1u) * tp.n_splits) * (uint32_t)kBlockN; };
+  // (past the last tile: the last one again into a buffer nobody reads, so that the wait counts stay fixed)
+  auto k_desc = [&](uint32_t i) {
+    return make_tile_load<D, false, false>(kbase, kstride_b, tile_t0(i), 0u, p.t_all, 0u,
+                                           (lds_char*)(smem + (i % NB) * L::K_BYTES), wave, lane);
+  };
+#pragma unroll
+  for (int i = 0; i < PF; ++i) issue_tile<D, false>(k_desc((uint32_t)i), wave, lane);
+
+  u32x4 qf[2][NSTEP];
+#pragma unroll
+  for (int b = 0; b < 2; ++b) {
+    const uint32_t r = min(row0 + 32u * b + l32, rows_total - 1u);   // (rows past the last copy it: tau is +inf there)
+    const uint32_t tok = tp.tok0 + r / p.group, qh = kvh * p.group + r % p.group;
+    const uint16_t* qp = (const uint16_t*)p.q + ((size_t)tok * p.hq + qh) * D + 8u * g2;
+#pragma unroll
+    for (int s = 0; s < NSTEP; ++s) {
+      u32x4 raw = *(const u32x4*)(qp + 16 * s);
+      if (F16 && p.q_is_bf16) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          raw[e] = pack2<true>(__uint_as_float(raw[e] << 16), __uint_as_float(raw[e] & 0xffff0000u));
+      }
+      qf[b][s] = raw;
+      asm volatile("" : "+a"(qf[b][s]));
+    }
+  }
+  // S = K.Q^T: the lane is a query row of the block, register e is key 8 (e >> 2) + 4 g2 + (e & 3) of the tile.  Each lane
+  // keeps lists of its own, one per block, so an entry's place is the lane's count and nothing is exchanged.
+  float tau[2];
+  uint32_t lane_base[2], count[2] = {0u, 0u};
+#pragma unroll
+  for (int b = 0; b < 2; ++b) {
+    const uint32_t r = row0 + 32u * b + l32;
+    tau[b] = r < rows_total ? tp.tau[(size_t)kvh * tp.n_mtiles * kTopkFilterRows + r] : INFINITY;
+    lane_base[b] = (64u * b + lane) * (kTopkSegAlloc * 8u);
+  }
+  char* const cbase = (char*)tp.cand + (size_t)seg * (kTopkSegAlloc * 8u);
+  const float scale = tp.scale;
+  // Comparison of the scores in four registers, in four parts (between the parts, products; side by side, because one wave
+  // per SIMD hides no latency of another's).  No branch, and exactly one store per register whose mask is never empty:
+  // lane 0 always writes, and where its score is too low, its next entry or nothing takes the place.  So a key tile
+  // is always 32 stores and NLD loads of the one memory counter, and the wait at a tile's start can tell its own loads
+  // from what was issued behind them.
+  // (With query rows in the registers and keys in the lanes an entry's place took a rank among the lanes and a scalar
+  // count per register, 15 instructions a score register instead of 8: 163 us instead of 141 for 256 rows over 33k keys.)
+  uint64_t mask[4];
+  uint32_t at[4];
+  u32x2 entry[16];          // (score, position) of register e: positions move on by a tile step, shared by the blocks
+  auto keep = [&](auto n_c, const f32x16 (&sc)[2]) {
+    constexpr int n0 = decltype(n_c)::value & ~3, part = decltype(n_c)::value & 3, b = n0 >> 4, e0 = n0 & 15;
+    if constexpr (part == 0) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float v = sc[b][e0 + i] * scale;
+        entry[e0 + i][0] = __float_as_uint(v);
+        mask[i] = __builtin_amdgcn_ballot_w64(v >= tau[b]);
+      }
+    } else if constexpr (part == 1) {
+      asm volatile("s_nop 1");       // a mask written by a comparison is a carry-in two wait states later at the earliest
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        at[i] = lane_base[b] + count[b] * 8u;
+        asm volatile("v_addc_co_u32_e64 %0, vcc, %0, 0, %1" : "+v"(count[b]) : "s"(mask[i]) : "vcc");
+      }
+    } else if constexpr (part == 2) {
+      store4_masked(mask, at, entry[e0], entry[e0 + 1], entry[e0 + 2], entry[e0 + 3], cbase);
+    } else if constexpr (e0 == 12) {
+      count[b] = min(count[b], kTopkSegCap);
+    }
+  };
+  auto positions = [&](uint32_t t0) {
+#pragma unroll
+    for (int e = 0; e < 16; ++e) entry[e][1] = t0 + 8u * (e >> 2) + (e & 3) + 4u * g2;
+  };
+
+  constexpr int CH = 8, NCHUNK = NSTEP / CH, LPC = NLD / NCHUNK;
+  // tile i: its products into s, the comparison of the tile before (sp) between them
+  auto tile_step = [&](uint32_t i, f32x16 (&s)[2], const f32x16 (&sp)[2]) {
+    positions(tile_t0(i - 1u));
+    // this wave's loads of K(i) have landed: they were issued PF tiles ago (or waited for before the loop), in front of at
+    // least two tiles' worth of loads and stores, which is more than the counter can hold back
+    static_assert((PF - 1) * (NLD + 32) >= 63, "operations issued behind a tile's loads");
+    wait_loads_then_barrier<63>();
+    const TileLoad tl_next = k_desc(i + PF);
+    lds_char* const kb = (lds_char*)(smem + (i % NB) * L::K_BYTES);
+    u32x4 fr[2][CH];
+    auto read_chunk = [&](int c, u32x4 (&dst)[CH]) {
+#pragma unroll
+      for (int x = 0; x < CH; ++x) dst[x] = *(lds_u32x4*)(kb + k_lane_off + 32 * (c * CH + x));
+    };
+    read_chunk(0, fr[0]);
+    static_for<0, NCHUNK>([&](auto c_c) {
+      constexpr int c = decltype(c_c)::value;
+      if constexpr (c + 1 < NCHUNK) read_chunk(c + 1, fr[(c + 1) & 1]);
+      __builtin_amdgcn_sched_barrier(0);
+      static_for<0, CH>([&](auto i_c) {
+        constexpr int x = decltype(i_c)::value, st = c * CH + x;
+        if constexpr (st + 1 < NSTEP) {
+          mfma_filter<F16, st == 0>(s[0], fr[c & 1][x], qf[0][st]);
+          mfma_filter<F16, st == 0>(s[1], fr[c & 1][x], qf[1][st]);
+        } else {
+          mfma_filter_last<F16>(s[0], s[1], fr[c & 1][x], qf[0][st], qf[1][st]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (x % (CH / LPC) == 1) issue_tile_part<D, false, c * LPC + x / (CH / LPC)>(tl_next, wave, lane);
+        keep(std::integral_constant<int, st>{}, sp);
+        __builtin_amdgcn_sched_barrier(0);
+      });
+    });
+  };
+  wait_vmem_all();      // the query rows and with them the first PF tiles
+  __builtin_amdgcn_s_waitcnt(0xC07F);     // (lgkmcnt(0): or scalar loads in flight here make the compiler wait for whole chunks below)
+  f32x16 sa[2], sb[2];
+#pragma unroll
+  for (int e = 0; e < 16; ++e) sb[0][e] = sb[1][e] = __uint_as_float(0x7fc00000u);   // (in front of the first tile: NaN passes nowhere)
+  for (uint32_t i = 0; i < n_tiles; i += 2) {
+    tile_step(i, sa, sb);
+    if (i + 1u < n_tiles) {
+      tile_step(i + 1u, sb, sa);
+    } else {
+      positions(tile_t0(i));
+      static_for<0, 32>([&](auto n_c) { keep(n_c, sa); });
+    }
+  }
+  if ((n_tiles & 1u) == 0u) {
+    positions(tile_t0(n_tiles - 1u));
+    static_for<0, 32>([&](auto n_c) { keep(n_c, sb); });
+  }
+  tp.cand_n[seg + lane] = count[0];
+  tp.cand_n[seg + 64u + lane] = count[1];
+  wait_vmem_all();   // no direct-to-LDS load may outlive the workgroup's LDS
+}
+
+// One wave per row: candidates from the row's segments, the k-th largest by bisection over registers (a ballot per 64
+// candidates and step; no histogram, no barrier), the kept keys in position order by ranking them in a bitmap, softmax,
+// gathered P.V.  In position order the waves of an XCD sweep the V plane together and share its rows through the L2.
+constexpr uint32_t kRankWords = 64 * 17;               // bitmap words, 17 per lane: an odd stride, no bank conflicts
+constexpr uint32_t kRankWindow = kRankWords * 32;      // positions per pass
+template <bool F16, int NR>
+__global__ void __launch_bounds__(256, NR <= 20 ? 4 : NR == 24 ? 3 : 2) topk_list_select_kernel(const TopkParams tp) {
+  constexpr int D = 512, PER = 8;
+  constexpr uint32_t CAP = 64u * NR;                   // candidates a wave can hold
+  constexpr uint32_t SEL = NR == 16 ? 160u : NR == 20 ? 272u : NR == 24 ? 384u : 512u;   // most keys kept
+  static_assert(CAP * 8u >= kRankWords * 6u + SEL * 8u, "bitmap, prefix counts and kept keys reuse the candidate list");
+  constexpr uint32_t GU = 8;
+  static_assert(SEL % GU == 0, "kept keys are padded to whole groups");
+  const AttnParams& p = tp.a;
+  __shared__ __attribute__((aligned(16))) u32x2 lists[4][CAP];
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t n_rows = tp.ntok * p.hq;
+  const uint32_t wg = (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);   // runs of rows, one per XCD
+  const uint32_t rid = wg * 4u + wave;
+  if (rid >= n_rows) return;
+  const uint32_t rows = tp.ntok * p.group;
+  const uint32_t kvh = rid / rows, rr = rid % rows;
+  const uint32_t tok_l = rr / p.group, qh = kvh * p.group + rr % p.group;
+  const uint32_t tok = tp.tok0 + tok_l;
+  const RowBounds rb = row_bounds(p, tok);
+  const uint32_t k = row_k(tp, tok, visible_count(rb, p.t_all));
+  u32x2* const list = lists[wave];
+
+  // ---- this row's candidates, packed ----
+  // (half a wave per segment: the two lanes that held the row in the filter kernel had a list each)
+  const uint32_t seg0 = ((kvh * tp.n_mtiles + (rr >> 8)) * tp.n_splits * 4u + ((rr >> 6) & 3u)) * kTopkSegs +
+                        ((rr >> 5) & 1u) * 64u + (rr & 31u) + (lane & 32u);
+  constexpr uint32_t seg_step = 4u * kTopkSegs;
+  const uint32_t l32 = lane & 31u;
+  const u32x2* const cand = (const u32x2*)tp.cand;
+  uint32_t n = 0u;
+  bool over = false;
+  auto take = [&](u32x2 v, bool in) {
+    const bool own = in && key_visible(rb, v[1], p.t_all);
+    const uint64_t m = __builtin_amdgcn_ballot_w64(own);
+    const uint32_t to = n + rank_in(m);
+    if (own && to < CAP) list[to] = u32x2{score_key(__uint_as_float(v[0])), v[1]};
+    n += (uint32_t)__builtin_popcountll(m);
+  };
+  constexpr uint32_t SB = 8;       // splits in flight
+  for (uint32_t s0 = 0; s0 < tp.n_splits; s0 += SB) {
+    u32x2 v[SB];
+    uint32_t c[SB];
+#pragma unroll
+    for (uint32_t i = 0; i < SB; ++i) {
+      c[i] = s0 + i < tp.n_splits ? tp.cand_n[seg0 + (s0 + i) * seg_step] : 0u;
+      // (the first 32 places of a segment exist whatever its count)
+      v[i] = cand[(size_t)(seg0 + min(s0 + i, tp.n_splits - 1u) * seg_step) * kTopkSegAlloc + l32];
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < SB; ++i) {
+      over |= c[i] >= kTopkSegCap;
+      take(v[i], l32 < c[i]);
+      for (uint32_t x = 32u; __builtin_amdgcn_ballot_w64(x < c[i]) != 0ull; x += 32u) {
+        u32x2 w = {0u, 0u};
+        if (l32 + x < c[i]) w = cand[(size_t)(seg0 + (s0 + i) * seg_step) * kTopkSegAlloc + l32 + x];
+        take(w, l32 + x < c[i]);
+      }
+    }
+  }
+  const bool fail = __builtin_amdgcn_ballot_w64(over) != 0ull || n < k || n > CAP;
+  if (lane == 0u) {
+    tp.fail_rows[(size_t)tok * p.hq + qh] = fail ? 1u : 0u;
+    if (fail) atomicAdd(&tp.fail_block[tok_l / tp.fail_block_tok], 1u);
+  }
+  if (fail) return;
+  wave_lds_fence();
+  const uint32_t nu = (n + 63u) >> 6;
+  uint32_t key[NR], pos[NR];
+#pragma unroll
+  for (int u = 0; u < NR; ++u) {
+    key[u] = 0u;           // (below every candidate: NaN never passes a threshold)
+    pos[u] = 0xffffffffu;
+    if ((uint32_t)u < nu && 64u * u + lane < n) {
+      const u32x2 v = list[64u * u + lane];
+      key[u] = v[0];
+      pos[u] = v[1];
+    }
+  }
+  wave_lds_fence();
+
+  // ---- the k-th largest ----
+  uint32_t top = 0u, bot = 0xffffffffu;
+#pragma unroll
+  for (int u = 0; u < NR; ++u) {
+    top = max(top, key[u]);
+    if (pos[u] != 0xffffffffu) bot = min(bot, key[u]);
+  }
+  top = wave_max(top);
+  bot = ~wave_max(~bot);
+  auto count_ge = [&](uint32_t x) {
+    uint32_t c = 0u;
+#pragma unroll
+    for (int u = 0; u < NR; u += 4) {
+      if ((uint32_t)u < nu) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) c += (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(key[u + i] >= x));
+      }
+    }
+    return c;
+  };
+  uint32_t lo = bot, hi = top + 1u, c_lo = n;      // count(>= lo) = c_lo >= k > count(>= hi)
+  while (hi - lo > 1u && c_lo != k) {
+    const uint32_t mid = lo + ((hi - lo) >> 1);
+    const uint32_t c = count_ge(mid);
+    if (c >= k) {
+      lo = mid;
+      c_lo = c;
+    } else {
+      hi = mid;
+    }
+  }
+  // equal scores at the threshold: the lower positions are kept, up to t_last
+  uint32_t t_last = 0xfffffffeu;
+  if (c_lo != k) {
+    const uint32_t drop = c_lo - k;              // this many of the highest positions among the equal ones go
+    uint32_t a = 0u, b = p.t_all;                // count(equal, position >= a) >= drop > ... >= b
+    while (b - a > 1u) {
+      const uint32_t mid = a + ((b - a) >> 1);
+      uint32_t c = 0u;
+#pragma unroll
+      for (int u = 0; u < NR; ++u) {
+        if ((uint32_t)u < nu) c += (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(key[u] == lo && pos[u] >= mid));
+      }
+      if (c >= drop) a = mid;
+      else b = mid;
+    }
+    t_last = a - 1u;      // (position a is the last one dropped; a > 0 because at least one equal key stays)
+  }
+#pragma unroll
+  for (int u = 0; u < NR; ++u) {
+    if (key[u] < lo || (key[u] == lo && pos[u] > t_last)) pos[u] = 0xffffffffu;      // not kept: in no window below
+  }
+
+  // ---- softmax over the kept scores (cpu.rs:95-104), and their order by position ----
+  uint32_t* const bits = (uint32_t*)list;
+  uint16_t* const before = (uint16_t*)(bits + kRankWords);
+  u32x2* const sel = list + kRankWords * 6u / 8u;          // (weight, byte offset of the key's V row)
+  const uint32_t v_step = (uint32_t)p.v_tok_stride * 2u;   // (offsets stay below 2^32: the host's rule)
+  const float mmax = key_score(top);
+  float l = 0.f;
+  uint32_t ranked = 0u;
+  for (uint32_t t0 = 0; t0 < p.t_all; t0 += kRankWindow) {
+#pragma unroll
+    for (uint32_t w = 0; w < 17u; ++w) bits[64u * w + lane] = 0u;
+    wave_lds_fence();
+#pragma unroll
+    for (int u = 0; u < NR; ++u) {
+      if ((uint32_t)u < nu && pos[u] - t0 < kRankWindow) atomicOr(&bits[(pos[u] - t0) >> 5], 1u << ((pos[u] - t0) & 31u));
+    }
+    wave_lds_fence();
+    uint32_t run = 0u;
+#pragma unroll
+    for (uint32_t w = 0; w < 17u; ++w) {
+      before[17u * lane + w] = (uint16_t)run;
+      run += (uint32_t)__builtin_popcount(bits[17u * lane + w]);
+    }
+    uint32_t incl = run;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const uint32_t v = (uint32_t)__shfl_up((int)incl, off, 64);
+      if (lane >= (uint32_t)off) incl += v;
+    }
+    const uint32_t excl = incl - run;
+    wave_lds_fence();
+#pragma unroll
+    for (int u = 0; u < NR; ++u) {
+      if ((uint32_t)u < nu) {
+        const bool in = pos[u] - t0 < kRankWindow;
+        const uint32_t w = in ? (pos[u] - t0) >> 5 : 0u;
+        const uint32_t base = (uint32_t)__shfl((int)excl, (int)(w / 17u), 64);
+        if (in) {
+          const uint32_t r = ranked + base + before[w] + (uint32_t)__builtin_popcount(bits[w] & ((1u << (pos[u] & 31u)) - 1u));
+          const float e = expf(key_score(key[u]) - mmax);
+          l += e;
+          if (r < SEL) sel[r] = u32x2{__float_as_uint(e), pos[u] * v_step};
+        }
+      }
+    }
+    ranked += (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+    wave_lds_fence();
+  }
+  l = wave_sum(l);
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  // up to a whole number of groups: the last key again, weight 0
+  if (lane < (0u - k) % GU) sel[k + lane] = u32x2{0u, sel[k - 1u][1]};
+  wave_lds_fence();
+
+  // ---- gathered P.V: a lane owns 8 consecutive d; weights are divided by their sum at the end.  All waves of an XCD
+  // sweep the keys in order, and a V row that four of its 512 rows want should be fetched into its L2 once: the nearer the waves
+  // keep together the better, so only GU rows are loaded ahead (256 rows over 33k keys, the whole kernel: 2 rows 99 us,
+  // 4 rows 110, 8 rows 131, 16 rows 142, the latter with half of the requests missing the L2) ----
+  float acc[PER];
+#pragma unroll
+  for (int i = 0; i < PER; ++i) acc[i] = 0.f;
+  const char* const vbase = (const char*)p.v + (int64_t)kvh * p.v_head_stride * 2;
+  const uint32_t lane_b = lane * 16u;
+  auto gather = [&](auto gu_c) {
+    constexpr uint32_t GU = decltype(gu_c)::value;
+    for (uint32_t j0 = 0; j0 < k; j0 += GU) {
+      float e[GU];
+      u32x4 raw[GU];
+#pragma unroll
+      for (uint32_t u = 0; u < GU; ++u) {
+        const u32x2 v = sel[j0 + u];
+        e[u] = __uint_as_float(v[0]);
+        raw[u] = *(const u32x4*)(vbase + (v[1] + lane_b));
+      }
+#pragma unroll
+      for (uint32_t u = 0; u < GU; ++u) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          acc[2 * i] = __builtin_fmaf(e[u], unpack_lo<F16>(raw[u][i]), acc[2 * i]);
+          acc[2 * i + 1] = __builtin_fmaf(e[u], unpack_hi<F16>(raw[u][i]), acc[2 * i + 1]);
+        }
+      }
+    }
+  };
+  if (n_rows > 2048u) gather(std::integral_constant<uint32_t, 2>{});
+  else gather(std::integral_constant<uint32_t, 8>{});
+#pragma unroll
+  for (int i = 0; i < PER; ++i) acc[i] *= inv;
+  const size_t out_off = ((size_t)tok * p.hq + qh) * D + lane * PER;
+  if (p.out_dtype == 2u) {
+    float* const o = (float*)p.out + out_off;
+    *(f32x4*)o = f32x4{acc[0], acc[1], acc[2], acc[3]};
+    *(f32x4*)(o + 4) = f32x4{acc[4], acc[5], acc[6], acc[7]};
+  } else {
+    u32x4 o;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      o[i] = (uint32_t)f32_to_bf16_bits(acc[2 * i], p.out_trunc != 0u) |
+             ((uint32_t)f32_to_bf16_bits(acc[2 * i + 1], p.out_trunc != 0u) << 16);
+    *(u32x4*)((uint16_t*)p.out + out_off) = o;
+  }
+}
+
 template <int D, bool F16>
 hipError_t launch_stage(const TopkParams& tp, int stage, hipStream_t s) {
   if (stage == 0) {
@@ -736,8 +1278,39 @@ hipError_t launch_by_dim(const TopkParams& tp, int stage, uint32_t head_dim, hip
   }
 }
 
+template <bool F16>
+hipError_t launch_filter(const TopkParams& tp, const TopkParams& sample, hipStream_t s) {
+  hipError_t rc = launch_stage<512, F16>(sample, 0, s);
+  if (rc != hipSuccess) return rc;
+  const uint32_t rows = tp.ntok * tp.a.hq;
+  const dim3 by_wave((rows + 3u) / 4u);
+  const uint32_t m = sample.a.t_all;
+  if (m <= 64u * 32u) hipLaunchKernelGGL((topk_tau_kernel<32>), by_wave, dim3(256), 0, s, tp);
+  else if (m <= 64u * 64u) hipLaunchKernelGGL((topk_tau_kernel<64>), by_wave, dim3(256), 0, s, tp);
+  else hipLaunchKernelGGL((topk_tau_kernel<128>), by_wave, dim3(256), 0, s, tp);
+  if ((rc = hipGetLastError()) != hipSuccess) return rc;
+  const uint32_t n_units = tp.a.hkv * tp.n_splits * tp.n_mtiles;
+  hipLaunchKernelGGL((topk_filter_kernel<F16>), dim3((n_units + 7u) / 8u * 8u), dim3(256), 0, s, tp);
+  return hipGetLastError();
+}
+template <bool F16>
+hipError_t launch_list_select(const TopkParams& tp, uint32_t k_most, hipStream_t s) {
+  const dim3 sel((tp.ntok * tp.a.hq + 31u) / 32u * 8u);
+  if (k_most <= 160u) hipLaunchKernelGGL((topk_list_select_kernel<F16, 16>), sel, dim3(256), 0, s, tp);
+  else if (k_most <= 272u) hipLaunchKernelGGL((topk_list_select_kernel<F16, 20>), sel, dim3(256), 0, s, tp);
+  else if (k_most <= 384u) hipLaunchKernelGGL((topk_list_select_kernel<F16, 24>), sel, dim3(256), 0, s, tp);
+  else hipLaunchKernelGGL((topk_list_select_kernel<F16, 32>), sel, dim3(256), 0, s, tp);
+  return hipGetLastError();
+}
+
 }  // namespace
 
+hipError_t launch_topk_filter(const TopkParams& tp, const TopkParams& sample, uint32_t kv_dtype, hipStream_t s) {
+  return kv_dtype == 1u ? launch_filter<true>(tp, sample, s) : launch_filter<false>(tp, sample, s);
+}
+hipError_t launch_topk_list_select(const TopkParams& tp, uint32_t k_most, uint32_t kv_dtype, hipStream_t s) {
+  return kv_dtype == 1u ? launch_list_select<true>(tp, k_most, s) : launch_list_select<false>(tp, k_most, s);
+}
 hipError_t launch_topk_scores(const TopkParams& tp, uint32_t head_dim, uint32_t kv_dtype, hipStream_t s) {
   return kv_dtype == 1u ? launch_by_dim<true>(tp, 0, head_dim, s) : launch_by_dim<false>(tp, 0, head_dim, s);
 }

@@ -6,6 +6,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstring>
 #include <mutex>
 #include <vector>
@@ -645,9 +646,84 @@ constexpr size_t kTopkPlaneBudget = (size_t)DG_TOPK_PLANE_MIB << 20;
 struct TopkPlan {
   uint32_t t_pad = 0, block_tok = 0;
   size_t total = 0;
+  // filtered path (pass_tok = 0: not taken): canvas rows per pass and, within a pass, per block of the general path
+  // behind it; sampled keys; key-range splits; byte offsets in the workspace
+  uint32_t pass_tok = 0, redo_tok = 0, stride = 0, sample_n = 0, sample_pad = 0, splits = 0, k_most = 0;
+  size_t off_block = 0, off_plane = 0, off_tau = 0, off_cand_n = 0, off_lists = 0;
 };
 
-int make_topk_plan(const dg_attn_desc* d, const uint32_t* k_cfg, const Plan& pl, TopkPlan* tk) {
+// Where the filtered path is taken: what its kernels are made for (head_dim 512, linear cache, every row sees all keys
+// up to its own or the last), at most 512 keys kept (what a wave holds of a row's list), prefixes long
+// enough that a pass over 1/17 of the keys tells where the k-th score lies, and calls with enough scores.  Its six and more
+// launches take about 75 us however small they are; the general path takes 50, and about 30 for every 2^23 scores once its
+// select kernel, a workgroup per (row, head), needs more than one round of the chip, 10 below that.  Measured, the layer
+// step with 16 heads, general -> filtered path: 64 rows over 20k keys 99 -> 104 us, 33k 152 -> 136, 50k 297 -> 179;
+// 128 rows over 3k keys 79 -> 81 us, 8k 99 -> 91, 33k 294 -> 185; 256 rows over 3k keys 136 -> 96 us, 33k 629 -> 290.
+constexpr uint32_t kTopkFilterMinPrefix = 2048;
+constexpr uint32_t kTopkFilterMaxK = 512;
+constexpr uint64_t kTopkFilterMinScores = 1ull << 23;         // three times that in one round of the select kernel
+
+size_t filter_bytes(const dg_attn_desc* d, const Plan& pl, uint32_t cus, uint32_t ntok, TopkPlan* tk) {
+  const uint32_t n_mtiles = (ntok * pl.group + dg::kTopkFilterRows - 1) / dg::kTopkFilterRows;
+  const uint32_t base = d->n_kv_heads * n_mtiles;
+  const uint32_t n_tiles = (pl.t_all + dg::kBlockN - 1) / dg::kBlockN;
+  // Enough workgroups for every CU, in whole rounds of the chip, but four key tiles each; and segments that expect half
+  // of what they hold.  A row's list is about k + 5 sqrt(stride k) + 3 stride long, in two segments per split.
+  const double list = tk->k_most + 5.0 * std::sqrt((double)tk->stride * tk->k_most) + 3.0 * tk->stride;
+  const uint32_t round = (cus + base - 1) / base;
+  const uint32_t fit = (uint32_t)(list / 2.0 / (dg::kTopkSegCap / 2)) + 1;
+  tk->splits = std::min({round * ((fit + round - 1) / round), std::max(fit, n_tiles / 4), dg::kMaxSplits});
+  const size_t segs = (size_t)base * tk->splits * 4 * dg::kTopkSegs;
+  tk->off_block = align_up((size_t)d->canvas * d->n_q_heads * sizeof(uint32_t));
+  tk->off_plane = tk->off_block + align_up((size_t)ntok * sizeof(uint32_t));
+  tk->off_tau = tk->off_plane;
+  tk->off_cand_n = tk->off_tau + align_up((size_t)base * dg::kTopkFilterRows * sizeof(float));
+  tk->off_lists = tk->off_cand_n + align_up(segs * sizeof(uint32_t));
+  // (the lists lie where the sampled scores were)
+  const size_t sample = (size_t)d->n_q_heads * ntok * tk->sample_pad * sizeof(float);
+  return tk->off_lists + align_up(std::max(segs * dg::kTopkSegAlloc * 8, sample));
+}
+
+void plan_filtered(const dg_attn_desc* d, const uint32_t* k_cfg, const Plan& pl, uint32_t cus, TopkPlan* tk) {
+  if (d->head_dim != 512 || pl.lo_nc != 0 || pl.win_m1 != 0xffffffffu || d->kv_ring_mask != 0) return;
+  if (d->kv_len < kTopkFilterMinPrefix || !std::isfinite(pl.scale) || (d->flags & DG_ATTN_F_TOPK_SCORE_PLANE)) return;
+  const uint64_t rows = (uint64_t)d->canvas * d->n_q_heads;
+  const bool one_round = rows <= 4ull * cus;
+  if (rows * pl.t_all < (one_round ? 3 : 1) * kTopkFilterMinScores && !(d->flags & DG_ATTN_F_TOPK_THRESHOLD)) return;
+  if (k_cfg[1] != 0u) {
+    const uint64_t gran = std::max(k_cfg[0], 1u);
+    const uint64_t most = (pl.t_all + gran - 1) / gran * gran / k_cfg[1];
+    tk->k_most = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(most, k_cfg[2]), k_cfg[3]);
+  } else {
+    tk->k_most = std::max(k_cfg[0], 1u);
+  }
+  if (tk->k_most == 0u || tk->k_most > kTopkFilterMaxK) return;
+  // (odd: sampled rows of a head-major cache, 1 KiB each, then fall on all memory channels)
+  tk->stride = std::max(17u, (pl.t_all + dg::kTopkSampleMax - 1) / dg::kTopkSampleMax | 1u);
+  if (tk->stride > 21u) return;       // (17 to 21: the list of a row that keeps 512 keys still fits)
+  // key rows of the sampled launch are `stride` rows apart, a tile's offsets have 31 bits
+  if ((uint64_t)d->k_tok_stride * 2 * tk->stride * dg::kBlockN >= (1ull << 31)) return;
+  if ((uint64_t)d->v_tok_stride * 2 * pl.t_all + 1024 >= (1ull << 32)) return;      // V rows are gathered by 32-bit offsets
+  tk->sample_n = (pl.t_all + tk->stride - 1) / tk->stride;
+  tk->sample_pad = (tk->sample_n + dg::kBlockN - 1) / dg::kBlockN * dg::kBlockN;
+  uint32_t ntok = d->canvas;
+  size_t need = filter_bytes(d, pl, cus, ntok, tk);
+  while (need > kTopkPlaneBudget && ntok > 32) {
+    ntok = ((ntok + 1) / 2 + 31) & ~31u;
+    need = filter_bytes(d, pl, cus, ntok, tk);
+  }
+  if (need > kTopkPlaneBudget) return;
+  const size_t per_tok = (size_t)d->n_q_heads * tk->t_pad * sizeof(float);
+  if (tk->block_tok == d->canvas) tk->total = std::max(tk->total, tk->off_plane + align_up((size_t)ntok * per_tok));
+  tk->total = std::max(tk->total, need);
+  const size_t fit = (tk->total - tk->off_plane) / per_tok;
+  if (fit == 0) return;
+  tk->pass_tok = ntok;
+  const uint32_t blocks = (uint32_t)((ntok + fit - 1) / fit);
+  tk->redo_tok = (ntok + blocks - 1) / blocks;
+}
+
+int make_topk_plan(const dg_attn_desc* d, const uint32_t* k_cfg, const Plan& pl, uint32_t cus, TopkPlan* tk) {
   if (!k_cfg) return DG_ERR_NULL;
   if (pl.scalar || d->q_dtype == DG_F32 || d->kv_dtype == DG_F32) return DG_ERR_UNSUPPORTED;
   if (k_cfg[1] == 0u) {
@@ -662,6 +738,7 @@ int make_topk_plan(const dg_attn_desc* d, const uint32_t* k_cfg, const Plan& pl,
   tk->block_tok = (uint32_t)std::min<size_t>(blk, d->canvas);
   tk->total = align_up((size_t)tk->block_tok * per_tok);
   if (tk->total / sizeof(float) >= (1ull << 32)) return DG_ERR_SHAPE;   // score rows are addressed with 32-bit offsets
+  plan_filtered(d, k_cfg, pl, cus, tk);
   return DG_OK;
 }
 }  // namespace
@@ -672,7 +749,7 @@ int dg_attn_topk_workspace_bytes(const dg_attn_desc* d, const uint32_t* k_cfg, s
   int rc = make_plan(d, plan_cus(), &pl);
   if (rc != DG_OK) return rc;
   TopkPlan tk;
-  rc = make_topk_plan(d, k_cfg, pl, &tk);
+  rc = make_topk_plan(d, k_cfg, pl, plan_cus(), &tk);
   if (rc != DG_OK) return rc;
   *out_bytes = tk.total;
   return DG_OK;
@@ -688,7 +765,7 @@ int dg_attn_topk_forward(const dg_attn_desc* d, const uint32_t* k_cfg, const voi
   rc = make_plan(d, plan_cus(), &pl);
   if (rc != DG_OK) return rc;
   TopkPlan tk;
-  rc = make_topk_plan(d, k_cfg, pl, &tk);
+  rc = make_topk_plan(d, k_cfg, pl, plan_cus(), &tk);
   if (rc != DG_OK) return rc;
   if (!workspace || workspace_bytes < tk.total || ((uintptr_t)workspace % 16) != 0) return DG_ERR_WORKSPACE;
   if (((uintptr_t)q % 16) != 0 || ((uintptr_t)kv_base % 16) != 0 || ((uintptr_t)out % 16) != 0) return DG_ERR_LAYOUT;
@@ -706,28 +783,84 @@ int dg_attn_topk_forward(const dg_attn_desc* d, const uint32_t* k_cfg, const voi
   for (int i = 0; i < 4; ++i) tp.k_cfg[i] = k_cfg[i];
   tp.scale = pl.scale;
   const uint32_t ntiles = std::max(1u, pl.tile_end - pl.tile_first);
-  for (uint32_t tok0 = 0; tok0 < d->canvas; tok0 += tk.block_tok) {
+  // (timing aid: one event pair per stage, scores first)
+  bool prof = false;
+  auto mark = [&](uint32_t i) {
+    if (prof) (void)hipEventRecord(g_prof.ev[2 * g_prof.used + i], s);
+  };
+  // the general path over canvas rows [tok0, tok0 + ntok)
+  auto block = [&](uint32_t tok0, uint32_t ntok, bool marks) -> hipError_t {
     tp.tok0 = tok0;
-    tp.ntok = std::min(tk.block_tok, d->canvas - tok0);
+    tp.ntok = ntok;
     tp.n_mtiles = (tp.ntok * pl.group + dg::kBlockM - 1) / dg::kBlockM;
     // enough workgroups for every CU, no split shorter than 8 key tiles; splits write disjoint
     // columns of the score plane, so there is nothing to merge
     const uint32_t base = d->n_kv_heads * tp.n_mtiles;
     uint32_t splits = std::max(1u, ((uint32_t)di.cus + base - 1u) / base);
     tp.n_splits = std::max(1u, std::min(splits, ntiles / 8u));
-    // (timing aid: one event pair per kernel, scores first)
-    const bool prof = g_prof.active && 2 * (size_t)g_prof.used + 3 < g_prof.ev.size();
-    if (prof) (void)hipEventRecord(g_prof.ev[2 * g_prof.used], s);
-    if (dg::launch_topk_scores(tp, d->head_dim, pl.e_dtype, s) != hipSuccess) return DG_ERR_LAUNCH;
-    if (prof) {
-      (void)hipEventRecord(g_prof.ev[2 * g_prof.used + 1], s);
-      (void)hipEventRecord(g_prof.ev[2 * g_prof.used + 2], s);
+    if (marks) mark(0);
+    hipError_t e = dg::launch_topk_scores(tp, d->head_dim, pl.e_dtype, s);
+    if (marks) {
+      mark(1);
+      mark(2);
     }
-    if (dg::launch_topk_select(tp, d->head_dim, pl.e_dtype, s) != hipSuccess) return DG_ERR_LAUNCH;
-    if (prof) {
-      (void)hipEventRecord(g_prof.ev[2 * g_prof.used + 3], s);
-      g_prof.used += 2;
+    if (e == hipSuccess) e = dg::launch_topk_select(tp, d->head_dim, pl.e_dtype, s);
+    return e;
+  };
+  const uint32_t step = tk.pass_tok ? tk.pass_tok : tk.block_tok;
+  for (uint32_t tok0 = 0; tok0 < d->canvas; tok0 += step) {
+    const uint32_t ntok = std::min(step, d->canvas - tok0);
+    prof = g_prof.active && 2 * (size_t)g_prof.used + 3 < g_prof.ev.size();
+    if (tk.pass_tok == 0) {
+      if (block(tok0, ntok, true) != hipSuccess) return DG_ERR_LAUNCH;
+    } else {
+      char* const ws = (char*)workspace;
+      dg::TopkParams fp = tp;
+      fp.tok0 = tok0;
+      fp.ntok = ntok;
+      fp.n_mtiles = (ntok * pl.group + dg::kTopkFilterRows - 1) / dg::kTopkFilterRows;
+      fp.n_splits = tk.splits;
+      fp.sample_stride = tk.stride;
+      fp.sample_n = tk.sample_n;
+      fp.sample_pad = tk.sample_pad;
+      fp.sample_plane = (float*)(ws + tk.off_lists);
+      fp.tau = (float*)(ws + tk.off_tau);
+      fp.cand_n = (uint32_t*)(ws + tk.off_cand_n);
+      fp.cand = ws + tk.off_lists;
+      fp.fail_rows = (uint32_t*)ws;
+      fp.fail_block = (uint32_t*)(ws + tk.off_block);
+      fp.fail_block_tok = tk.redo_tok;
+      // the sampled keys as a cache of their own: every stride-th row of K, all of them scored
+      dg::TopkParams sp = tp;
+      sp.a.k_tok_stride *= tk.stride;
+      sp.a.causal_rows = 0u;
+      sp.a.t_all = tk.sample_n;
+      sp.a.t_clip_lo = 0u;
+      sp.a.t_clip_hi = sp.a.extra_lo = tk.sample_n;
+      sp.s_plane = fp.sample_plane;
+      sp.tok0 = tok0;
+      sp.ntok = ntok;
+      sp.t_pad = tk.sample_pad;
+      sp.n_mtiles = (ntok * pl.group + dg::kBlockM - 1) / dg::kBlockM;
+      sp.tile_first = 0u;
+      sp.tile_end = tk.sample_pad / dg::kBlockN;
+      const uint32_t base = d->n_kv_heads * sp.n_mtiles;
+      sp.n_splits = std::max(1u, std::min(((uint32_t)di.cus + base - 1u) / base, sp.tile_end / 4u));
+      mark(0);
+      if (dg::launch_topk_filter(fp, sp, pl.e_dtype, s) != hipSuccess) return DG_ERR_LAUNCH;
+      mark(1);
+      mark(2);
+      if (dg::launch_topk_list_select(fp, tk.k_most, pl.e_dtype, s) != hipSuccess) return DG_ERR_LAUNCH;
+      tp.s_plane = (float*)(ws + tk.off_plane);
+      tp.fail_rows = fp.fail_rows;
+      for (uint32_t b = 0; b * tk.redo_tok < ntok; ++b) {
+        tp.fail_block = fp.fail_block + b;
+        const uint32_t at = b * tk.redo_tok;
+        if (block(tok0 + at, std::min(tk.redo_tok, ntok - at), false) != hipSuccess) return DG_ERR_LAUNCH;
+      }
     }
+    mark(3);
+    if (prof) g_prof.used += 2;
   }
   return DG_OK;
 }

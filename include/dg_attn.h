@@ -104,6 +104,12 @@ typedef enum dg_kernel_sel {
                                               launch), as does an explicit n_splits.  Results agree to the rounding
                                               of the probabilities; the flag is there to compare the two. */
 
+#define DG_ATTN_F_TOPK_THRESHOLD 0x200u  /* top-k attention, wherever its thresholds-and-lists path can run (head_dim 512, linear
+                                              cache, no window, prefix of at least 2048, at most 512 keys kept): take it,
+                                              also where the library would score into a plane.  Both give the same kept keys;
+                                              the flags are there to compare the two. */
+#define DG_ATTN_F_TOPK_SCORE_PLANE 0x400u /* top-k attention: always through the score plane. */
+
 typedef struct dg_attn_desc {
   uint32_t canvas;        /* query rows; the reference passes active_canvas (256/128/64) */
   uint32_t n_q_heads;

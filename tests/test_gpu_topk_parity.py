@@ -49,7 +49,7 @@ def test_ragged_causal_tail(gpu_ready, po):
 
 # ------------------------------------------------------------------ generic runner
 def run_topk(po, canvas, hq, hkv, hd, kv_len, k_cfg, *, causal_rows=0, window=0, q=None, kv=None, seed=0, toks=None,
-             kv_dtype=capi.DG_BF16):
+             kv_dtype=capi.DG_BF16, flags=0):
     """bf16 (or f16) storage, fp32 output: isolates selection and arithmetic from the output store."""
     import torch
     rng = np.random.default_rng(seed)
@@ -63,7 +63,7 @@ def run_topk(po, canvas, hq, hkv, hd, kv_len, k_cfg, *, causal_rows=0, window=0,
                           else (R.f32_to_f16_bits_rne, R.f16_bits_to_f32))
     qb, kb = R.f32_to_bf16_bits_rne(q), to_bits(kv)
     d = A.make_desc(canvas, hq, hkv, hd, kv_len, causal_rows=causal_rows, window=window, q_dtype=capi.DG_BF16,
-                    kv_dtype=kv_dtype, out_dtype=capi.DG_F32)
+                    kv_dtype=kv_dtype, out_dtype=capi.DG_F32, flags=flags)
     out = torch.zeros(canvas * hq * hd, dtype=torch.float32, device="cuda")
     T.forward(d, k_cfg, A.to_device_bits(qb.reshape(-1)), A.to_device_bits(kb.reshape(-1)), out, T.alloc_workspace(d, k_cfg))
     torch.cuda.synchronize()
@@ -206,6 +206,89 @@ def test_edge_cases(gpu_ready, po, case):
                         toks=toks)
     assert np.isfinite(got).all()
     assert max_abs_diff(got, ref) <= 2e-2 and mean_abs_diff(got, ref) <= 2e-3
+
+
+# ------------------------------------------------------------------ thresholds instead of a score plane (head_dim 512, long rows)
+FILTERED = [
+    # canvas, hq, hkv, kv_len, causal_rows, k_cfg, what the keys look like
+    (40, 16, 2, 2048, 0, T.adaptive_k(), "unit"),         # shortest prefix taken; 320 stacked rows: the second row tile is ragged
+    (3, 6, 2, 2500, 2, (64, 0, 0, 0), "unit"),            # 9 stacked rows per KV head, group 3
+    (17, 4, 1, 4077, 17, (512, 0, 0, 0), "unit"),         # odd key count, most keys kept, causal rows
+    (8, 8, 8, 3001, 0, (1, 0, 0, 0), "unit"),             # no sharing, one key kept
+    (6, 16, 2, 2100, 3, (100, 0, 0, 0), "ties"),          # exact scores full of ties: lists overflow or end inside a tie
+    (6, 16, 2, 6000, 0, (100, 0, 0, 0), "few ties"),      # ties, but lists that fit: the tie-break inside the list
+    (4, 4, 2, 3000, 0, (50, 0, 0, 0), "zero"),            # a zero query: every row is left to the general path
+    (9, 16, 2, 5000, 0, (64, 0, 0, 0), "cluster"),        # the best keys are neighbours
+    (9, 16, 2, 5000, 0, (64, 0, 0, 0), "half"),           # some rows left over, the others not
+    (5, 16, 2, 36000, 5, T.adaptive_k(), "unit"),         # positions ranked in two windows
+]
+
+
+@pytest.mark.parametrize("case", FILTERED)
+def test_thresholds_and_lists(gpu_ready, po, case):
+    canvas, hq, hkv, kvl, cr, k_cfg, keys = case
+    rng = np.random.default_rng(sum(case[:5]))
+    t_all, hd = kvl + canvas, 512
+    rms = lambda x: (x / np.sqrt(np.mean(x * x, axis=-1, keepdims=True))).astype(np.float32)
+    q, kv = rms(rng.standard_normal((canvas, hq, hd))), rms(rng.standard_normal((t_all, 2, hkv, hd)))
+    exact = keys in ("ties", "few ties", "zero", "half")
+    if exact:       # few-bit dyadic values in a few dimensions: scores exact in fp32 whatever the order of summation
+        live = {"ties": 8, "half": 128}.get(keys, 256)
+        q[:], kv[:, 0] = 0, 0
+        q[..., :live] = rng.integers(-2, 3, (canvas, hq, live)) / 4
+        kv[:, 0, :, :live] = rng.integers(-2, 3, (t_all, hkv, live)) / 4
+        if keys == "zero":
+            q[:] = 0
+        if keys == "half":
+            q[::2] = 0
+    if keys == "cluster":
+        kv[3000:3200, 0] *= 4
+    run = lambda flag: run_topk(po, canvas, hq, hkv, hd, kvl, k_cfg, causal_rows=cr, q=q, kv=kv, flags=flag)
+    got, ref = run(capi.DG_ATTN_F_TOPK_THRESHOLD)
+    assert np.isfinite(got).all()
+    if exact:       # same kept sets: outputs agree to fp32 summation error
+        assert max_abs_diff(got, ref) < 2e-5
+    else:
+        assert max_abs_diff(got, ref) <= 2e-2 and mean_abs_diff(got, ref) <= 2e-3
+        # both paths sum a score over d in the same order, so they keep the same keys: fp32 summation error again
+        assert max_abs_diff(got, run(capi.DG_ATTN_F_TOPK_SCORE_PLANE)[0]) < 2e-5
+
+
+
+def test_thresholds_and_lists_replay_in_a_graph(gpu_ready):
+    """Recorded once, replayed over other queries in the same buffers (one of them zero: rows left to the general path)."""
+    import torch
+    w = W.Workload("rep2", 64, 16, 2, 512, 5000, seed=32)
+    q, kv = W.generate(w)
+    qd, kd = W.device_arrays(w, q, kv)
+    d = w.desc(flags=capi.DG_ATTN_F_TOPK_THRESHOLD)
+    k_cfg = T.adaptive_k()
+    ws = T.alloc_workspace(d, k_cfg)
+    out = torch.zeros(w.canvas * w.n_q_heads * w.head_dim, dtype=torch.int16, device="cuda")
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        T.forward(d, k_cfg, qd, kd, out, ws)
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        T.forward(d, k_cfg, qd, kd, out, ws)
+    first = qd.clone()
+    half = qd.numel() // 2
+    for change in ("none", "half zero", "none", "shifted"):
+        qd.copy_(first)
+        if change == "half zero":
+            qd.view(-1)[:half] = 0
+        elif change == "shifted":
+            qd.copy_(first.view(-1).roll(512 * 16).view(first.shape))
+        out.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        want = torch.zeros_like(out)
+        T.forward(d, k_cfg, qd, kd, want, T.alloc_workspace(d, k_cfg))
+        torch.cuda.synchronize()
+        assert torch.equal(out, want) and bool((out != 0).any())
 
 
 def test_ring_cache(gpu_ready, po):
