@@ -832,6 +832,7 @@ int dg_attn_topk_forward(const dg_attn_desc* d, const uint32_t* k_cfg, const voi
       fp.fail_block_tok = tk.redo_tok;
       // the sampled keys as a cache of their own: every stride-th row of K, all of them scored
       dg::TopkParams sp = tp;
+      sp.fail_rows = sp.fail_block = nullptr;      // (the last pass's)
       sp.a.k_tok_stride *= tk.stride;
       sp.a.causal_rows = 0u;
       sp.a.t_all = tk.sample_n;

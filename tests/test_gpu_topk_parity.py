@@ -221,6 +221,7 @@ FILTERED = [
     (9, 16, 2, 5000, 0, (64, 0, 0, 0), "cluster"),        # the best keys are neighbours
     (9, 16, 2, 5000, 0, (64, 0, 0, 0), "half"),           # some rows left over, the others not
     (5, 16, 2, 36000, 5, T.adaptive_k(), "unit"),         # positions ranked in two windows
+    (320, 16, 2, 40000, 320, T.adaptive_k(), "unit"),     # more rows than a pass takes
 ]
 
 
@@ -243,7 +244,8 @@ def test_thresholds_and_lists(gpu_ready, po, case):
             q[::2] = 0
     if keys == "cluster":
         kv[3000:3200, 0] *= 4
-    run = lambda flag: run_topk(po, canvas, hq, hkv, hd, kvl, k_cfg, causal_rows=cr, q=q, kv=kv, flags=flag)
+    toks = None if canvas <= 64 else np.array([0, 159, 160, 161, 319])
+    run = lambda flag: run_topk(po, canvas, hq, hkv, hd, kvl, k_cfg, causal_rows=cr, q=q, kv=kv, flags=flag, toks=toks)
     got, ref = run(capi.DG_ATTN_F_TOPK_THRESHOLD)
     assert np.isfinite(got).all()
     if exact:       # same kept sets: outputs agree to fp32 summation error
@@ -253,6 +255,22 @@ def test_thresholds_and_lists(gpu_ready, po, case):
         # both paths sum a score over d in the same order, so they keep the same keys: fp32 summation error again
         assert max_abs_diff(got, run(capi.DG_ATTN_F_TOPK_SCORE_PLANE)[0]) < 2e-5
 
+
+
+def test_random_rows_are_not_left_over(gpu_ready):
+    """Five-sigma thresholds: on random rows the lists suffice, in every pass over the canvas rows (the workspace begins with
+    a word per row and head that says whether the general path had to redo it)."""
+    import torch
+    w = W.Workload("left", 320, 16, 2, 512, 40000, causal_rows=320, seed=6)
+    q, kv = W.generate(w)
+    qd, kd = W.device_arrays(w, q, kv)
+    d = w.desc(flags=capi.DG_ATTN_F_TOPK_THRESHOLD)
+    k_cfg = T.adaptive_k()
+    ws = T.alloc_workspace(d, k_cfg)
+    T.forward(d, k_cfg, qd, kd, torch.zeros(w.canvas * w.n_q_heads * w.head_dim, dtype=torch.int16, device="cuda"), ws)
+    torch.cuda.synchronize()
+    left = ws.view(torch.int32)[:w.canvas * w.n_q_heads]
+    assert int(((left != 0) & (left != 1)).sum()) == 0 and int(left.sum()) <= 8      # (5120 rows at 1e-5 each)
 
 
 def test_thresholds_and_lists_replay_in_a_graph(gpu_ready):
