@@ -69,6 +69,8 @@ struct TopkParams {
   float* tau;            // [hkv][n_mtiles * 256]: a row's threshold
   uint32_t* cand_n;      // [hkv][n_mtiles][n_splits][4 waves][kTopkSegs]: entries in a segment
   void* cand;            // the same index space, kTopkSegAlloc entries of 8 bytes each
+  void* kept;            // [row of the pass][kept_pad]: (weight, byte offset of the key's V row), in order of position
+  uint32_t kept_pad;
   uint32_t* fail_rows;   // [canvas][hq]: rows the filtered path has left over (null: every row takes the general path)
   uint32_t* fail_block;  // rows left over per block of canvas rows (general path: of this block)
   uint32_t fail_block_tok;   // canvas rows per block
@@ -78,6 +80,7 @@ struct TopkParams {
 constexpr uint32_t kTopkSegs = 128;         // per wave of the filter kernel and split: two blocks of 32 rows, two lanes per row
 constexpr uint32_t kTopkSegCap = 80, kTopkSegAlloc = kTopkSegCap + 16;
 constexpr uint32_t kTopkFilterRows = 256;   // stacked rows per workgroup of the filter kernel
+constexpr uint32_t kTopkGather = 8;         // a row's list of kept keys is padded to a multiple
 constexpr uint32_t kTopkSampleMax = 8192;   // most sampled keys per row
 
 // Merging attention states of key-range partials (dg_attn_merge).  A state holds, per row

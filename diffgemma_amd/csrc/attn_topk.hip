@@ -729,9 +729,9 @@ __global__ void __launch_bounds__(256) topk_select_kernel(const TopkParams tp) {
 // two to four times k entries that one wave holds in registers.  Whatever tau is, the result is exact: a row whose
 // list holds fewer than k entries, or more than fit, is marked, and the general path redoes the marked rows (its
 // launches end at once where no row of the block is marked, 1.5 us each).
-// 256 rows x 16 heads over 33024 keys, layer step: 646 -> 283 us.  Launches: sampled scores 24 us (was: scores and plane, 4 x 55),
-// thresholds 16, filter 141 (0.98 PFLOP/s; the products alone, with their LDS reads and nothing else, 101), selection 99
-// (was 4 x 94; 70 of the 99 are the gathered V rows, 1.08 GB through the L2s).
+// 256 rows x 16 heads over 33024 keys, layer step: 646 -> 279 us.  Launches: sampled scores 24 us (was: scores and plane, 4 x 55),
+// thresholds 16, filter 141 (0.98 PFLOP/s; the products alone, with their LDS reads and nothing else, 101), selection 30
+// and gathered P.V 55 (both: was 4 x 94).
 
 // scores through an ordinary-register accumulator, query fragment in accumulation registers (256 of them hold the 64
 // query rows of a wave; a comparison cannot read that file)
@@ -1012,18 +1012,14 @@ __global__ void __launch_bounds__(256) topk_filter_kernel(const TopkParams tp) {
 }
 
 // One wave per row: candidates from the row's segments, the k-th largest by bisection over registers (a ballot per 64
-// candidates and step; no histogram, no barrier), the kept keys in position order by ranking them in a bitmap, softmax,
-// gathered P.V.  In position order the waves of an XCD sweep the V plane together and share its rows through the L2.
+// candidates and step; no histogram, no barrier), the kept keys in position order by ranking them in a bitmap, softmax.
 constexpr uint32_t kRankWords = 64 * 17;               // bitmap words, 17 per lane: an odd stride, no bank conflicts
 constexpr uint32_t kRankWindow = kRankWords * 32;      // positions per pass
-template <bool F16, int NR>
+template <int NR>
 __global__ void __launch_bounds__(256, NR <= 20 ? 4 : NR == 24 ? 3 : 2) topk_list_select_kernel(const TopkParams tp) {
-  constexpr int D = 512, PER = 8;
   constexpr uint32_t CAP = 64u * NR;                   // candidates a wave can hold
   constexpr uint32_t SEL = NR == 16 ? 160u : NR == 20 ? 272u : NR == 24 ? 384u : 512u;   // most keys kept
   static_assert(CAP * 8u >= kRankWords * 6u + SEL * 8u, "bitmap, prefix counts and kept keys reuse the candidate list");
-  constexpr uint32_t GU = 8;
-  static_assert(SEL % GU == 0, "kept keys are padded to whole groups");
   const AttnParams& p = tp.a;
   __shared__ __attribute__((aligned(16))) u32x2 lists[4][CAP];
   const uint32_t lane = threadIdx.x & 63u;
@@ -1201,14 +1197,36 @@ __global__ void __launch_bounds__(256, NR <= 20 ? 4 : NR == 24 ? 3 : 2) topk_lis
   }
   l = wave_sum(l);
   const float inv = l > 0.f ? 1.f / l : 0.f;
-  // up to a whole number of groups: the last key again, weight 0
-  if (lane < (0u - k) % GU) sel[k + lane] = u32x2{0u, sel[k - 1u][1]};
-  wave_lds_fence();
+  // the kept keys, up to a whole number of the gather's groups: the last key again, weight 0
+  u32x2* const out = (u32x2*)tp.kept + (size_t)rid * tp.kept_pad;
+  const uint32_t k_up = (k + kTopkGather - 1u) / kTopkGather * kTopkGather;
+  for (uint32_t j = lane; j < k_up; j += 64u) {
+    const u32x2 v = sel[min(j, k - 1u)];
+    out[j] = u32x2{j < k ? __float_as_uint(__uint_as_float(v[0]) * inv) : 0u, v[1]};
+  }
+}
 
-  // ---- gathered P.V: a lane owns 8 consecutive d; weights are divided by their sum at the end.  All waves of an XCD
-  // sweep the keys in order, and a V row that four of its 512 rows want should be fetched into its L2 once: the nearer the waves
-  // keep together the better, so only GU rows are loaded ahead (256 rows over 33k keys, the whole kernel: 2 rows 99 us,
-  // 4 rows 110, 8 rows 131, 16 rows 142, the latter with half of the requests missing the L2) ----
+// Gathered P.V of the rows the selection has listed, one wave each: a lane owns 8 consecutive d, keys in order of position.
+// A launch of its own so that its waves begin together: all waves of an XCD sweep the keys in order, and a V row
+// that four of its 512 rows want should be fetched into its L2 once.  For the same reason only four rows are loaded ahead where
+// there are waves enough.  256 rows over 33k keys: 1 row ahead 101 us, 2 rows 68, 4 rows 55 (20 TB/s out of the L2s), 8 rows 88;
+// as the tail of the selection, its waves apart by what came before, 2 rows 70 and 16 rows 110 us, half of the
+// requests missing the L2.  64 rows, a wave per SIMD: 8 rows ahead.
+template <bool F16>
+__global__ void __launch_bounds__(256) topk_gather_kernel(const TopkParams tp) {
+  constexpr int D = 512, PER = 8;
+  const AttnParams& p = tp.a;
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t n_rows = tp.ntok * p.hq;
+  const uint32_t wg = (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);   // runs of rows, one per XCD
+  const uint32_t rid = __builtin_amdgcn_readfirstlane(wg * 4u + (threadIdx.x >> 6));
+  if (rid >= n_rows) return;
+  const uint32_t rows = tp.ntok * p.group;
+  const uint32_t kvh = rid / rows, rr = rid % rows;
+  const uint32_t tok = tp.tok0 + rr / p.group, qh = kvh * p.group + rr % p.group;
+  if (tp.fail_rows[(size_t)tok * p.hq + qh] != 0u) return;       // (the general path's)
+  const uint32_t k = row_k(tp, tok, visible_count(row_bounds(p, tok), p.t_all));
+  const u32x2* const kept = (const u32x2*)tp.kept + (size_t)rid * tp.kept_pad;
   float acc[PER];
 #pragma unroll
   for (int i = 0; i < PER; ++i) acc[i] = 0.f;
@@ -1217,28 +1235,27 @@ __global__ void __launch_bounds__(256, NR <= 20 ? 4 : NR == 24 ? 3 : 2) topk_lis
   auto gather = [&](auto gu_c) {
     constexpr uint32_t GU = decltype(gu_c)::value;
     for (uint32_t j0 = 0; j0 < k; j0 += GU) {
-      float e[GU];
+      float w[GU];
       u32x4 raw[GU];
 #pragma unroll
       for (uint32_t u = 0; u < GU; ++u) {
-        const u32x2 v = sel[j0 + u];
-        e[u] = __uint_as_float(v[0]);
+        const u32x2 v = kept[j0 + u];
+        w[u] = __uint_as_float(v[0]);
         raw[u] = *(const u32x4*)(vbase + (v[1] + lane_b));
       }
 #pragma unroll
       for (uint32_t u = 0; u < GU; ++u) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          acc[2 * i] = __builtin_fmaf(e[u], unpack_lo<F16>(raw[u][i]), acc[2 * i]);
-          acc[2 * i + 1] = __builtin_fmaf(e[u], unpack_hi<F16>(raw[u][i]), acc[2 * i + 1]);
+          acc[2 * i] = __builtin_fmaf(w[u], unpack_lo<F16>(raw[u][i]), acc[2 * i]);
+          acc[2 * i + 1] = __builtin_fmaf(w[u], unpack_hi<F16>(raw[u][i]), acc[2 * i + 1]);
         }
       }
     }
   };
-  if (n_rows > 2048u) gather(std::integral_constant<uint32_t, 2>{});
+  static_assert(kTopkGather % 8 == 0, "lists are padded to whole groups");
+  if (n_rows > 2048u) gather(std::integral_constant<uint32_t, 4>{});
   else gather(std::integral_constant<uint32_t, 8>{});
-#pragma unroll
-  for (int i = 0; i < PER; ++i) acc[i] *= inv;
   const size_t out_off = ((size_t)tok * p.hq + qh) * D + lane * PER;
   if (p.out_dtype == 2u) {
     float* const o = (float*)p.out + out_off;
@@ -1296,10 +1313,13 @@ hipError_t launch_filter(const TopkParams& tp, const TopkParams& sample, hipStre
 template <bool F16>
 hipError_t launch_list_select(const TopkParams& tp, uint32_t k_most, hipStream_t s) {
   const dim3 sel((tp.ntok * tp.a.hq + 31u) / 32u * 8u);
-  if (k_most <= 160u) hipLaunchKernelGGL((topk_list_select_kernel<F16, 16>), sel, dim3(256), 0, s, tp);
-  else if (k_most <= 272u) hipLaunchKernelGGL((topk_list_select_kernel<F16, 20>), sel, dim3(256), 0, s, tp);
-  else if (k_most <= 384u) hipLaunchKernelGGL((topk_list_select_kernel<F16, 24>), sel, dim3(256), 0, s, tp);
-  else hipLaunchKernelGGL((topk_list_select_kernel<F16, 32>), sel, dim3(256), 0, s, tp);
+  if (k_most <= 160u) hipLaunchKernelGGL((topk_list_select_kernel<16>), sel, dim3(256), 0, s, tp);
+  else if (k_most <= 272u) hipLaunchKernelGGL((topk_list_select_kernel<20>), sel, dim3(256), 0, s, tp);
+  else if (k_most <= 384u) hipLaunchKernelGGL((topk_list_select_kernel<24>), sel, dim3(256), 0, s, tp);
+  else hipLaunchKernelGGL((topk_list_select_kernel<32>), sel, dim3(256), 0, s, tp);
+  const hipError_t rc = hipGetLastError();
+  if (rc != hipSuccess) return rc;
+  hipLaunchKernelGGL((topk_gather_kernel<F16>), sel, dim3(256), 0, s, tp);
   return hipGetLastError();
 }
 

@@ -649,19 +649,20 @@ struct TopkPlan {
   // filtered path (pass_tok = 0: not taken): canvas rows per pass and, within a pass, per block of the general path
   // behind it; sampled keys; key-range splits; byte offsets in the workspace
   uint32_t pass_tok = 0, redo_tok = 0, stride = 0, sample_n = 0, sample_pad = 0, splits = 0, k_most = 0;
-  size_t off_block = 0, off_plane = 0, off_tau = 0, off_cand_n = 0, off_lists = 0;
+  size_t off_block = 0, off_plane = 0, off_tau = 0, off_cand_n = 0, off_kept = 0, off_lists = 0;
+  uint32_t kept_pad = 0;
 };
 
 // Where the filtered path is taken: what its kernels are made for (head_dim 512, linear cache, every row sees all keys
 // up to its own or the last), at most 512 keys kept (what a wave holds of a row's list), prefixes long
-// enough that a pass over 1/17 of the keys tells where the k-th score lies, and calls with enough scores.  Its six and more
-// launches take about 75 us however small they are; the general path takes 50, and about 30 for every 2^23 scores once its
-// select kernel, a workgroup per (row, head), needs more than one round of the chip, 10 below that.  Measured, the layer
-// step with 16 heads, general -> filtered path: 64 rows over 20k keys 99 -> 104 us, 33k 152 -> 136, 50k 297 -> 179;
-// 128 rows over 3k keys 79 -> 81 us, 8k 99 -> 91, 33k 294 -> 185; 256 rows over 3k keys 136 -> 96 us, 33k 629 -> 290.
+// enough that a pass over 1/17 of the keys tells where the k-th score lies, and calls large enough.  Its seven and more
+// launches take about 75 us however small they are; the general path, a workgroup per (row, head) in the end, takes 50 and its
+// time grows with the rounds of the chip those workgroups need.  Measured, the layer step with 16 heads, general -> filtered
+// path: 64 rows (one round) over 20k keys 99 -> 108 us, 33k 152 -> 141, 50k 297 -> 190; 128 rows (two) over 5k keys
+// 87 -> 89 us, 8k 99.5 -> 98, 12k 123 -> 107, 33k 294 -> 175; 256 rows over 3k keys 136 -> 100 us, 33k 592 -> 269.
 constexpr uint32_t kTopkFilterMinPrefix = 2048;
 constexpr uint32_t kTopkFilterMaxK = 512;
-constexpr uint64_t kTopkFilterMinScores = 1ull << 23;         // three times that in one round of the select kernel
+constexpr uint32_t kTopkFilterMinKeys[3] = {24576, 8192, 0};   // one round, two rounds, more
 
 size_t filter_bytes(const dg_attn_desc* d, const Plan& pl, uint32_t cus, uint32_t ntok, TopkPlan* tk) {
   const uint32_t n_mtiles = (ntok * pl.group + dg::kTopkFilterRows - 1) / dg::kTopkFilterRows;
@@ -678,7 +679,9 @@ size_t filter_bytes(const dg_attn_desc* d, const Plan& pl, uint32_t cus, uint32_
   tk->off_plane = tk->off_block + align_up((size_t)ntok * sizeof(uint32_t));
   tk->off_tau = tk->off_plane;
   tk->off_cand_n = tk->off_tau + align_up((size_t)base * dg::kTopkFilterRows * sizeof(float));
-  tk->off_lists = tk->off_cand_n + align_up(segs * sizeof(uint32_t));
+  tk->off_kept = tk->off_cand_n + align_up(segs * sizeof(uint32_t));
+  tk->kept_pad = (tk->k_most + dg::kTopkGather - 1) / dg::kTopkGather * dg::kTopkGather;
+  tk->off_lists = tk->off_kept + align_up((size_t)ntok * d->n_q_heads * tk->kept_pad * 8);
   // (the lists lie where the sampled scores were)
   const size_t sample = (size_t)d->n_q_heads * ntok * tk->sample_pad * sizeof(float);
   return tk->off_lists + align_up(std::max(segs * dg::kTopkSegAlloc * 8, sample));
@@ -688,8 +691,8 @@ void plan_filtered(const dg_attn_desc* d, const uint32_t* k_cfg, const Plan& pl,
   if (d->head_dim != 512 || pl.lo_nc != 0 || pl.win_m1 != 0xffffffffu || d->kv_ring_mask != 0) return;
   if (d->kv_len < kTopkFilterMinPrefix || !std::isfinite(pl.scale) || (d->flags & DG_ATTN_F_TOPK_SCORE_PLANE)) return;
   const uint64_t rows = (uint64_t)d->canvas * d->n_q_heads;
-  const bool one_round = rows <= 4ull * cus;
-  if (rows * pl.t_all < (one_round ? 3 : 1) * kTopkFilterMinScores && !(d->flags & DG_ATTN_F_TOPK_THRESHOLD)) return;
+  const uint32_t min_keys = kTopkFilterMinKeys[rows <= 4ull * cus ? 0 : rows <= 8ull * cus ? 1 : 2];
+  if (pl.t_all < min_keys && !(d->flags & DG_ATTN_F_TOPK_THRESHOLD)) return;
   if (k_cfg[1] != 0u) {
     const uint64_t gran = std::max(k_cfg[0], 1u);
     const uint64_t most = (pl.t_all + gran - 1) / gran * gran / k_cfg[1];
@@ -827,6 +830,8 @@ int dg_attn_topk_forward(const dg_attn_desc* d, const uint32_t* k_cfg, const voi
       fp.tau = (float*)(ws + tk.off_tau);
       fp.cand_n = (uint32_t*)(ws + tk.off_cand_n);
       fp.cand = ws + tk.off_lists;
+      fp.kept = ws + tk.off_kept;
+      fp.kept_pad = tk.kept_pad;
       fp.fail_rows = (uint32_t*)ws;
       fp.fail_block = (uint32_t*)(ws + tk.off_block);
       fp.fail_block_tok = tk.redo_tok;
