@@ -11,7 +11,7 @@ import pytest
 import isa_hazards as H
 from diffgemma_amd import build
 
-UNITS = {"attn_mfma.hip": 100, "attn_wsplit.hip": 50}   # file -> at least this many assembly MFMAs expected
+UNITS = {"attn_mfma.hip": 100, "attn_topk.hip": 100, "attn_wsplit.hip": 50}   # file -> at least this many assembly MFMAs expected
 
 
 def _emit(src, out_dir):
