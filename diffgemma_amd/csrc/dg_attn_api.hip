@@ -646,6 +646,7 @@ constexpr size_t kTopkPlaneBudget = (size_t)DG_TOPK_PLANE_MIB << 20;
 struct TopkPlan {
   uint32_t t_pad = 0, block_tok = 0;
   size_t total = 0;
+  size_t general = 0;      // what the general path alone needs: with less than `total` it is taken
   // filtered path (pass_tok = 0: not taken): canvas rows per pass and, within a pass, per block of the general path
   // behind it; sampled keys; key-range splits; byte offsets in the workspace
   uint32_t pass_tok = 0, redo_tok = 0, stride = 0, sample_n = 0, sample_pad = 0, splits = 0, k_most = 0;
@@ -717,10 +718,11 @@ void plan_filtered(const dg_attn_desc* d, const uint32_t* k_cfg, const Plan& pl,
   }
   if (need > kTopkPlaneBudget) return;
   const size_t per_tok = (size_t)d->n_q_heads * tk->t_pad * sizeof(float);
-  if (tk->block_tok == d->canvas) tk->total = std::max(tk->total, tk->off_plane + align_up((size_t)ntok * per_tok));
-  tk->total = std::max(tk->total, need);
-  const size_t fit = (tk->total - tk->off_plane) / per_tok;
+  size_t total = std::max(tk->total, need);
+  if (tk->block_tok == d->canvas) total = std::max(total, tk->off_plane + align_up((size_t)ntok * per_tok));
+  const size_t fit = (total - tk->off_plane) / per_tok;
   if (fit == 0) return;
+  tk->total = total;
   tk->pass_tok = ntok;
   const uint32_t blocks = (uint32_t)((ntok + fit - 1) / fit);
   tk->redo_tok = (ntok + blocks - 1) / blocks;
@@ -741,6 +743,7 @@ int make_topk_plan(const dg_attn_desc* d, const uint32_t* k_cfg, const Plan& pl,
   tk->block_tok = (uint32_t)std::min<size_t>(blk, d->canvas);
   tk->total = align_up((size_t)tk->block_tok * per_tok);
   if (tk->total / sizeof(float) >= (1ull << 32)) return DG_ERR_SHAPE;   // score rows are addressed with 32-bit offsets
+  tk->general = tk->total;
   plan_filtered(d, k_cfg, pl, cus, tk);
   return DG_OK;
 }
@@ -770,7 +773,8 @@ int dg_attn_topk_forward(const dg_attn_desc* d, const uint32_t* k_cfg, const voi
   TopkPlan tk;
   rc = make_topk_plan(d, k_cfg, pl, plan_cus(), &tk);
   if (rc != DG_OK) return rc;
-  if (!workspace || workspace_bytes < tk.total || ((uintptr_t)workspace % 16) != 0) return DG_ERR_WORKSPACE;
+  if (workspace_bytes < tk.total) tk.pass_tok = 0;
+  if (!workspace || workspace_bytes < tk.general || ((uintptr_t)workspace % 16) != 0) return DG_ERR_WORKSPACE;
   if (((uintptr_t)q % 16) != 0 || ((uintptr_t)kv_base % 16) != 0 || ((uintptr_t)out % 16) != 0) return DG_ERR_LAYOUT;
   hipStream_t s = (hipStream_t)stream;
 

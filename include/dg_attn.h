@@ -323,7 +323,10 @@ int dg_attention_block_state_bytes(const dg_layer_offsets* L, const dg_attn_dims
  * (src/flags/accessors.rs:210-221, attention_topk.metal:160-182): divisor 0 keeps k_cfg[0] keys
  * (at least 1); otherwise a row keeps clamp(t_equiv / divisor, k_min, k_max) keys, t_equiv being
  * its number of visible keys, rounded up to the grid for causal rows.  Never more than the row
- * sees, never more than 1024. */
+ * sees, never more than 1024.
+ *
+ * dg_attn_topk_forward also takes less scratch than dg_attn_topk_workspace_bytes asks for, down to what the
+ * descriptor with DG_ATTN_F_TOPK_SCORE_PLANE needs, and then scores into the plane. */
 int dg_attn_topk_workspace_bytes(const dg_attn_desc* d, const uint32_t* k_cfg, size_t* out_bytes);
 int dg_attn_topk_forward(const dg_attn_desc* d, const uint32_t* k_cfg, const void* q, const void* kv_base,
                          void* out, void* workspace, size_t workspace_bytes, void* stream);

@@ -273,6 +273,25 @@ def test_random_rows_are_not_left_over(gpu_ready):
     assert int(((left != 0) & (left != 1)).sum()) == 0 and int(left.sum()) <= 8      # (5120 rows at 1e-5 each)
 
 
+def test_workspace_of_the_score_plane_alone_is_enough(gpu_ready):
+    """A caller with scratch for the score plane and no more gets the score plane's path, byte for byte."""
+    import torch
+    w = W.Workload("small_ws", 256, 16, 2, 512, 4000, seed=8)
+    q, kv = W.generate(w)
+    qd, kd = W.device_arrays(w, q, kv)
+    k_cfg = T.adaptive_k()
+    outs = []
+    plane = w.desc(flags=capi.DG_ATTN_F_TOPK_SCORE_PLANE)
+    need = T.workspace_bytes(plane, k_cfg)
+    assert need < T.workspace_bytes(w.desc(), k_cfg)
+    for d in (plane, w.desc()):
+        ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+        outs.append(torch.zeros(w.canvas * w.n_q_heads * w.head_dim, dtype=torch.int16, device="cuda"))
+        T.forward(d, k_cfg, qd, kd, outs[-1], ws)
+    torch.cuda.synchronize()
+    assert torch.equal(outs[0], outs[1]) and bool((outs[0] != 0).any())
+
+
 def test_thresholds_and_lists_replay_in_a_graph(gpu_ready):
     """Recorded once, replayed over other queries in the same buffers (one of them zero: rows left to the general path)."""
     import torch
