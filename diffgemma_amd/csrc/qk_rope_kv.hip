@@ -209,6 +209,7 @@ __global__ void __launch_bounds__(256) qk_rope_kv_kernel(const RopeParams p) {
   const uint32_t half_lanes = min(hd, 64u) / 2u;
   const uint32_t pd = (lane & (half_lanes - 1u)) * PER;
   const bool first = lane < half_lanes;
+  const bool rotated = pd < half_rot;   // (half_rot is a multiple of PER: all of a lane's elements or none)
   float cs[PER], sn[PER];   // sn signed: the first member becomes x0 cos - x1 sin, the second x1 cos + x0 sin
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
@@ -255,7 +256,9 @@ __global__ void __launch_bounds__(256) qk_rope_kv_kernel(const RopeParams p) {
       } else {
         other = __shfl_xor(y[i], 16, 64);
       }
-      y[i] = y[i] * cs[i] + other * sn[i];
+      // (selected, not multiplied by cos 1 and sin 0: an infinite or NaN partner, or a zero's sign, must not cross to an
+      // element that is left alone)
+      y[i] = rotated ? y[i] * cs[i] + other * sn[i] : y[i];
     }
     if (!active) continue;
     if (is_k && kv_write)

@@ -132,6 +132,41 @@ def test_debug_status_names_the_producer(gpu_ready):
     assert value == tok and tg_id == (tok << 16) | head
 
 
+@pytest.mark.parametrize("is_full", [False, True])
+@pytest.mark.parametrize("hd", [32, 64, 128, 256, 512])
+def test_nonfinite_elements_stay_where_the_rotation_leaves_them(gpu_ready, po, hd, is_full):
+    """An infinite element reaches its rotation partner and no other element: three quarters of a proportional head
+    (pairs d >= hd / 8) are left alone (cpu.rs:31-65), so neither a NaN nor the sign of a zero may cross there.  A row with
+    an infinity has 1/rms = 0: the element itself becomes NaN, the others zeros with the sign of x * w; an infinite
+    weight makes one infinite element of a finite row."""
+    half, half_rot = hd // 2, hd // 8 if is_full else hd // 2
+    elems = sorted({0, half_rot - 1, half_rot % hd, half - 1, half, half + half_rot - 1, (half + half_rot) % hd, hd - 1})
+    f = QR.random_fixture(len(elems), 3, 2, hd, 40, is_full=is_full, v_proj=1, seed=hd)
+    q, k, v = (x.reshape(len(elems), -1, hd) for x in (f.q, f.k, f.v))
+    for tok, e in enumerate(elems):       # head 0: an infinity, head 1 as well but for K / V; head 2 of Q: what the weights do
+        q[tok, 0, e] = np.inf
+        q[tok, 1, e] = -np.inf
+        k[tok, 0, e] = np.inf
+        v[tok, 1, e] = np.inf
+    f.q_norm_w[half - 1] = np.inf
+    f.k_norm_w[hd - 1] = np.inf
+    with np.errstate(invalid="ignore", over="ignore"):
+        want = reference_cpu(po, f)
+    rig = QR.RopeRig(f)
+    rig.run_dispatch()
+    unrotated = np.ones(hd, bool)
+    unrotated[:half_rot] = unrotated[half:half + half_rot] = False
+    for g, r in zip(rig.read(), want):
+        g, r = g.reshape(-1, hd), r.reshape(-1, hd)
+        r = np.where(np.abs(r) == 65504, np.copysign(np.float32(np.inf), r), r)   # (the host's conversion to f16 clamps; kv_store does not)
+        assert np.array_equal(np.isnan(g), np.isnan(r)) and np.array_equal(np.isposinf(g), np.isposinf(r))
+        assert np.array_equal(np.isneginf(g), np.isneginf(r))
+        finite = np.isfinite(r)
+        assert np.all(np.abs(g[finite] - r[finite]) <= storage_tolerance(r[finite], 7))
+        zero = (r == 0) & unrotated       # (or an f16 subnormal, which the host's conversion flushes)
+        assert np.array_equal(np.signbit(g[zero]), np.signbit(r[zero]))
+
+
 def test_write_suppression_and_untouched_rows(gpu_ready, po):
     """kv_write_end (qk_rope_kv.metal:56-60): pad rows are normed and rotated in place but never reach
     the cache; every slot the launch does not own keeps its bits."""
