@@ -607,11 +607,13 @@ __global__ void __launch_bounds__(256) attn_wsplit_kernel(const WsArgs args) {
     if (rr >= p.rows_total) break;
     const uint32_t tok = fast_div(rr, args.div_group), g = rr - tok * p.group;
     if (p.dbg) {   // a NaN or infinity among the chunk's elements: an all-ones exponent carries into the top bit
-      uint32_t t = 0;
+      uint32_t t[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e)
-        t |= f32_out ? ((h[e] & 0x7fffffffu) + 0x00800000u) & 0x80000000u : ((h[e] & 0x7fff7fffu) + 0x00800080u) & 0x80008000u;
-      if (t) dbg_report(p.dbg, DBG_ERR_NONFINITE, DBG_KERNEL_ATTENTION, (tok << 16) | (kvh * p.group + g), ch * (f32_out ? 4u : 8u));
+        t[e] = f32_out ? ((h[e] & 0x7fffffffu) + 0x00800000u) & 0x80000000u : ((h[e] & 0x7fff7fffu) + 0x00800080u) & 0x80008000u;
+      if ((t[0] | t[1]) | (t[2] | t[3]))   // (named by fours, as an accumulator holds them: a chunk of 16-bit elements is two)
+        dbg_report(p.dbg, DBG_ERR_NONFINITE, DBG_KERNEL_ATTENTION, (tok << 16) | (kvh * p.group + g),
+                   f32_out ? ch * 4u : ch * 8u + (t[0] | t[1] ? 0u : 4u));
     }
     wt_store16(out_win, (((tok - tok0) * p.hq + g) * cpr + ch) * 16u, h);
   }

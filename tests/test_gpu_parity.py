@@ -667,6 +667,22 @@ def test_debug_status_reports_nonfinite_output(gpu_ready, fixture):
     assert np.isnan(bad.read_out_f32()).any()
 
 
+@pytest.mark.parametrize("fixture,element", [("tiny", 6), ("wide", 37), ("sliding_hd256", 5), ("sliding_hd256", 254)])
+def test_debug_status_of_the_one_launch_kernel_names_four_elements(gpu_ready, fixture, element):
+    """The index in the record is that of the first of the four elements an accumulator group holds, as from the general
+    kernel's single pass: not of the eight that one store moves."""
+    f = FIXTURES[fixture][0]()
+    kv = f.kvcache.copy()
+    hd, nkv = f.head_dim(), f.n_kv()
+    kv[f.kv_len * 2 * nkv * hd + nkv * hd + element] = np.float32(np.nan)   # V of KV head 0, first canvas key
+    rig = A.AttnRig.from_fixture(A.Fixture(q=f.q, kvcache=kv, layer=f.layer, canvas=f.canvas, n_q_heads=f.n_q_heads, kv_len=f.kv_len))
+    assert capi.workspace_bytes(rig.desc()) == 0        # one launch
+    rig.run_dispatch(causal=0)
+    st = rig.read_debug_status()
+    assert (st.code, st.kernel_id) == (capi.DG_DBG_ERR_NONFINITE, capi.DG_DBG_KERNEL_ATTENTION)
+    assert st.value == element // 4 * 4
+
+
 def test_row_without_visible_keys(gpu_ready):
     """An empty key range stores zeros and LSE = -inf instead of NaN (attention_mma2.metal:297)."""
     import torch
