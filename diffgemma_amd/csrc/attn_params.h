@@ -169,6 +169,26 @@ __device__ __forceinline__ bool key_visible(const RowBounds& b, uint32_t t, uint
   return t < t_all && ((t >= b.lo && t < b.hi) || t >= b.extra);
 }
 
+// Rows of the key tile at position t0 that the kernels may read, as row numbers in the tile: [first, last].  Any other
+// row is replaced by the nearest of these.  Past the last key there may be no memory; before `lo`, the first key a row of
+// the workgroup sees, a dead ring slot may hold anything, and a holder of a key range (dg_attn_partial) who passes a
+// shifted base has no memory there either.
+struct TileRows {
+  uint32_t first, last;
+};
+__host__ __device__ __forceinline__ TileRows tile_rows(uint32_t t0, uint32_t lo, uint32_t t_all) {
+  const uint32_t left = t_all - 1u - t0;
+  TileRows r;
+  r.last = left < (uint32_t)kBlockN - 1u ? left : (uint32_t)kBlockN - 1u;
+  // (a first visible key at or past t_all, i.e. rows that see nothing, must not move the clamp past the last key)
+  r.first = lo <= t0 ? 0u : lo - t0 < r.last ? lo - t0 : r.last;
+  return r;
+}
+// whether some row of the tile may not be read
+__host__ __device__ __forceinline__ bool tile_is_edge(uint32_t t0, uint32_t lo, uint32_t t_all) {
+  return t0 < lo || t0 + (uint32_t)kBlockN > t_all;
+}
+
 __device__ __forceinline__ uint32_t kv_slot(uint32_t ring_mask, uint32_t t) {
   return ring_mask ? (t & ring_mask) : t;
 }

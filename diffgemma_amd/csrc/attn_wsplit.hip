@@ -196,10 +196,8 @@ __global__ void __launch_bounds__(256) attn_wsplit_kernel(const WsArgs args) {
   const uint32_t voff = lgrp * (uint32_t)NBLK * (uint32_t)vstride_b + lcol;
   const uint32_t lds0 = (uint32_t)(size_t)(lds_char*)smem;
   const uint32_t my_k = lds0 + wave * (uint32_t)L::SLICE, my_v = my_k + (uint32_t)L::K_BYTES;
-  // Tiles with rows that must not be read.  Past the last key there may be no memory; before the first visible key a dead
-  // ring slot may hold anything, which only V minds (0 * NaN; a score of such a key is masked whatever it is).
-  auto k_is_edge = [&](uint32_t tile) { return tile * kBlockN + kBlockN > p.t_all; };
-  auto v_is_edge = [&](uint32_t tile) { return tile * kBlockN < lo_min || tile * kBlockN + kBlockN > p.t_all; };
+  // a tile with rows that must not be read (tile_rows): of K as of V
+  auto is_edge = [&](uint32_t tile) { return tile_is_edge(tile * kBlockN, lo_min, p.t_all); };
   auto tile_base = [&](auto is_v_c, uint32_t tile) __attribute__((always_inline)) -> uint64_t {
     constexpr bool IS_V = decltype(is_v_c)::value;
     return uniform_address((IS_V ? vbase : kbase) + (int64_t)kv_slot(p.ring_mask, tile * kBlockN) * (IS_V ? vstride_b : kstride_b));
@@ -211,17 +209,15 @@ __global__ void __launch_bounds__(256) attn_wsplit_kernel(const WsArgs args) {
     const uint64_t stride_b = IS_V ? vstride_b : kstride_b;
     ws_issue<G, g * G * BLK, BLK>(base + (uint64_t)(g * G) * stride_b, stride_b - BLK, IS_V ? voff : koff, IS_V ? my_v : my_k);
   };
-  // The same for a tile with rows that must not be read: every row outside [rmin, rmax] is replaced by the nearest one inside.
+  // The same for an edge tile: every row that must not be read is replaced by the nearest one that may.
   auto issue_edge = [&](auto is_v_c, uint32_t tile) __attribute__((always_inline)) {
     constexpr bool IS_V = decltype(is_v_c)::value;
     constexpr int BLK = IS_V ? L::V_BLK : L::K_BLK, G = NBLK >= 4 ? 4 : NBLK;
     constexpr uint32_t BIAS = 4096;   // keeps the compensated offsets positive
-    const uint32_t t0 = tile * kBlockN, stride_b = (uint32_t)(IS_V ? vstride_b : kstride_b);
+    const uint32_t stride_b = (uint32_t)(IS_V ? vstride_b : kstride_b);
     const uint64_t base = tile_base(is_v_c, tile) - BIAS;
-    const uint32_t rmax = min(p.t_all - 1u - t0, (uint32_t)kBlockN - 1u);
-    // (a first visible key at or past t_all, i.e. rows that see nothing, must not move the clamp past the last key)
-    const uint32_t rmin = IS_V && lo_min > t0 ? min(lo_min - t0, rmax) : 0u;
-    const uint32_t lo = rmin * stride_b + lcol, hi = rmax * stride_b + lcol;
+    const TileRows rows = tile_rows(tile * kBlockN, lo_min, p.t_all);
+    const uint32_t lo = rows.first * stride_b + lcol, hi = rows.last * stride_b + lcol;
     static_for<0, NBLK / G>([&](auto g_c) {
       constexpr int g = decltype(g_c)::value;
       uint32_t off[4];
@@ -233,9 +229,9 @@ __global__ void __launch_bounds__(256) attn_wsplit_kernel(const WsArgs args) {
       ws_issue_clamped<G, g * G * BLK, BLK>(base, off, IS_V ? my_v : my_k);
     });
   };
-    constexpr int GK = NBLK >= 4 ? 4 : NBLK, GV = 2;
+  constexpr int GK = NBLK >= 4 ? 4 : NBLK, GV = 2;
   auto issue_k = [&](uint32_t tile) __attribute__((always_inline)) {
-    if (__builtin_expect(k_is_edge(tile), 0)) {
+    if (__builtin_expect(is_edge(tile), 0)) {
       issue_edge(std::false_type{}, tile);
     } else {
       const uint64_t base = tile_base(std::false_type{}, tile);
@@ -460,7 +456,7 @@ __global__ void __launch_bounds__(256) attn_wsplit_kernel(const WsArgs args) {
   // scores of `tile` (its K has landed) with the loads of its V, two at a time, between them: they have the rest of the
   // scores, the issue of the next K tile and the softmax to land
   auto scores_and_v = [&](uint32_t tile) __attribute__((always_inline)) {
-    const bool edge = v_is_edge(tile);
+    const bool edge = is_edge(tile);
     uint64_t base = 0;
     if (__builtin_expect(edge, 0)) issue_edge(std::true_type{}, tile);
     else base = tile_base(std::true_type{}, tile);

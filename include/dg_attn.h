@@ -209,7 +209,12 @@ size_t dg_attn_static_scratch_bytes(void);
  * l = 0 for a row that saw no key.  (The reference keeps the same three quantities head-major;
  * nothing outside the kernels reads its planes.)  dg_attn_partial leaves states in the normal
  * form l = 1, acc = the normalised row.  The workspace of a partial is sized by
- * dg_attn_partial_workspace_bytes for the same range. */
+ * dg_attn_partial_workspace_bytes for the same range.
+ *
+ * Rows a partial reads of a linear cache: none before t_begin, none at or past the last key (kv_len + canvas); where
+ * t_end is neither a multiple of 32 nor past the last key, also the rows up to the next multiple, which must then hold
+ * finite numbers (their weight is zero).  A caller that holds the rows [t_begin, t_end) alone passes kv_base shifted back
+ * by t_begin rows (not with an f32 cache, which is converted from its first row on). */
 int dg_attn_state_bytes(const dg_attn_desc* d, size_t* out_bytes);
 int dg_attn_partial_workspace_bytes(const dg_attn_desc* d, uint32_t t_begin, uint32_t t_end, size_t* out_bytes);
 int dg_attn_partial(const dg_attn_desc* d, uint32_t t_begin, uint32_t t_end, const void* q, const void* kv_base,

@@ -79,6 +79,36 @@ def test_partials_match_the_oracle_and_merge_to_the_single_call(gpu_ready, po, n
     assert np.all(np.abs(lg - one_lse.cpu().numpy()) <= np.maximum(1e-3 * np.abs(ref_lse), 2.0 ** -8))
 
 
+@pytest.mark.parametrize("hkv,hd,window", [(8, 256, 1024), (4, 64, 0), (2, 512, 0)])
+@pytest.mark.parametrize("a,b", [(1001, 1312), (1030, 1056), (1279, 1601)])
+def test_a_holder_of_a_key_range_needs_no_other_rows(gpu_ready, hkv, hd, window, a, b):
+    """A buffer with the rows [a, b) alone, passed with its base shifted back by a rows, gives the whole cache's state bit for
+    bit: no row before a is read (a not on a key tile), and none past b (on a key tile, or the last key)."""
+    import torch
+    w = W.Workload("holder", 64, 16, hkv, hd, 1537, window=window, layout="reference", seed=a)
+    q, kv = W.generate(w)
+    assert b % 32 == 0 or b == w.t_all
+    d = w.desc()
+    row = 2 * hkv * hd
+    qd, kd = W.device_arrays(w, q, kv)
+    whole = A.alloc_state(d)
+    A.partial(d, a, b, qd, kd, whole)
+    guard = 64 * row                       # (NaN on both sides, inside the allocation)
+    held = torch.full((2 * guard + (b - a) * row,), 0x7fc0, dtype=torch.int16, device="cuda")
+    held[guard:guard + (b - a) * row] = kd.view(-1)[a * row:b * row]
+
+    class Shifted:                         # where row 0 would lie
+        def data_ptr(self):
+            return held.data_ptr() + 2 * (guard - a * row)
+    part = A.alloc_state(d)
+    A.partial(d, a, b, qd, Shifted(), part)
+    torch.cuda.synchronize()
+    m, l, acc = A.read_state(d, part)
+    assert np.isfinite(acc).all() and (l > 0).any()
+    for got, want in zip((m, l, acc), A.read_state(d, whole)):
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
 def test_merge_into_a_state_in_place_equals_merge_of_all(gpu_ready):
     """Folding states one at a time into a carried state (state_out = an input) gives the rows a
     single merge of all of them gives, to fp32 rounding."""

@@ -1,0 +1,49 @@
+"""Which cache rows a key tile's loads touch: the arithmetic every tile loader shares (tile_rows, tile_is_edge in
+csrc/attn_params.h), compiled for the host.  A row before the first key the workgroup sees, or past the last key, may lie
+outside the caller's allocation (a holder of a key range passes a shifted base) and must not be read."""
+import subprocess
+
+from diffgemma_amd import build
+
+PROGRAM = r"""
+#include "attn_params.h"
+#include <cstdio>
+int main() {
+  using namespace dg;
+  const uint32_t span = 3 * kBlockN + 2;
+  for (uint32_t t_all = 1; t_all <= span; ++t_all)
+    for (uint32_t lo = 0; lo <= t_all + kBlockN; ++lo)
+      for (uint32_t t0 = 0; t0 < t_all; t0 += kBlockN) {
+        const TileRows r = tile_rows(t0, lo, t_all);
+        const uint32_t see = lo < t_all ? lo : t_all - 1u;      // (rows that see nothing: any row that exists)
+        bool clamped = false;
+        for (uint32_t i = 0; i < (uint32_t)kBlockN; ++i) {
+          const uint32_t row = t0 + (i < r.first ? r.first : i > r.last ? r.last : i);
+          clamped |= row != t0 + i;
+          // inside the keys that exist, and not before the first visible one unless the whole tile is
+          if (row >= t_all || (row < see && see < t0 + kBlockN)) return std::printf("t_all %u lo %u t0 %u row %u\n", t_all, lo, t0, row), 1;
+          if (t0 + i >= lo && t0 + i < t_all && row != t0 + i) return std::printf("moved a visible row %u\n", t0 + i), 1;
+        }
+        if (clamped && !tile_is_edge(t0, lo, t_all)) return std::printf("t_all %u lo %u t0 %u: no edge tile\n", t_all, lo, t0), 1;
+      }
+  std::puts("ok");
+  return 0;
+}
+"""
+
+
+def test_no_row_outside_the_visible_keys_is_read(tmp_path):
+    src, exe = tmp_path / "rows.hip", tmp_path / "rows"
+    src.write_text(PROGRAM)
+    res = subprocess.run([build.hipcc_path(), *build.HIP_FLAGS, "-I", str(build.CSRC), str(src), "-o", str(exe)],
+                         stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    assert res.returncode == 0, res.stdout[-2000:]
+    res = subprocess.run([str(exe)], stdout=subprocess.PIPE, text=True)
+    assert res.returncode == 0 and res.stdout == "ok\n", res.stdout
+
+
+def test_k_and_v_tiles_of_the_one_launch_kernel_share_the_rule():
+    """The one-launch kernel once clamped V's first tile and not K's."""
+    text = (build.CSRC / "attn_wsplit.hip").read_text()
+    assert text.count("tile_is_edge(") == 1 and text.count("tile_rows(tile * kBlockN, lo_min, p.t_all)") == 1
+    assert text.count("is_edge(tile)") == 2        # where K's loads go out and where V's do
