@@ -51,7 +51,6 @@ def test_ragged_causal_tail(gpu_ready, po):
 def run_topk(po, canvas, hq, hkv, hd, kv_len, k_cfg, *, causal_rows=0, window=0, q=None, kv=None, seed=0, toks=None,
              kv_dtype=capi.DG_BF16, flags=0):
     """bf16 (or f16) storage, fp32 output: isolates selection and arithmetic from the output store."""
-    import torch
     rng = np.random.default_rng(seed)
     t_all = kv_len + canvas
     if q is None:
@@ -59,20 +58,29 @@ def run_topk(po, canvas, hq, hkv, hd, kv_len, k_cfg, *, causal_rows=0, window=0,
         kv = rng.standard_normal((t_all, 2, hkv, hd)).astype(np.float32)
         rms = lambda x: x / np.sqrt(np.mean(x * x, axis=-1, keepdims=True) + 1e-6)
         q, kv = rms(q).astype(np.float32), rms(kv).astype(np.float32)
-    to_bits, from_bits = ((R.f32_to_bf16_bits_rne, R.bf16_bits_to_f32) if kv_dtype == capi.DG_BF16
-                          else (R.f32_to_f16_bits_rne, R.f16_bits_to_f32))
+    from_bits = R.bf16_bits_to_f32 if kv_dtype == capi.DG_BF16 else R.f16_bits_to_f32
+    got, qb, kb, _ = device_topk(canvas, hq, hkv, hd, kv_len, k_cfg, q, kv, causal_rows=causal_rows, window=window,
+                                 kv_dtype=kv_dtype, flags=flags)
+    od = po.make_desc(canvas, hq, hkv, hd, kv_len, causal_rows=causal_rows, window=window,
+                      causal_sees_masked=int(bool(flags & capi.DG_ATTN_F_CAUSAL_SEES_MASKED)))
+    ref = po.attention_topk_f32(od, k_cfg, R.bf16_bits_to_f32(qb).reshape(q.shape), from_bits(kb).reshape(kv.shape),
+                                tok_list=toks)
+    rows = np.arange(canvas) if toks is None else np.asarray(toks)
+    return got[rows], ref[rows]
+
+
+def device_topk(canvas, hq, hkv, hd, kv_len, k_cfg, q, kv, *, causal_rows=0, window=0, kv_dtype=capi.DG_BF16, flags=0):
+    """(fp32 rows, the storage bits of q and kv, the workspace as the call left it) of one dg_attn_topk_forward."""
+    import torch
+    to_bits = R.f32_to_bf16_bits_rne if kv_dtype == capi.DG_BF16 else R.f32_to_f16_bits_rne
     qb, kb = R.f32_to_bf16_bits_rne(q), to_bits(kv)
     d = A.make_desc(canvas, hq, hkv, hd, kv_len, causal_rows=causal_rows, window=window, q_dtype=capi.DG_BF16,
                     kv_dtype=kv_dtype, out_dtype=capi.DG_F32, flags=flags)
     out = torch.zeros(canvas * hq * hd, dtype=torch.float32, device="cuda")
-    T.forward(d, k_cfg, A.to_device_bits(qb.reshape(-1)), A.to_device_bits(kb.reshape(-1)), out, T.alloc_workspace(d, k_cfg))
+    ws = T.alloc_workspace(d, k_cfg)
+    T.forward(d, k_cfg, A.to_device_bits(qb.reshape(-1)), A.to_device_bits(kb.reshape(-1)), out, ws)
     torch.cuda.synchronize()
-    od = po.make_desc(canvas, hq, hkv, hd, kv_len, causal_rows=causal_rows, window=window)
-    ref = po.attention_topk_f32(od, k_cfg, R.bf16_bits_to_f32(qb).reshape(q.shape), from_bits(kb).reshape(kv.shape),
-                                tok_list=toks)
-    got = out.cpu().numpy().reshape(canvas, hq, hd)
-    rows = np.arange(canvas) if toks is None else np.asarray(toks)
-    return got[rows], ref[rows]
+    return out.cpu().numpy().reshape(canvas, hq, hd), qb, kb, ws
 
 
 # ------------------------------------------------------------------ selection exactness
@@ -225,8 +233,7 @@ FILTERED = [
 ]
 
 
-@pytest.mark.parametrize("case", FILTERED)
-def test_thresholds_and_lists(gpu_ready, po, case):
+def check_thresholds_and_lists(po, case, kv_dtype=capi.DG_BF16, more_flags=0):
     canvas, hq, hkv, kvl, cr, k_cfg, keys = case
     rng = np.random.default_rng(sum(case[:5]))
     t_all, hd = kvl + canvas, 512
@@ -245,7 +252,8 @@ def test_thresholds_and_lists(gpu_ready, po, case):
     if keys == "cluster":
         kv[3000:3200, 0] *= 4
     toks = None if canvas <= 64 else np.array([0, 159, 160, 161, 319])
-    run = lambda flag: run_topk(po, canvas, hq, hkv, hd, kvl, k_cfg, causal_rows=cr, q=q, kv=kv, flags=flag, toks=toks)
+    run = lambda flag: run_topk(po, canvas, hq, hkv, hd, kvl, k_cfg, causal_rows=cr, q=q, kv=kv, flags=flag | more_flags, toks=toks,
+                                kv_dtype=kv_dtype)
     got, ref = run(capi.DG_ATTN_F_TOPK_THRESHOLD)
     assert np.isfinite(got).all()
     if exact:       # same kept sets: outputs agree to fp32 summation error
@@ -255,6 +263,105 @@ def test_thresholds_and_lists(gpu_ready, po, case):
         # both paths sum a score over d in the same order, so they keep the same keys: fp32 summation error again
         assert max_abs_diff(got, run(capi.DG_ATTN_F_TOPK_SCORE_PLANE)[0]) < 2e-5
 
+
+@pytest.mark.parametrize("case", FILTERED)
+def test_thresholds_and_lists(gpu_ready, po, case):
+    check_thresholds_and_lists(po, case)
+
+
+@pytest.mark.parametrize("case", [c for c in FILTERED if c[0] <= 64])
+def test_thresholds_and_lists_over_an_f16_cache(gpu_ready, po, case):
+    """The storage of the reference's own boundary: bf16 queries converted in the kernel, f16 K and V."""
+    check_thresholds_and_lists(po, case, kv_dtype=capi.DG_F16)
+
+
+@pytest.mark.parametrize("case", [
+    (40, 16, 2, 2100, 25, T.adaptive_k(), "unit"),        # causal rows see the prefix, themselves and the masked canvas keys
+    (33, 8, 2, 2069, 7, (200, 0, 0, 0), "unit"),          # the second range begins inside a key tile
+    (6, 16, 2, 2100, 3, (100, 0, 0, 0), "ties"),
+    (24, 4, 1, 5001, 23, (64, 0, 0, 0), "few ties"),      # a second range of one key
+])
+@pytest.mark.parametrize("kv_dtype", [capi.DG_BF16, capi.DG_F16])
+def test_thresholds_and_lists_with_a_second_key_range(gpu_ready, po, case, kv_dtype):
+    check_thresholds_and_lists(po, case, kv_dtype=kv_dtype, more_flags=capi.DG_ATTN_F_CAUSAL_SEES_MASKED)
+
+
+def rows_left_over(ws, rows):
+    """The marks the thresholds-and-lists path leaves at the workspace's start, one word per row and head: 0, or 1 where
+    the general path redid it.  None where the words are no marks: the score plane begins there."""
+    import torch
+    left = ws.view(torch.int32)[:rows].cpu().numpy()
+    return int(left.sum()) if ((left == 0) | (left == 1)).all() else None
+
+
+@pytest.mark.parametrize("t_all,stride", [(8192 * 17, 17), (8192 * 17 + 1, 19), (8192 * 19, 19), (8192 * 19 + 1, 21), (8192 * 21, 21),
+                                          (8192 * 21 + 1, None)])
+def test_sample_strides_of_very_long_rows(gpu_ready, po, t_all, stride):
+    """8192 sampled keys at most: every 17th, 19th or 21st key, and past that the score plane."""
+    canvas, hq, hkv, hd, k_cfg = 3, 2, 1, 512, T.adaptive_k()
+    rng = np.random.default_rng(t_all)
+    rms = lambda x: x / np.sqrt(np.mean(x * x, axis=-1, keepdims=True))
+    q = rms(rng.standard_normal((canvas, hq, hd), dtype=np.float32))
+    kv = rms(rng.standard_normal((t_all, 2, hkv, hd), dtype=np.float32))
+    args = (canvas, hq, hkv, hd, t_all - canvas, k_cfg, q, kv)
+    got, qb, kb, ws = device_topk(*args, flags=capi.DG_ATTN_F_TOPK_THRESHOLD)
+    assert rows_left_over(ws, canvas * hq) == (None if stride is None else 0)
+    plane = device_topk(*args, flags=capi.DG_ATTN_F_TOPK_SCORE_PLANE)[0]
+    assert np.isfinite(got).all() and max_abs_diff(got, plane) < 2e-5
+    if stride in (None, 21):
+        od = po.make_desc(canvas, hq, hkv, hd, t_all - canvas)
+        ref = po.attention_topk_f32(od, k_cfg, R.bf16_bits_to_f32(qb).reshape(q.shape), R.bf16_bits_to_f32(kb).reshape(kv.shape))
+        assert max_abs_diff(got, ref) <= 2e-2 and mean_abs_diff(got, ref) <= 2e-3
+
+
+@pytest.mark.parametrize("kv_dtype", [capi.DG_BF16, capi.DG_F16])
+def test_nonfinite_scores_go_the_score_planes_way(gpu_ready, kv_dtype):
+    """NaN scores sort below every other (never kept while enough others are visible), an infinite score is kept and
+    makes its row NaN, -inf sorts low, a query row of NaN keeps the lowest positions: the same through both paths."""
+    canvas, hq, hkv, hd, kvl = 12, 4, 1, 512, 3000
+    rng = np.random.default_rng(5)
+    rms = lambda x: (x / np.sqrt(np.mean(x * x, axis=-1, keepdims=True))).astype(np.float32)
+    q, kv = rms(rng.standard_normal((canvas, hq, hd))), rms(rng.standard_normal((kvl + canvas, 2, hkv, hd)))
+    kv[[0, 17, 31, 34, 1000, kvl + 3], 0] = np.nan              # sampled positions (multiples of 17) and others
+    kv[2000:2040, 0] = np.nan
+    kv[[51, 500], 0, :, 3] = np.inf                             # +inf or -inf, by the sign of the query's element 3
+    q[:6, :, 3] = -np.abs(q[:6, :, 3])
+    q[6:, :, 3] = np.abs(q[6:, :, 3])
+    q[2, 1] = np.nan
+    for k_cfg in (T.adaptive_k(), (1, 0, 0, 0), (512, 0, 0, 0)):
+        args = (canvas, hq, hkv, hd, kvl, k_cfg, q, kv)
+        with np.errstate(invalid="ignore"):
+            got, _, _, ws = device_topk(*args, kv_dtype=kv_dtype, flags=capi.DG_ATTN_F_TOPK_THRESHOLD)
+            plane = device_topk(*args, kv_dtype=kv_dtype, flags=capi.DG_ATTN_F_TOPK_SCORE_PLANE)[0]
+        assert rows_left_over(ws, canvas * hq) == 1             # the NaN query's
+        assert np.isfinite(np.delete(got[:6].reshape(24, hd), 2 * hq + 1, axis=0)).all()
+        assert np.isnan(got[6:]).all() and np.isnan(got[2, 1]).all()
+        assert np.array_equal(np.isnan(got), np.isnan(plane))
+        assert max_abs_diff(got[~np.isnan(got)], plane[~np.isnan(got)]) < 2e-5
+
+
+def test_dispatch_over_a_long_prefix_keeps_lists(gpu_ready, po):
+    """The reference's argument block on rows long enough for thresholds: f16 slot-major cache, truncating store."""
+    kvl, canvas, hq, hkv, hd = 2500, 160, 16, 2, 512
+    rng = np.random.default_rng(77)
+    rms = lambda x: (x / np.sqrt(np.mean(x * x, axis=-1, keepdims=True))).astype(np.float32)
+    q = rms(rng.standard_normal((canvas, hq, hd), dtype=np.float32))
+    kv = rms(rng.standard_normal((kvl + canvas, 2, hkv, hd), dtype=np.float32))
+    f = A.Fixture(q.reshape(-1), kv.reshape(-1), A.LayerAttnParams(hd, hkv, True, 0), canvas, hq, kvl)
+    for causal in (False, True):
+        rig = A.AttnRig.from_fixture(f)
+        T.run_dispatch(rig, causal, T.adaptive_k())
+        got = rig.read_out_f32().reshape(canvas, hq, hd)
+        (ws,) = rig._ws.values()
+        assert rows_left_over(ws, canvas * hq) == 0
+        toks = np.array([0, 1, 79, 127, 128, 159], dtype=np.uint32)
+        d = po.make_desc(canvas, hq, hkv, hd, kvl, causal_rows=canvas if causal else 0)
+        ref = po.attention_topk_f32(d, T.adaptive_k(), R.bf16_bits_to_f32(R.f32_to_bf16_bits_trunc(q)).reshape(q.shape),
+                                    R.f16_bits_to_f32(R.f32_to_f16_bits_trunc(kv)).reshape(kv.shape), tok_list=toks)
+        assert np.isfinite(got).all()
+        # on top of the fp32 comparison's bounds the truncating store takes up to 2^-7 of a value, half of that on average
+        err, mag = np.abs(got[toks] - ref[toks]), np.abs(ref[toks])
+        assert np.all(err <= 2e-2 + mag * 2.0 ** -7) and err.mean() <= 2e-3 + mag.mean() * 2.0 ** -8
 
 
 def test_random_rows_are_not_left_over(gpu_ready):
