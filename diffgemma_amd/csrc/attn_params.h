@@ -43,7 +43,8 @@ struct AttnParams {
   uint32_t q_is_bf16;    // Q holds bf16 although E is f16 (reference: bf16 activations, f16 cache)
   uint32_t out_dtype, out_trunc;
   uint32_t part_half;    // split partials are normalised f16 rows instead of unnormalised fp32 ones
-  uint32_t touch_ahead;  // head_dim 512: touch key/value tiles into the L2 some tiles before they are loaded
+  uint32_t touch_ahead;  // the rows will come from HBM: at head_dim 512 key/value tiles are touched into the L2 some tiles
+                         // before they are loaded, in the one-launch kernel the key range at its start
   uint32_t lo_explicit;  // lo_nc was given by the caller (not the window rule)
   uint32_t cus;          // compute units of the device
   uint32_t sees_masked;  // causal rows also see the canvas keys behind the causal rows

@@ -28,7 +28,9 @@
 // table, scalar address arithmetic, divisions by multiplication, accumulators stored to LDS without passing through vector
 // registers, the shares of a row exchanged in register order).
 // Measured (GPU time of producer + attention, before and after these): a sliding layer over 1279 keys 23.1 -> 21.3 us, over
-// an f16 cache 25.6 -> 22.6; 64 rows behind 22 keys 13.4 -> 9.5; 901 causal rows 50.2 -> 36.4.
+// an f16 cache 25.6 -> 22.5; 64 rows behind 22 keys 13.4 -> 9.6; 901 causal rows 50.2 -> 34.9.  Of a launch over 1279 keys
+// 1.5 us go before the first scores, 1.6 into the first tile (cold code), 1.07 into each later one (the compute unit's load
+// path alone takes 0.85), 2.1 into the shares of the four waves and the rows.
 // Softmax arithmetic (lazy reference max, exponent offset under which negligible weights become exact zeros,
 // row sum over the rounded probabilities) is that of attn_mfma.hip, without its explicit zeroing of weights
 // far below the running max (a power device of the long kernel; here it would only cost instructions).
@@ -635,7 +637,7 @@ template <int D, bool F16>
 hipError_t launch_ws(const AttnParams& p, hipStream_t s) {
   // 32 rows per workgroup while they are one round of the chip's compute units (one workgroup each: LDS); past that 64
   // rows, whose workgroups take 1.6 x as long for twice the rows, where that is fewer rounds' time.  (Sliding layer, step
-  // in us, 32 | 64 rows: 256 canvas rows = 128 workgroups of 32: 21.3 | 31.0; 901 rows = 456: 41.7 | 36.4.)
+  // in us, 32 | 64 rows: 256 canvas rows = 128 workgroups of 32: 21.2 | 31.0; 901 rows = 456: 40.3 | 34.9.)
   const uint32_t cus = p.cus, r1 = (p.hkv * ((p.rows_total + 31u) / 32u) + cus - 1u) / cus;
   const uint32_t r2 = (p.hkv * ((p.rows_total + 63u) / 64u) + cus - 1u) / cus;
   if (8u * r2 < 5u * r1) return launch_rows<D, F16, 2>(p, s);

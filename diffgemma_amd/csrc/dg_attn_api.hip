@@ -661,6 +661,9 @@ struct TopkPlan {
 // time grows with the rounds of the chip those workgroups need.  Measured, the layer step with 16 heads, general -> filtered
 // path: 64 rows (one round) over 20k keys 99 -> 108 us, 33k 152 -> 141, 50k 297 -> 190; 128 rows (two) over 5k keys
 // 87 -> 89 us, 8k 99.5 -> 98, 12k 123 -> 107, 33k 294 -> 175; 256 rows over 3k keys 136 -> 100 us, 33k 592 -> 269.
+// That is for rows the lists hold.  A row they do not (thousands of equal scores) has its block of canvas rows scored again:
+// the attention call alone, 256 rows over 33k keys, general | filtered: one such row 706 | 462 us, one in every canvas row
+// 975 | 1300, all of them 1947 | 3120; 64 rows over 33k: 233 | 380, 235 | 384, 489 | 766.  The host cannot tell.
 constexpr uint32_t kTopkFilterMinPrefix = 2048;
 constexpr uint32_t kTopkFilterMaxK = 512;
 constexpr uint32_t kTopkFilterMinKeys[3] = {24576, 8192, 0};   // one round, two rounds, more

@@ -105,10 +105,13 @@ typedef enum dg_kernel_sel {
                                               of the probabilities; the flag is there to compare the two. */
 
 #define DG_ATTN_F_TOPK_THRESHOLD 0x200u  /* top-k attention, wherever its thresholds-and-lists path can run (head_dim 512, linear
-                                              cache, no window, prefix of at least 2048, at most 512 keys kept): take it,
-                                              also where the library would score into a plane.  Both give the same kept keys;
+                                              cache, no window, prefix of at least 2048, at most 172032 keys with the canvas
+                                              (8192 sampled keys, every 21st at most), at most 512 keys kept, 32-bit byte offsets
+                                              to every V row): take it, also where the library would score into a plane.
+                                              Otherwise the plane is used without a word.  Both give the same kept keys;
                                               the flags are there to compare the two. */
-#define DG_ATTN_F_TOPK_SCORE_PLANE 0x400u /* top-k attention: always through the score plane. */
+#define DG_ATTN_F_TOPK_SCORE_PLANE 0x400u /* top-k attention: always through the score plane (faster where most rows hold
+                                              thousands of equal scores, which lists cannot). */
 
 typedef struct dg_attn_desc {
   uint32_t canvas;        /* query rows; the reference passes active_canvas (256/128/64) */
