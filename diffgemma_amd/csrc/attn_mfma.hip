@@ -165,14 +165,11 @@ __global__ void __launch_bounds__(256) attn_mfma_kernel(const MfmaArgs args) {
   const uint32_t row0 = mt * kBlockM;
   const uint32_t r = row0 + wave * 32u + l32;
   const bool row_ok = r < p.rows_total;
-  const uint32_t tok = row_ok ? fast_div(r, args.div_group) : 0u;
-  const uint32_t qh = kvh * p.group + (row_ok ? r - tok * p.group : 0u);
-  RowBounds rb = row_bounds(p, tok);
-  if (!row_ok) {
-    rb.lo = 0;
-    rb.hi = 0;
-    rb.extra = p.t_all;
-  }
+  // (rows past the last one are copies of it that nobody stores: with bounds of their own, seeing nothing, every tile of
+  // a ragged row tile needs the mask, and the launch is as long as that row tile: 1.57 -> 2.2 us a key tile)
+  const uint32_t tok = fast_div(min(r, p.rows_total - 1u), args.div_group);
+  const uint32_t qh = kvh * p.group + min(r, p.rows_total - 1u) - tok * p.group;
+  const RowBounds rb = row_bounds(p, tok);
 
   // ---- tile-uniform bounds: which key tiles to visit, which need the per-element mask ----
   uint32_t lo_min, lo_max, hi_min, hi_max;
@@ -192,7 +189,6 @@ __global__ void __launch_bounds__(256) attn_mfma_kernel(const MfmaArgs args) {
       hi_max = max(hi_max, max(bc.hi, bd.hi));
     }
     if (tok_a < p.causal_rows && p.extra_lo < p.t_clip_hi) hi_max = p.t_clip_hi;
-    if (row0 + kBlockM > p.rows_total) hi_min = 0;  // ragged tile: always take the masked path
     // all four are the same in every lane; say so, so that they live in scalar registers
     lo_min = __builtin_amdgcn_readfirstlane(lo_min);
     lo_max = __builtin_amdgcn_readfirstlane(lo_max);
