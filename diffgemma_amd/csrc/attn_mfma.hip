@@ -141,7 +141,7 @@ __global__ void __launch_bounds__(256) attn_mfma_kernel(const MfmaArgs args) {
   static_assert(LDS_BYTES <= 160 * 1024, "LDS of one compute unit");
   static_assert(L::K_BYTES % 16 == 0 && L::V_BYTES % 16 == 0, "buffer alignment");
   __shared__ __attribute__((aligned(1024))) char smem[LDS_BYTES];
-  float* const sml = (float*)(smem + OFF_ML);
+  float* const sinv = (float*)(smem + OFF_ML);
 
   // ---- which (KV head, split, row tile) this workgroup owns ----
   // Workgroup ids go round-robin over the 8 XCDs, each with its own L2.  The units, ordered
@@ -163,6 +163,7 @@ __global__ void __launch_bounds__(256) attn_mfma_kernel(const MfmaArgs args) {
 
   // ---- row-owner role: this lane's query row and its key bounds ----
   const uint32_t row0 = mt * kBlockM;
+  const uint32_t tok0 = fast_div(row0, args.div_group);
   const uint32_t r = row0 + wave * 32u + l32;
   const bool row_ok = r < p.rows_total;
   // (rows past the last one are copies of it that nobody stores: with bounds of their own, seeing nothing, every tile of
@@ -202,7 +203,31 @@ __global__ void __launch_bounds__(256) attn_mfma_kernel(const MfmaArgs args) {
   const uint32_t per_split = (mt_end - mt_begin + p.n_splits - 1u) / p.n_splits;
   const uint32_t tb = __builtin_amdgcn_readfirstlane(min(mt_begin + split * per_split, mt_end));
   const uint32_t te = __builtin_amdgcn_readfirstlane(min(tb + per_split, mt_end));
-  const uint32_t ntile = te > tb ? te - tb : 0u;
+  const uint32_t ntile = te - tb;
+
+  // first partial row of this workgroup; partial rows and their (m, l) are written through (wt_store.h)
+  const size_t wg_prow0 = ((size_t)split * p.hkv + kvh) * p.rows_pad + row0;
+  // No key tile to visit: the rows' share is nothing, (m, l, O) = (-inf, 0, 0).  An exit of its own, so that the epilogue
+  // has one predecessor and takes O from the registers the tile loop leaves it in (with a second one the compiler moved
+  // all 256 accumulation registers at the loop's exit, 512 instructions).
+  if (ntile == 0u) {
+    const uint32_t row_b = D * (p.n_splits > 1 ? (p.part_half ? 2u : 4u) : p.out_dtype == DT_F32 ? 4u : 2u);
+    const u32x4 zero = {0u, 0u, 0u, 0u};
+    if (p.n_splits > 1) {
+      if (threadIdx.x < (uint32_t)kBlockM)
+        wt_store8(wt_window(p.part_ml + wg_prow0 * 2), threadIdx.x * 8u, u32x2{__float_as_uint(-INFINITY), 0u});
+      const auto win = wt_window((const char*)p.part_o + wg_prow0 * row_b);
+      for (uint32_t c = threadIdx.x; c < (uint32_t)kBlockM * row_b / 16u; c += 256u) wt_store16(win, c * 16u, zero);
+      return;
+    }
+    if (row_ok && g2 == 0u) {
+      if (p.lse) p.lse[(size_t)tok * p.hq + qh] = -INFINITY;
+      if (p.dbg) dbg_report(p.dbg, DBG_ERR_SOFTMAX_NORM_ZERO, DBG_KERNEL_ATTENTION, (tok << 16) | qh, (tok << 16) | qh);
+    }
+    if (row_ok)
+      for (uint32_t b = g2 * 16u; b < row_b; b += 32u) *(u32x4*)((char*)p.out + ((size_t)tok * p.hq + qh) * row_b + b) = zero;
+    return;
+  }
 
   const char* kbase = (const char*)p.k + (int64_t)kvh * p.k_head_stride * 2;
   const char* vbase = (const char*)p.v + (int64_t)kvh * p.v_head_stride * 2;
@@ -259,6 +284,14 @@ __global__ void __launch_bounds__(256) attn_mfma_kernel(const MfmaArgs args) {
     return make_tile_load<D, true, true>(vbase, vstride_b, tb * kBlockN, lo_min, p.t_all, p.ring_mask, buf, wave, lane);
   };
 
+  // d-owner accumulators: o[i * NRBW + j] = O^T block (d-block dgrp*NDBW+i, row-block rgrp*NRBW+j);
+  // register e of a block is d offset 8*(e>>2) + 4*g2 + (e&3), the lane is the row (l32).
+  f32x16 o[NACC];
+#pragma unroll
+  for (int i = 0; i < NACC; ++i)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) o[i][e] = 0.f;
+
   // ---- Q fragments: B operand of S^T = K.Q^T, lane = row, 8 consecutive d per step ----
   // The operand layout gives a lane 16 bytes of its own row per step, so loading the fragments
   // straight from memory touches 32 bytes of 32 different cache lines per instruction, and the
@@ -300,13 +333,12 @@ __global__ void __launch_bounds__(256) attn_mfma_kernel(const MfmaArgs args) {
       };
       lds_char* const ql = qb + i16 * PAIR + h16 * (uint32_t)D + g2 * 16u;
       load_half(0u);
-      if (ntile > 0) {
-        issue_tile<D, false>(k_load_first(k0), wave, lane);
-        issue_tile<D, false>(k_load((tb + 1) * kBlockN, k1, lane), wave, lane);
-        wait_vmem_but<2 * L::NLD>();
-      } else {
-        wait_vmem_all();
-      }
+      issue_tile<D, false>(k_load_first(k0), wave, lane);
+      issue_tile<D, false>(k_load((tb + 1) * kBlockN, k1, lane), wave, lane);
+      // O is cleared here, while the loads are on their way (left to the compiler: in front of the first tile)
+#pragma unroll
+      for (int i = 0; i < NACC; ++i) asm volatile("" : "+a"(o[i]));
+      wait_vmem_but<2 * L::NLD>();
 #pragma unroll
       for (int st = 0; st < NSTEP / 2; ++st) q_to_frag(*(lds_u32x4*)(ql + 32 * st), qf[st]);
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (read before the second half lands there)
@@ -335,13 +367,6 @@ __global__ void __launch_bounds__(256) attn_mfma_kernel(const MfmaArgs args) {
     __syncthreads();
   }
 
-  // d-owner accumulators: o[i * NRBW + j] = O^T block (d-block dgrp*NDBW+i, row-block rgrp*NRBW+j);
-  // register e of a block is d offset 8*(e>>2) + 4*g2 + (e&3), the lane is the row (l32).
-  f32x16 o[NACC];
-#pragma unroll
-  for (int i = 0; i < NACC; ++i)
-#pragma unroll
-    for (int e = 0; e < 16; ++e) o[i][e] = 0.f;
   float m_ref = -INFINITY;  // running reference max, log2 units (scale folded in)
   float m_run = -INFINITY;  // running max itself
   float x_drop = -INFINITY; // exponents below this are dropped: m_run - kDrop, relative to the reference in use
@@ -388,297 +413,303 @@ __global__ void __launch_bounds__(256) attn_mfma_kernel(const MfmaArgs args) {
     return u32x4{lo[0], lo[1], hi[0], hi[1]};
   };
 
-  if (ntile > 0) {
-    // ---- softmax of one tile, cut into NCH pieces ----
-    // The pieces of tile jj run between the score MFMAs of tile jj+1: one wave per SIMD issues
-    // in order, so vector work only overlaps the matrix pipe if it sits between MFMAs in
-    // program order.  A vector instruction that needs the result of the one before it waits
-    // about 8 cycles, an independent one issues after 4, so every piece is written as a group of
-    // independent operations (four scores at a time, two partial row sums).
-    // State that lives across pieces:
-    float tmax = 0.f, m_use = 0.f;
-    float ex[4] = {0.f, 0.f, 0.f, 0.f};
-    u32x4 pk4 = {0, 0, 0, 0};
-    auto softmax_piece = [&](auto c_c, f32x16& s, uint32_t t0, uint32_t par) {
-      constexpr int c = decltype(c_c)::value;
-      if constexpr (c == 0) {
-        // mask (edge tiles only)
-        const bool masked = !(t0 >= lo_max && t0 + kBlockN <= hi_min);
-        if (__builtin_expect(masked, 0)) {
+  // ---- softmax of one tile, cut into NCH pieces ----
+  // The pieces of tile jj run between the score MFMAs of tile jj+1: one wave per SIMD issues
+  // in order, so vector work only overlaps the matrix pipe if it sits between MFMAs in
+  // program order.  A vector instruction that needs the result of the one before it waits
+  // about 8 cycles, an independent one issues after 4, so every piece is written as a group of
+  // independent operations (four scores at a time, two partial row sums).
+  // State that lives across pieces:
+  float tmax = 0.f, m_use = 0.f;
+  float ex[4] = {0.f, 0.f, 0.f, 0.f};
+  u32x4 pk4 = {0, 0, 0, 0};
+  auto softmax_piece = [&](auto c_c, f32x16& s, uint32_t t0, uint32_t par) {
+    constexpr int c = decltype(c_c)::value;
+    if constexpr (c == 0) {
+      // mask (edge tiles only)
+      const bool masked = !(t0 >= lo_max && t0 + kBlockN <= hi_min);
+      if (__builtin_expect(masked, 0)) {
 #pragma unroll
-          for (int e = 0; e < 16; ++e) {
-            const uint32_t t = t0 + 8u * (e >> 2) + 4u * g2 + (e & 3);
-            if (!key_visible(rb, t, p.t_clip_hi)) s[e] = -INFINITY;
-          }
-        }
-      } else if constexpr (c == 1) {
-        // tile max of the row, as a tree
-        const float a0 = fmaxf(fmaxf(s[0], s[1]), s[2]), a1 = fmaxf(fmaxf(s[3], s[4]), s[5]);
-        const float a2 = fmaxf(fmaxf(s[6], s[7]), s[8]), a3 = fmaxf(fmaxf(s[9], s[10]), s[11]);
-        const float a4 = fmaxf(fmaxf(s[12], s[13]), s[14]);
-        tmax = fmaxf(fmaxf(fmaxf(a0, a1), a2), fmaxf(fmaxf(a3, a4), s[15]));
-      } else if constexpr (c == 2) {
-        // online softmax with a lazily raised reference max
-        tmax = max_across_halves(tmax) * p.scale_log2;
-        const bool raise = __builtin_amdgcn_ballot_w64(tmax > m_ref + kTau<F16>) != 0ull;
-        bool rescale = false;   // some row of the block has accumulated something that changes
-        m_run = fmaxf(m_run, tmax);
-        if (__builtin_expect(raise, 0)) {
-          // When one row of the block has to raise its reference the whole block is rescaled anyway,
-          // so every row moves its reference up to its running max: the next raise is then as far
-          // away as it can be (with f16 operands, where the threshold is low, this halves the raises).
-          const float m_new = fmaxf(m_ref, m_run);
-          const float corr = (m_new == -INFINITY) ? 1.f : __builtin_amdgcn_exp2f(m_ref - m_new);
-          rescale = __builtin_amdgcn_ballot_w64(m_ref != -INFINITY && corr != 1.f) != 0ull;
-          l_part *= corr;
-          l_part2 *= corr;
-          // the d owners rescale O after the barrier
-          if (g2 == 0) ((float*)(smem + OFF_CORR + par * CORR_BYTES))[wave * 32u + l32] = corr;
-          m_ref = m_new;
-        }
-        if (lane == 0) ((uint32_t*)(smem + OFF_FLAG + par * FLAG_BYTES))[wave] = rescale ? 1u : 0u;
-        m_use = (m_ref == -INFINITY) ? 0.f : m_ref + kPOff<F16>;
-        if constexpr (!F16) x_drop = m_run - kDrop - m_use;
-      } else {
-        // scores 4 q .. 4 q + 3 in two steps: (a) scale and subtract, first two exponentials;
-        // (b) the other two exponentials, rounding to the MFMA operand type, and for every
-        // second q the store of a k-step's B operand and its share of the row sum
-        constexpr int q = (c - 3) / 2;
-        if constexpr ((c - 3) % 2 == 0) {
-#pragma unroll
-          for (int i = 0; i < 4; ++i) ex[i] = __builtin_fmaf(s[4 * q + i], p.scale_log2, -m_use);
-          const bool keep0 = F16 || ex[0] >= x_drop, keep1 = F16 || ex[1] >= x_drop;
-          ex[0] = __builtin_amdgcn_exp2f(ex[0]);
-          ex[1] = __builtin_amdgcn_exp2f(ex[1]);
-          ex[0] = keep0 ? ex[0] : 0.f;
-          ex[1] = keep1 ? ex[1] : 0.f;
-        } else {
-          const bool keep2 = F16 || ex[2] >= x_drop, keep3 = F16 || ex[3] >= x_drop;
-          ex[2] = __builtin_amdgcn_exp2f(ex[2]);
-          ex[3] = __builtin_amdgcn_exp2f(ex[3]);
-          ex[2] = keep2 ? ex[2] : 0.f;
-          ex[3] = keep3 ? ex[3] : 0.f;
-          pk4[(2 * q) % 4] = pack2<F16>(ex[0], ex[1]);
-          pk4[(2 * q + 1) % 4] = pack2<F16>(ex[2], ex[3]);
-          if constexpr (q % 2 == 1) {
-            // register image of the B operand of MFMA k-step q/2 for (row l32, lane half g2)
-            *(lds_u32x4*)((lds_char*)(smem + OFF_P) + par * P_BYTES + (((uint32_t)(q / 2) * 4u + wave) * 64u + lane) * 16u) =
-                pk4;
-            // the row sum uses the rounded probabilities, the same numbers P.V multiplies
-            l_part = add_pair<F16>(pk4[0], l_part);
-            l_part2 = add_pair<F16>(pk4[1], l_part2);
-            l_part = add_pair<F16>(pk4[2], l_part);
-            l_part2 = add_pair<F16>(pk4[3], l_part2);
-          }
+        for (int e = 0; e < 16; ++e) {
+          const uint32_t t = t0 + 8u * (e >> 2) + 4u * g2 + (e & 3);
+          if (!key_visible(rb, t, p.t_clip_hi)) s[e] = -INFINITY;
         }
       }
-    };
-    constexpr int NCH = 3 + 8;   // pieces the softmax of a tile is cut into
-
-    // S^T = K.Q^T, MFMA steps [ST0, ST1) of the tile in kb.  The K fragments of steps
-    // 0 .. PFK-1 are already in (or on their way to) kf; fragment reads run PFK ahead of the
-    // MFMA that consumes them.  With SOFTMAX, the softmax of the previous tile (scores in
-    // s_prev) is spread over the steps below NSPLIT.  The scheduling barriers keep the
-    // interleaving as written.
-    constexpr int NSPLIT = NQK - PFK;   // steps before the tile's barrier; the rest need no more LDS reads
-    u32x4 kf[PFK];
-    auto kf_preload = [&](lds_char* kb) {
-#pragma unroll
-      for (int i = 0; i < PFK; ++i) kf[i] = k_frag(kb, i);
-    };
-    auto qk_steps = [&](auto st0_c, auto st1_c, lds_char* kb, auto softmax_c, auto wait_c, f32x16& s, f32x16& s_prev,
-                        uint32_t t0_prev, uint32_t par, auto&& after) {
-      constexpr bool SOFTMAX = decltype(softmax_c)::value, WAIT = decltype(wait_c)::value;
-      static_for<decltype(st0_c)::value, decltype(st1_c)::value>([&](auto st_c) {
-        constexpr int st = decltype(st_c)::value;
-        __builtin_amdgcn_sched_barrier(0);
-        if constexpr (st == 0) mfma_scores_first<F16>(s, kf[0], qf[0]);
-        else if constexpr (WAIT && st == NQK - 1) mfma_scores_last<F16>(s, kf[st % PFK], qf[st]);
-        else mfma_scores_acc<F16>(s, kf[st % PFK], qf[st]);
-        if constexpr (st + PFK < NQK) kf[st % PFK] = k_frag(kb, st + PFK);
-        if constexpr (SOFTMAX && st < NSPLIT) {
-          // pieces [st NCH / NSPLIT, (st+1) NCH / NSPLIT) follow MFMA st
-          static_for<st * NCH / (NSPLIT > 0 ? NSPLIT : 1), (st + 1) * NCH / (NSPLIT > 0 ? NSPLIT : 1)>(
-              [&](auto c_c) {
-                softmax_piece(c_c, s_prev, t0_prev, par); });
-        }
-        after(st_c);
-      });
-      __builtin_amdgcn_sched_barrier(0);
-    };
-    using I0 = std::integral_constant<int, 0>;
-    using ISPLIT = std::integral_constant<int, NSPLIT>;
-    using IQK = std::integral_constant<int, NQK>;
-
-    if constexpr (L::PAD) {
-      issue_tile<D, true>(v_load_first(v0), wave, lane);   // (waited for in front of the first tile's P.V)
+    } else if constexpr (c == 1) {
+      // tile max of the row, as a tree
+      const float a0 = fmaxf(fmaxf(s[0], s[1]), s[2]), a1 = fmaxf(fmaxf(s[3], s[4]), s[5]);
+      const float a2 = fmaxf(fmaxf(s[6], s[7]), s[8]), a3 = fmaxf(fmaxf(s[9], s[10]), s[11]);
+      const float a4 = fmaxf(fmaxf(s[12], s[13]), s[14]);
+      tmax = fmaxf(fmaxf(fmaxf(a0, a1), a2), fmaxf(fmaxf(a3, a4), s[15]));
+    } else if constexpr (c == 2) {
+      // online softmax with a lazily raised reference max
+      tmax = max_across_halves(tmax) * p.scale_log2;
+      const bool raise = __builtin_amdgcn_ballot_w64(tmax > m_ref + kTau<F16>) != 0ull;
+      bool rescale = false;   // some row of the block has accumulated something that changes
+      m_run = fmaxf(m_run, tmax);
+      if (__builtin_expect(raise, 0)) {
+        // When one row of the block has to raise its reference the whole block is rescaled anyway,
+        // so every row moves its reference up to its running max: the next raise is then as far
+        // away as it can be (with f16 operands, where the threshold is low, this halves the raises).
+        const float m_new = fmaxf(m_ref, m_run);
+        const float corr = (m_new == -INFINITY) ? 1.f : __builtin_amdgcn_exp2f(m_ref - m_new);
+        rescale = __builtin_amdgcn_ballot_w64(m_ref != -INFINITY && corr != 1.f) != 0ull;
+        l_part *= corr;
+        l_part2 *= corr;
+        // the d owners rescale O after the barrier
+        if (g2 == 0) ((float*)(smem + OFF_CORR + par * CORR_BYTES))[wave * 32u + l32] = corr;
+        m_ref = m_new;
+      }
+      if (lane == 0) ((uint32_t*)(smem + OFF_FLAG + par * FLAG_BYTES))[wave] = rescale ? 1u : 0u;
+      m_use = (m_ref == -INFINITY) ? 0.f : m_ref + kPOff<F16>;
+      if constexpr (!F16) x_drop = m_run - kDrop - m_use;
     } else {
-      issue_tile<D, false>(k_load_first(k0), wave, lane);
-      issue_tile<D, false>(k_load((tb + 1) * kBlockN, k1, lane), wave, lane);
-      issue_tile<D, true>(v_load_first(v0), wave, lane);
-      wait_vmem_all();
-      __syncthreads();
-    }
-    // s_a: scores of the tile whose softmax is due; s_b: scores being accumulated for the next.
-    // s_b is copied into s_a during each tile's P.V by copy_scores_part(), not by an assignment:
-    // the compiler would merge the two and place its own copy right behind (or before) the last
-    // score MFMA, reading the registers before the MFMA has written them.
-    f32x16 s_a, s_b;
-    kf_preload(k0);
-    auto nothing = [](auto) {};
-    qk_steps(I0{}, IQK{}, k0, std::false_type{}, std::true_type{}, s_a, s_b, 0u, 0u, nothing);
-    __syncthreads();   // every wave is done with K(tb): its buffer takes K(tb+2)
-    issue_tile<D, false>(k_load((tb + 2) * kBlockN, k0, lane), wave, lane);
-    if constexpr (PREFETCH) touch_tile(tb + PF_AHEAD - 1, lane);
-    kf_preload(k1);
-
-    for (uint32_t jj = 0; jj < ntile; ++jj) {
-      const uint32_t par = jj & 1u;
-      const uint32_t t0 = (tb + jj) * kBlockN;
-      lds_char* const kb_next = par ? k0 : k1;    // holds K(jj+1); takes K(jj+3) after the barrier
-      lds_char* const kb_next2 = par ? k1 : k0;   // holds K(jj+2) once the barrier is passed
-      lds_char* const vb_cur = par ? v1 : v0;     // holds V(jj)
-      lds_char* const vb_free = par ? v0 : v1;    // takes V(jj+1)
-
-      // ---- row-owner role: scores of the next tile, softmax of this one ----
-      // (K(jj+1) has landed everywhere: its loads were waited for before the previous barrier,
-      // and its first fragments were read during the previous tile's P.V.  For the last tile
-      // the "next" scores are those of a repeated tile and go unused.)
-      if constexpr (NSPLIT == 0)
-        static_for<0, NCH>([&](auto c_c) { softmax_piece(c_c, s_a, t0, par); });
-      qk_steps(I0{}, ISPLIT{}, kb_next, std::true_type{}, std::false_type{}, s_b, s_a, t0, par, nothing);
-      // The one barrier of the tile.  Before it: this wave's loads of V(jj) and K(jj+2), issued
-      // during the previous tile's P.V, have landed, its P is written and the last K fragments
-      // of the tile are in registers (the barrier's fence waits for all three).  After it: P,
-      // the rescale words and V(jj) of this tile are visible to the d owners; every wave is done
-      // reading K(jj+1), V(jj-1) and the previous tile's P (which has its own buffer), so their
-      // buffers can be refilled.
-      if constexpr (PREFETCH) wait_vmem_but<1>();   // (the touch of the previous tile may be on its way)
-      else wait_vmem_all();
-      __syncthreads();
-
-      // ---- d-owner role ----
-      lds_char* const pbuf = (lds_char*)(smem + OFF_P) + par * P_BYTES;
-      auto p_frag = [&](int ks, uint32_t rbk) -> u32x4 {
-        return *(lds_u32x4*)(pbuf + (((uint32_t)ks * 4u + rbk) * 64u + lane) * 16u);
-      };
-      constexpr int NVF = 2 * NDBW;                    // V^T fragments per tile and wave
-      constexpr int PFV = NVF - 1 < 3 ? NVF - 1 : 3;   // fragment reads in flight ahead of the MFMAs
-      auto v_frag_n = [&](int f) { return v_frag(vb_cur, f / NDBW, dgrp * NDBW + f % NDBW); };
-      // first reads of the P.V phase; the last score MFMAs of the next tile cover their latency
-      u32x4 fl = *(lds_u32x4*)((lds_char*)(smem + OFF_FLAG) + par * FLAG_BYTES);
-      u32x4 pbv[NRBW];
+      // scores 4 q .. 4 q + 3 in two steps: (a) scale and subtract, first two exponentials;
+      // (b) the other two exponentials, rounding to the MFMA operand type, and for every
+      // second q the store of a k-step's B operand and its share of the row sum
+      constexpr int q = (c - 3) / 2;
+      if constexpr ((c - 3) % 2 == 0) {
 #pragma unroll
-      for (int j = 0; j < NRBW; ++j) pbv[j] = p_frag(0, rgrp * NRBW + j);
-      u32x4 va[PFV + 1];
-#pragma unroll
-      for (int f = 0; f <= PFV; ++f) va[f] = v_frag_n(f);
-      // The descriptors of this tile's global loads are worked out between those MFMAs, not
-      // behind the branch below, where nothing would overlap them.  The per-lane offsets are
-      // re-derived in every iteration: hoisted out of the loop they would cost more live VGPRs
-      // than this kernel has.
-      const uint32_t lane_l = opaque(lane);
-      TileLoad next_v, next_k;
-      Touch next_touch{nullptr, 0u};
-      qk_steps(ISPLIT{}, IQK{}, kb_next, std::true_type{}, std::false_type{}, s_b, s_a, t0, par, [&](auto st_c) {
-        constexpr int st = decltype(st_c)::value;
-        if constexpr (st == NSPLIT) next_v = pinned(v_load(t0 + kBlockN, vb_free, lane_l));
-        if constexpr (st == (NSPLIT + 1 < NQK ? NSPLIT + 1 : NSPLIT))
-          next_k = pinned(k_load(t0 + 3 * kBlockN, kb_next, lane_l));
-      });
-      // keep every use of the flags behind those MFMAs: they are what hides the latency of the read
-      fl = opaque4(fl);
-      if (__builtin_expect(__builtin_amdgcn_readfirstlane(fl[0] | fl[1] | fl[2] | fl[3]) != 0u, 0)) {
-        // O lives in accumulator registers, which only MFMA and the accvgpr moves can touch.
-        // Spelling the multiply out keeps the values in that register class on both sides of
-        // this rarely taken branch; a plain `o[i] *= corr` makes the allocator shuttle all of
-        // O through VGPRs and spill.
-        const float* const scorr = (const float*)(smem + OFF_CORR + par * CORR_BYTES);
-#pragma unroll
-        for (int j = 0; j < NRBW; ++j) {
-          const uint32_t rbk = rgrp * NRBW + j;
-          if (__builtin_amdgcn_readfirstlane(fl[rbk]) == 0u) continue;
-          const float corr = scorr[rbk * 32u + l32];
-#pragma unroll
-          for (int i = 0; i < NDBW; ++i)
-#pragma unroll
-            for (int e = 0; e < 16; e += 8) {
-              f32x16& a = o[i * NRBW + j];
-              float x0 = a[e], x1 = a[e + 1], x2 = a[e + 2], x3 = a[e + 3];
-              float x4 = a[e + 4], x5 = a[e + 5], x6 = a[e + 6], x7 = a[e + 7];
-              scale_acc8(x0, x1, x2, x3, x4, x5, x6, x7, corr);
-              a[e] = x0;
-              a[e + 1] = x1;
-              a[e + 2] = x2;
-              a[e + 3] = x3;
-              a[e + 4] = x4;
-              a[e + 5] = x5;
-              a[e + 6] = x6;
-              a[e + 7] = x7;
-            }
-          scale_acc_done();
+        for (int i = 0; i < 4; ++i) ex[i] = __builtin_fmaf(s[4 * q + i], p.scale_log2, -m_use);
+        const bool keep0 = F16 || ex[0] >= x_drop, keep1 = F16 || ex[1] >= x_drop;
+        ex[0] = __builtin_amdgcn_exp2f(ex[0]);
+        ex[1] = __builtin_amdgcn_exp2f(ex[1]);
+        ex[0] = keep0 ? ex[0] : 0.f;
+        ex[1] = keep1 ? ex[1] : 0.f;
+      } else {
+        const bool keep2 = F16 || ex[2] >= x_drop, keep3 = F16 || ex[3] >= x_drop;
+        ex[2] = __builtin_amdgcn_exp2f(ex[2]);
+        ex[3] = __builtin_amdgcn_exp2f(ex[3]);
+        ex[2] = keep2 ? ex[2] : 0.f;
+        ex[3] = keep3 ? ex[3] : 0.f;
+        pk4[(2 * q) % 4] = pack2<F16>(ex[0], ex[1]);
+        pk4[(2 * q + 1) % 4] = pack2<F16>(ex[2], ex[3]);
+        if constexpr (q % 2 == 1) {
+          // register image of the B operand of MFMA k-step q/2 for (row l32, lane half g2)
+          *(lds_u32x4*)((lds_char*)(smem + OFF_P) + par * P_BYTES + (((uint32_t)(q / 2) * 4u + wave) * 64u + lane) * 16u) =
+              pk4;
+          // the row sum uses the rounded probabilities, the same numbers P.V multiplies
+          l_part = add_pair<F16>(pk4[0], l_part);
+          l_part2 = add_pair<F16>(pk4[1], l_part2);
+          l_part = add_pair<F16>(pk4[2], l_part);
+          l_part2 = add_pair<F16>(pk4[3], l_part2);
         }
       }
-      // O^T += V^T . P^T: per k-step, NDBW V^T fragments x NRBW P fragments.  The P fragments
-      // of a k-step stay in registers for the whole step; V^T fragments are fetched PFV ahead
-      // of the one that multiplies, and each P fragment of k-step 1 replaces its k-step 0
-      // counterpart right after that one's last use.  Spread between the MFMAs: the global
-      // loads of V(jj+1) and K(jj+3), alternating; the copy of the next tile's scores to where
-      // the softmax expects them; behind the last MFMAs, the reads of the first K fragments of
-      // tile jj+2 (pinned there: at the loop end the compiler would move them to the top of the
-      // next iteration, in front of the MFMAs that wait for them).
-      constexpr int COPY_AT = NPV >= 16 ? NPV / 2 : 0;   // MFMA index after which the copy starts
-      static_for<0, NVF>([&](auto f_c) {
-        constexpr int f = decltype(f_c)::value, ks = f / NDBW, i = f % NDBW;
-        static_for<0, NRBW>([&](auto j_c) {
-          constexpr int j = decltype(j_c)::value, n = f * NRBW + j;   // n: MFMA index within the tile
-          __builtin_amdgcn_sched_barrier(0);
-          o[i * NRBW + j] = mfma16<F16>(va[f % (PFV + 1)], pbv[j], o[i * NRBW + j]);
-          if constexpr (ks == 0 && i == NDBW - 1) pbv[j] = p_frag(1, rgrp * NRBW + j);
-          if constexpr (n % LD_EVERY == 0 && n / LD_EVERY < 2 * NLD) {
-            constexpr int q = n / LD_EVERY;
-            if constexpr (q % 2 == 0) issue_tile_part<D, true, q / 2>(next_v, wave, lane_l);
-            else issue_tile_part<D, false, q / 2>(next_k, wave, lane_l);
-          }
-          if constexpr (NPV >= 16 && n >= COPY_AT && n < COPY_AT + 8) copy_scores_part<n - COPY_AT>(s_a, s_b);
-          if constexpr (NPV >= PFK && n >= NPV - PFK) kf[n - (NPV - PFK)] = k_frag(kb_next2, n - (NPV - PFK));
-          // the touch itself behind the tile's last load, its address worked out a few MFMAs earlier
-          // (behind the last MFMA nothing would overlap the arithmetic)
-          if constexpr (PREFETCH && n == NPV - 6) {
-            next_touch = touch_address(tb + jj + PF_AHEAD, lane_l);
-            uint64_t b = (uint64_t)next_touch.base;
-            uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)b);
-            uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(b >> 32));
-            asm volatile("" : "+s"(lo), "+s"(hi), "+v"(next_touch.voff));
-            next_touch.base = (const char*)(((uint64_t)hi << 32) | lo);
-          }
-          if constexpr (PREFETCH && n == NPV - 1) {
-            static_assert(!PREFETCH || (2 * NLD - 1) * LD_EVERY < NPV - 1, "the touch follows the tile's last load");
-            touch(next_touch);
-          }
-        });
-        if constexpr (f + PFV + 1 < NVF) va[f % (PFV + 1)] = v_frag_n(f + PFV + 1);
-      });
-      __builtin_amdgcn_sched_barrier(0);
-      if constexpr (NPV < 16) static_for<0, 8>([&](auto i_c) { copy_scores_part<decltype(i_c)::value>(s_a, s_b); });
-      if constexpr (NPV < PFK) kf_preload(kb_next2);
     }
-    // the loads issued for tiles after the last one must not outlive this workgroup's LDS
+  };
+  constexpr int NCH = 3 + 8;   // pieces the softmax of a tile is cut into
+
+  // S^T = K.Q^T, MFMA steps [ST0, ST1) of the tile in kb.  The K fragments of steps
+  // 0 .. PFK-1 are already in (or on their way to) kf; fragment reads run PFK ahead of the
+  // MFMA that consumes them.  With SOFTMAX, the softmax of the previous tile (scores in
+  // s_prev) is spread over the steps below NSPLIT.  The scheduling barriers keep the
+  // interleaving as written.
+  constexpr int NSPLIT = NQK - PFK;   // steps before the tile's barrier; the rest need no more LDS reads
+  u32x4 kf[PFK];
+  auto kf_preload = [&](lds_char* kb) {
+#pragma unroll
+    for (int i = 0; i < PFK; ++i) kf[i] = k_frag(kb, i);
+  };
+  auto qk_steps = [&](auto st0_c, auto st1_c, lds_char* kb, auto softmax_c, auto wait_c, f32x16& s, f32x16& s_prev,
+                      uint32_t t0_prev, uint32_t par, auto&& after) {
+    constexpr bool SOFTMAX = decltype(softmax_c)::value, WAIT = decltype(wait_c)::value;
+    static_for<decltype(st0_c)::value, decltype(st1_c)::value>([&](auto st_c) {
+      constexpr int st = decltype(st_c)::value;
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (st == 0) mfma_scores_first<F16>(s, kf[0], qf[0]);
+      else if constexpr (WAIT && st == NQK - 1) mfma_scores_last<F16>(s, kf[st % PFK], qf[st]);
+      else mfma_scores_acc<F16>(s, kf[st % PFK], qf[st]);
+      if constexpr (st + PFK < NQK) kf[st % PFK] = k_frag(kb, st + PFK);
+      if constexpr (SOFTMAX && st < NSPLIT) {
+        // pieces [st NCH / NSPLIT, (st+1) NCH / NSPLIT) follow MFMA st
+        static_for<st * NCH / (NSPLIT > 0 ? NSPLIT : 1), (st + 1) * NCH / (NSPLIT > 0 ? NSPLIT : 1)>(
+            [&](auto c_c) {
+              softmax_piece(c_c, s_prev, t0_prev, par); });
+      }
+      after(st_c);
+    });
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  using I0 = std::integral_constant<int, 0>;
+  using ISPLIT = std::integral_constant<int, NSPLIT>;
+  using IQK = std::integral_constant<int, NQK>;
+
+  if constexpr (L::PAD) {
+    issue_tile<D, true>(v_load_first(v0), wave, lane);   // (waited for in front of the first tile's P.V)
+  } else {
+    issue_tile<D, false>(k_load_first(k0), wave, lane);
+    issue_tile<D, false>(k_load((tb + 1) * kBlockN, k1, lane), wave, lane);
+    issue_tile<D, true>(v_load_first(v0), wave, lane);
     wait_vmem_all();
+    __syncthreads();
+  }
+  // s_a: scores of the tile whose softmax is due; s_b: scores being accumulated for the next.
+  // s_b is copied into s_a during each tile's P.V by copy_scores_part(), not by an assignment:
+  // the compiler would merge the two and place its own copy right behind (or before) the last
+  // score MFMA, reading the registers before the MFMA has written them.
+  f32x16 s_a, s_b;
+  kf_preload(k0);
+  auto nothing = [](auto) {};
+  qk_steps(I0{}, IQK{}, k0, std::false_type{}, std::true_type{}, s_a, s_b, 0u, 0u, nothing);
+  __syncthreads();   // every wave is done with K(tb): its buffer takes K(tb+2)
+  issue_tile<D, false>(k_load((tb + 2) * kBlockN, k0, lane), wave, lane);
+  if constexpr (PREFETCH) touch_tile(tb + PF_AHEAD - 1, lane);
+  kf_preload(k1);
+
+  for (uint32_t jj = 0; jj < ntile; ++jj) {
+    const uint32_t par = jj & 1u;
+    const uint32_t t0 = (tb + jj) * kBlockN;
+    lds_char* const kb_next = par ? k0 : k1;    // holds K(jj+1); takes K(jj+3) after the barrier
+    lds_char* const kb_next2 = par ? k1 : k0;   // holds K(jj+2) once the barrier is passed
+    lds_char* const vb_cur = par ? v1 : v0;     // holds V(jj)
+    lds_char* const vb_free = par ? v0 : v1;    // takes V(jj+1)
+
+    // ---- row-owner role: scores of the next tile, softmax of this one ----
+    // (K(jj+1) has landed everywhere: its loads were waited for before the previous barrier,
+    // and its first fragments were read during the previous tile's P.V.  For the last tile
+    // the "next" scores are those of a repeated tile and go unused.)
+    if constexpr (NSPLIT == 0)
+      static_for<0, NCH>([&](auto c_c) { softmax_piece(c_c, s_a, t0, par); });
+    qk_steps(I0{}, ISPLIT{}, kb_next, std::true_type{}, std::false_type{}, s_b, s_a, t0, par, nothing);
+    // The one barrier of the tile.  Before it: this wave's loads of V(jj) and K(jj+2), issued
+    // during the previous tile's P.V, have landed, its P is written and the last K fragments
+    // of the tile are in registers (the barrier's fence waits for all three).  After it: P,
+    // the rescale words and V(jj) of this tile are visible to the d owners; every wave is done
+    // reading K(jj+1), V(jj-1) and the previous tile's P (which has its own buffer), so their
+    // buffers can be refilled.
+    if constexpr (PREFETCH) wait_vmem_but<1>();   // (the touch of the previous tile may be on its way)
+    else wait_vmem_all();
+    __syncthreads();
+
+    // ---- d-owner role ----
+    lds_char* const pbuf = (lds_char*)(smem + OFF_P) + par * P_BYTES;
+    auto p_frag = [&](int ks, uint32_t rbk) -> u32x4 {
+      return *(lds_u32x4*)(pbuf + (((uint32_t)ks * 4u + rbk) * 64u + lane) * 16u);
+    };
+    constexpr int NVF = 2 * NDBW;                    // V^T fragments per tile and wave
+    constexpr int PFV = NVF - 1 < 3 ? NVF - 1 : 3;   // fragment reads in flight ahead of the MFMAs
+    auto v_frag_n = [&](int f) { return v_frag(vb_cur, f / NDBW, dgrp * NDBW + f % NDBW); };
+    // first reads of the P.V phase; the last score MFMAs of the next tile cover their latency
+    u32x4 fl = *(lds_u32x4*)((lds_char*)(smem + OFF_FLAG) + par * FLAG_BYTES);
+    u32x4 pbv[NRBW];
+#pragma unroll
+    for (int j = 0; j < NRBW; ++j) pbv[j] = p_frag(0, rgrp * NRBW + j);
+    u32x4 va[PFV + 1];
+#pragma unroll
+    for (int f = 0; f <= PFV; ++f) va[f] = v_frag_n(f);
+    // The descriptors of this tile's global loads are worked out between those MFMAs, not
+    // behind the branch below, where nothing would overlap them.  The per-lane offsets are
+    // re-derived in every iteration: hoisted out of the loop they would cost more live VGPRs
+    // than this kernel has.
+    const uint32_t lane_l = opaque(lane);
+    TileLoad next_v, next_k;
+    Touch next_touch{nullptr, 0u};
+    qk_steps(ISPLIT{}, IQK{}, kb_next, std::true_type{}, std::false_type{}, s_b, s_a, t0, par, [&](auto st_c) {
+      constexpr int st = decltype(st_c)::value;
+      if constexpr (st == NSPLIT) next_v = pinned(v_load(t0 + kBlockN, vb_free, lane_l));
+      if constexpr (st == (NSPLIT + 1 < NQK ? NSPLIT + 1 : NSPLIT))
+        next_k = pinned(k_load(t0 + 3 * kBlockN, kb_next, lane_l));
+    });
+    // keep every use of the flags behind those MFMAs: they are what hides the latency of the read
+    fl = opaque4(fl);
+    if (__builtin_expect(__builtin_amdgcn_readfirstlane(fl[0] | fl[1] | fl[2] | fl[3]) != 0u, 0)) {
+      // O lives in accumulator registers, which only MFMA and the accvgpr moves can touch.
+      // Spelling the multiply out keeps the values in that register class on both sides of
+      // this rarely taken branch; a plain `o[i] *= corr` makes the allocator shuttle all of
+      // O through VGPRs and spill.
+      const float* const scorr = (const float*)(smem + OFF_CORR + par * CORR_BYTES);
+#pragma unroll
+      for (int j = 0; j < NRBW; ++j) {
+        const uint32_t rbk = rgrp * NRBW + j;
+        if (__builtin_amdgcn_readfirstlane(fl[rbk]) == 0u) continue;
+        const float corr = scorr[rbk * 32u + l32];
+#pragma unroll
+        for (int i = 0; i < NDBW; ++i)
+#pragma unroll
+          for (int e = 0; e < 16; e += 8) {
+            f32x16& a = o[i * NRBW + j];
+            float x0 = a[e], x1 = a[e + 1], x2 = a[e + 2], x3 = a[e + 3];
+            float x4 = a[e + 4], x5 = a[e + 5], x6 = a[e + 6], x7 = a[e + 7];
+            scale_acc8(x0, x1, x2, x3, x4, x5, x6, x7, corr);
+            a[e] = x0;
+            a[e + 1] = x1;
+            a[e + 2] = x2;
+            a[e + 3] = x3;
+            a[e + 4] = x4;
+            a[e + 5] = x5;
+            a[e + 6] = x6;
+            a[e + 7] = x7;
+          }
+        scale_acc_done();
+      }
+    }
+    // O^T += V^T . P^T: per k-step, NDBW V^T fragments x NRBW P fragments.  The P fragments
+    // of a k-step stay in registers for the whole step; V^T fragments are fetched PFV ahead
+    // of the one that multiplies, and each P fragment of k-step 1 replaces its k-step 0
+    // counterpart right after that one's last use.  Spread between the MFMAs: the global
+    // loads of V(jj+1) and K(jj+3), alternating; the copy of the next tile's scores to where
+    // the softmax expects them; behind the last MFMAs, the reads of the first K fragments of
+    // tile jj+2 (pinned there: at the loop end the compiler would move them to the top of the
+    // next iteration, in front of the MFMAs that wait for them).
+    constexpr int COPY_AT = NPV >= 16 ? NPV / 2 : 0;   // MFMA index after which the copy starts
+    static_for<0, NVF>([&](auto f_c) {
+      constexpr int f = decltype(f_c)::value, ks = f / NDBW, i = f % NDBW;
+      static_for<0, NRBW>([&](auto j_c) {
+        constexpr int j = decltype(j_c)::value, n = f * NRBW + j;   // n: MFMA index within the tile
+        __builtin_amdgcn_sched_barrier(0);
+        o[i * NRBW + j] = mfma16<F16>(va[f % (PFV + 1)], pbv[j], o[i * NRBW + j]);
+        if constexpr (ks == 0 && i == NDBW - 1) pbv[j] = p_frag(1, rgrp * NRBW + j);
+        if constexpr (n % LD_EVERY == 0 && n / LD_EVERY < 2 * NLD) {
+          constexpr int q = n / LD_EVERY;
+          if constexpr (q % 2 == 0) issue_tile_part<D, true, q / 2>(next_v, wave, lane_l);
+          else issue_tile_part<D, false, q / 2>(next_k, wave, lane_l);
+        }
+        if constexpr (NPV >= 16 && n >= COPY_AT && n < COPY_AT + 8) copy_scores_part<n - COPY_AT>(s_a, s_b);
+        if constexpr (NPV >= PFK && n >= NPV - PFK) kf[n - (NPV - PFK)] = k_frag(kb_next2, n - (NPV - PFK));
+        // the touch itself behind the tile's last load, its address worked out a few MFMAs earlier
+        // (behind the last MFMA nothing would overlap the arithmetic)
+        if constexpr (PREFETCH && n == NPV - 6) {
+          next_touch = touch_address(tb + jj + PF_AHEAD, lane_l);
+          uint64_t b = (uint64_t)next_touch.base;
+          uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)b);
+          uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(b >> 32));
+          asm volatile("" : "+s"(lo), "+s"(hi), "+v"(next_touch.voff));
+          next_touch.base = (const char*)(((uint64_t)hi << 32) | lo);
+        }
+        if constexpr (PREFETCH && n == NPV - 1) {
+          static_assert(!PREFETCH || (2 * NLD - 1) * LD_EVERY < NPV - 1, "the touch follows the tile's last load");
+          touch(next_touch);
+        }
+      });
+      if constexpr (f + PFV + 1 < NVF) va[f % (PFV + 1)] = v_frag_n(f + PFV + 1);
+    });
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (NPV < 16) static_for<0, 8>([&](auto i_c) { copy_scores_part<decltype(i_c)::value>(s_a, s_b); });
+    if constexpr (NPV < PFK) kf_preload(kb_next2);
   }
 
   // ---- epilogue ----
+  // Row owners publish (m, l) of their rows; d owners pass their slice of O through LDS, a 32-row block at a time, and store
+  // whole pieces of rows (the accumulators hold a row per lane: stored as they are, every instruction would scatter 32 pieces
+  // of it).  A wave alone on its SIMD takes about 8 cycles per instruction here, so it is their number that counts: 512 of
+  // the 700 read the accumulators and round them.
+  //   f16 partial rows: each accumulator divided by the split's row sum first (a weighted mean of V rows, no larger than the
+  //     largest |V|); the merge weighs the rows by l 2^(m - m_max) instead of 2^(m - m_max)
+  //   fp32 partial rows: the accumulators as they are
+  //   result rows (one split): divided by the row sum
+  const bool parts = p.n_splits > 1;
+  const bool rows16 = parts ? p.part_half != 0u : p.out_dtype != DT_F32;
+  constexpr int STG16 = NDBW * 64 + 16;   // bytes of a staged row slice, padded (the 16-byte pieces of 8 rows fall on distinct banks)
+  // The loads issued for tiles behind the last one are still on their way to the buffers of V(last + 1) and K(last + 1 .. 3).
+  // 16-bit rows at head_dim 512 fit the V buffer of the last tile, which none of them goes to; otherwise they are waited for.
+  constexpr bool IN_V = L::PAD && 4 * 32 * STG16 <= L::V_BYTES;
+  if (!IN_V || !rows16) wait_vmem_all();
   if (p.part_half) f16_saturate();
-  // row owners publish (m, l) of their rows; d owners normalise and store their slice of O
   const float l_tot = sum_across_halves(l_part + l_part2);
   const float m_pub = m_ref + kPOff<F16>;   // the exponent the sums are relative to
-  // first partial row of this workgroup; partial rows and their (m, l) are written through (wt_store.h)
-  const size_t wg_prow0 = ((size_t)split * p.hkv + kvh) * p.rows_pad + row0;
-  __syncthreads();   // the last tile's readers are done with LDS
   if (g2 == 0) {
-    sml[(wave * 32u + l32) * 2u] = m_pub;
-    sml[(wave * 32u + l32) * 2u + 1u] = l_tot;
-    if (p.n_splits > 1) {
+    sinv[wave * 32u + l32] = l_tot > 0.f ? 1.f / l_tot : 0.f;
+    if (parts) {
       const u32x2 ml2 = {__float_as_uint(m_pub), __float_as_uint(l_tot)};
       wt_store8(wt_window(p.part_ml + wg_prow0 * 2), (r - row0) * 8u, ml2);
     } else if (row_ok) {
@@ -686,100 +717,104 @@ __global__ void __launch_bounds__(256) attn_mfma_kernel(const MfmaArgs args) {
       if (p.dbg && !(l_tot > 0.f)) dbg_report(p.dbg, DBG_ERR_SOFTMAX_NORM_ZERO, DBG_KERNEL_ATTENTION, (tok << 16) | qh, (tok << 16) | qh);
     }
   }
-  __syncthreads();
+  __syncthreads();   // the row sums are there and the last tile's readers are done with LDS
+  auto rows_out = [&](auto part_c, auto b16_c, auto trunc_c) __attribute__((always_inline)) {
+    constexpr bool PART = decltype(part_c)::value, B16 = decltype(b16_c)::value, TRUNC = decltype(trunc_c)::value;
+    constexpr int ESZ = B16 ? 2 : 4, STG_ROW = NDBW * 32 * ESZ + 16;
+    constexpr int LPR = NDBW * 2 * ESZ, RPI = 64 / LPR, NIT = 32 / RPI;   // lanes per row slice (16 B each), rows per store, stores
+    static_assert(4 * 32 * STG_ROW <= OFF_ML, "staging must not reach the row sums");
+    lds_char* const stg = (lds_char*)smem + (IN_V && B16 ? ((ntile & 1u) ? OFF_V0 : OFF_V1) : 0) + wave * (uint32_t)(32 * STG_ROW);
+    lds_char* const wr = stg + l32 * (uint32_t)STG_ROW + g2 * (4u * ESZ);
+    lds_char* const rd = stg + lane / LPR * (uint32_t)STG_ROW + (lane % LPR) * 16u;
+    const uint32_t d_off = 32u * ESZ * (dgrp * NDBW) + (lane % LPR) * 16u;   // of the lane's piece in its row, bytes
+    const auto win = PART ? wt_window((const char*)p.part_o + wg_prow0 * (D * ESZ))
+                          : wt_window((const char*)p.out + ((size_t)tok0 * p.hq + kvh * p.group) * (D * ESZ));
+    // (a window reaches 2 GiB: with thousands of heads a row tile's result rows are further apart than that)
+    const bool in_win = PART || (uint64_t)p.hq * (uint32_t)(kBlockM * D * ESZ) < 0x7fffffffull;
+    constexpr int G = PART || NIT < 4 ? NIT : 4;   // pieces fetched from LDS at a time
+    u32x4 held[G];
+    auto fetch = [&](uint32_t it0) __attribute__((always_inline)) {
 #pragma unroll
-  for (int j = 0; j < NRBW; ++j) {
-    const uint32_t rbk = rgrp * NRBW + j;
-    const uint32_t rr = row0 + rbk * 32u + l32;
-    if (p.n_splits > 1 && p.part_half) {
-      // Same route through LDS as below, for partial rows kept as f16: each accumulator is divided
-      // by the split's row sum first (a weighted mean of V rows: no larger than the largest |V|),
-      // and the merge weighs the rows by l 2^(m - m_max) instead of 2^(m - m_max).
-      constexpr int STG_ROW = NDBW * 64 + 16;             // bytes of a staged row slice, padded
-      constexpr int LPR = NDBW * 4, RPI = 64 / LPR;       // lanes per row slice (16 B each), rows per store
-      lds_char* const stg = (lds_char*)smem + wave * (32 * STG_ROW);
-      const float l_row = sml[(rbk * 32u + l32) * 2u + 1u];
-      const float inv = l_row > 0.f ? 1.f / l_row : 0.f;
+      for (int u = 0; u < G; ++u) held[u] = *(lds_u32x4*)(rd + it0 * (uint32_t)(RPI * STG_ROW) + u * (RPI * STG_ROW));
+    };
+    auto put = [&](uint32_t rbk, uint32_t it0) __attribute__((always_inline)) {
 #pragma unroll
-      for (int i = 0; i < NDBW; ++i) {
-        const f32x16& a = o[i * NRBW + j];
-#pragma unroll
-        for (int q4 = 0; q4 < 4; ++q4) {
-          const f32x4 x = acc_read4<D == 512>(a, 4 * q4);
-          const u32x2 h2 = {mul_pack_f16(x[0], x[1], inv), mul_pack_f16(x[2], x[3], inv)};
-          *(__attribute__((address_space(3))) u32x2*)(stg + l32 * STG_ROW + (32 * i + 8 * q4 + 4 * g2) * 2) = h2;
-        }
-      }
-      const auto win = wt_window((const uint16_t*)p.part_o + wg_prow0 * D);
-      const uint32_t po = ((rbk * 32u) * D + 32u * (dgrp * NDBW) + (lane % LPR) * 8u) * 2u;   // bytes
-#pragma unroll
-      for (int it = 0; it < 32 / RPI; ++it) {
-        const uint32_t rl = it * RPI + lane / LPR;        // row within the block
-        const u32x4 v4 = *(lds_u32x4*)(stg + rl * STG_ROW + (lane % LPR) * 16);
-        wt_store16(win, po + rl * (D * 2u), v4);
-      }
-      continue;
-    }
-    if (p.n_splits > 1) {
-      // The accumulators hold a row per lane: stored as they are, every instruction would
-      // scatter 32-byte pieces over 32 rows.  Each wave passes its 32 rows x (NDBW x 32) d through
-      // its own piece of LDS (the tile buffers are free now) and writes whole rows instead.
-      constexpr int STG_ROW = NDBW * 128 + 16;            // bytes; the pad keeps the 16-byte writes of 8 rows apart
-      constexpr int LPR = NDBW * 8, RPI = 64 / LPR;       // lanes per row slice, rows per store instruction
-      static_assert(4 * 32 * STG_ROW <= OFF_ML, "staging must not reach the (m, l) words");
-      lds_char* const stg = (lds_char*)smem + wave * (32 * STG_ROW);
-#pragma unroll
-      for (int i = 0; i < NDBW; ++i) {
-        const f32x16& a = o[i * NRBW + j];
-#pragma unroll
-        for (int q4 = 0; q4 < 4; ++q4) {
-          const f32x4 v4 = acc_read4<D == 512>(a, 4 * q4);
-          *(__attribute__((address_space(3))) f32x4*)(stg + l32 * STG_ROW + (32 * i + 8 * q4 + 4 * g2) * 4) = v4;
-        }
-      }
-      const auto win = wt_window(p.part_o + wg_prow0 * D);
-      const uint32_t po = ((rbk * 32u) * D + 32u * (dgrp * NDBW) + (lane % LPR) * 4u) * 4u;   // bytes
-#pragma unroll
-      for (int it = 0; it < 32 / RPI; ++it) {
-        const uint32_t rl = it * RPI + lane / LPR;        // row within the block
-        const u32x4 v4 = *(lds_u32x4*)(stg + rl * STG_ROW + (lane % LPR) * 16);
-        wt_store16(win, po + rl * (D * 4u), v4);
-      }
-      continue;
-    }
-    if (rr >= p.rows_total) continue;
-    const float l_row = sml[(rbk * 32u + l32) * 2u + 1u];
-    const float inv = l_row > 0.f ? 1.f / l_row : 0.f;
-    const uint32_t tok_o = fast_div(rr, args.div_group), qh_o = kvh * p.group + rr - tok_o * p.group;
-#pragma unroll
-    for (int i = 0; i < NDBW; ++i) {
-      const size_t idx0 = ((size_t)tok_o * p.hq + qh_o) * D + 32u * (dgrp * NDBW + i) + 4u * g2;
-#pragma unroll
-      for (int q4 = 0; q4 < 4; ++q4) {
-        const f32x16& a = o[i * NRBW + j];
-        const f32x4 x = acc_read4<D == 512>(a, 4 * q4);
-        const float y0 = x[0] * inv, y1 = x[1] * inv;
-        const float y2 = x[2] * inv, y3 = x[3] * inv;
-        const size_t idx = idx0 + 8 * q4;
-        if (p.dbg && !(fabsf(y0) + fabsf(y1) + fabsf(y2) + fabsf(y3) <= 3.402823466e38f))   // NaN or infinity
-          dbg_report(p.dbg, DBG_ERR_NONFINITE, DBG_KERNEL_ATTENTION, (tok_o << 16) | qh_o, 32u * (dgrp * NDBW + i) + 4u * g2 + 8u * q4);
-        if (p.out_dtype == DT_F32) {
-          f32x4 v4 = {y0, y1, y2, y3};
-          *(f32x4*)((float*)p.out + idx) = v4;
+      for (int u = 0; u < G; ++u) {
+        const u32x4 h = held[u];
+        const uint32_t rl = rbk * 32u + (it0 + u) * RPI + lane / LPR;   // row within the tile
+        if constexpr (PART) {
+          wt_store16(win, rl * (uint32_t)(D * ESZ) + d_off, h);
         } else {
-          u32x2 pk;
-          if (p.out_trunc) {
-            pk[0] = (__float_as_uint(y0) >> 16) | (__float_as_uint(y1) & 0xffff0000u);
-            pk[1] = (__float_as_uint(y2) >> 16) | (__float_as_uint(y3) & 0xffff0000u);
-          } else {
-            pk[0] = pack2<false>(y0, y1);
-            pk[1] = pack2<false>(y2, y3);
+          const uint32_t rr = row0 + rl;
+          if (rr >= p.rows_total) break;
+          const uint32_t tk = fast_div(rr, args.div_group), g = rr - tk * p.group;
+          if (p.dbg) {   // a NaN or infinity among the piece's elements: an all-ones exponent carries into the top bit
+            uint32_t t[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              t[e] = B16 ? ((h[e] & 0x7fff7fffu) + 0x00800080u) & 0x80008000u : ((h[e] & 0x7fffffffu) + 0x00800000u) & 0x80000000u;
+            if ((t[0] | t[1]) | (t[2] | t[3]))   // (named by fours, as an accumulator holds them)
+              dbg_report(p.dbg, DBG_ERR_NONFINITE, DBG_KERNEL_ATTENTION, (tk << 16) | (kvh * p.group + g),
+                         B16 ? d_off / 2u + (t[0] | t[1] ? 0u : 4u) : d_off / 4u);
           }
-          *(u32x2*)((uint16_t*)p.out + idx) = pk;
+          if (in_win) wt_store16(win, ((tk - tok0) * p.hq + g) * (uint32_t)(D * ESZ) + d_off, h);
+          else *(u32x4*)((char*)p.out + ((size_t)tk * p.hq + kvh * p.group + g) * (D * ESZ) + d_off) = h;
         }
       }
-    }
+    };
+    auto stage = [&](auto j_c, float inv) __attribute__((always_inline)) {
+      constexpr int j = decltype(j_c)::value;
+      static_for<0, NDBW>([&](auto i_c) {
+        constexpr int i = decltype(i_c)::value;
+        const f32x16& a = o[i * NRBW + j];
+        static_for<0, 2>([&](auto h_c) {   // eight registers: d 32 i + 16 h + 4 g2 .. + 3 and the four 8 further on
+          constexpr int h = decltype(h_c)::value;
+          lds_char* const to = wr + (32 * i + 16 * h) * ESZ;
+          if constexpr (B16 && PART) {
+            const u32x4 v = acc_scale_pack8<D == 512>(a, 8 * h, inv);
+            *(lds_u32x2*)to = u32x2{v[0], v[1]};
+            *(lds_u32x2*)(to + 8 * ESZ) = u32x2{v[2], v[3]};
+          } else {
+            static_for<0, 2>([&](auto q_c) {
+              constexpr int q = decltype(q_c)::value;
+              const f32x4 x = acc_read4<D == 512>(a, 8 * h + 4 * q) * inv;
+              if constexpr (!B16) *(__attribute__((address_space(3))) f32x4*)(to + 8 * q * ESZ) = x;
+              else if constexpr (TRUNC)
+                *(lds_u32x2*)(to + 8 * q * ESZ) = u32x2{__builtin_amdgcn_perm(__float_as_uint(x[1]), __float_as_uint(x[0]), 0x07060302u),
+                                                        __builtin_amdgcn_perm(__float_as_uint(x[3]), __float_as_uint(x[2]), 0x07060302u)};
+              else *(lds_u32x2*)(to + 8 * q * ESZ) = u32x2{pack2<false>(x[0], x[1]), pack2<false>(x[2], x[3])};
+            });
+          }
+        });
+      });
+    };
+    static_for<0, NRBW>([&](auto j_c) {
+      constexpr int j = decltype(j_c)::value;
+      const uint32_t rbk = rgrp * NRBW + j;
+      stage(j_c, PART && !B16 ? 1.f : sinv[rbk * 32u + l32]);
+      if constexpr (PART) {   // the rows of block j are stored behind the staging of block j + 1
+        if constexpr (j > 0) put(rbk - 1u, 0u);
+        fetch(0u);
+      } else {
+#pragma unroll 1
+        for (uint32_t it0 = 0; it0 < (uint32_t)NIT; it0 += G) {
+          fetch(it0);
+          put(rbk, it0);
+        }
+      }
+    });
+    if constexpr (PART) put(rgrp * NRBW + NRBW - 1, 0u);
+  };
+  if (parts) {
+    if (rows16) rows_out(std::true_type{}, std::true_type{}, std::false_type{});
+    else rows_out(std::true_type{}, std::false_type{}, std::false_type{});
+  } else if (rows16) {
+    if (p.out_trunc) rows_out(std::false_type{}, std::true_type{}, std::true_type{});
+    else rows_out(std::false_type{}, std::true_type{}, std::false_type{});
+  } else {
+    rows_out(std::false_type{}, std::false_type{}, std::false_type{});
   }
+  wait_vmem_all();   // (tile loads must not outlive this workgroup's LDS)
 }
 
 template <int D, bool F16>

@@ -28,6 +28,7 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 typedef __attribute__((address_space(3))) char lds_char;
 typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
+typedef __attribute__((address_space(3))) u32x2 lds_u32x2;
 typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
 typedef __attribute__((address_space(1))) const void gbl_void;
 typedef __attribute__((address_space(3))) void lds_void;
@@ -127,6 +128,24 @@ __device__ __forceinline__ uint32_t mul_pack_f16(float a, float b, float c) {
   asm("v_fma_mixlo_f16 %0, %1, %2, 0" : "=v"(d) : "v"(a), "v"(c));
   asm("v_fma_mixhi_f16 %0, %1, %2, 0" : "+v"(d) : "v"(b), "v"(c));
   return d;
+}
+// Eight values out of accumulation registers (see acc_read4), times c, as four packed pairs of halves.  Independent
+// instructions next to each other: one that needs the result of the one before it waits twice as long to issue.
+template <bool FROM_ACC>
+__device__ __forceinline__ u32x4 acc_scale_pack8(const f32x16& a, int e, float c) {
+  if constexpr (!FROM_ACC)
+    return u32x4{mul_pack_f16(a[e], a[e + 1], c), mul_pack_f16(a[e + 2], a[e + 3], c), mul_pack_f16(a[e + 4], a[e + 5], c),
+                 mul_pack_f16(a[e + 6], a[e + 7], c)};
+  uint32_t d0, d1, d2, d3;
+  float t0, t1, t2, t3, t4, t5, t6, t7;
+  asm volatile(
+      "v_accvgpr_read_b32 %4, %12\n\tv_accvgpr_read_b32 %5, %13\n\tv_accvgpr_read_b32 %6, %14\n\tv_accvgpr_read_b32 %7, %15\n\t"
+      "v_accvgpr_read_b32 %8, %16\n\tv_accvgpr_read_b32 %9, %17\n\tv_accvgpr_read_b32 %10, %18\n\tv_accvgpr_read_b32 %11, %19\n\t"
+      "v_fma_mixlo_f16 %0, %4, %20, 0\n\tv_fma_mixlo_f16 %1, %6, %20, 0\n\tv_fma_mixlo_f16 %2, %8, %20, 0\n\tv_fma_mixlo_f16 %3, %10, %20, 0\n\t"
+      "v_fma_mixhi_f16 %0, %5, %20, 0\n\tv_fma_mixhi_f16 %1, %7, %20, 0\n\tv_fma_mixhi_f16 %2, %9, %20, 0\n\tv_fma_mixhi_f16 %3, %11, %20, 0"
+      : "=&v"(d0), "=&v"(d1), "=&v"(d2), "=&v"(d3), "=&v"(t0), "=&v"(t1), "=&v"(t2), "=&v"(t3), "=&v"(t4), "=&v"(t5), "=&v"(t6), "=&v"(t7)
+      : "a"(a[e]), "a"(a[e + 1]), "a"(a[e + 2]), "a"(a[e + 3]), "a"(a[e + 4]), "a"(a[e + 5]), "a"(a[e + 6]), "a"(a[e + 7]), "v"(c));
+  return u32x4{d0, d1, d2, d3};
 }
 // From here on the wave's f16 results saturate to +-65504 instead of overflowing (FP16_OVFL; an infinite operand still
 // gives an infinity).
