@@ -161,9 +161,52 @@ __global__ void __launch_bounds__(256) attn_mfma_kernel(const MfmaArgs args) {
   const uint32_t g2 = lane >> 5, l32 = lane & 31u, h16 = (lane >> 4) & 1u, i16 = lane & 15u;
   const uint32_t dgrp = wave % DSPLIT, rgrp = wave / DSPLIT;
 
-  // ---- row-owner role: this lane's query row and its key bounds ----
   const uint32_t row0 = mt * kBlockM;
   const uint32_t tok0 = fast_div(row0, args.div_group);
+
+  // ---- query rows, on their way before anything else is worked out ----
+  const char* const q_base = (const char*)p.q + (size_t)kvh * p.group * (2 * D);
+  // byte offset of a stacked row; below 4 GiB, which the host checks
+  auto q_row_off = [&](uint32_t rq) -> uint32_t {
+    return (rq + fast_div(rq, args.div_group) * (p.hq - p.group)) * (uint32_t)(2 * D);
+  };
+  // head_dim 512: in two halves of head_dim, through the V tiles' LDS: the first K tiles can then be on their way at the same
+  // time.  One instruction = half of rows i and i + 16, 16 bytes apart from the next pair.  A wave reads what it loaded
+  // itself, so there is no barrier between the halves.  A wave alone on its SIMD takes 5 to 9 cycles per instruction, so 16
+  // loads with an address each took 0.7 us; where a KV head has a multiple of eight heads, eight rows are next to each other
+  // and one offset per lane serves them, and the loads go at what the compute unit's 64 bytes a cycle allow.  The second K
+  // tile, not needed before the first tile's scores, follows the query rows.  (Scores of the first tile begin 3.5 us into a
+  // workgroup instead of 3.9, call 28.3 -> 27.5 us for 256 rows over 1033 keys, 15.4 -> 14.6 for 64 over 86.)
+  constexpr uint32_t Q_PAIR = 1024 + 16;
+  static_assert(!L::PAD || 4 * 16 * Q_PAIR <= 2 * L::V_BYTES, "the V tiles hold half of the query rows");
+  lds_char* const q_stage = (lds_char*)(smem + OFF_V0) + wave * (16u * Q_PAIR);
+  const uint32_t q_row = row0 + wave * 32u + g2 * 16u;   // (rows past the last one: copies of it, or of its token's; finite values)
+  const bool q_eights = (p.group & 7u) == 0u;
+  uint32_t q_off[2] = {0u, 0u};
+  if constexpr (L::PAD) {
+    if (q_eights) {
+      q_off[0] = q_row_off(min(q_row, p.rows_total - 8u)) + l32 * 16u;
+      q_off[1] = q_row_off(min(q_row + 8u, p.rows_total - 8u)) + l32 * 16u;
+    }
+  }
+  auto q_load_half = [&](uint32_t half) __attribute__((always_inline)) {
+    const uint32_t lds = (uint32_t)(size_t)q_stage;
+    if (q_eights) {
+      const uint64_t b = uniform_address(q_base) + half * (uint32_t)D;
+      constexpr uint64_t STEP = 1024 - (uint64_t)Q_PAIR;
+      lds_dma_group<4, 0, Q_PAIR>(b, STEP, q_off[0], lds);
+      lds_dma_group<4, 4 * Q_PAIR, Q_PAIR>(b + 4096, STEP, q_off[0], lds);
+      lds_dma_group<4, 8 * Q_PAIR, Q_PAIR>(b, STEP, q_off[1], lds);
+      lds_dma_group<4, 12 * Q_PAIR, Q_PAIR>(b + 4096, STEP, q_off[1], lds);
+    } else {
+#pragma unroll 1
+      for (uint32_t i = 0; i < 16u; ++i)
+        lds_dma_16<0>(q_base, q_row_off(min(q_row + i, p.rows_total - 1u)) + half * (uint32_t)D + l32 * 16u, lds + i * Q_PAIR);
+    }
+  };
+  if constexpr (L::PAD) q_load_half(0u);
+
+  // ---- row-owner role: this lane's query row and its key bounds ----
   const uint32_t r = row0 + wave * 32u + l32;
   const bool row_ok = r < p.rows_total;
   // (rows past the last one are copies of it that nobody stores: with bounds of their own, seeing nothing, every tile of
@@ -211,6 +254,7 @@ __global__ void __launch_bounds__(256) attn_mfma_kernel(const MfmaArgs args) {
   // has one predecessor and takes O from the registers the tile loop leaves it in (with a second one the compiler moved
   // all 256 accumulation registers at the loop's exit, 512 instructions).
   if (ntile == 0u) {
+    wait_vmem_all();   // (the query rows; loads must not outlive this workgroup's LDS)
     const uint32_t row_b = D * (p.n_splits > 1 ? (p.part_half ? 2u : 4u) : p.out_dtype == DT_F32 ? 4u : 2u);
     const u32x4 zero = {0u, 0u, 0u, 0u};
     if (p.n_splits > 1) {
@@ -287,10 +331,12 @@ __global__ void __launch_bounds__(256) attn_mfma_kernel(const MfmaArgs args) {
   // d-owner accumulators: o[i * NRBW + j] = O^T block (d-block dgrp*NDBW+i, row-block rgrp*NRBW+j);
   // register e of a block is d offset 8*(e>>2) + 4*g2 + (e&3), the lane is the row (l32).
   f32x16 o[NACC];
+  if constexpr (!L::PAD) {
 #pragma unroll
-  for (int i = 0; i < NACC; ++i)
+    for (int i = 0; i < NACC; ++i)
 #pragma unroll
-    for (int e = 0; e < 16; ++e) o[i][e] = 0.f;
+      for (int e = 0; e < 16; ++e) o[i][e] = 0.f;
+  }
 
   // ---- Q fragments: B operand of S^T = K.Q^T, lane = row, 8 consecutive d per step ----
   // The operand layout gives a lane 16 bytes of its own row per step, so loading the fragments
@@ -298,15 +344,8 @@ __global__ void __launch_bounds__(256) attn_mfma_kernel(const MfmaArgs args) {
   // four waves' 128 KiB pass through the compute unit's first-level cache several times over
   // (measured: 4.7 us until the rows had landed, 3.0 us this way).  Instead each wave brings its
   // 32 rows into LDS as whole pieces of rows and reads the fragments from there the way it reads K fragments.
-  // (Rows past the last one repeat it: finite values, and the rows are masked everywhere.)
   u32x4 qf[NSTEP];
   {
-    const char* const q_base = (const char*)p.q + (size_t)kvh * p.group * (2 * D);
-    // byte offset of a stacked row; below 4 GiB, which the host checks
-    auto q_row_off = [&](uint32_t row) -> uint32_t {
-      const uint32_t rq = min(row, p.rows_total - 1u);
-      return (rq + fast_div(rq, args.div_group) * (p.hq - p.group)) * (uint32_t)(2 * D);
-    };
     auto q_to_frag = [&](u32x4 raw, u32x4& f) {
       if (F16 && p.q_is_bf16) {
 #pragma unroll
@@ -317,33 +356,19 @@ __global__ void __launch_bounds__(256) attn_mfma_kernel(const MfmaArgs args) {
       }
     };
     if constexpr (L::PAD) {
-      // In two halves of head_dim, through the V tiles' LDS: the first K tiles can then be on their way at the same time
-      // (256 rows over 1033 keys: 33.9 -> 31.2 us with the divisions by reciprocals and the rolled loops; this part is run
-      // once, from code fetched cold at about 10 cycles an instruction, so its length counts as much as its waits).
-      // One instruction = half of rows i and i + 16, 16 bytes apart from the next pair.  A wave reads what it loaded
-      // itself, so there is no barrier between the halves.
-      constexpr uint32_t PAIR = 1024 + 16;
-      static_assert(4 * 16 * PAIR <= 2 * L::V_BYTES, "the V tiles hold half of the query rows");
-      lds_char* const qb = v0 + wave * (16u * PAIR);
-      auto load_half = [&](uint32_t half) {
-        const uint32_t rq = r - l32 + (lane >> 5) * 16u;
-#pragma unroll 1
-        for (uint32_t i = 0; i < 16u; ++i)
-          lds_dma_16<0>(q_base, q_row_off(rq + i) + half * (uint32_t)D + l32 * 16u, (uint32_t)(size_t)qb + i * PAIR);
-      };
-      lds_char* const ql = qb + i16 * PAIR + h16 * (uint32_t)D + g2 * 16u;
-      load_half(0u);
+      lds_char* const ql = q_stage + i16 * Q_PAIR + h16 * (uint32_t)D + g2 * 16u;
       issue_tile<D, false>(k_load_first(k0), wave, lane);
-      issue_tile<D, false>(k_load((tb + 1) * kBlockN, k1, lane), wave, lane);
-      // O is cleared here, while the loads are on their way (left to the compiler: in front of the first tile)
+      // O is cleared here, while the loads are on their way (left to the compiler: in front of the first tile), by 16 MFMAs
+      // instead of 256 register writes
 #pragma unroll
-      for (int i = 0; i < NACC; ++i) asm volatile("" : "+a"(o[i]));
-      wait_vmem_but<2 * L::NLD>();
+      for (int i = 0; i < NACC; ++i) mfma_zero(o[i]);
+      wait_vmem_but<L::NLD>();
 #pragma unroll
       for (int st = 0; st < NSTEP / 2; ++st) q_to_frag(*(lds_u32x4*)(ql + 32 * st), qf[st]);
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (read before the second half lands there)
-      load_half(1u);
-      wait_vmem_all();
+      q_load_half(1u);
+      issue_tile<D, false>(k_load((tb + 1) * kBlockN, k1, lane), wave, lane);   // (not waited for here)
+      wait_vmem_but<L::NLD>();
 #pragma unroll
       for (int st = 0; st < NSTEP / 2; ++st) q_to_frag(*(lds_u32x4*)(ql + 32 * st), qf[NSTEP / 2 + st]);
     } else {
@@ -355,15 +380,15 @@ __global__ void __launch_bounds__(256) attn_mfma_kernel(const MfmaArgs args) {
         constexpr int blk = decltype(b_c)::value;
         const uint32_t pch = blk * 64 + lane;
         const uint32_t rl = pch / L::CPR, pc = pch % L::CPR;
-        lds_dma_16<blk * 1024>(q_base, q_row_off(row0 + wave * 32u + rl) + (pc ^ L::swz_k(rl)) * 16u, (uint32_t)(size_t)qb);
+        lds_dma_16<blk * 1024>(q_base, q_row_off(min(row0 + wave * 32u + rl, p.rows_total - 1u)) + (pc ^ L::swz_k(rl)) * 16u, (uint32_t)(size_t)qb);
       });
       wait_vmem_all();
       const uint32_t q_lane_off = l32 * L::K_STRIDE, q_swz = L::swz_k(l32);
 #pragma unroll
       for (int st = 0; st < NSTEP; ++st) q_to_frag(*(lds_u32x4*)(qb + q_lane_off + ((((uint32_t)(2 * st) + g2) ^ q_swz) << 4)), qf[st]);
     }
-    // every wave has its fragments before the next tiles overwrite the rows (head_dim 512: and everybody's first K tiles
-    // have landed)
+    // every wave has its fragments before the next tiles overwrite the rows (head_dim 512: and everybody's first K tile
+    // has landed)
     __syncthreads();
   }
 
@@ -551,6 +576,7 @@ __global__ void __launch_bounds__(256) attn_mfma_kernel(const MfmaArgs args) {
   kf_preload(k0);
   auto nothing = [](auto) {};
   qk_steps(I0{}, IQK{}, k0, std::false_type{}, std::true_type{}, s_a, s_b, 0u, 0u, nothing);
+  if constexpr (L::PAD) wait_vmem_but<L::NLD>();   // K(tb+1) has landed; V(tb) may be on its way
   __syncthreads();   // every wave is done with K(tb): its buffer takes K(tb+2)
   issue_tile<D, false>(k_load((tb + 2) * kBlockN, k0, lane), wave, lane);
   if constexpr (PREFETCH) touch_tile(tb + PF_AHEAD - 1, lane);

@@ -87,28 +87,7 @@ struct WsLay {
   }
 };
 
-// G consecutive KiB blocks of a tile whose rows all exist, from one setting of M0: the instruction's immediate offset moves
-// the LDS address and, compensated in the scalar bases, the memory address.  A wave stands still until a load is accepted
-// (64 cycles when all four waves stream).
-template <int G, int LDS_OFF, int BLK>
-__device__ __forceinline__ void ws_issue(uint64_t b0, uint64_t step, uint32_t voff, uint32_t lds) {
-  const uint64_t b1 = b0 + step, b2 = b1 + step, b3 = b2 + step;
-  if constexpr (G == 1)
-    asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(b0), "n"(LDS_OFF)
-                 : "memory", "scc");
-  else if constexpr (G == 2)
-    asm volatile("s_add_u32 m0, %0, %4\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\t"
-                 "global_load_lds_dwordx4 %1, %3 offset:%5" ::"s"(lds), "v"(voff), "s"(b0), "s"(b1), "n"(LDS_OFF), "n"(BLK)
-                 : "memory", "scc");
-  else
-    asm volatile("s_add_u32 m0, %0, %6\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\t"
-                 "global_load_lds_dwordx4 %1, %3 offset:%7\n\tglobal_load_lds_dwordx4 %1, %4 offset:%8\n\t"
-                 "global_load_lds_dwordx4 %1, %5 offset:%9" ::"s"(lds), "v"(voff), "s"(b0), "s"(b1), "s"(b2), "s"(b3),
-                 "n"(LDS_OFF), "n"(BLK), "n"(2 * BLK), "n"(3 * BLK)
-                 : "memory", "scc");
-}
-
-// The same with an offset of its own for every block.
+// lds_dma_group (mfma_tile.h) with an offset of its own for every block.
 template <int G, int LDS_OFF, int BLK>
 __device__ __forceinline__ void ws_issue_clamped(uint64_t base, const uint32_t (&voff)[4], uint32_t lds) {
   if constexpr (G == 1)
@@ -209,7 +188,7 @@ __global__ void __launch_bounds__(256) attn_wsplit_kernel(const WsArgs args) {
     constexpr bool IS_V = decltype(is_v_c)::value;
     constexpr int G = decltype(size_c)::value, g = decltype(g_c)::value, BLK = IS_V ? L::V_BLK : L::K_BLK;
     const uint64_t stride_b = IS_V ? vstride_b : kstride_b;
-    ws_issue<G, g * G * BLK, BLK>(base + (uint64_t)(g * G) * stride_b, stride_b - BLK, IS_V ? voff : koff, IS_V ? my_v : my_k);
+    lds_dma_group<G, g * G * BLK, BLK>(base + (uint64_t)(g * G) * stride_b, stride_b - BLK, IS_V ? voff : koff, IS_V ? my_v : my_k);
   };
   // The same for an edge tile: every row that must not be read is replaced by the nearest one that may.
   auto issue_edge = [&](auto is_v_c, uint32_t tile) __attribute__((always_inline)) {

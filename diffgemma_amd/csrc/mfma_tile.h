@@ -74,6 +74,13 @@ __device__ __forceinline__ void mfma_scores_last(f32x16& s, u32x4 a, u32x4 b) {
     asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0\n\ts_nop 11" : "+v"(s) : "v"(a), "v"(b));
 }
 
+// acc = 0, one instruction for the 16 registers of a block.  The compiler does not know it for an MFMA: the zeros are two wait
+// states old when it reads them, and nothing may touch the block for 12 (callers wait for memory in between).
+__device__ __forceinline__ void mfma_zero(f32x16& acc) {
+  const u32x4 z = {0u, 0u, 0u, 0u};
+  asm volatile("s_nop 1\n\tv_mfma_f32_32x32x16_bf16 %0, %1, %1, 0" : "=a"(acc) : "v"(z));
+}
+
 // x *= c for values that live in accumulation registers, without the register allocator moving
 // them into the VGPR class.  Eight at a time: eight independent read / multiply / write chains in flight.
 __device__ __forceinline__ void scale_acc8(float& x0, float& x1, float& x2, float& x3, float& x4, float& x5, float& x6,
@@ -296,6 +303,27 @@ __device__ __forceinline__ void lds_dma_16(const char* base_uniform, uint32_t vo
                  "s"(base), "n"(LDS_IMM)
                  : "memory", "scc");
   }
+}
+
+// G direct-to-LDS loads, block i from b0 + i (step + BLK) + voff to lds + LDS_OFF + i BLK, from one setting of M0: the
+// instruction's immediate offset moves the LDS address and, compensated in the scalar bases, the memory address.  A wave stands still until a load is accepted
+// (64 cycles when all four waves stream).
+template <int G, int LDS_OFF, int BLK>
+__device__ __forceinline__ void lds_dma_group(uint64_t b0, uint64_t step, uint32_t voff, uint32_t lds) {
+  const uint64_t b1 = b0 + step, b2 = b1 + step, b3 = b2 + step;
+  if constexpr (G == 1)
+    asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(b0), "n"(LDS_OFF)
+                 : "memory", "scc");
+  else if constexpr (G == 2)
+    asm volatile("s_add_u32 m0, %0, %4\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\t"
+                 "global_load_lds_dwordx4 %1, %3 offset:%5" ::"s"(lds), "v"(voff), "s"(b0), "s"(b1), "n"(LDS_OFF), "n"(BLK)
+                 : "memory", "scc");
+  else
+    asm volatile("s_add_u32 m0, %0, %6\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\t"
+                 "global_load_lds_dwordx4 %1, %3 offset:%7\n\tglobal_load_lds_dwordx4 %1, %4 offset:%8\n\t"
+                 "global_load_lds_dwordx4 %1, %5 offset:%9" ::"s"(lds), "v"(voff), "s"(b0), "s"(b1), "s"(b2), "s"(b3),
+                 "n"(LDS_OFF), "n"(BLK), "n"(2 * BLK), "n"(3 * BLK)
+                 : "memory", "scc");
 }
 
 // lane l: 4 bytes from base + voff -> a dump area in LDS (64 words) that nobody reads.  What the load
