@@ -313,7 +313,7 @@ __global__ void __launch_bounds__(256) attn_mfma_kernel(const MfmaArgs args) {
   lds_char* const k1 = (lds_char*)(smem + OFF_K1);
   lds_char* const v0 = (lds_char*)(smem + OFF_V0);
   lds_char* const v1 = (lds_char*)(smem + OFF_V1);
-  const uint32_t t_last = (te - 1u) * kBlockN;
+  const uint32_t t_last = past_end_pos((te - 1u) * kBlockN, lo_min, p.t_all, p.ring_mask);
   // (in the loop only tiles behind the workgroup's first one are loaded)
   auto k_load = [&](uint32_t t0, lds_char* buf, uint32_t ln) {
     return make_tile_load<D, false, false>(kbase, kstride_b, min(t0, t_last), 0u, p.t_all, p.ring_mask, buf, wave, ln);

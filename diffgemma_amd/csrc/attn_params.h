@@ -185,6 +185,13 @@ __host__ __device__ __forceinline__ TileRows tile_rows(uint32_t t0, uint32_t lo,
   r.first = lo <= t0 ? 0u : lo - t0 < r.last ? lo - t0 : r.last;
   return r;
 }
+// Where loads issued for tiles behind a row tile's last one (at t_last) go, so that the tile loop need not branch around them:
+// the last tile again, its rows clamped at the end alone.  Where that tile begins before `lo` (it is then the only one), the
+// rows from `lo` on instead; a ring has memory for every slot, and 32 rows from an arbitrary slot could run past its end.
+__host__ __device__ __forceinline__ uint32_t past_end_pos(uint32_t t_last, uint32_t lo, uint32_t t_all, uint32_t ring_mask) {
+  const uint32_t see = lo < t_all ? lo : t_all - 1u;
+  return ring_mask == 0u && see > t_last ? see : t_last;
+}
 // whether some row of the tile may not be read
 __host__ __device__ __forceinline__ bool tile_is_edge(uint32_t t0, uint32_t lo, uint32_t t_all) {
   return t0 < lo || t0 + (uint32_t)kBlockN > t_all;

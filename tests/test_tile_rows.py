@@ -24,6 +24,11 @@ int main() {
           if (row >= t_all || (row < see && see < t0 + kBlockN)) return std::printf("t_all %u lo %u t0 %u row %u\n", t_all, lo, t0, row), 1;
           if (t0 + i >= lo && t0 + i < t_all && row != t0 + i) return std::printf("moved a visible row %u\n", t0 + i), 1;
         }
+        // loads for tiles behind t0, the last one: nothing before the first visible key where t0 is the first tile too
+        const uint32_t pos = past_end_pos(t0, lo, t_all, 0u);
+        const TileRows past = tile_rows(pos, 0u, t_all);
+        if (pos >= t_all || pos + past.last >= t_all || pos < t0 || (see < t0 + kBlockN && pos < see) || past_end_pos(t0, lo, t_all, 63u) != t0)
+          return std::printf("t_all %u lo %u t0 %u: past the end at %u\n", t_all, lo, t0, pos), 1;
         if (clamped && !tile_is_edge(t0, lo, t_all)) return std::printf("t_all %u lo %u t0 %u: no edge tile\n", t_all, lo, t0), 1;
       }
   std::puts("ok");
