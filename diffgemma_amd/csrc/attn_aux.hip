@@ -249,51 +249,65 @@ __global__ void __launch_bounds__(256) attn_merge_kernel(const AttnParams p, con
   }
 }
 
-// The same merge for at most 8 splits of f16 partial rows whose total is small (a sliding layer:
-// 6 splits x 4096 rows x 512 bytes): there the kernel is as long as one wave's chain of memory round
-// trips, not bandwidth.  So a wave asks for everything at once, the (m, l) pairs and the partial rows
-// of all splits (an absent split repeats the last one, weight zero), instead of weights first and
-// only the rows of splits that count; and the weights come from lane-to-scalar reads, every lane
-// doing the same arithmetic, instead of a dozen dependent shuffles.  The sum of the weights pairs
-// its terms as the butterfly over the lanes does, ((0+4)+(2+6))+((1+5)+(3+7)), and the rows are
-// added in the same order with the same cut, so both kernels give the same bits.
+// The same merge for at most 8 splits of f16 partial rows whose total is small: there the kernel is as long as one wave's
+// chain of memory round trips, not bandwidth.  So a wave asks for everything at once, the (m, l) pairs and the partial rows
+// of all splits, instead of weights first and then rows four at a time; and the weights come from lane-to-scalar reads, every
+// lane doing the same arithmetic, instead of a dozen dependent shuffles.  One instance per split count: with eight loads
+// whatever the count, the repeated ones filled the load path (2 or 3 splits: 0.4 to 0.7 us of a call of 20 to 30).  The sum of the weights pairs its
+// terms as the butterfly over the lanes does, ((0+4)+(2+6))+((1+5)+(3+7)), and the rows are added in the same order with the
+// same cut, so both kernels give the same bits.  (Past 8 splits fetching every row loses to skipping the ones that do
+// not count: 128 rows in 14 splits 20.4 -> 27.1 us on peaked rows.)
 constexpr uint32_t kMergeFewSplits = 8;
-__global__ void __launch_bounds__(256) attn_merge_few_kernel(const AttnParams p, const uint32_t hd) {
-  const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+struct MergeArgs {
+  AttnParams p;
+  FastDiv div_rows, div_group;   // by the rows of a KV head and by the GQA group
+  uint32_t hd;
+};
+template <uint32_t N>
+__global__ void __launch_bounds__(256) attn_merge_few_kernel(const MergeArgs args) {
+  const AttnParams& p = args.p;
+  const uint32_t hd = args.hd;
+  const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
   const uint32_t gr = blockIdx.x * 4 + wave;  // global stacked row over all KV heads
   if (gr >= p.hkv * p.rows_total) return;
-  const uint32_t kvh = gr / p.rows_total, r = gr % p.rows_total;
-  const uint32_t tok = r / p.group, qh = kvh * p.group + r % p.group;
+  const uint32_t kvh = fast_div(gr, args.div_rows), r = gr - kvh * p.rows_total;
+  const uint32_t tok = fast_div(r, args.div_group), qh = kvh * p.group + r - tok * p.group;
   const size_t split_stride = (size_t)p.hkv * p.rows_pad;
   const size_t row = (size_t)kvh * p.rows_pad + r;
-  const uint32_t n = p.n_splits;
-  const float2 ml = *(const float2*)(p.part_ml + ((size_t)min(lane, n - 1u) * split_stride + row) * 2);
+  const float2 ml = *(const float2*)(p.part_ml + ((size_t)min(lane, N - 1u) * split_stride + row) * 2);
   const bool live = lane < hd / 8;
   const uint32_t d8 = live ? lane : 0u;
   const uint16_t* const hbase = (const uint16_t*)p.part_o + row * hd;
   const size_t sstride = split_stride * hd;
-  uint4 a[kMergeFewSplits];
+  uint4 a[N];
 #pragma unroll
-  for (uint32_t u = 0; u < kMergeFewSplits; ++u) a[u] = ((const uint4*)(hbase + min(u, n - 1u) * sstride))[d8];
-  float msu[kMergeFewSplits], wlu[kMergeFewSplits];
+  for (uint32_t u = 0; u < N; ++u) a[u] = ((const uint4*)(hbase + u * sstride))[d8];
+  float msu[N], wlu[N], sum[kMergeFewSplits];
   float mx = -INFINITY;
 #pragma unroll
-  for (uint32_t u = 0; u < kMergeFewSplits; ++u) {
-    msu[u] = u < n ? __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(ml.x), (int)u)) : -INFINITY;
+  for (uint32_t u = 0; u < N; ++u) {
+    msu[u] = __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(ml.x), (int)u));
     mx = fmaxf(mx, msu[u]);
   }
 #pragma unroll
   for (uint32_t u = 0; u < kMergeFewSplits; ++u) {
-    const float lsu = u < n ? __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(ml.y), (int)u)) : 0.f;
-    wlu[u] = lsu > 0.f ? lsu * exp2f(msu[u] - mx) : 0.f;
+    sum[u] = 0.f;
+    if (u < N) {
+      const float lsu = __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(ml.y), (int)u));
+      sum[u] = wlu[u] = lsu > 0.f ? lsu * exp2f(msu[u] - mx) : 0.f;
+    }
   }
-  const float den = ((wlu[0] + wlu[4]) + (wlu[2] + wlu[6])) + ((wlu[1] + wlu[5]) + (wlu[3] + wlu[7]));
+#pragma unroll
+  for (uint32_t w = kMergeFewSplits / 2; w > 0; w >>= 1)
+#pragma unroll
+    for (uint32_t u = 0; u < w; ++u) sum[u] += sum[u + w];
+  const float den = sum[0];
   const float inv = den > 0.f ? 1.f / den : 0.f;
   float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (uint32_t u = 0; u < kMergeFewSplits; ++u) {
+  for (uint32_t u = 0; u < N; ++u) {
     const float w = wlu[u] * inv;
-    if (u < n && w >= 5.9604645e-8f) {   // the same in every lane
+    if (w >= 5.9604645e-8f) {   // the same in every lane
       const uint32_t wd[4] = {a[u].x, a[u].y, a[u].z, a[u].w};
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
@@ -303,29 +317,30 @@ __global__ void __launch_bounds__(256) attn_merge_few_kernel(const AttnParams p,
     }
   }
   const size_t ooff = ((size_t)tok * p.hq + qh) * hd;
-  if (live) {
+  if (live) {   // (16-bit partial rows: the output is bf16)
     if (p.dbg) {
       bool bad = false;
 #pragma unroll
       for (int e = 0; e < 8; ++e) bad = bad || nonfinite(acc[e]);
       if (bad) dbg_report(p.dbg, DBG_ERR_NONFINITE, DBG_KERNEL_ATTENTION, (tok << 16) | qh, d8 * 8u);
     }
-    if (p.out_dtype == DT_BF16) {
-      const bool tr = p.out_trunc != 0;
-      const wt_u32x4 pk4 = {(uint32_t)f32_to_bf16_bits(acc[0], tr) | ((uint32_t)f32_to_bf16_bits(acc[1], tr) << 16),
-                            (uint32_t)f32_to_bf16_bits(acc[2], tr) | ((uint32_t)f32_to_bf16_bits(acc[3], tr) << 16),
-                            (uint32_t)f32_to_bf16_bits(acc[4], tr) | ((uint32_t)f32_to_bf16_bits(acc[5], tr) << 16),
-                            (uint32_t)f32_to_bf16_bits(acc[6], tr) | ((uint32_t)f32_to_bf16_bits(acc[7], tr) << 16)};
-      wt_store16(wt_window_wave((const uint16_t*)p.out + ooff), d8 * 16u, pk4);
-    } else {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) store_out(p, ooff + d8 * 8 + e, acc[e]);
-    }
+    const bool tr = p.out_trunc != 0;
+    const wt_u32x4 pk4 = {(uint32_t)f32_to_bf16_bits(acc[0], tr) | ((uint32_t)f32_to_bf16_bits(acc[1], tr) << 16),
+                          (uint32_t)f32_to_bf16_bits(acc[2], tr) | ((uint32_t)f32_to_bf16_bits(acc[3], tr) << 16),
+                          (uint32_t)f32_to_bf16_bits(acc[4], tr) | ((uint32_t)f32_to_bf16_bits(acc[5], tr) << 16),
+                          (uint32_t)f32_to_bf16_bits(acc[6], tr) | ((uint32_t)f32_to_bf16_bits(acc[7], tr) << 16)};
+    wt_store16(wt_window_wave((const uint16_t*)p.out + ooff), d8 * 16u, pk4);
   }
   if (lane == 0) {
     if (!(den > 0.f)) dbg_report(p.dbg, DBG_ERR_SOFTMAX_NORM_ZERO, DBG_KERNEL_ATTENTION, (tok << 16) | qh, (tok << 16) | qh);
     if (p.lse) p.lse[(size_t)tok * p.hq + qh] = den > 0.f ? mx * kLn2 + logf(den) : -INFINITY;
   }
+}
+
+template <uint32_t N>
+hipError_t launch_merge_few(const MergeArgs& a, uint32_t rows, hipStream_t s) {
+  hipLaunchKernelGGL((attn_merge_few_kernel<N>), dim3((rows + 3) / 4), dim3(256), 0, s, a);
+  return hipGetLastError();
 }
 
 __device__ __forceinline__ float load_any(const void* src, uint32_t dt, size_t i) {
@@ -564,12 +579,26 @@ hipError_t launch_state_merge(const StateMergeParams& p, hipStream_t s) {
 
 hipError_t launch_attn_merge(const AttnParams& p, uint32_t head_dim, bool streamed, hipStream_t s) {
   const uint32_t rows = p.hkv * p.rows_total;
-  // a few splits of a small workspace: the variant that asks for every partial row up front
+  // not many splits, not many bytes: the variant that asks for every partial row up front
   const size_t part_bytes = (size_t)p.n_splits * p.hkv * p.rows_pad * head_dim * 2;
-  if (!streamed && p.part_half && p.n_splits <= kMergeFewSplits && head_dim % 8 == 0 && head_dim <= 512 && part_bytes < ((size_t)32 << 20))
-    hipLaunchKernelGGL(attn_merge_few_kernel, dim3((rows + 3) / 4), dim3(256), 0, s, p, head_dim);
-  else
-    hipLaunchKernelGGL(attn_merge_kernel, dim3((rows + 3) / 4), dim3(256), 0, s, p, head_dim);
+  if (!streamed && p.part_half && p.n_splits <= kMergeFewSplits && head_dim % 8 == 0 && head_dim <= 512 && part_bytes < ((size_t)32 << 20)) {
+    MergeArgs a;
+    a.p = p;
+    a.div_rows = make_fast_div(p.rows_total);
+    a.div_group = make_fast_div(p.group);
+    a.hd = head_dim;
+    switch (p.n_splits) {
+      case 2: return launch_merge_few<2>(a, rows, s);
+      case 3: return launch_merge_few<3>(a, rows, s);
+      case 4: return launch_merge_few<4>(a, rows, s);
+      case 5: return launch_merge_few<5>(a, rows, s);
+      case 6: return launch_merge_few<6>(a, rows, s);
+      case 7: return launch_merge_few<7>(a, rows, s);
+      case 8: return launch_merge_few<8>(a, rows, s);
+      default: break;
+    }
+  }
+  hipLaunchKernelGGL(attn_merge_kernel, dim3((rows + 3) / 4), dim3(256), 0, s, p, head_dim);
   return hipGetLastError();
 }
 
