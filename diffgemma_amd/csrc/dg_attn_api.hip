@@ -143,7 +143,32 @@ struct Plan {
   float scale = 1.0f;
 };
 
-int make_plan(const dg_attn_desc* d, int cus, Plan* pl, const uint32_t* key_range = nullptr) {
+// Key tiles per split of the split kernel where the library chooses.  `base` = workgroups of one split, `room` = splits that
+// keep it one round of the chip.
+//
+// head_dim 512: a tile takes c = 1.3 to 1.6 us, and a split costs what its partial rows cost, written and read back, about
+// m = 0.12 us per 16 row tiles and key range, i.e. 9 c m / room for `base` of them: c n / s + m' s is least at
+// s = sqrt(n room / 9).  The curve is flat around it.  Attention call, us, splits of 6 tiles and more | this rule:
+// 64 rows (room 32) over 86 keys 14.6 | 13.3, over 364 20.0 | 15.5, 841 21.0 | 18.1, 2064 23.7 | 22.6, 5064 29.2 | 29.2; 128 rows
+// (16) over 428 keys 21.7 | 18.6, 905 23.8 | 22.9, 2128 29.0 | 30.1; 256 rows (8) over 278 22.2 | 20.5, 356 23.3 | 21.9,
+// 556 24.4 | 24.5, 1033 26.7 | 27.0; 300 causal rows (6) 22.8 | 19.4.
+//
+// Smaller head_dim: no split shorter than 6 tiles (a sliding layer's 40 tiles, step in us: 4 splits 25.7, 5 splits 24.8,
+// 6 and 7 splits 23.7, 8 splits 24.5, 10 splits 33.4).
+uint32_t tiles_of_split(uint32_t ntiles, uint32_t room, uint32_t hd, bool long_splits) {
+  room = std::max(1u, std::min(room, kMaxSplits));
+  if (hd != 512 || long_splits) {
+    const uint32_t s = std::min(room, std::max(1u, ntiles / 6u));
+    return (ntiles + s - 1) / s;
+  }
+  const double s = std::sqrt((double)ntiles * room / 9.0);
+  const uint32_t t = std::max(1u, (uint32_t)(ntiles / s + 0.5));
+  return std::max(t, (ntiles + room - 1) / room);
+}
+
+// Scratch a split count takes, and the count for a call that has `scratch` bytes of it: what the rule asks for, or, where
+// that is more, splits of at least 6 tiles (a caller may hold what an earlier library asked for).
+int make_plan(const dg_attn_desc* d, int cus, Plan* pl, const uint32_t* key_range = nullptr, size_t scratch = SIZE_MAX) {
   if (!d) return DG_ERR_NULL;
   pl->cus = (uint32_t)cus;
   const uint32_t hd = d->head_dim;
@@ -249,42 +274,40 @@ int make_plan(const dg_attn_desc* d, int cus, Plan* pl, const uint32_t* key_rang
     pl->wsplit = !pl->scalar && hd <= 256 && d->n_splits == 0 && !(d->flags & DG_ATTN_F_SPLIT_OVER_WORKGROUPS) &&
                  span_tiles <= kWsplitMaxTiles;
   }
-  uint32_t splits = d->n_splits;
+  const uint32_t room = (uint32_t)cus / std::max(1u, d->n_kv_heads * pl->n_mtiles);
+  // workspace carve-up, with splits of `tps` key tiles
+  auto carve = [&](uint32_t tps) {
+    pl->tiles_per_split = tps;
+    pl->n_splits = (ntiles + tps - 1) / tps;
+    size_t off = 0;
+    if (pl->convert_q) {
+      pl->off_q = off;
+      off += align_up((size_t)d->canvas * d->n_q_heads * hd * 2);
+    }
+    if (pl->gather_kv) {
+      pl->off_kv = off;
+      off += align_up((size_t)2 * d->n_kv_heads * pl->t_all * hd * 2);
+    }
+    // f16 partial rows need |V| <= 65504: an f16 cache guarantees it, for a bf16 cache the caller says so
+    pl->part_half = pl->n_splits > 1 && d->out_dtype != DG_F32 && !(d->flags & DG_ATTN_F_F32_PARTIALS) &&
+                    (pl->e_dtype == DG_F16 || (d->flags & DG_ATTN_F_F16_PARTIALS));
+    if (pl->n_splits > 1) {
+      pl->off_part_o = off;
+      off += align_up((size_t)pl->n_splits * d->n_kv_heads * pl->rows_pad * hd * (pl->part_half ? 2 : 4));
+      pl->off_part_ml = off;
+      off += align_up((size_t)pl->n_splits * d->n_kv_heads * pl->rows_pad * 2 * 4);
+    }
+    pl->total = off;
+  };
   if (pl->scalar || pl->wsplit) {
-    splits = 1;
-  } else if (splits == 0) {
-    // enough workgroups for every CU, but no split shorter than 6 tiles: below that the partial
-    // rows a split writes (and the merge reads back) cost more than the idle CUs do (a sliding
-    // layer's 40 tiles, step in us: 4 splits 25.7, 5 splits 24.8, 6 and 7 splits 23.7, 8 splits 24.5,
-    // 10 splits 33.4)
-    const uint32_t base = d->n_kv_heads * pl->n_mtiles;
-    splits = std::max(1u, (uint32_t)cus / std::max(1u, base));
-    splits = std::min(splits, std::max(1u, ntiles / 6u));
+    carve(ntiles);
+  } else if (d->n_splits != 0) {
+    const uint32_t splits = std::min(std::min(d->n_splits, kMaxSplits), ntiles);
+    carve((ntiles + splits - 1) / splits);
+  } else {
+    carve(tiles_of_split(ntiles, room, hd, false));
+    if (pl->total > scratch) carve(tiles_of_split(ntiles, room, hd, true));
   }
-  splits = std::min(std::min(splits, kMaxSplits), ntiles);
-  pl->tiles_per_split = (ntiles + splits - 1) / splits;
-  pl->n_splits = (ntiles + pl->tiles_per_split - 1) / pl->tiles_per_split;
-
-  // workspace carve-up
-  size_t off = 0;
-  if (pl->convert_q) {
-    pl->off_q = off;
-    off += align_up((size_t)d->canvas * d->n_q_heads * hd * 2);
-  }
-  if (pl->gather_kv) {
-    pl->off_kv = off;
-    off += align_up((size_t)2 * d->n_kv_heads * pl->t_all * hd * 2);
-  }
-  // f16 partial rows need |V| <= 65504: an f16 cache guarantees it, for a bf16 cache the caller says so
-  pl->part_half = pl->n_splits > 1 && d->out_dtype != DG_F32 && !(d->flags & DG_ATTN_F_F32_PARTIALS) &&
-                  (pl->e_dtype == DG_F16 || (d->flags & DG_ATTN_F_F16_PARTIALS));
-  if (pl->n_splits > 1) {
-    pl->off_part_o = off;
-    off += align_up((size_t)pl->n_splits * d->n_kv_heads * pl->rows_pad * hd * (pl->part_half ? 2 : 4));
-    pl->off_part_ml = off;
-    off += align_up((size_t)pl->n_splits * d->n_kv_heads * pl->rows_pad * 2 * 4);
-  }
-  pl->total = off;
   return DG_OK;
 }
 
@@ -505,7 +528,7 @@ int dg_attn_forward(const dg_attn_desc* d, const void* q, const void* kv_base, v
   int rc = device_info(&di);
   if (rc != DG_OK) return rc;
   Plan pl;
-  rc = make_plan(d, di.cus, &pl);
+  rc = make_plan(d, di.cus, &pl, nullptr, workspace ? workspace_bytes : 0);
   if (rc != DG_OK) return rc;
   return forward_planned(d, pl, q, kv_base, out, lse, workspace, workspace_bytes, stream);
 }
@@ -518,7 +541,7 @@ int dg_attn_forward_dev(const dg_attn_desc* d, const dg_step_params* step_dev, c
   int rc = device_info(&di);
   if (rc != DG_OK) return rc;
   Plan pl;
-  rc = make_plan(d, di.cus, &pl);
+  rc = make_plan(d, di.cus, &pl, nullptr, workspace ? workspace_bytes : 0);
   if (rc != DG_OK) return rc;
   return forward_planned(d, pl, q, kv_base, out, lse, workspace, workspace_bytes, stream, (const uint32_t*)step_dev);
 }
@@ -532,7 +555,7 @@ int dg_attn_forward_static(const dg_attn_desc* d, const void* q, const void* kv_
   int rc = device_info(&di);
   if (rc != DG_OK) return rc;
   Plan pl;
-  rc = make_plan(d, di.cus, &pl);
+  rc = make_plan(d, di.cus, &pl, nullptr, kStaticScratchBytes);
   if (rc != DG_OK) return rc;
   if (pl.total > kStaticScratchBytes) return DG_ERR_SCRATCH_LIMIT;
   void* ptr = nullptr;
@@ -588,7 +611,7 @@ int dg_attn_partial(const dg_attn_desc* d, uint32_t t_begin, uint32_t t_end, con
   const dg_attn_desc pd = partial_desc(d);
   const uint32_t range[2] = {t_begin, t_end};
   Plan pl;
-  rc = make_plan(&pd, di.cus, &pl, range);
+  rc = make_plan(&pd, di.cus, &pl, range, workspace ? workspace_bytes : 0);
   if (rc != DG_OK) return rc;
   if (state_bytes < state_bytes_of(d) || ((uintptr_t)state % 16) != 0) return DG_ERR_WORKSPACE;
   // The attention kernels leave the row normalised (acc / l) and its log-sum-exp: the state's normal
@@ -937,24 +960,26 @@ int dg_attention_block_state_bytes(const dg_layer_offsets* L, const dg_attn_dims
   size_t ws_full = 0;
   int rc = dg_attn_workspace_bytes(&d, &ws_full);
   if (rc != DG_OK) return rc;
-  // The partial of a block [a, b) is split over workgroups like a whole call, and the number of splits a
-  // range resolves to is not monotone in its length (ceil(n / ceil(n / s)) jumps up and down with n), so a
-  // shorter range can take more splits than the whole one.  What bounds every range is the cap the split
-  // count is cut to before that rounding; the partial workspace is sized for it, with fp32 partial rows
-  // (a partial's result is fp32 accumulators).
+  // The partial of a block [a, b) is split over workgroups like a whole call, and the number of splits a range resolves to
+  // is not monotone in its length (ceil(n / ceil(n / s)) jumps up and down with n), so a shorter range can take more splits
+  // than the whole one.  The partial workspace is sized for the most any range takes, with fp32 partial rows (a partial's
+  // result is fp32 accumulators).  (`room` is reached within a few thousand tiles.)
   const dg_attn_desc pd = partial_desc(&d);
   Plan pl;
   const int cus = plan_cus();
   rc = make_plan(&pd, cus, &pl);
   if (rc != DG_OK) return rc;
   const uint32_t ntiles_full = std::max(1u, (pl.t_all + dg::kBlockN - 1) / dg::kBlockN);
-  const uint32_t base = d.n_kv_heads * pl.n_mtiles;
-  const uint32_t cap = std::min(std::min(std::max(1u, (uint32_t)cus / std::max(1u, base)), std::max(1u, ntiles_full / 6u)),
-                                kMaxSplits);
+  const uint32_t room = (uint32_t)cus / std::max(1u, d.n_kv_heads * pl.n_mtiles);
+  uint32_t most = 1;
+  for (uint32_t n = 1; n <= ntiles_full && most < std::min(room, kMaxSplits); ++n) {
+    const uint32_t t = tiles_of_split(n, room, d.head_dim, false);
+    most = std::max(most, (n + t - 1) / t);
+  }
   size_t ws_part = 0;
-  if (cap > 1)
-    ws_part = align_up((size_t)cap * d.n_kv_heads * pl.rows_pad * d.head_dim * 4) +
-              align_up((size_t)cap * d.n_kv_heads * pl.rows_pad * 2 * 4);
+  if (most > 1)
+    ws_part = align_up((size_t)most * d.n_kv_heads * pl.rows_pad * d.head_dim * 4) +
+              align_up((size_t)most * d.n_kv_heads * pl.rows_pad * 2 * 4);
   *out_bytes = 2 * align_up(state_bytes_of(&d)) + std::max(ws_full, ws_part);
   return DG_OK;
 }
