@@ -1302,7 +1302,9 @@ hipError_t launch_filter(const TopkParams& tp, const TopkParams& sample, hipStre
   const uint32_t rows = tp.ntok * tp.a.hq;
   const dim3 by_wave((rows + 3u) / 4u);
   const uint32_t m = sample.a.t_all;
-  if (m <= 64u * 32u) hipLaunchKernelGGL((topk_tau_kernel<32>), by_wave, dim3(256), 0, s, tp);
+  if (m <= 64u * 8u) hipLaunchKernelGGL((topk_tau_kernel<8>), by_wave, dim3(256), 0, s, tp);
+  else if (m <= 64u * 16u) hipLaunchKernelGGL((topk_tau_kernel<16>), by_wave, dim3(256), 0, s, tp);
+  else if (m <= 64u * 32u) hipLaunchKernelGGL((topk_tau_kernel<32>), by_wave, dim3(256), 0, s, tp);
   else if (m <= 64u * 64u) hipLaunchKernelGGL((topk_tau_kernel<64>), by_wave, dim3(256), 0, s, tp);
   else hipLaunchKernelGGL((topk_tau_kernel<128>), by_wave, dim3(256), 0, s, tp);
   if ((rc = hipGetLastError()) != hipSuccess) return rc;
