@@ -881,7 +881,7 @@ int dg_attn_topk_forward(const dg_attn_desc* d, const uint32_t* k_cfg, const voi
       sp.tile_first = 0u;
       sp.tile_end = tk.sample_pad / dg::kBlockN;
       const uint32_t base = d->n_kv_heads * sp.n_mtiles;
-      sp.n_splits = std::max(1u, std::min(((uint32_t)di.cus + base - 1u) / base, sp.tile_end / 4u));
+      sp.n_splits = std::max(1u, std::min(((uint32_t)di.cus + base - 1u) / base, sp.tile_end / 2u));
       mark(0);
       if (dg::launch_topk_filter(fp, sp, pl.e_dtype, s) != hipSuccess) return DG_ERR_LAUNCH;
       mark(1);
