@@ -51,6 +51,21 @@ struct AttnParams {
   float scale_log2;      // softmax_scale * log2(e)
 };
 
+// Division of n < 2^31 by a divisor the host knows: q = (mulhi(n, mul) + n) >> shift (the round-up method: mul =
+// floor(2^32 (2^shift - d) / d) + 1 with shift = ceil(log2 d)).  Three scalar instructions where a run-time division is
+// two dozen on the vector unit.
+struct FastDiv {
+  uint32_t mul, shift;
+};
+inline FastDiv make_fast_div(uint32_t d) {
+  uint32_t shift = 0;
+  while ((1ull << shift) < d) ++shift;
+  return FastDiv{(uint32_t)((((1ull << shift) - d) << 32) / d + 1u), shift};
+}
+__host__ __device__ __forceinline__ uint32_t fast_div(uint32_t n, FastDiv d) {
+  return ((uint32_t)(((uint64_t)n * d.mul) >> 32) + n) >> d.shift;
+}
+
 // One pass of top-k sparse attention over canvas rows [tok0, tok0 + ntok).
 constexpr int kTopkMaxK = 1024;   // most keys a row may keep
 struct TopkParams {
@@ -75,6 +90,7 @@ struct TopkParams {
   uint32_t* fail_rows;   // [canvas][hq]: rows the filtered path has left over (null: every row takes the general path)
   uint32_t* fail_block;  // rows left over per block of canvas rows (general path: of this block)
   uint32_t fail_block_tok;   // canvas rows per block
+  FastDiv div_mtiles, div_splits, div_group, div_rows;   // by n_mtiles, n_splits, the GQA group, ntok * group (set at the launch)
 };
 // A segment holds the candidates that one lane finds for one query row: half of the row's in a key-range split.  The spare
 // places behind the limit take what one more key tile may bring before the count is looked at.
@@ -124,21 +140,6 @@ __device__ __forceinline__ AttnParams resolve_step(const AttnParams& in) {
   p.tile_first = lo_all / (uint32_t)kBlockN;
   p.tile_end = max(p.tile_first, (p.t_all + (uint32_t)kBlockN - 1u) / (uint32_t)kBlockN);
   return p;
-}
-
-// Division of n < 2^31 by a divisor the host knows: q = (mulhi(n, mul) + n) >> shift (the round-up method: mul =
-// floor(2^32 (2^shift - d) / d) + 1 with shift = ceil(log2 d)).  Three scalar instructions where a run-time division is
-// two dozen on the vector unit.
-struct FastDiv {
-  uint32_t mul, shift;
-};
-inline FastDiv make_fast_div(uint32_t d) {
-  uint32_t shift = 0;
-  while ((1ull << shift) < d) ++shift;
-  return FastDiv{(uint32_t)((((1ull << shift) - d) << 32) / d + 1u), shift};
-}
-__host__ __device__ __forceinline__ uint32_t fast_div(uint32_t n, FastDiv d) {
-  return ((uint32_t)(((uint64_t)n * d.mul) >> 32) + n) >> d.shift;
 }
 
 struct RowBounds {

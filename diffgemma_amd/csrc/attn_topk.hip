@@ -63,10 +63,8 @@ __global__ void __launch_bounds__(256) topk_scores_kernel(const TopkParams tp) {
   const uint32_t wg = blockIdx.x;
   const uint32_t unit = (wg & 7u) * per_xcd + (wg >> 3);
   if (unit >= n_units) return;
-  const uint32_t stream = __builtin_amdgcn_readfirstlane(unit / tp.n_mtiles);
-  const uint32_t mt = __builtin_amdgcn_readfirstlane(unit % tp.n_mtiles);
-  const uint32_t kvh = __builtin_amdgcn_readfirstlane(stream / tp.n_splits);
-  const uint32_t split = __builtin_amdgcn_readfirstlane(stream % tp.n_splits);
+  const uint32_t stream = fast_div(unit, tp.div_mtiles), mt = unit - stream * tp.n_mtiles;
+  const uint32_t kvh = fast_div(stream, tp.div_splits), split = stream - kvh * tp.n_splits;
 
   const uint32_t lane = threadIdx.x & 63u;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -76,15 +74,15 @@ __global__ void __launch_bounds__(256) topk_scores_kernel(const TopkParams tp) {
   const uint32_t row0 = mt * kBlockM;
   const uint32_t r = row0 + wave * 32u + l32;
   const bool row_ok = r < rows_total;
-  const uint32_t tok_l = row_ok ? r / p.group : 0u;           // row within this pass
+  const uint32_t tok_l = row_ok ? fast_div(r, tp.div_group) : 0u;           // row within this pass
   const uint32_t tok = tp.tok0 + tok_l;
-  const uint32_t qh = kvh * p.group + (row_ok ? r % p.group : 0u);
+  const uint32_t qh = kvh * p.group + (row_ok ? r - tok_l * p.group : 0u);
 
   // key tiles some row of this row tile can see
   uint32_t lo_min, hi_max;
   {
     const uint32_t last_row = min(row0 + kBlockM, rows_total) - 1u;
-    const uint32_t tok_a = tp.tok0 + row0 / p.group, tok_b = tp.tok0 + last_row / p.group;
+    const uint32_t tok_a = tp.tok0 + fast_div(row0, tp.div_group), tok_b = tp.tok0 + fast_div(last_row, tp.div_group);
     const RowBounds ba = row_bounds(p, tok_a), bb = row_bounds(p, tok_b);
     lo_min = min(ba.lo, bb.lo);
     hi_max = max(ba.hi, bb.hi);
@@ -106,21 +104,30 @@ __global__ void __launch_bounds__(256) topk_scores_kernel(const TopkParams tp) {
 
   // Q fragments: lane = row, 8 consecutive d per step
   u32x4 qf[NSTEP];
-  {
+  const bool convert = F16 && p.q_is_bf16;
+  auto to_frag = [&](u32x4 raw) -> u32x4 {
+    if (convert) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        raw[e] = pack2<true>(__uint_as_float(raw[e] << 16), __uint_as_float(raw[e] & 0xffff0000u));
+    }
+    return raw;
+  };
+  if constexpr (D == 512) {   // through the K buffers' LDS
+    static_assert(4 * 32 * kQRowLds <= NB * L::K_BYTES, "the tile buffers hold the query rows");
+    lds_char* const qb = (lds_char*)smem + wave * (32u * kQRowLds);
+    issue_q_rows((const char*)p.q + ((size_t)tp.tok0 * p.hq + kvh * p.group) * (2 * D), row0 + wave * 32u, rows_total, p.group,
+                 (uint32_t)(size_t)qb, lane,
+                 [&](uint32_t rq) { return (rq + fast_div(rq, tp.div_group) * (p.hq - p.group)) * (uint32_t)(2 * D); });
+    wait_vmem_all();
+#pragma unroll
+    for (int st = 0; st < NSTEP; ++st) qf[st] = to_frag(*(lds_u32x4*)(qb + l32 * kQRowLds + g2 * 16u + 32 * st));
+    __syncthreads();   // the first tiles may take the rows' place
+  } else {
     const size_t qoff = ((size_t)tok * p.hq + qh) * D + 8u * g2;
     const uint16_t* qp = (const uint16_t*)p.q + qoff;
-    if (F16 && p.q_is_bf16) {
 #pragma unroll
-      for (int s = 0; s < NSTEP; ++s) {
-        u32x4 raw = row_ok ? *(const u32x4*)(qp + 16 * s) : u32x4{0, 0, 0, 0};
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          qf[s][e] = pack2<true>(__uint_as_float(raw[e] << 16), __uint_as_float(raw[e] & 0xffff0000u));
-      }
-    } else {
-#pragma unroll
-      for (int s = 0; s < NSTEP; ++s) qf[s] = row_ok ? *(const u32x4*)(qp + 16 * s) : u32x4{0, 0, 0, 0};
-    }
+    for (int st = 0; st < NSTEP; ++st) qf[st] = to_frag(row_ok ? *(const u32x4*)(qp + 16 * st) : u32x4{0, 0, 0, 0});
   }
 
   const char* kbase = (const char*)p.k + (int64_t)kvh * p.k_head_stride * 2;
@@ -148,8 +155,8 @@ __global__ void __launch_bounds__(256) topk_scores_kernel(const TopkParams tp) {
   for (int e = 0; e < 16; ++e) {
     const uint32_t rr = row0 + wave * 32u + 8u * (e >> 2) + 4u * g2 + (e & 3);
     const bool ok = rr < rows_total;
-    const uint32_t tl = ok ? rr / p.group : 0u;
-    const uint32_t hh = kvh * p.group + (ok ? rr % p.group : 0u);
+    const uint32_t tl = ok ? fast_div(rr, tp.div_group) : 0u;
+    const uint32_t hh = kvh * p.group + (ok ? rr - tl * p.group : 0u);
     row_off[e] = ((hh * tp.ntok + tl) * tp.t_pad + l32) * 4u;
     row_mask |= ok ? 1u << e : 0u;
   }
@@ -797,8 +804,8 @@ __global__ void __launch_bounds__(256) topk_tau_kernel(const TopkParams tp) {
   const uint32_t rid = __builtin_amdgcn_readfirstlane(blockIdx.x * 4u + (threadIdx.x >> 6));
   if (rid >= tp.ntok * p.hq) return;
   const uint32_t rows = tp.ntok * p.group;
-  const uint32_t kvh = rid / rows, rr = rid % rows;
-  const uint32_t tok_l = rr / p.group, qh = kvh * p.group + rr % p.group;
+  const uint32_t kvh = fast_div(rid, tp.div_rows), rr = rid - kvh * rows;
+  const uint32_t tok_l = fast_div(rr, tp.div_group), qh = kvh * p.group + rr - tok_l * p.group;
   const uint32_t tok = tp.tok0 + tok_l;
   if (qh == 0u && tok_l % tp.fail_block_tok == 0u && lane == 0u) tp.fail_block[tok_l / tp.fail_block_tok] = 0u;
   const RowBounds rb = row_bounds(p, tok);
@@ -858,16 +865,15 @@ __global__ void __launch_bounds__(256) topk_filter_kernel(const TopkParams tp) {
   const uint32_t unit = (blockIdx.x & 7u) * per_xcd + (blockIdx.x >> 3);
   if (unit >= n_units) return;
   // row tiles of one (KV head, split) next to each other: they read the same keys through one L2
-  const uint32_t mt = __builtin_amdgcn_readfirstlane(unit % tp.n_mtiles);
-  const uint32_t kvh = __builtin_amdgcn_readfirstlane(unit / tp.n_mtiles / tp.n_splits);
-  const uint32_t split = __builtin_amdgcn_readfirstlane(unit / tp.n_mtiles % tp.n_splits);
+  const uint32_t stream = fast_div(unit, tp.div_mtiles), mt = unit - stream * tp.n_mtiles;
+  const uint32_t kvh = fast_div(stream, tp.div_splits), split = stream - kvh * tp.n_splits;
   const uint32_t lane = threadIdx.x & 63u;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t g2 = lane >> 5, l32 = lane & 31u;
   const uint32_t rows_total = tp.ntok * p.group;
   const uint32_t row0 = mt * kTopkFilterRows + wave * 64u;
   const uint32_t n_tiles_all = (p.t_all + kBlockN - 1u) / kBlockN;
-  const uint32_t n_tiles = split < n_tiles_all ? (n_tiles_all - split + tp.n_splits - 1u) / tp.n_splits : 0u;
+  const uint32_t n_tiles = split < n_tiles_all ? fast_div(n_tiles_all - split + tp.n_splits - 1u, tp.div_splits) : 0u;
   const uint32_t seg = (((kvh * tp.n_mtiles + mt) * tp.n_splits + split) * 4u + wave) * kTopkSegs;   // this wave's first segment
   if (n_tiles == 0u) {
     tp.cand_n[seg + lane] = tp.cand_n[seg + 64u + lane] = 0u;
@@ -883,27 +889,35 @@ __global__ void __launch_bounds__(256) topk_filter_kernel(const TopkParams tp) {
     return make_tile_load<D, false, false>(kbase, kstride_b, tile_t0(i), 0u, p.t_all, 0u,
                                            (lds_char*)(smem + (i % NB) * L::K_BYTES), wave, lane);
   };
+  // Query rows through the K buffers' LDS, a block of 32 at a time, into accumulation registers.
+  u32x4 qf[2][NSTEP];
+  {
+    static_assert(4 * 32 * kQRowLds <= NB * L::K_BYTES, "the tile buffers hold a block of every wave's query rows");
+    lds_char* const qb = (lds_char*)smem + wave * (32u * kQRowLds);
+    const char* const q_base = (const char*)p.q + ((size_t)tp.tok0 * p.hq + kvh * p.group) * (2 * D);
+    const bool convert = F16 && p.q_is_bf16;
+    static_for<0, 2>([&](auto b_c) {
+      constexpr int b = decltype(b_c)::value;
+      issue_q_rows(q_base, row0 + 32u * b, rows_total, p.group, (uint32_t)(size_t)qb, lane,
+                   [&](uint32_t rq) { return (rq + fast_div(rq, tp.div_group) * (p.hq - p.group)) * (uint32_t)(2 * D); });
+      wait_vmem_all();
+      static_for<0, NSTEP>([&](auto st_c) {
+        constexpr int st = decltype(st_c)::value;
+        u32x4 raw = *(lds_u32x4*)(qb + l32 * kQRowLds + g2 * 16u + 32 * st);
+        if (convert) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            raw[e] = pack2<true>(__uint_as_float(raw[e] << 16), __uint_as_float(raw[e] & 0xffff0000u));
+        }
+        qf[b][st] = raw;
+        asm volatile("" : "+a"(qf[b][st]));
+      });
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (read before the next rows land there)
+    });
+  }
+  __syncthreads();
 #pragma unroll
   for (int i = 0; i < PF; ++i) issue_tile<D, false>(k_desc((uint32_t)i), wave, lane);
-
-  u32x4 qf[2][NSTEP];
-#pragma unroll
-  for (int b = 0; b < 2; ++b) {
-    const uint32_t r = min(row0 + 32u * b + l32, rows_total - 1u);   // (rows past the last copy it: tau is +inf there)
-    const uint32_t tok = tp.tok0 + r / p.group, qh = kvh * p.group + r % p.group;
-    const uint16_t* qp = (const uint16_t*)p.q + ((size_t)tok * p.hq + qh) * D + 8u * g2;
-#pragma unroll
-    for (int s = 0; s < NSTEP; ++s) {
-      u32x4 raw = *(const u32x4*)(qp + 16 * s);
-      if (F16 && p.q_is_bf16) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          raw[e] = pack2<true>(__uint_as_float(raw[e] << 16), __uint_as_float(raw[e] & 0xffff0000u));
-      }
-      qf[b][s] = raw;
-      asm volatile("" : "+a"(qf[b][s]));
-    }
-  }
   // S = K.Q^T: the lane is a query row of the block, register e is key 8 (e >> 2) + 4 g2 + (e & 3) of the tile.  Each lane
   // keeps lists of its own, one per block, so an entry's place is the lane's count and nothing is exchanged.
   float tau[2];
@@ -988,7 +1002,7 @@ __global__ void __launch_bounds__(256) topk_filter_kernel(const TopkParams tp) {
       });
     });
   };
-  wait_vmem_all();      // the query rows and with them the first PF tiles
+  wait_vmem_all();      // the first PF tiles
   __builtin_amdgcn_s_waitcnt(0xC07F);     // (lgkmcnt(0): or scalar loads in flight here make the compiler wait for whole chunks below)
   f32x16 sa[2], sb[2];
 #pragma unroll
@@ -1029,8 +1043,8 @@ __global__ void __launch_bounds__(256, NR <= 20 ? 4 : NR == 24 ? 3 : 2) topk_lis
   const uint32_t rid = wg * 4u + wave;
   if (rid >= n_rows) return;
   const uint32_t rows = tp.ntok * p.group;
-  const uint32_t kvh = rid / rows, rr = rid % rows;
-  const uint32_t tok_l = rr / p.group, qh = kvh * p.group + rr % p.group;
+  const uint32_t kvh = fast_div(rid, tp.div_rows), rr = rid - kvh * rows;
+  const uint32_t tok_l = fast_div(rr, tp.div_group), qh = kvh * p.group + rr - tok_l * p.group;
   const uint32_t tok = tp.tok0 + tok_l;
   const RowBounds rb = row_bounds(p, tok);
   const uint32_t k = row_k(tp, tok, visible_count(rb, p.t_all));
@@ -1222,8 +1236,8 @@ __global__ void __launch_bounds__(256) topk_gather_kernel(const TopkParams tp) {
   const uint32_t rid = __builtin_amdgcn_readfirstlane(wg * 4u + (threadIdx.x >> 6));
   if (rid >= n_rows) return;
   const uint32_t rows = tp.ntok * p.group;
-  const uint32_t kvh = rid / rows, rr = rid % rows;
-  const uint32_t tok = tp.tok0 + rr / p.group, qh = kvh * p.group + rr % p.group;
+  const uint32_t kvh = fast_div(rid, tp.div_rows), rr = rid - kvh * rows;
+  const uint32_t tok_l = fast_div(rr, tp.div_group), tok = tp.tok0 + tok_l, qh = kvh * p.group + rr - tok_l * p.group;
   if (tp.fail_rows[(size_t)tok * p.hq + qh] != 0u) return;       // (the general path's)
   const uint32_t k = row_k(tp, tok, visible_count(row_bounds(p, tok), p.t_all));
   const u32x2* const kept = (const u32x2*)tp.kept + (size_t)rid * tp.kept_pad;
@@ -1271,8 +1285,16 @@ __global__ void __launch_bounds__(256) topk_gather_kernel(const TopkParams tp) {
   }
 }
 
+void set_dividers(TopkParams* tp) {
+  tp->div_mtiles = make_fast_div(tp->n_mtiles);
+  tp->div_splits = make_fast_div(tp->n_splits);
+  tp->div_group = make_fast_div(tp->a.group);
+  tp->div_rows = make_fast_div(tp->ntok * tp->a.group);
+}
+
 template <int D, bool F16>
-hipError_t launch_stage(const TopkParams& tp, int stage, hipStream_t s) {
+hipError_t launch_stage(TopkParams tp, int stage, hipStream_t s) {
+  set_dividers(&tp);
   if (stage == 0) {
     const uint32_t n_units = tp.a.hkv * tp.n_splits * tp.n_mtiles;
     const uint32_t grid = ((n_units + 7u) / 8u) * 8u;
@@ -1296,7 +1318,8 @@ hipError_t launch_by_dim(const TopkParams& tp, int stage, uint32_t head_dim, hip
 }
 
 template <bool F16>
-hipError_t launch_filter(const TopkParams& tp, const TopkParams& sample, hipStream_t s) {
+hipError_t launch_filter(TopkParams tp, const TopkParams& sample, hipStream_t s) {
+  set_dividers(&tp);
   hipError_t rc = launch_stage<512, F16>(sample, 0, s);
   if (rc != hipSuccess) return rc;
   const uint32_t rows = tp.ntok * tp.a.hq;
@@ -1313,7 +1336,8 @@ hipError_t launch_filter(const TopkParams& tp, const TopkParams& sample, hipStre
   return hipGetLastError();
 }
 template <bool F16>
-hipError_t launch_list_select(const TopkParams& tp, uint32_t k_most, hipStream_t s) {
+hipError_t launch_list_select(TopkParams tp, uint32_t k_most, hipStream_t s) {
+  set_dividers(&tp);
   const dim3 sel((tp.ntok * tp.a.hq + 31u) / 32u * 8u);
   if (k_most <= 160u) hipLaunchKernelGGL((topk_list_select_kernel<16>), sel, dim3(256), 0, s, tp);
   else if (k_most <= 272u) hipLaunchKernelGGL((topk_list_select_kernel<20>), sel, dim3(256), 0, s, tp);

@@ -326,6 +326,31 @@ __device__ __forceinline__ void lds_dma_group(uint64_t b0, uint64_t step, uint32
                  : "memory", "scc");
 }
 
+// 32 stacked query rows of 1 KiB (head_dim 512) by one wave, rows `first` .. first + 31 of a KV head (`first` a multiple of 8),
+// 16 bytes apart at `lds`: fragments are read like K fragments.  `row_off` gives a row's byte offset from q_base, the same
+// in every lane.  Where the GQA group is a multiple of eight, eight rows lie next to each other.  Rows past the last one
+// are copies of it, or of its token's.  (The operand layout gives a lane 16 bytes of its own row per step: loaded straight
+// from memory, 64 rows a wave took 9 us of the top-k filter kernel.)
+constexpr uint32_t kQRowLds = 1024 + 16;
+template <typename RowOff>
+__device__ __forceinline__ void issue_q_rows(const char* q_base, uint32_t first, uint32_t rows_total, uint32_t group, uint32_t lds,
+                                             uint32_t lane, RowOff&& row_off) {
+  const uint64_t base = uniform_address(q_base);
+  if ((group & 7u) == 0u) {
+    constexpr uint64_t STEP = 1024 - (uint64_t)kQRowLds;
+    static_for<0, 4>([&](auto i_c) {
+      constexpr int i = decltype(i_c)::value;
+      const uint64_t b = base + (uint32_t)__builtin_amdgcn_readfirstlane((int)row_off(min(first + 8u * i, rows_total - 8u)));
+      lds_dma_group<4, 8 * i * (int)kQRowLds, (int)kQRowLds>(b, STEP, lane * 16u, lds);
+      lds_dma_group<4, (8 * i + 4) * (int)kQRowLds, (int)kQRowLds>(b + 4096, STEP, lane * 16u, lds);
+    });
+  } else {
+#pragma unroll 1
+    for (uint32_t i = 0; i < 32u; ++i)
+      lds_dma_16<0>(q_base + (uint32_t)__builtin_amdgcn_readfirstlane((int)row_off(min(first + i, rows_total - 1u))), lane * 16u, lds + i * kQRowLds);
+  }
+}
+
 // lane l: 4 bytes from base + voff -> a dump area in LDS (64 words) that nobody reads.  What the load
 // is for is its side effect: the 128-byte line it touches is in the L2 afterwards.  A load without a
 // register destination, so nothing has to stay reserved until it lands.
