@@ -283,13 +283,20 @@ __global__ void __launch_bounds__(256) attn_wsplit_kernel(const WsArgs args) {
   const uint32_t v_row = 4u * g2 + (i16 >> 2);   // below 8
   const uint32_t v_lane_off = (v_row & (uint32_t)(NBLK - 1)) * L::V_BLK + v_row / NBLK * L::ROWB + (2u * h16 + ((i16 & 3u) >> 1)) * 16u +
                               (i16 & 1u) * 8u;
+  // (Over a bf16 cache at head_dim 256 by MFMAs: the compiler put the 128 register writes between the first scores and the
+  // first tile, 0.2 - 0.3 us of a launch.  Over an f16 cache its other choices with them cost 0.3, and 64 rows spill.)
   f32x16 o[MR][NDB];
 #pragma unroll
   for (int m = 0; m < MR; ++m)
 #pragma unroll
-    for (int i = 0; i < NDB; ++i)
+    for (int i = 0; i < NDB; ++i) {
+      if constexpr (D == 256 && MR == 1 && !F16) {
+        mfma_zero(o[m][i]);
+      } else {
 #pragma unroll
-      for (int e = 0; e < 16; ++e) o[m][i][e] = 0.f;
+        for (int e = 0; e < 16; ++e) o[m][i][e] = 0.f;
+      }
+    }
   __builtin_amdgcn_sched_barrier(0);   // (all of the above while the loads are on their way)
   wait_vmem_all();
   __syncthreads();
