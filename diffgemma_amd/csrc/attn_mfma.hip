@@ -346,15 +346,19 @@ __global__ void __launch_bounds__(256) attn_mfma_kernel(const MfmaArgs args) {
   // 32 rows into LDS as whole pieces of rows and reads the fragments from there the way it reads K fragments.
   u32x4 qf[NSTEP];
   {
-    auto q_to_frag = [&](u32x4 raw, u32x4& f) {
+    // bf16 queries over an f16 cache: fragments [ST0, ST1) converted in place
+    auto convert = [&](auto st0_c, auto st1_c) {
       if (F16 && p.q_is_bf16) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-          f[e] = pack2<true>(__uint_as_float(raw[e] << 16), __uint_as_float(raw[e] & 0xffff0000u));
-      } else {
-        f = raw;
+        for (int st = decltype(st0_c)::value; st < decltype(st1_c)::value; ++st)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            qf[st][e] = pack2<true>(__uint_as_float(qf[st][e] << 16), __uint_as_float(qf[st][e] & 0xffff0000u));
       }
     };
+    using C0 = std::integral_constant<int, 0>;
+    using CHALF = std::integral_constant<int, NSTEP / 2>;
+    using CALL = std::integral_constant<int, NSTEP>;
     if constexpr (L::PAD) {
       lds_char* const ql = q_stage + i16 * Q_PAIR + h16 * (uint32_t)D + g2 * 16u;
       issue_tile<D, false>(k_load_first(k0), wave, lane);
@@ -364,13 +368,15 @@ __global__ void __launch_bounds__(256) attn_mfma_kernel(const MfmaArgs args) {
       for (int i = 0; i < NACC; ++i) mfma_zero(o[i]);
       wait_vmem_but<L::NLD>();
 #pragma unroll
-      for (int st = 0; st < NSTEP / 2; ++st) q_to_frag(*(lds_u32x4*)(ql + 32 * st), qf[st]);
+      for (int st = 0; st < NSTEP / 2; ++st) qf[st] = *(lds_u32x4*)(ql + 32 * st);
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (read before the second half lands there)
       q_load_half(1u);
       issue_tile<D, false>(k_load((tb + 1) * kBlockN, k1, lane), wave, lane);   // (not waited for here)
+      convert(C0{}, CHALF{});   // (192 instructions, while the second half is on its way)
       wait_vmem_but<L::NLD>();
 #pragma unroll
-      for (int st = 0; st < NSTEP / 2; ++st) q_to_frag(*(lds_u32x4*)(ql + 32 * st), qf[NSTEP / 2 + st]);
+      for (int st = 0; st < NSTEP / 2; ++st) qf[NSTEP / 2 + st] = *(lds_u32x4*)(ql + 32 * st);
+      convert(CHALF{}, CALL{});
     } else {
       // in the layout of a K tile, through the tile buffers
       static_assert(4 * L::K_BYTES <= LDS_BYTES, "the four waves' query rows are staged in the tile buffers");
@@ -385,7 +391,8 @@ __global__ void __launch_bounds__(256) attn_mfma_kernel(const MfmaArgs args) {
       wait_vmem_all();
       const uint32_t q_lane_off = l32 * L::K_STRIDE, q_swz = L::swz_k(l32);
 #pragma unroll
-      for (int st = 0; st < NSTEP; ++st) q_to_frag(*(lds_u32x4*)(qb + q_lane_off + ((((uint32_t)(2 * st) + g2) ^ q_swz) << 4)), qf[st]);
+      for (int st = 0; st < NSTEP; ++st) qf[st] = *(lds_u32x4*)(qb + q_lane_off + ((((uint32_t)(2 * st) + g2) ^ q_swz) << 4));
+      convert(C0{}, CALL{});
     }
     // every wave has its fragments before the next tiles overwrite the rows (head_dim 512: and everybody's first K tile
     // has landed)
