@@ -121,8 +121,8 @@ __global__ void __launch_bounds__(256) topk_scores_kernel(const TopkParams tp) {
                  [&](uint32_t rq) { return (rq + fast_div(rq, tp.div_group) * (p.hq - p.group)) * (uint32_t)(2 * D); });
     wait_vmem_all();
 #pragma unroll
-    for (int st = 0; st < NSTEP; ++st) qf[st] = to_frag(*(lds_u32x4*)(qb + l32 * kQRowLds + g2 * 16u + 32 * st));
-    __syncthreads();   // the first tiles may take the rows' place
+    for (int st = 0; st < NSTEP; ++st) qf[st] = *(lds_u32x4*)(qb + l32 * kQRowLds + g2 * 16u + 32 * st);
+    __syncthreads();   // the first tiles may take the rows' place (converted behind their loads, below)
   } else {
     const size_t qoff = ((size_t)tok * p.hq + qh) * D + 8u * g2;
     const uint16_t* qp = (const uint16_t*)p.q + qoff;
@@ -162,6 +162,10 @@ __global__ void __launch_bounds__(256) topk_scores_kernel(const TopkParams tp) {
   }
 #pragma unroll
   for (int i = 0; i < PF; ++i) issue_k(tb + i);
+  if constexpr (D == 512) {
+#pragma unroll
+    for (int st = 0; st < NSTEP; ++st) qf[st] = to_frag(qf[st]);
+  }
   // lane l32 holds key t0 + l32 of sixteen rows; element e of a tile's scores goes to
   // (uniform tile base) + (per-lane 32-bit offset)
   auto store_elem = [&](auto e_c, const f32x16& sc, uint32_t tile) {
@@ -895,29 +899,37 @@ __global__ void __launch_bounds__(256) topk_filter_kernel(const TopkParams tp) {
     static_assert(4 * 32 * kQRowLds <= NB * L::K_BYTES, "the tile buffers hold a block of every wave's query rows");
     lds_char* const qb = (lds_char*)smem + wave * (32u * kQRowLds);
     const char* const q_base = (const char*)p.q + ((size_t)tp.tok0 * p.hq + kvh * p.group) * (2 * D);
-    const bool convert = F16 && p.q_is_bf16;
-    static_for<0, 2>([&](auto b_c) {
-      constexpr int b = decltype(b_c)::value;
-      issue_q_rows(q_base, row0 + 32u * b, rows_total, p.group, (uint32_t)(size_t)qb, lane,
-                   [&](uint32_t rq) { return (rq + fast_div(rq, tp.div_group) * (p.hq - p.group)) * (uint32_t)(2 * D); });
+    auto row_off = [&](uint32_t rq) { return (rq + fast_div(rq, tp.div_group) * (p.hq - p.group)) * (uint32_t)(2 * D); };
+    u32x4 raw[NSTEP];
+    auto read_rows = [&]() {
       wait_vmem_all();
-      static_for<0, NSTEP>([&](auto st_c) {
-        constexpr int st = decltype(st_c)::value;
-        u32x4 raw = *(lds_u32x4*)(qb + l32 * kQRowLds + g2 * 16u + 32 * st);
-        if (convert) {
+#pragma unroll
+      for (int st = 0; st < NSTEP; ++st) raw[st] = *(lds_u32x4*)(qb + l32 * kQRowLds + g2 * 16u + 32 * st);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (before the next loads land there)
+    };
+    // (bf16 queries over an f16 cache: 384 conversions a block, while the next loads are on their way)
+    auto to_frags = [&](auto b_c) {
+#pragma unroll
+      for (int st = 0; st < NSTEP; ++st) {
+        if (F16 && p.q_is_bf16) {
 #pragma unroll
           for (int e = 0; e < 4; ++e)
-            raw[e] = pack2<true>(__uint_as_float(raw[e] << 16), __uint_as_float(raw[e] & 0xffff0000u));
+            raw[st][e] = pack2<true>(__uint_as_float(raw[st][e] << 16), __uint_as_float(raw[st][e] & 0xffff0000u));
         }
-        qf[b][st] = raw;
-        asm volatile("" : "+a"(qf[b][st]));
-      });
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (read before the next rows land there)
-    });
-  }
-  __syncthreads();
+        qf[decltype(b_c)::value][st] = raw[st];
+        asm volatile("" : "+a"(qf[decltype(b_c)::value][st]));
+      }
+    };
+    issue_q_rows(q_base, row0, rows_total, p.group, (uint32_t)(size_t)qb, lane, row_off);
+    read_rows();
+    issue_q_rows(q_base, row0 + 32u, rows_total, p.group, (uint32_t)(size_t)qb, lane, row_off);
+    to_frags(std::integral_constant<int, 0>{});
+    read_rows();
+    __syncthreads();
 #pragma unroll
-  for (int i = 0; i < PF; ++i) issue_tile<D, false>(k_desc((uint32_t)i), wave, lane);
+    for (int i = 0; i < PF; ++i) issue_tile<D, false>(k_desc((uint32_t)i), wave, lane);
+    to_frags(std::integral_constant<int, 1>{});
+  }
   // S = K.Q^T: the lane is a query row of the block, register e is key 8 (e >> 2) + 4 g2 + (e & 3) of the tile.  Each lane
   // keeps lists of its own, one per block, so an entry's place is the lane's count and nothing is exchanged.
   float tau[2];
