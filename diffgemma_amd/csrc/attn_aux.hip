@@ -263,7 +263,8 @@ struct MergeArgs {
   FastDiv div_rows, div_group;   // by the rows of a KV head and by the GQA group
   uint32_t hd;
 };
-template <uint32_t N>
+// MAPPED: row tiles have split counts of their own (AttnParams.map), at most N; rows of one split are in the output already.
+template <uint32_t N, bool MAPPED>
 __global__ void __launch_bounds__(256) attn_merge_few_kernel(const MergeArgs args) {
   const AttnParams& p = args.p;
   const uint32_t hd = args.hd;
@@ -272,28 +273,41 @@ __global__ void __launch_bounds__(256) attn_merge_few_kernel(const MergeArgs arg
   if (gr >= p.hkv * p.rows_total) return;
   const uint32_t kvh = fast_div(gr, args.div_rows), r = gr - kvh * p.rows_total;
   const uint32_t tok = fast_div(r, args.div_group), qh = kvh * p.group + r - tok * p.group;
-  const size_t split_stride = (size_t)p.hkv * p.rows_pad;
-  const size_t row = (size_t)kvh * p.rows_pad + r;
-  const float2 ml = *(const float2*)(p.part_ml + ((size_t)min(lane, N - 1u) * split_stride + row) * 2);
   const bool live = lane < hd / 8;
   const uint32_t d8 = live ? lane : 0u;
-  const uint16_t* const hbase = (const uint16_t*)p.part_o + row * hd;
-  const size_t sstride = split_stride * hd;
+  const uint32_t mt = r / (uint32_t)kBlockM;
+  uint32_t n = N, prow[N];   // partial row of each split; past n the first one's, with weight zero
+  if constexpr (MAPPED) {
+    n = map_splits(p.map, mt);
+    if (n == 1u) return;
+#pragma unroll
+    for (uint32_t u = 0; u < N; ++u) {
+      const uint32_t i = u < n ? u : 0u;
+      prow[u] = (kvh * p.map.units + p.map.cum[i] + mt - p.map.first[i]) * (uint32_t)kBlockM + r % (uint32_t)kBlockM;
+    }
+  } else {
+#pragma unroll
+    for (uint32_t u = 0; u < N; ++u) prow[u] = (u * p.hkv + kvh) * p.rows_pad + r;
+  }
+  uint32_t my_row = prow[0];
+#pragma unroll
+  for (uint32_t u = 1; u < N; ++u) my_row = lane == u ? prow[u] : my_row;
+  const float2 ml = *(const float2*)(p.part_ml + (size_t)my_row * 2);
   uint4 a[N];
 #pragma unroll
-  for (uint32_t u = 0; u < N; ++u) a[u] = ((const uint4*)(hbase + u * sstride))[d8];
+  for (uint32_t u = 0; u < N; ++u) a[u] = ((const uint4*)((const uint16_t*)p.part_o + (size_t)prow[u] * hd))[d8];
   float msu[N], wlu[N], sum[kMergeFewSplits];
   float mx = -INFINITY;
 #pragma unroll
   for (uint32_t u = 0; u < N; ++u) {
-    msu[u] = __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(ml.x), (int)u));
+    msu[u] = u < n ? __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(ml.x), (int)u)) : -INFINITY;
     mx = fmaxf(mx, msu[u]);
   }
 #pragma unroll
   for (uint32_t u = 0; u < kMergeFewSplits; ++u) {
     sum[u] = 0.f;
     if (u < N) {
-      const float lsu = __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(ml.y), (int)u));
+      const float lsu = u < n ? __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(ml.y), (int)u)) : 0.f;
       sum[u] = wlu[u] = lsu > 0.f ? lsu * exp2f(msu[u] - mx) : 0.f;
     }
   }
@@ -339,7 +353,8 @@ __global__ void __launch_bounds__(256) attn_merge_few_kernel(const MergeArgs arg
 
 template <uint32_t N>
 hipError_t launch_merge_few(const MergeArgs& a, uint32_t rows, hipStream_t s) {
-  hipLaunchKernelGGL((attn_merge_few_kernel<N>), dim3((rows + 3) / 4), dim3(256), 0, s, a);
+  if (a.p.map.n) hipLaunchKernelGGL((attn_merge_few_kernel<N, true>), dim3((rows + 3) / 4), dim3(256), 0, s, a);
+  else hipLaunchKernelGGL((attn_merge_few_kernel<N, false>), dim3((rows + 3) / 4), dim3(256), 0, s, a);
   return hipGetLastError();
 }
 
@@ -581,13 +596,13 @@ hipError_t launch_attn_merge(const AttnParams& p, uint32_t head_dim, bool stream
   const uint32_t rows = p.hkv * p.rows_total;
   // not many splits, not many bytes: the variant that asks for every partial row up front
   const size_t part_bytes = (size_t)p.n_splits * p.hkv * p.rows_pad * head_dim * 2;
-  if (!streamed && p.part_half && p.n_splits <= kMergeFewSplits && head_dim % 8 == 0 && head_dim <= 512 && part_bytes < ((size_t)32 << 20)) {
+  if (p.map.n || (!streamed && p.part_half && p.n_splits <= kMergeFewSplits && head_dim % 8 == 0 && head_dim <= 512 && part_bytes < ((size_t)32 << 20))) {
     MergeArgs a;
     a.p = p;
     a.div_rows = make_fast_div(p.rows_total);
     a.div_group = make_fast_div(p.group);
     a.hd = head_dim;
-    switch (p.n_splits) {
+    switch (p.map.n ? p.map.n : p.n_splits) {
       case 2: return launch_merge_few<2>(a, rows, s);
       case 3: return launch_merge_few<3>(a, rows, s);
       case 4: return launch_merge_few<4>(a, rows, s);

@@ -42,6 +42,8 @@
 #include "mfma_tile.h"
 #include "wt_store.h"
 
+#include <algorithm>
+
 namespace dg {
 namespace {
 
@@ -102,6 +104,7 @@ __device__ __forceinline__ float add_pair(uint32_t pk, float acc) {
 struct MfmaArgs {
   AttnParams p;
   FastDiv div_mtiles, div_splits, div_group;
+  FastDiv div_units, div_n[kMapSplits];   // with a split map: by the units of a KV head, by 1 .. 8
 };
 
 template <int D, bool F16, bool TOUCH>
@@ -148,13 +151,27 @@ __global__ void __launch_bounds__(256) attn_mfma_kernel(const MfmaArgs args) {
   // (KV head, split) first and row tile second, are cut into 8 equal runs, one per XCD, so the
   // row tiles that stream the same keys sit behind one L2 and every XCD has work whatever
   // the number of (KV head, split) pairs.
-  const uint32_t n_units = p.hkv * p.n_splits * p.n_mtiles;
+  const SplitMap& map = args.p.map;
+  const bool mapped = map.n != 0u;
+  const uint32_t n_units = p.hkv * (mapped ? map.units : p.n_splits * p.n_mtiles);
   const uint32_t per_xcd = (n_units + 7u) >> 3;
   const uint32_t wg = blockIdx.x;
   const uint32_t unit = (wg & 7u) * per_xcd + (wg >> 3);
   if (unit >= n_units) return;
-  const uint32_t stream = fast_div(unit, args.div_mtiles), mt = unit - stream * p.n_mtiles;
-  const uint32_t kvh = fast_div(stream, args.div_splits), split = stream - kvh * p.n_splits;
+  uint32_t mt, kvh, split, n_splits;
+  if (mapped) {
+    kvh = fast_div(unit, args.div_units);
+    const uint32_t u = unit - kvh * map.units;
+    split = map_split_of(map, u);
+    mt = map.first[split] + u - map.cum[split];
+    n_splits = map_splits(map, mt);
+  } else {
+    const uint32_t stream = fast_div(unit, args.div_mtiles);
+    mt = unit - stream * p.n_mtiles;
+    kvh = fast_div(stream, args.div_splits);
+    split = stream - kvh * p.n_splits;
+    n_splits = p.n_splits;
+  }
 
   const uint32_t lane = threadIdx.x & 63u;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -240,24 +257,24 @@ __global__ void __launch_bounds__(256) attn_mfma_kernel(const MfmaArgs args) {
     hi_max = __builtin_amdgcn_readfirstlane(hi_max);
   }
   // the key tiles this row tile can see, cut into n_splits equal runs (a causal or windowed row
-  // tile sees only part of the launch's key range: cutting its own range keeps the splits even)
+  // tile sees only part of the launch's key range: cutting its own range keeps the splits even; a split map goes further)
   const uint32_t mt_begin = max(lo_min / kBlockN, p.tile_first);
   const uint32_t mt_end = max(min((hi_max + kBlockN - 1) / kBlockN, p.tile_end), mt_begin);
-  const uint32_t per_split = (mt_end - mt_begin + p.n_splits - 1u) / p.n_splits;
+  const uint32_t per_split = fast_div(mt_end - mt_begin + n_splits - 1u, mapped ? args.div_n[n_splits - 1u] : args.div_splits);
   const uint32_t tb = __builtin_amdgcn_readfirstlane(min(mt_begin + split * per_split, mt_end));
   const uint32_t te = __builtin_amdgcn_readfirstlane(min(tb + per_split, mt_end));
   const uint32_t ntile = te - tb;
 
   // first partial row of this workgroup; partial rows and their (m, l) are written through (wt_store.h)
-  const size_t wg_prow0 = ((size_t)split * p.hkv + kvh) * p.rows_pad + row0;
+  const size_t wg_prow0 = mapped ? (size_t)unit * kBlockM : ((size_t)split * p.hkv + kvh) * p.rows_pad + row0;
   // No key tile to visit: the rows' share is nothing, (m, l, O) = (-inf, 0, 0).  An exit of its own, so that the epilogue
   // has one predecessor and takes O from the registers the tile loop leaves it in (with a second one the compiler moved
   // all 256 accumulation registers at the loop's exit, 512 instructions).
   if (ntile == 0u) {
     wait_vmem_all();   // (the query rows; loads must not outlive this workgroup's LDS)
-    const uint32_t row_b = D * (p.n_splits > 1 ? (p.part_half ? 2u : 4u) : p.out_dtype == DT_F32 ? 4u : 2u);
+    const uint32_t row_b = D * (n_splits > 1 ? (p.part_half ? 2u : 4u) : p.out_dtype == DT_F32 ? 4u : 2u);
     const u32x4 zero = {0u, 0u, 0u, 0u};
-    if (p.n_splits > 1) {
+    if (n_splits > 1) {
       if (threadIdx.x < (uint32_t)kBlockM)
         wt_store8(wt_window(p.part_ml + wg_prow0 * 2), threadIdx.x * 8u, u32x2{__float_as_uint(-INFINITY), 0u});
       const auto win = wt_window((const char*)p.part_o + wg_prow0 * row_b);
@@ -730,7 +747,7 @@ __global__ void __launch_bounds__(256) attn_mfma_kernel(const MfmaArgs args) {
   //     largest |V|); the merge weighs the rows by l 2^(m - m_max) instead of 2^(m - m_max)
   //   fp32 partial rows: the accumulators as they are
   //   result rows (one split): divided by the row sum
-  const bool parts = p.n_splits > 1;
+  const bool parts = n_splits > 1;
   const bool rows16 = parts ? p.part_half != 0u : p.out_dtype != DT_F32;
   constexpr int STG16 = NDBW * 64 + 16;   // bytes of a staged row slice, padded (the 16-byte pieces of 8 rows fall on distinct banks)
   // The loads issued for tiles behind the last one are still on their way to the buffers of V(last + 1) and K(last + 1 .. 3).
@@ -857,7 +874,10 @@ hipError_t launch_one(const AttnParams& p, hipStream_t s) {
   a.div_mtiles = make_fast_div(p.n_mtiles);
   a.div_splits = make_fast_div(p.n_splits);
   a.div_group = make_fast_div(p.group);
-  const uint32_t grid = ((p.hkv * p.n_splits * p.n_mtiles + 7u) / 8u) * 8u;
+  a.div_units = make_fast_div(std::max(1u, p.map.units));
+  for (uint32_t i = 0; i < kMapSplits; ++i) a.div_n[i] = make_fast_div(i + 1u);
+  const uint32_t n_units = p.hkv * (p.map.n ? p.map.units : p.n_splits * p.n_mtiles);
+  const uint32_t grid = (n_units + 7u) / 8u * 8u;
   if constexpr (D == 512) {
     if (p.touch_ahead) {
       hipLaunchKernelGGL((attn_mfma_kernel<D, F16, true>), dim3(grid), dim3(256), 0, s, a);

@@ -14,6 +14,47 @@ constexpr int kBlockN = 32;    // keys per tile
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
 
+// Row tiles with split counts of their own (causal rows: a row tile sees as many key tiles as lie before it, and with one
+// count for all the launch is as long as the last row tile's share).  The counts do not fall with the row tile, so they
+// are given by where each begins: row tile mt has more than i splits from mt = first[i] on.  The units of a KV head are
+// ordered by split, then row tile: split i of row tile mt is unit cum[i] + mt - first[i], which also numbers its partial rows.
+constexpr uint32_t kMapSplits = 8;
+struct SplitMap {
+  uint32_t n;                     // most splits of a row tile; 0: every row tile has n_splits
+  uint32_t units;                 // of a KV head
+  uint32_t first[kMapSplits], cum[kMapSplits];   // past n: no row tile, no unit
+};
+__host__ __device__ __forceinline__ uint32_t map_splits(const SplitMap& m, uint32_t mt) {
+  uint32_t s = 0;
+#pragma unroll
+  for (uint32_t i = 0; i < kMapSplits; ++i) s += mt >= m.first[i] ? 1u : 0u;
+  return s;
+}
+// split of unit u of a KV head; its row tile is first[split] + u - cum[split]
+__host__ __device__ __forceinline__ uint32_t map_split_of(const SplitMap& m, uint32_t u) {
+  uint32_t s = 0;
+#pragma unroll
+  for (uint32_t i = 1; i < kMapSplits; ++i) s = u >= m.cum[i] ? i : s;
+  return s;
+}
+// The map for row tiles that see tiles(mt) key tiles (not falling with mt), none of whose shares is longer than `len`;
+// false where one needs more than kMapSplits.
+template <typename Tiles>
+inline bool make_split_map(uint32_t n_mtiles, uint32_t len, Tiles&& tiles, SplitMap* m) {
+  m->n = m->units = 0;
+  for (uint32_t i = 0; i < kMapSplits; ++i) m->first[i] = m->cum[i] = 0xffffffffu;
+  for (uint32_t mt = 0; mt < n_mtiles; ++mt) {
+    const uint32_t s = (tiles(mt) + len - 1) / len;
+    if (s > kMapSplits) return false;
+    while (m->n < s) m->first[m->n++] = mt;
+  }
+  for (uint32_t i = 0; i < m->n; ++i) {
+    m->cum[i] = m->units;
+    m->units += n_mtiles - m->first[i];
+  }
+  return true;
+}
+
 // Stacked row r of a KV head = tok * group + g: the `group` query heads that share one KV
 // head sit next to each other, so a 128-row tile covers 128/group consecutive canvas rows.
 struct AttnParams {
@@ -49,6 +90,7 @@ struct AttnParams {
   uint32_t cus;          // compute units of the device
   uint32_t sees_masked;  // causal rows also see the canvas keys behind the causal rows
   float scale_log2;      // softmax_scale * log2(e)
+  SplitMap map;          // (split kernel and its merge)
 };
 
 // Division of n < 2^31 by a divisor the host knows: q = (mulhi(n, mul) + n) >> shift (the round-up method: mul =

@@ -140,6 +140,7 @@ struct Plan {
   bool wsplit = false;          // short key range, head_dim <= 256: keys split over the waves of a workgroup, one launch
   bool part_half = false;       // split partial rows travel as normalised f16 rows
   size_t off_q = 0, off_kv = 0, off_part_o = 0, off_part_ml = 0, total = 0;
+  dg::SplitMap map = {};        // row tiles with split counts of their own (n = 0: none)
   float scale = 1.0f;
 };
 
@@ -166,9 +167,34 @@ uint32_t tiles_of_split(uint32_t ntiles, uint32_t room, uint32_t hd, bool long_s
   return std::max(t, (ntiles + room - 1) / room);
 }
 
+// Row tiles that see different numbers of key tiles (causal rows of a global layer): split counts of their own, so that no
+// share is longer than the smallest length that leaves one round of the chip.  With 16-bit partial rows (what the merge for
+// them reads) and a prefix the host knows.  Taken where that shortens the longest share by a tenth and by two key tiles: attention
+// call, us, one count for all | split map: 1024 causal rows behind 0 keys 50.7 | 45.1 (shares of 16 tiles become 12), behind 300
+// 60.4 | 55.8, 901 behind 0 43.4 | 38.7, 700 behind 0 36.0 | 31.8, behind 700 51.5 | 45.6; by one tile: 512 behind 0 26.0 | 26.5,
+// 300 20.5 | 19.9, 200 17.2 | 18.0, 256 rows, 128 of them causal, behind 300 23.9 | 25.0.
+bool plan_split_map(const dg_attn_desc* d, const Plan& pl, int cus, uint32_t ntiles, dg::SplitMap* out) {
+  if (d->head_dim != 512 || d->causal_rows == 0 || d->window != 0 || (d->flags & DG_ATTN_F_T_LO_EXPLICIT) || !pl.part_half) return false;
+  const uint32_t budget = (uint32_t)cus / d->n_kv_heads;
+  if (pl.tiles_per_split >= ntiles || budget < pl.n_mtiles || ntiles >= 65536u) return false;
+  auto tiles = [&](uint32_t mt) -> uint32_t {   // as the kernel cuts them
+    const uint32_t a = mt * dg::kBlockM / pl.group, b = (std::min((mt + 1) * dg::kBlockM, pl.rows_total) - 1) / pl.group;
+    uint32_t hi = b < d->causal_rows ? std::min(pl.t_all, d->kv_len + b + 1) : pl.t_all;
+    if (a < d->causal_rows && pl.extra_lo < pl.t_all) hi = pl.t_all;
+    return (hi + dg::kBlockN - 1) / dg::kBlockN;
+  };
+  const double s = std::sqrt((double)ntiles * budget / pl.n_mtiles / 9.0);
+  uint32_t len = std::max(1u, (uint32_t)(ntiles / std::max(1.0, s)));
+  for (; 10u * len <= 9u * pl.tiles_per_split && len + 2u <= pl.tiles_per_split; ++len)
+    if (dg::make_split_map(pl.n_mtiles, len, tiles, out) && out->units <= budget) return out->n > 1;
+  return false;
+}
+
 // Scratch a split count takes, and the count for a call that has `scratch` bytes of it: what the rule asks for, or, where
 // that is more, splits of at least 6 tiles (a caller may hold what an earlier library asked for).
-int make_plan(const dg_attn_desc* d, int cus, Plan* pl, const uint32_t* key_range = nullptr, size_t scratch = SIZE_MAX) {
+// `on_device`: the prefix length is read when the kernels run, so every row tile has the same count.
+int make_plan(const dg_attn_desc* d, int cus, Plan* pl, const uint32_t* key_range = nullptr, size_t scratch = SIZE_MAX,
+              bool on_device = false) {
   if (!d) return DG_ERR_NULL;
   pl->cus = (uint32_t)cus;
   const uint32_t hd = d->head_dim;
@@ -306,6 +332,18 @@ int make_plan(const dg_attn_desc* d, int cus, Plan* pl, const uint32_t* key_rang
     carve((ntiles + splits - 1) / splits);
   } else {
     carve(tiles_of_split(ntiles, room, hd, false));
+    dg::SplitMap map;
+    if (!key_range && plan_split_map(d, *pl, cus, ntiles, &map)) {
+      // (sized for either, so that one workspace serves the entry points with and without a host-known prefix)
+      const size_t rows = (size_t)d->n_kv_heads * map.units * dg::kBlockM, equal = pl->total;
+      const size_t ml = pl->off_part_o + align_up(rows * hd * 2), both = std::max(equal, ml + align_up(rows * 8));
+      if (!on_device && both <= scratch) {
+        pl->map = map;
+        pl->n_splits = map.n;
+        pl->off_part_ml = ml;
+        pl->total = both;
+      }
+    }
     if (pl->total > scratch) carve(tiles_of_split(ntiles, room, hd, true));
   }
   return DG_OK;
@@ -457,6 +495,7 @@ int fill_params(const dg_attn_desc* d, const Plan& pl, const void* q, const void
   p.rows_pad = pl.rows_pad;
   p.n_mtiles = pl.n_mtiles;
   p.n_splits = pl.n_splits;
+  p.map = pl.map;
   p.tile_first = pl.tile_first;
   p.tiles_per_split = pl.tiles_per_split;
   p.tile_end = pl.tile_end;
@@ -541,7 +580,7 @@ int dg_attn_forward_dev(const dg_attn_desc* d, const dg_step_params* step_dev, c
   int rc = device_info(&di);
   if (rc != DG_OK) return rc;
   Plan pl;
-  rc = make_plan(d, di.cus, &pl, nullptr, workspace ? workspace_bytes : 0);
+  rc = make_plan(d, di.cus, &pl, nullptr, workspace ? workspace_bytes : 0, true);
   if (rc != DG_OK) return rc;
   return forward_planned(d, pl, q, kv_base, out, lse, workspace, workspace_bytes, stream, (const uint32_t*)step_dev);
 }

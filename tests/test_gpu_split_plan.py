@@ -50,3 +50,47 @@ def test_smaller_scratch_takes_fewer_splits(gpu_ready):
     assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2]) and not torch.equal(outs[0], outs[3])
     with pytest.raises(RuntimeError):
         A.forward(d, qd, kd, outs[0], None, torch.empty(least - 256, dtype=torch.uint8, device="cuda"))
+
+
+@pytest.mark.parametrize("canvas,kv_len,causal_rows,f16,sees_masked", [
+    (1024, 0, 1024, False, False), (1024, 300, 1024, True, False), (901, 0, 901, False, False), (700, 700, 700, True, False),
+    (1000, 5, 1000, False, True), (800, 0, 500, False, False)])
+def test_split_counts_per_row_tile(gpu_ready, po, canvas, kv_len, causal_rows, f16, sees_masked):
+    """Causal rows behind a short prefix: row tiles of one split go straight to the output, the others are merged by counts of
+    their own.  Rows at the edges of row tiles against the oracle; the same bits on every run."""
+    import torch
+    w = dataclasses.replace(W.Workload("map", canvas, 16, 2, 512, kv_len, causal_rows=causal_rows, sees_masked=sees_masked, seed=canvas),
+                            kv_f16=f16)
+    toks = np.unique(np.concatenate([np.arange(0, canvas, 61), np.arange(15, canvas, 160), np.arange(16, canvas, 160),
+                                     [causal_rows - 1, min(causal_rows, canvas - 1), canvas - 1]])).astype(np.uint32)
+    check_tolerances(*run_workload(po, w, toks=toks))
+    q, kv = W.generate(w)
+    qd, kd = W.device_arrays(w, q, kv)
+    d, first = w.desc(), None
+    ws = A.alloc_workspace(d)
+    for _ in range(3):
+        out = torch.full((canvas * 16 * 512,), -1, dtype=torch.int16, device="cuda")
+        A.forward(d, qd, kd, out, None, ws)
+        torch.cuda.synchronize()
+        first = out if first is None else first
+        assert torch.equal(out, first)
+        ws.fill_(255)      # NaN everywhere: nothing of an earlier call is read
+
+
+def test_device_prefix_with_the_scratch_of_a_split_map(gpu_ready, po):
+    """The entry point that reads the prefix on the device has one count for all row tiles and runs in the same scratch."""
+    import torch
+    w = W.Workload("map_dev", 1024, 16, 2, 512, 0, causal_rows=1024, seed=2)
+    q, kv = W.generate(w)
+    qd, kd = W.device_arrays(w, q, kv)
+    d = w.desc()
+    outs = []
+    for run in (lambda o: A.forward(d, qd, kd, o, None, A.alloc_workspace(d)),
+                lambda o: A.forward_dev(d, A.device_step_params(0), qd, kd, o, None, A.alloc_workspace(d)),
+                lambda o: A.forward(w.desc(n_splits=2), qd, kd, o, None, A.alloc_workspace(w.desc(n_splits=2)))):
+        out = torch.zeros(w.canvas * 16 * 512, dtype=torch.int16, device="cuda")
+        run(out)
+        torch.cuda.synchronize()
+        outs.append(out.view(torch.bfloat16).float())
+    assert torch.equal(outs[1], outs[2])
+    assert (outs[0] - outs[1]).abs().max() <= 2.0 ** -7 * outs[1].abs().max()

@@ -1,0 +1,63 @@
+"""Split counts per row tile (SplitMap in csrc/attn_params.h), compiled for the host: every (row tile, split) is one unit of a
+KV head, found again from its number, and the longest share keeps the asked-for length."""
+import subprocess
+
+from diffgemma_amd import attention as A, build, capi
+
+PROGRAM = r"""
+#include "attn_params.h"
+#include <algorithm>
+#include <cstdio>
+#include <vector>
+int main() {
+  using namespace dg;
+  for (uint32_t n = 1; n <= 70; n += n < 6 ? 1 : 13)
+    for (uint32_t len = 1; len <= 20; ++len)
+      for (uint32_t base = 0; base <= 40; base += 8)
+        for (uint32_t per = 0; per <= 3; ++per) {
+          auto tiles = [&](uint32_t mt) { return base + 1 + mt * per / 2; };
+          SplitMap m;
+          const uint32_t most = (tiles(n - 1) + len - 1) / len;
+          if (make_split_map(n, len, tiles, &m) != (most <= kMapSplits)) return std::printf("n %u len %u most %u\n", n, len, most), 1;
+          if (most > kMapSplits) continue;
+          if (m.n != most) return std::printf("n %u len %u: %u splits\n", n, len, m.n), 1;
+          std::vector<uint32_t> seen(n, 0);
+          uint32_t units = 0;
+          for (uint32_t mt = 0; mt < n; ++mt) {
+            if (map_splits(m, mt) != (tiles(mt) + len - 1) / len) return std::printf("mt %u: %u splits\n", mt, map_splits(m, mt)), 1;
+            units += map_splits(m, mt);
+          }
+          if (units != m.units) return std::printf("units %u %u\n", units, m.units), 1;
+          for (uint32_t u = 0; u < m.units; ++u) {
+            const uint32_t s = map_split_of(m, u), mt = m.first[s] + u - m.cum[s];
+            if (mt >= n || s >= map_splits(m, mt) || (seen[mt] & (1u << s))) return std::printf("unit %u: mt %u split %u\n", u, mt, s), 1;
+            seen[mt] |= 1u << s;
+          }
+        }
+  std::puts("ok");
+  return 0;
+}
+"""
+
+
+def test_units_of_a_split_map(tmp_path):
+    src, exe = tmp_path / "map.hip", tmp_path / "map"
+    src.write_text(PROGRAM)
+    res = subprocess.run([build.hipcc_path(), *build.HIP_FLAGS, "-I", str(build.CSRC), str(src), "-o", str(exe)],
+                         stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    assert res.returncode == 0, res.stdout[-2000:]
+    res = subprocess.run([str(exe)], stdout=subprocess.PIPE, text=True)
+    assert res.returncode == 0 and res.stdout == "ok\n", res.stdout
+
+
+def test_where_a_split_map_is_planned():
+    """Causal rows behind a short prefix, 16-bit partial rows; not behind a long one, not with a window, fp32 partial rows, an
+    explicit count or equal rows.  The scratch covers the entry points that read the prefix on the device, too."""
+    half = capi.DG_ATTN_F_F16_PARTIALS
+    desc = lambda rows, kv, cr, **kw: A.make_desc(rows, 16, 2, 512, kv, causal_rows=cr, **{"flags": half, **kw})
+    assert capi.resolved_splits(desc(1024, 0, 1024)) == 3 and capi.resolved_splits(desc(700, 700, 700)) == 4
+    assert capi.resolved_splits(desc(1024, 0, 1024, kv_dtype=capi.DG_F16, flags=0)) == 3
+    for d in (desc(1024, 0, 1024, flags=0), desc(1024, 20000, 1024), desc(1024, 0, 0), desc(1024, 0, 1024, n_splits=2)):
+        assert capi.resolved_splits(d) == 2
+    row_tiles = 2 * 64 * 128
+    assert capi.workspace_bytes(desc(1024, 0, 1024)) >= 2 * row_tiles * (512 * 2 + 8)      # two equal splits
