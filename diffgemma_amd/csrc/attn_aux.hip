@@ -289,9 +289,12 @@ __global__ void __launch_bounds__(256) attn_merge_few_kernel(const MergeArgs arg
 #pragma unroll
     for (uint32_t u = 0; u < N; ++u) prow[u] = (u * p.hkv + kvh) * p.rows_pad + r;
   }
-  uint32_t my_row = prow[0];
+  uint32_t my_row = prow[0] + min(lane, N - 1u) * p.hkv * p.rows_pad;   // lane u reads split u's (m, l)
+  if constexpr (MAPPED) {
+    my_row = prow[0];
 #pragma unroll
-  for (uint32_t u = 1; u < N; ++u) my_row = lane == u ? prow[u] : my_row;
+    for (uint32_t u = 1; u < N; ++u) my_row = lane == u ? prow[u] : my_row;
+  }
   const float2 ml = *(const float2*)(p.part_ml + (size_t)my_row * 2);
   uint4 a[N];
 #pragma unroll

@@ -107,7 +107,8 @@ struct MfmaArgs {
   FastDiv div_units, div_n[kMapSplits];   // with a split map: by the units of a KV head, by 1 .. 8
 };
 
-template <int D, bool F16, bool TOUCH>
+// MAPPED: with a split map (an instance of its own: what the map takes at a workgroup's start is 0.3 us of a short call)
+template <int D, bool F16, bool TOUCH, bool MAPPED>
 __global__ void __launch_bounds__(256) attn_mfma_kernel(const MfmaArgs args) {
   const AttnParams p = resolve_step(args.p);
   using L = Lay<D>;
@@ -152,19 +153,20 @@ __global__ void __launch_bounds__(256) attn_mfma_kernel(const MfmaArgs args) {
   // row tiles that stream the same keys sit behind one L2 and every XCD has work whatever
   // the number of (KV head, split) pairs.
   const SplitMap& map = args.p.map;
-  const bool mapped = map.n != 0u;
-  const uint32_t n_units = p.hkv * (mapped ? map.units : p.n_splits * p.n_mtiles);
+  const uint32_t n_units = p.hkv * (MAPPED ? map.units : p.n_splits * p.n_mtiles);
   const uint32_t per_xcd = (n_units + 7u) >> 3;
   const uint32_t wg = blockIdx.x;
   const uint32_t unit = (wg & 7u) * per_xcd + (wg >> 3);
   if (unit >= n_units) return;
   uint32_t mt, kvh, split, n_splits;
-  if (mapped) {
+  FastDiv div_n = args.div_splits;
+  if constexpr (MAPPED) {
     kvh = fast_div(unit, args.div_units);
     const uint32_t u = unit - kvh * map.units;
     split = map_split_of(map, u);
     mt = map.first[split] + u - map.cum[split];
     n_splits = map_splits(map, mt);
+    div_n = args.div_n[n_splits - 1u];
   } else {
     const uint32_t stream = fast_div(unit, args.div_mtiles);
     mt = unit - stream * p.n_mtiles;
@@ -260,13 +262,13 @@ __global__ void __launch_bounds__(256) attn_mfma_kernel(const MfmaArgs args) {
   // tile sees only part of the launch's key range: cutting its own range keeps the splits even; a split map goes further)
   const uint32_t mt_begin = max(lo_min / kBlockN, p.tile_first);
   const uint32_t mt_end = max(min((hi_max + kBlockN - 1) / kBlockN, p.tile_end), mt_begin);
-  const uint32_t per_split = fast_div(mt_end - mt_begin + n_splits - 1u, mapped ? args.div_n[n_splits - 1u] : args.div_splits);
+  const uint32_t per_split = fast_div(mt_end - mt_begin + n_splits - 1u, div_n);
   const uint32_t tb = __builtin_amdgcn_readfirstlane(min(mt_begin + split * per_split, mt_end));
   const uint32_t te = __builtin_amdgcn_readfirstlane(min(tb + per_split, mt_end));
   const uint32_t ntile = te - tb;
 
   // first partial row of this workgroup; partial rows and their (m, l) are written through (wt_store.h)
-  const size_t wg_prow0 = mapped ? (size_t)unit * kBlockM : ((size_t)split * p.hkv + kvh) * p.rows_pad + row0;
+  const size_t wg_prow0 = MAPPED ? (size_t)unit * kBlockM : ((size_t)split * p.hkv + kvh) * p.rows_pad + row0;
   // No key tile to visit: the rows' share is nothing, (m, l, O) = (-inf, 0, 0).  An exit of its own, so that the epilogue
   // has one predecessor and takes O from the registers the tile loop leaves it in (with a second one the compiler moved
   // all 256 accumulation registers at the loop's exit, 512 instructions).
@@ -878,14 +880,15 @@ hipError_t launch_one(const AttnParams& p, hipStream_t s) {
   for (uint32_t i = 0; i < kMapSplits; ++i) a.div_n[i] = make_fast_div(i + 1u);
   const uint32_t n_units = p.hkv * (p.map.n ? p.map.units : p.n_splits * p.n_mtiles);
   const uint32_t grid = (n_units + 7u) / 8u * 8u;
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), 0, s, a);
+    return hipGetLastError();
+  };
   if constexpr (D == 512) {
-    if (p.touch_ahead) {
-      hipLaunchKernelGGL((attn_mfma_kernel<D, F16, true>), dim3(grid), dim3(256), 0, s, a);
-      return hipGetLastError();
-    }
+    if (p.map.n) return p.touch_ahead ? launch(attn_mfma_kernel<D, F16, true, true>) : launch(attn_mfma_kernel<D, F16, false, true>);
+    if (p.touch_ahead) return launch(attn_mfma_kernel<D, F16, true, false>);
   }
-  hipLaunchKernelGGL((attn_mfma_kernel<D, F16, false>), dim3(grid), dim3(256), 0, s, a);
-  return hipGetLastError();
+  return launch(attn_mfma_kernel<D, F16, false, false>);
 }
 
 }  // namespace
