@@ -249,15 +249,13 @@ __global__ void __launch_bounds__(256) attn_merge_kernel(const AttnParams p, con
   }
 }
 
-// The same merge for at most 8 splits of f16 partial rows whose total is small: there the kernel is as long as one wave's
-// chain of memory round trips, not bandwidth.  So a wave asks for everything at once, the (m, l) pairs and the partial rows
-// of all splits, instead of weights first and then rows four at a time; and the weights come from lane-to-scalar reads, every
-// lane doing the same arithmetic, instead of a dozen dependent shuffles.  One instance per split count: with eight loads
-// whatever the count, the repeated ones filled the load path (2 or 3 splits: 0.4 to 0.7 us of a call of 20 to 30).  The sum of the weights pairs its
-// terms as the butterfly over the lanes does, ((0+4)+(2+6))+((1+5)+(3+7)), and the rows are added in the same order with the
-// same cut, so both kernels give the same bits.  (Past 8 splits fetching every row loses to skipping the ones that do
-// not count: 128 rows in 14 splits 20.4 -> 27.1 us on peaked rows.)
-constexpr uint32_t kMergeFewSplits = 8;
+// The same merge for few splits of f16 partial rows whose total is small (merge_at_once): there the kernel is as long as one
+// wave's chain of memory round trips, not bandwidth.  So a wave asks for everything at once, the (m, l) pairs and the partial
+// rows of all splits, instead of weights first and then rows four at a time; and the weights come from lane-to-scalar
+// reads, every lane doing the same arithmetic, instead of a dozen dependent shuffles.  One instance per split count up to 8,
+// every second from there (with eight loads whatever the count, the repeated ones filled the load path: 2 or 3 splits, 0.4 to
+// 0.7 us of a call of 20 to 30).  The sum of the weights pairs its terms as the butterfly over the lanes does, i with i + 8,
+// then i + 4, ..., and the rows are added in the same order with the same cut, so both kernels give the same bits.
 struct MergeArgs {
   AttnParams p;
   FastDiv div_rows, div_group;   // by the rows of a KV head and by the GQA group
@@ -276,7 +274,7 @@ __global__ void __launch_bounds__(256) attn_merge_few_kernel(const MergeArgs arg
   const bool live = lane < hd / 8;
   const uint32_t d8 = live ? lane : 0u;
   const uint32_t mt = r / (uint32_t)kBlockM;
-  uint32_t n = N, prow[N];   // partial row of each split; past n the first one's, with weight zero
+  uint32_t n = N <= 8 ? N : p.n_splits, prow[N];   // partial row of each split; past n one that exists, with weight zero
   if constexpr (MAPPED) {
     n = map_splits(p.map, mt);
     if (n == 1u) return;
@@ -287,9 +285,9 @@ __global__ void __launch_bounds__(256) attn_merge_few_kernel(const MergeArgs arg
     }
   } else {
 #pragma unroll
-    for (uint32_t u = 0; u < N; ++u) prow[u] = (u * p.hkv + kvh) * p.rows_pad + r;
+    for (uint32_t u = 0; u < N; ++u) prow[u] = (min(u, n - 1u) * p.hkv + kvh) * p.rows_pad + r;
   }
-  uint32_t my_row = prow[0] + min(lane, N - 1u) * p.hkv * p.rows_pad;   // lane u reads split u's (m, l)
+  uint32_t my_row = prow[0] + min(lane, n - 1u) * p.hkv * p.rows_pad;   // lane u reads split u's (m, l)
   if constexpr (MAPPED) {
     my_row = prow[0];
 #pragma unroll
@@ -299,7 +297,8 @@ __global__ void __launch_bounds__(256) attn_merge_few_kernel(const MergeArgs arg
   uint4 a[N];
 #pragma unroll
   for (uint32_t u = 0; u < N; ++u) a[u] = ((const uint4*)((const uint16_t*)p.part_o + (size_t)prow[u] * hd))[d8];
-  float msu[N], wlu[N], sum[kMergeFewSplits];
+  constexpr uint32_t W = N <= 8 ? 8 : 16;
+  float msu[N], wlu[N], sum[W];
   float mx = -INFINITY;
 #pragma unroll
   for (uint32_t u = 0; u < N; ++u) {
@@ -307,7 +306,7 @@ __global__ void __launch_bounds__(256) attn_merge_few_kernel(const MergeArgs arg
     mx = fmaxf(mx, msu[u]);
   }
 #pragma unroll
-  for (uint32_t u = 0; u < kMergeFewSplits; ++u) {
+  for (uint32_t u = 0; u < W; ++u) {
     sum[u] = 0.f;
     if (u < N) {
       const float lsu = u < n ? __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(ml.y), (int)u)) : 0.f;
@@ -315,7 +314,7 @@ __global__ void __launch_bounds__(256) attn_merge_few_kernel(const MergeArgs arg
     }
   }
 #pragma unroll
-  for (uint32_t w = kMergeFewSplits / 2; w > 0; w >>= 1)
+  for (uint32_t w = W / 2; w > 0; w >>= 1)
 #pragma unroll
     for (uint32_t u = 0; u < w; ++u) sum[u] += sum[u + w];
   const float den = sum[0];
@@ -599,7 +598,7 @@ hipError_t launch_attn_merge(const AttnParams& p, uint32_t head_dim, bool stream
   const uint32_t rows = p.hkv * p.rows_total;
   // not many splits, not many bytes: the variant that asks for every partial row up front
   const size_t part_bytes = (size_t)p.n_splits * p.hkv * p.rows_pad * head_dim * 2;
-  if (p.map.n || (!streamed && p.part_half && p.n_splits <= kMergeFewSplits && head_dim % 8 == 0 && head_dim <= 512 && part_bytes < ((size_t)32 << 20))) {
+  if (p.map.n || (!streamed && p.part_half && head_dim % 8 == 0 && head_dim <= 512 && merge_at_once(p.n_splits, part_bytes))) {
     MergeArgs a;
     a.p = p;
     a.div_rows = make_fast_div(p.rows_total);
@@ -613,6 +612,10 @@ hipError_t launch_attn_merge(const AttnParams& p, uint32_t head_dim, bool stream
       case 6: return launch_merge_few<6>(a, rows, s);
       case 7: return launch_merge_few<7>(a, rows, s);
       case 8: return launch_merge_few<8>(a, rows, s);
+      case 9: case 10: return launch_merge_few<10>(a, rows, s);
+      case 11: case 12: return launch_merge_few<12>(a, rows, s);
+      case 13: case 14: return launch_merge_few<14>(a, rows, s);
+      case 15: case 16: return launch_merge_few<16>(a, rows, s);
       default: break;
     }
   }

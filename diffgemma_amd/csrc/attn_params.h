@@ -280,6 +280,15 @@ __device__ __forceinline__ void dbg_report(uint32_t* dbg, uint32_t code, uint32_
   }
 }
 
+// Where the merge that asks for all of a row's 16-bit partial rows at once beats the one that looks at the weights first, four
+// rows at a time: up to 8 splits while they are less than 32 MiB in all; up to 16 where they are few bytes.  Attention call, us,
+// weights first | at once, flat and peaked rows (of which the first fetches a part): 64 rows over 841 keys in 9 splits 20.4 | 18.3,
+// 19.1 | 18.0, over 5064 in 16 32.2 | 29.4, 31.7 | 28.9; past 17 MiB 128 rows over 428 keys in 14 splits 20.4 | 27.1 on peaked rows.
+constexpr uint32_t kMergeFewSplits = 16;
+inline bool merge_at_once(uint32_t n_splits, size_t bytes) {
+  return n_splits <= 8 ? bytes < ((size_t)32 << 20) : n_splits <= kMergeFewSplits && bytes <= ((size_t)17 << 20);
+}
+
 // host-side launchers (defined next to their kernels)
 hipError_t launch_attn_scalar(const AttnParams& p, uint32_t head_dim, uint32_t kv_dtype, hipStream_t s);
 hipError_t launch_attn_mfma(const AttnParams& p, uint32_t head_dim, uint32_t kv_dtype, hipStream_t s);

@@ -147,24 +147,28 @@ struct Plan {
 // Key tiles per split of the split kernel where the library chooses.  `base` = workgroups of one split, `room` = splits that
 // keep it one round of the chip.
 //
-// head_dim 512: a tile takes c = 1.3 to 1.6 us, and a split costs what its partial rows cost, written and read back, about
-// m = 0.12 us per 16 row tiles and key range, i.e. 9 c m / room for `base` of them: c n / s + m' s is least at
-// s = sqrt(n room / 9).  The curve is flat around it.  Attention call, us, splits of 6 tiles and more | this rule:
-// 64 rows (room 32) over 86 keys 14.6 | 13.3, over 364 20.0 | 15.5, 841 21.0 | 18.1, 2064 23.7 | 22.6, 5064 29.2 | 29.2; 128 rows
-// (16) over 428 keys 21.7 | 18.6, 905 23.8 | 22.9, 2128 29.0 | 30.1; 256 rows (8) over 278 22.2 | 20.5, 356 23.3 | 21.9,
-// 556 24.4 | 24.5, 1033 26.7 | 27.0; 300 causal rows (6) 22.8 | 19.4.
+// head_dim 512: a tile takes c = 1.3 to 1.6 us, and a split what its partial rows take, written and read back, about 9 c / room:
+// c n / s + 9 c s / room is least at s = sqrt(n room / 9).  The curve is flat around it; where it leads past the splits that
+// are merged at once, fewer are taken as long as that makes a share at most three tiles longer.  Attention call, us, splits
+// of 6 tiles and more | this rule: 64 rows (room 32) over 86 keys 14.6 | 13.3, over 364 20.0 | 15.5, 841 21.0 | 18.3, 2064 25.9 | 23.7,
+// 5064 31.2 | 29.4; 128 rows (16) over 428 keys 21.7 | 18.6, 905 23.8 | 22.9, 2128 28.7 | 28.1; 256 rows (8) over 278 22.2 | 20.5,
+// 356 23.3 | 21.9, 556 24.4 | 24.5, 1033 26.7 | 27.0; 300 causal rows (6) 22.8 | 19.4.
 //
 // Smaller head_dim: no split shorter than 6 tiles (a sliding layer's 40 tiles, step in us: 4 splits 25.7, 5 splits 24.8,
 // 6 and 7 splits 23.7, 8 splits 24.5, 10 splits 33.4).
-uint32_t tiles_of_split(uint32_t ntiles, uint32_t room, uint32_t hd, bool long_splits) {
-  room = std::max(1u, std::min(room, kMaxSplits));
+uint32_t tiles_of_split(uint32_t ntiles, uint32_t base, uint32_t cus, uint32_t hd, bool long_splits) {
+  const uint32_t room = std::max(1u, std::min(cus / std::max(1u, base), kMaxSplits));
   if (hd != 512 || long_splits) {
     const uint32_t s = std::min(room, std::max(1u, ntiles / 6u));
     return (ntiles + s - 1) / s;
   }
+  auto of = [&](uint32_t splits) { return (ntiles + splits - 1) / splits; };
   const double s = std::sqrt((double)ntiles * room / 9.0);
-  const uint32_t t = std::max(1u, (uint32_t)(ntiles / s + 0.5));
-  return std::max(t, (ntiles + room - 1) / room);
+  const uint32_t t = std::max(std::max(1u, (uint32_t)(ntiles / s + 0.5)), of(room));
+  const size_t split_bytes = (size_t)base * dg::kBlockM * hd * 2;
+  for (uint32_t few = dg::kMergeFewSplits; few >= 8u && !dg::merge_at_once(of(t), of(t) * split_bytes); few -= 8u)
+    if (dg::merge_at_once(of(of(few)), of(of(few)) * split_bytes)) return of(few) > t && of(few) <= t + 3u ? of(few) : t;
+  return t;
 }
 
 // Row tiles that see different numbers of key tiles (causal rows of a global layer): split counts of their own, so that no
@@ -300,7 +304,7 @@ int make_plan(const dg_attn_desc* d, int cus, Plan* pl, const uint32_t* key_rang
     pl->wsplit = !pl->scalar && hd <= 256 && d->n_splits == 0 && !(d->flags & DG_ATTN_F_SPLIT_OVER_WORKGROUPS) &&
                  span_tiles <= kWsplitMaxTiles;
   }
-  const uint32_t room = (uint32_t)cus / std::max(1u, d->n_kv_heads * pl->n_mtiles);
+  const uint32_t base = d->n_kv_heads * pl->n_mtiles;
   // workspace carve-up, with splits of `tps` key tiles
   auto carve = [&](uint32_t tps) {
     pl->tiles_per_split = tps;
@@ -331,7 +335,7 @@ int make_plan(const dg_attn_desc* d, int cus, Plan* pl, const uint32_t* key_rang
     const uint32_t splits = std::min(std::min(d->n_splits, kMaxSplits), ntiles);
     carve((ntiles + splits - 1) / splits);
   } else {
-    carve(tiles_of_split(ntiles, room, hd, false));
+    carve(tiles_of_split(ntiles, base, (uint32_t)cus, hd, false));
     dg::SplitMap map;
     if (!key_range && plan_split_map(d, *pl, cus, ntiles, &map)) {
       // (sized for either, so that one workspace serves the entry points with and without a host-known prefix)
@@ -344,7 +348,7 @@ int make_plan(const dg_attn_desc* d, int cus, Plan* pl, const uint32_t* key_rang
         pl->total = both;
       }
     }
-    if (pl->total > scratch) carve(tiles_of_split(ntiles, room, hd, true));
+    if (pl->total > scratch) carve(tiles_of_split(ntiles, base, (uint32_t)cus, hd, true));
   }
   return DG_OK;
 }
@@ -1009,10 +1013,10 @@ int dg_attention_block_state_bytes(const dg_layer_offsets* L, const dg_attn_dims
   rc = make_plan(&pd, cus, &pl);
   if (rc != DG_OK) return rc;
   const uint32_t ntiles_full = std::max(1u, (pl.t_all + dg::kBlockN - 1) / dg::kBlockN);
-  const uint32_t room = (uint32_t)cus / std::max(1u, d.n_kv_heads * pl.n_mtiles);
+  const uint32_t base = d.n_kv_heads * pl.n_mtiles, room = (uint32_t)cus / std::max(1u, base);
   uint32_t most = 1;
   for (uint32_t n = 1; n <= ntiles_full && most < std::min(room, kMaxSplits); ++n) {
-    const uint32_t t = tiles_of_split(n, room, d.head_dim, false);
+    const uint32_t t = tiles_of_split(n, base, (uint32_t)cus, d.head_dim, false);
     most = std::max(most, (n + t - 1) / t);
   }
   size_t ws_part = 0;
