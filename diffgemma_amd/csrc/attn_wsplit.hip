@@ -376,7 +376,7 @@ __global__ void __launch_bounds__(256) attn_wsplit_kernel(const WsArgs args) {
   };
   // ---- online softmax with a lazily raised reference max: the tile's probabilities in the MFMA's operand layout ----
   u32x4 pk[MR][2];
-  auto softmax = [&](auto m_c, float tmax) __attribute__((always_inline)) {
+  auto raise_reference = [&](auto m_c, float tmax) __attribute__((always_inline)) {
     constexpr int m = decltype(m_c)::value;
     tmax = max_across_halves(tmax) * p.scale_log2;
     const bool raise = __builtin_amdgcn_ballot_w64(tmax > m_ref[m] + kWsTau<F16>) != 0ull;
@@ -410,36 +410,32 @@ __global__ void __launch_bounds__(256) attn_wsplit_kernel(const WsArgs args) {
       }
       m_ref[m] = m_new;
     }
-    // The probabilities are 2^(score - reference - offset): with bf16 the offset puts a weight 2^40 below the
-    // reference (and so below the row's largest) under the smallest normal number, an exact zero.
+  };
+  // The probabilities are 2^(score - reference - offset): with bf16 the offset puts a weight 2^40 below the
+  // reference (and so below the row's largest) under the smallest normal number, an exact zero.  Scores 4 q .. 4 q + 3.
+  auto probs = [&](auto m_c, auto q_c) __attribute__((always_inline)) {
+    constexpr int m = decltype(m_c)::value, q = decltype(q_c)::value;
     const float m_use = (m_ref[m] == -INFINITY) ? 0.f : m_ref[m] + kWsPOff<F16>;
-    static_for<0, 4>([&](auto q_c) {
-      constexpr int q = decltype(q_c)::value;
-      float ex[4];
+    float ex[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) ex[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[m][4 * q + i], p.scale_log2, -m_use));
-      pk[m][q >> 1][(2 * q) & 3] = pack2<F16>(ex[0], ex[1]);
-      pk[m][q >> 1][(2 * q + 1) & 3] = pack2<F16>(ex[2], ex[3]);
-    });
+    for (int i = 0; i < 4; ++i) ex[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[m][4 * q + i], p.scale_log2, -m_use));
+    const uint32_t a = pack2<F16>(ex[0], ex[1]), b = pack2<F16>(ex[2], ex[3]);
+    pk[m][q >> 1][(2 * q) & 3] = a;
+    pk[m][q >> 1][(2 * q + 1) & 3] = b;
     // the row sum uses the rounded probabilities, the same numbers P.V multiplies
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      l_part[m] = ws_add_pair<F16>(pk[m][ks][0], l_part[m]);
-      l_part2[m] = ws_add_pair<F16>(pk[m][ks][1], l_part2[m]);
-      l_part[m] = ws_add_pair<F16>(pk[m][ks][2], l_part[m]);
-      l_part2[m] = ws_add_pair<F16>(pk[m][ks][3], l_part2[m]);
-    }
+    l_part[m] = ws_add_pair<F16>(a, l_part[m]);
+    l_part2[m] = ws_add_pair<F16>(b, l_part2[m]);
   };
   // O^T += V^T.P^T, a V fragment serving every row block
-  auto pv = [&]() __attribute__((always_inline)) {
+  auto pv = [&](auto ks_c, auto&& between) __attribute__((always_inline)) {
+    constexpr int ks = decltype(ks_c)::value;
+    static_for<0, NDB>([&](auto db_c) {
+      constexpr int db = decltype(db_c)::value;
+      const u32x4 vf = v_frag(ks, db);
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-      for (int db = 0; db < NDB; ++db) {
-        const u32x4 vf = v_frag(ks, db);
-#pragma unroll
-        for (int m = 0; m < MR; ++m) o[m][db] = mfma16<F16>(vf, pk[m][ks], o[m][db]);
-      }
+      for (int m = 0; m < MR; ++m) o[m][db] = mfma16<F16>(vf, pk[m][ks], o[m][db]);
+      between(db_c);
+    });
   };
   // scores of `tile` (its K has landed) with the loads of its V, two at a time, between them: they have the rest of the
   // scores, the issue of the next K tile and the softmax to land
@@ -466,11 +462,31 @@ __global__ void __launch_bounds__(256) attn_wsplit_kernel(const WsArgs args) {
     // them here, behind the tile max and ahead of everything that depends on it.  (Between the softmax and P.V
     // instructions, one at a time, they land too late for the next scores: 22.4 -> 24.3 us for a sliding layer's step.)
     if (more) issue_k(tile + 1u);
-    static_for<0, MR>([&](auto m_c) { softmax(m_c, tmax[decltype(m_c)::value]); });
+    static_for<0, MR>([&](auto m_c) { raise_reference(m_c, tmax[decltype(m_c)::value]); });
+    static_for<0, MR>([&](auto m_c) {
+      probs(m_c, std::integral_constant<int, 0>{});
+      probs(m_c, std::integral_constant<int, 1>{});
+    });
     // V(jj) has landed (the loads of K(jj+1), issued after it, may still be on their way)
     if (more) wait_vmem_but<NBLK>();
     else wait_vmem_all();
-    pv();
+    // With 64 rows the probabilities of the last 16 keys are worked out between the products of the first 16 (901 causal rows 27.6
+    // -> 26.7 us, 700 over an f16 cache 36.5 -> 35.1); with 32 rows the load path sets the pace, and the wave gets to the next
+    // loads' wait that much earlier for nothing (256 rows 17.8 -> 18.1).
+    constexpr int PIECES = 2 * MR, PER = NDB >= PIECES ? NDB / PIECES : 1;
+    constexpr bool BETWEEN = MR > 1 && NDB >= PIECES;
+    if constexpr (!BETWEEN)
+      static_for<0, PIECES>([&](auto x_c) {
+        probs(std::integral_constant<int, decltype(x_c)::value / 2>{}, std::integral_constant<int, 2 + decltype(x_c)::value % 2>{});
+      });
+    pv(std::integral_constant<int, 0>{}, [&](auto db_c) {
+      constexpr int db = decltype(db_c)::value;
+      if constexpr (BETWEEN && db % PER == 0 && db / PER < PIECES) {
+        probs(std::integral_constant<int, db / PER / 2>{}, std::integral_constant<int, 2 + db / PER % 2>{});
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    });
+    pv(std::integral_constant<int, 1>{}, [](auto) {});
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the V buffer is free for the next tile's loads
     if (more) {
       wait_vmem_all();   // K(jj+1), the only load outstanding
