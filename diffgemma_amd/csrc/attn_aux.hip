@@ -260,8 +260,9 @@ struct MergeArgs {
   AttnParams p;
   FastDiv div_rows, div_group;   // by the rows of a KV head and by the GQA group
   uint32_t hd;
+  SplitMap map;
 };
-// MAPPED: row tiles have split counts of their own (AttnParams.map), at most N; rows of one split are in the output already.
+// MAPPED: row tiles have split counts of their own (a split map), at most N; rows of one split are in the output already.
 template <uint32_t N, bool MAPPED>
 __global__ void __launch_bounds__(256) attn_merge_few_kernel(const MergeArgs args) {
   const AttnParams& p = args.p;
@@ -276,12 +277,12 @@ __global__ void __launch_bounds__(256) attn_merge_few_kernel(const MergeArgs arg
   const uint32_t mt = r / (uint32_t)kBlockM;
   uint32_t n = N <= 8 ? N : p.n_splits, prow[N];   // partial row of each split; past n one that exists, with weight zero
   if constexpr (MAPPED) {
-    n = map_splits(p.map, mt);
+    n = map_splits(args.map, mt);
     if (n == 1u) return;
 #pragma unroll
     for (uint32_t u = 0; u < N; ++u) {
       const uint32_t i = u < n ? u : 0u;
-      prow[u] = (kvh * p.map.units + p.map.cum[i] + mt - p.map.first[i]) * (uint32_t)kBlockM + r % (uint32_t)kBlockM;
+      prow[u] = (kvh * args.map.units + args.map.cum[i] + mt - args.map.first[i]) * (uint32_t)kBlockM + r % (uint32_t)kBlockM;
     }
   } else {
 #pragma unroll
@@ -355,7 +356,7 @@ __global__ void __launch_bounds__(256) attn_merge_few_kernel(const MergeArgs arg
 
 template <uint32_t N>
 hipError_t launch_merge_few(const MergeArgs& a, uint32_t rows, hipStream_t s) {
-  if (a.p.map.n) hipLaunchKernelGGL((attn_merge_few_kernel<N, true>), dim3((rows + 3) / 4), dim3(256), 0, s, a);
+  if (a.map.n) hipLaunchKernelGGL((attn_merge_few_kernel<N, true>), dim3((rows + 3) / 4), dim3(256), 0, s, a);
   else hipLaunchKernelGGL((attn_merge_few_kernel<N, false>), dim3((rows + 3) / 4), dim3(256), 0, s, a);
   return hipGetLastError();
 }
@@ -594,17 +595,18 @@ hipError_t launch_state_merge(const StateMergeParams& p, hipStream_t s) {
   return hipGetLastError();
 }
 
-hipError_t launch_attn_merge(const AttnParams& p, uint32_t head_dim, bool streamed, hipStream_t s) {
+hipError_t launch_attn_merge(const AttnParams& p, const SplitMap& map, uint32_t head_dim, bool streamed, hipStream_t s) {
   const uint32_t rows = p.hkv * p.rows_total;
   // not many splits, not many bytes: the variant that asks for every partial row up front
   const size_t part_bytes = (size_t)p.n_splits * p.hkv * p.rows_pad * head_dim * 2;
-  if (p.map.n || (!streamed && p.part_half && head_dim % 8 == 0 && head_dim <= 512 && merge_at_once(p.n_splits, part_bytes))) {
+  if (map.n || (!streamed && p.part_half && head_dim % 8 == 0 && head_dim <= 512 && merge_at_once(p.n_splits, part_bytes))) {
     MergeArgs a;
     a.p = p;
     a.div_rows = make_fast_div(p.rows_total);
     a.div_group = make_fast_div(p.group);
     a.hd = head_dim;
-    switch (p.map.n ? p.map.n : p.n_splits) {
+    a.map = map;
+    switch (map.n ? map.n : p.n_splits) {
       case 2: return launch_merge_few<2>(a, rows, s);
       case 3: return launch_merge_few<3>(a, rows, s);
       case 4: return launch_merge_few<4>(a, rows, s);

@@ -105,6 +105,7 @@ struct MfmaArgs {
   AttnParams p;
   FastDiv div_mtiles, div_splits, div_group;
   FastDiv div_units, div_n[kMapSplits];   // with a split map: by the units of a KV head, by 1 .. 8
+  SplitMap map;
 };
 
 // MAPPED: with a split map (an instance of its own: what the map takes at a workgroup's start is 0.3 us of a short call)
@@ -152,7 +153,7 @@ __global__ void __launch_bounds__(256) attn_mfma_kernel(const MfmaArgs args) {
   // (KV head, split) first and row tile second, are cut into 8 equal runs, one per XCD, so the
   // row tiles that stream the same keys sit behind one L2 and every XCD has work whatever
   // the number of (KV head, split) pairs.
-  const SplitMap& map = args.p.map;
+  const SplitMap& map = args.map;
   const uint32_t n_units = p.hkv * (MAPPED ? map.units : p.n_splits * p.n_mtiles);
   const uint32_t per_xcd = (n_units + 7u) >> 3;
   const uint32_t wg = blockIdx.x;
@@ -870,22 +871,23 @@ __global__ void __launch_bounds__(256) attn_mfma_kernel(const MfmaArgs args) {
 }
 
 template <int D, bool F16>
-hipError_t launch_one(const AttnParams& p, hipStream_t s) {
+hipError_t launch_one(const AttnParams& p, const SplitMap& map, hipStream_t s) {
   MfmaArgs a;
   a.p = p;
+  a.map = map;
   a.div_mtiles = make_fast_div(p.n_mtiles);
   a.div_splits = make_fast_div(p.n_splits);
   a.div_group = make_fast_div(p.group);
-  a.div_units = make_fast_div(std::max(1u, p.map.units));
+  a.div_units = make_fast_div(std::max(1u, map.units));
   for (uint32_t i = 0; i < kMapSplits; ++i) a.div_n[i] = make_fast_div(i + 1u);
-  const uint32_t n_units = p.hkv * (p.map.n ? p.map.units : p.n_splits * p.n_mtiles);
+  const uint32_t n_units = p.hkv * (map.n ? map.units : p.n_splits * p.n_mtiles);
   const uint32_t grid = (n_units + 7u) / 8u * 8u;
   auto launch = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), 0, s, a);
     return hipGetLastError();
   };
   if constexpr (D == 512) {
-    if (p.map.n) return p.touch_ahead ? launch(attn_mfma_kernel<D, F16, true, true>) : launch(attn_mfma_kernel<D, F16, false, true>);
+    if (map.n) return p.touch_ahead ? launch(attn_mfma_kernel<D, F16, true, true>) : launch(attn_mfma_kernel<D, F16, false, true>);
     if (p.touch_ahead) return launch(attn_mfma_kernel<D, F16, true, false>);
   }
   return launch(attn_mfma_kernel<D, F16, false, false>);
@@ -893,14 +895,14 @@ hipError_t launch_one(const AttnParams& p, hipStream_t s) {
 
 }  // namespace
 
-hipError_t launch_attn_mfma(const AttnParams& p, uint32_t head_dim, uint32_t kv_dtype, hipStream_t s) {
+hipError_t launch_attn_mfma(const AttnParams& p, const SplitMap& map, uint32_t head_dim, uint32_t kv_dtype, hipStream_t s) {
   const bool f16 = kv_dtype == DT_F16;
   switch (head_dim) {
-    case 32: return f16 ? launch_one<32, true>(p, s) : launch_one<32, false>(p, s);
-    case 64: return f16 ? launch_one<64, true>(p, s) : launch_one<64, false>(p, s);
-    case 128: return f16 ? launch_one<128, true>(p, s) : launch_one<128, false>(p, s);
-    case 256: return f16 ? launch_one<256, true>(p, s) : launch_one<256, false>(p, s);
-    case 512: return f16 ? launch_one<512, true>(p, s) : launch_one<512, false>(p, s);
+    case 32: return f16 ? launch_one<32, true>(p, map, s) : launch_one<32, false>(p, map, s);
+    case 64: return f16 ? launch_one<64, true>(p, map, s) : launch_one<64, false>(p, map, s);
+    case 128: return f16 ? launch_one<128, true>(p, map, s) : launch_one<128, false>(p, map, s);
+    case 256: return f16 ? launch_one<256, true>(p, map, s) : launch_one<256, false>(p, map, s);
+    case 512: return f16 ? launch_one<512, true>(p, map, s) : launch_one<512, false>(p, map, s);
     default: return hipErrorInvalidValue;
   }
 }

@@ -90,7 +90,6 @@ struct AttnParams {
   uint32_t cus;          // compute units of the device
   uint32_t sees_masked;  // causal rows also see the canvas keys behind the causal rows
   float scale_log2;      // softmax_scale * log2(e)
-  SplitMap map;          // (split kernel and its merge)
 };
 
 // Division of n < 2^31 by a divisor the host knows: q = (mulhi(n, mul) + n) >> shift (the round-up method: mul =
@@ -291,9 +290,12 @@ inline bool merge_at_once(uint32_t n_splits, size_t bytes) {
 
 // host-side launchers (defined next to their kernels)
 hipError_t launch_attn_scalar(const AttnParams& p, uint32_t head_dim, uint32_t kv_dtype, hipStream_t s);
-hipError_t launch_attn_mfma(const AttnParams& p, uint32_t head_dim, uint32_t kv_dtype, hipStream_t s);
+// (map: row tiles with split counts of their own, head_dim 512; n = 0 for none. It stands behind AttnParams in the
+// arguments of these two and not inside it: its 72 bytes pushed what the one-launch kernel reads first to a further
+// line of the arguments, and a call with 64 canvas rows on a sliding layer took 9.77 us for 9.52.)
+hipError_t launch_attn_mfma(const AttnParams& p, const SplitMap& map, uint32_t head_dim, uint32_t kv_dtype, hipStream_t s);
 hipError_t launch_attn_wsplit(const AttnParams& p, uint32_t head_dim, uint32_t kv_dtype, hipStream_t s);
-hipError_t launch_attn_merge(const AttnParams& p, uint32_t head_dim, bool streamed, hipStream_t s);
+hipError_t launch_attn_merge(const AttnParams& p, const SplitMap& map, uint32_t head_dim, bool streamed, hipStream_t s);
 hipError_t launch_state_merge(const StateMergeParams& p, hipStream_t s);
 // l[row] = 1 where m[row] is finite, else 0: completes a state whose rows are already normalised
 hipError_t launch_state_unit_l(float* m_plane, float* l_plane, uint32_t rows, hipStream_t s);

@@ -499,7 +499,6 @@ int fill_params(const dg_attn_desc* d, const Plan& pl, const void* q, const void
   p.rows_pad = pl.rows_pad;
   p.n_mtiles = pl.n_mtiles;
   p.n_splits = pl.n_splits;
-  p.map = pl.map;
   p.tile_first = pl.tile_first;
   p.tiles_per_split = pl.tiles_per_split;
   p.tile_end = pl.tile_end;
@@ -553,13 +552,13 @@ int forward_planned(const dg_attn_desc* d, const Plan& pl, const void* q, const 
   }
   const bool prof = g_prof.active && 2 * (size_t)g_prof.used + 1 < g_prof.ev.size();
   if (prof) (void)hipEventRecord(g_prof.ev[2 * g_prof.used], s);
-  if ((pl.wsplit ? dg::launch_attn_wsplit(p, hd, pl.e_dtype, s) : dg::launch_attn_mfma(p, hd, pl.e_dtype, s)) != hipSuccess)
+  if ((pl.wsplit ? dg::launch_attn_wsplit(p, hd, pl.e_dtype, s) : dg::launch_attn_mfma(p, pl.map, hd, pl.e_dtype, s)) != hipSuccess)
     return DG_ERR_LAUNCH;
   if (prof) {
     (void)hipEventRecord(g_prof.ev[2 * g_prof.used + 1], s);
     ++g_prof.used;
   }
-  if (pl.n_splits > 1 && dg::launch_attn_merge(p, hd, (d->flags & DG_ATTN_F_STREAMED_MERGE) != 0, s) != hipSuccess) return DG_ERR_LAUNCH;
+  if (pl.n_splits > 1 && dg::launch_attn_merge(p, pl.map, hd, (d->flags & DG_ATTN_F_STREAMED_MERGE) != 0, s) != hipSuccess) return DG_ERR_LAUNCH;
   return DG_OK;
 }
 }  // namespace
