@@ -249,7 +249,7 @@ __global__ void __launch_bounds__(256) attn_merge_kernel(const AttnParams p, con
   }
 }
 
-// The same merge for few splits of f16 partial rows whose total is small (merge_at_once): there the kernel is as long as one
+// The same merge for few splits whose partial rows are small in total (merge_at_once): there the kernel is as long as one
 // wave's chain of memory round trips, not bandwidth.  So a wave asks for everything at once, the (m, l) pairs and the partial
 // rows of all splits, instead of weights first and then rows four at a time; and the weights come from lane-to-scalar
 // reads, every lane doing the same arithmetic, instead of a dozen dependent shuffles.  One instance per split count up to 8,
@@ -263,7 +263,9 @@ struct MergeArgs {
   SplitMap map;
 };
 // MAPPED: row tiles have split counts of their own (a split map), at most N; rows of one split are in the output already.
-template <uint32_t N, bool MAPPED>
+// F32_CH > 0: fp32 partial rows in at most 8 splits, four elements of each of F32_CH runs of 256 to a lane, added as the other
+// kernel adds them.  (head_dim 512, 64 rows, us, streamed | at once: over 184 keys in 3 splits 18.3 | 17.3, over 314 in 5 18.8 | 18.4.)
+template <uint32_t N, bool MAPPED, uint32_t F32_CH = 0>
 __global__ void __launch_bounds__(256) attn_merge_few_kernel(const MergeArgs args) {
   const AttnParams& p = args.p;
   const uint32_t hd = args.hd;
@@ -275,6 +277,7 @@ __global__ void __launch_bounds__(256) attn_merge_few_kernel(const MergeArgs arg
   const bool live = lane < hd / 8;
   const uint32_t d8 = live ? lane : 0u;
   const uint32_t mt = r / (uint32_t)kBlockM;
+  const size_t ooff = ((size_t)tok * p.hq + qh) * hd;
   uint32_t n = N <= 8 ? N : p.n_splits, prow[N];   // partial row of each split; past n one that exists, with weight zero
   if constexpr (MAPPED) {
     n = map_splits(args.map, mt);
@@ -296,8 +299,16 @@ __global__ void __launch_bounds__(256) attn_merge_few_kernel(const MergeArgs arg
   }
   const float2 ml = *(const float2*)(p.part_ml + (size_t)my_row * 2);
   uint4 a[N];
+  float4 f[N][F32_CH ? F32_CH : 1];
 #pragma unroll
-  for (uint32_t u = 0; u < N; ++u) a[u] = ((const uint4*)((const uint16_t*)p.part_o + (size_t)prow[u] * hd))[d8];
+  for (uint32_t u = 0; u < N; ++u) {
+    if constexpr (F32_CH == 0) {
+      a[u] = ((const uint4*)((const uint16_t*)p.part_o + (size_t)prow[u] * hd))[d8];
+    } else {
+#pragma unroll
+      for (uint32_t c = 0; c < F32_CH; ++c) f[u][c] = ((const float4*)(p.part_o + (size_t)prow[u] * hd))[min(c * 64u + lane, hd / 4u - 1u)];
+    }
+  }
   constexpr uint32_t W = N <= 8 ? 8 : 16;
   float msu[N], wlu[N], sum[W];
   float mx = -INFINITY;
@@ -320,9 +331,47 @@ __global__ void __launch_bounds__(256) attn_merge_few_kernel(const MergeArgs arg
     for (uint32_t u = 0; u < w; ++u) sum[u] += sum[u + w];
   const float den = sum[0];
   const float inv = den > 0.f ? 1.f / den : 0.f;
+  if constexpr (F32_CH > 0) {
+    float w[N];
+#pragma unroll
+    for (uint32_t u = 0; u < N; ++u) w[u] = wlu[u] > 0.f ? exp2f(msu[u] - mx) * inv : 0.f;
+#pragma unroll
+    for (uint32_t c = 0; c < F32_CH; ++c) {
+      float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
+      constexpr uint32_t N4 = N / 4 * 4;
+#pragma unroll
+      for (uint32_t u = 0; u < N4; u += 4) {
+        o.x += w[u] * f[u][c].x + w[u + 1] * f[u + 1][c].x + w[u + 2] * f[u + 2][c].x + w[u + 3] * f[u + 3][c].x;
+        o.y += w[u] * f[u][c].y + w[u + 1] * f[u + 1][c].y + w[u + 2] * f[u + 2][c].y + w[u + 3] * f[u + 3][c].y;
+        o.z += w[u] * f[u][c].z + w[u + 1] * f[u + 1][c].z + w[u + 2] * f[u + 2][c].z + w[u + 3] * f[u + 3][c].z;
+        o.w += w[u] * f[u][c].w + w[u + 1] * f[u + 1][c].w + w[u + 2] * f[u + 2][c].w + w[u + 3] * f[u + 3][c].w;
+      }
+#pragma unroll
+      for (uint32_t u = N4; u < N; ++u) {
+        o.x += w[u] * f[u][c].x;
+        o.y += w[u] * f[u][c].y;
+        o.z += w[u] * f[u][c].z;
+        o.w += w[u] * f[u][c].w;
+      }
+      const uint32_t d4 = c * 64u + lane;
+      if (d4 >= hd / 4) break;
+      if (p.dbg && (nonfinite(o.x) || nonfinite(o.y) || nonfinite(o.z) || nonfinite(o.w)))
+        dbg_report(p.dbg, DBG_ERR_NONFINITE, DBG_KERNEL_ATTENTION, (tok << 16) | qh, d4 * 4u);
+      if (p.out_dtype == DT_F32) {
+        const wt_u32x4 o4 = {__float_as_uint(o.x), __float_as_uint(o.y), __float_as_uint(o.z), __float_as_uint(o.w)};
+        wt_store16(wt_window_wave((const float*)p.out + ooff), d4 * 16u, o4);
+      } else {
+        const bool tr = p.out_trunc != 0;
+        const wt_u32x2 pk2 = {(uint32_t)f32_to_bf16_bits(o.x, tr) | ((uint32_t)f32_to_bf16_bits(o.y, tr) << 16),
+                              (uint32_t)f32_to_bf16_bits(o.z, tr) | ((uint32_t)f32_to_bf16_bits(o.w, tr) << 16)};
+        wt_store8(wt_window_wave((const uint16_t*)p.out + ooff), d4 * 8u, pk2);
+      }
+    }
+  }
   float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (uint32_t u = 0; u < N; ++u) {
+    if constexpr (F32_CH > 0) break;
     const float w = wlu[u] * inv;
     if (w >= 5.9604645e-8f) {   // the same in every lane
       const uint32_t wd[4] = {a[u].x, a[u].y, a[u].z, a[u].w};
@@ -333,8 +382,7 @@ __global__ void __launch_bounds__(256) attn_merge_few_kernel(const MergeArgs arg
       }
     }
   }
-  const size_t ooff = ((size_t)tok * p.hq + qh) * hd;
-  if (live) {   // (16-bit partial rows: the output is bf16)
+  if (F32_CH == 0 && live) {   // (16-bit partial rows: the output is bf16)
     if (p.dbg) {
       bool bad = false;
 #pragma unroll
@@ -356,7 +404,11 @@ __global__ void __launch_bounds__(256) attn_merge_few_kernel(const MergeArgs arg
 
 template <uint32_t N>
 hipError_t launch_merge_few(const MergeArgs& a, uint32_t rows, hipStream_t s) {
-  if (a.map.n) hipLaunchKernelGGL((attn_merge_few_kernel<N, true>), dim3((rows + 3) / 4), dim3(256), 0, s, a);
+  if (!a.p.part_half) {
+    if constexpr (N > 8) return hipErrorInvalidValue;   // (not asked for)
+    else if (a.hd <= 256) hipLaunchKernelGGL((attn_merge_few_kernel<N, false, 1>), dim3((rows + 3) / 4), dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((attn_merge_few_kernel<N, false, 2>), dim3((rows + 3) / 4), dim3(256), 0, s, a);
+  } else if (a.map.n) hipLaunchKernelGGL((attn_merge_few_kernel<N, true>), dim3((rows + 3) / 4), dim3(256), 0, s, a);
   else hipLaunchKernelGGL((attn_merge_few_kernel<N, false>), dim3((rows + 3) / 4), dim3(256), 0, s, a);
   return hipGetLastError();
 }
@@ -598,8 +650,8 @@ hipError_t launch_state_merge(const StateMergeParams& p, hipStream_t s) {
 hipError_t launch_attn_merge(const AttnParams& p, const SplitMap& map, uint32_t head_dim, bool streamed, hipStream_t s) {
   const uint32_t rows = p.hkv * p.rows_total;
   // not many splits, not many bytes: the variant that asks for every partial row up front
-  const size_t part_bytes = (size_t)p.n_splits * p.hkv * p.rows_pad * head_dim * 2;
-  if (map.n || (!streamed && p.part_half && head_dim % 8 == 0 && head_dim <= 512 && merge_at_once(p.n_splits, part_bytes))) {
+  const size_t part_bytes = (size_t)p.n_splits * p.hkv * p.rows_pad * head_dim * (p.part_half ? 2 : 4);
+  if (map.n || (!streamed && (p.part_half || p.n_splits <= 8) && head_dim % 8 == 0 && head_dim <= 512 && merge_at_once(p.n_splits, part_bytes))) {
     MergeArgs a;
     a.p = p;
     a.div_rows = make_fast_div(p.rows_total);

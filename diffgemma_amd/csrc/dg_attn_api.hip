@@ -150,12 +150,18 @@ struct Plan {
 // head_dim 512: a tile takes c = 1.3 to 1.6 us, and a split what its partial rows take, written and read back, about 9 c / room:
 // c n / s + 9 c s / room is least at s = sqrt(n room / 9).  The curve is flat around it; where it leads past the splits that
 // are merged at once, fewer are taken as long as that makes a share at most three tiles longer.  Attention call, us, splits
-// of 6 tiles and more | this rule: 64 rows (room 32) over 86 keys 14.6 | 13.3, over 364 20.0 | 15.5, 841 21.0 | 18.3, 2064 25.9 | 23.7,
-// 5064 31.2 | 29.4; 128 rows (16) over 428 keys 21.7 | 18.6, 905 23.8 | 22.9, 2128 28.7 | 28.1; 256 rows (8) over 278 22.2 | 20.5,
-// 356 23.3 | 21.9, 556 24.4 | 24.5, 1033 26.7 | 27.0; 300 causal rows (6) 22.8 | 19.4.
+// of 6 tiles and more | this rule: 64 rows (room 32) over 841 keys 21.0 | 18.3, 2064 25.9 | 23.7,
+// 5064 31.2 | 29.4; 128 rows (16) over 428 keys 21.7 | 18.6, 905 23.8 | 22.9, 2128 28.7 | 28.1; 256 rows (8) over 556 24.4 | 24.5, 1033 26.7 | 27.0.
+//
+// Fewer than kF32PartTiles tiles were one split as long as none was shorter than 6, and its rows fp32 until they are rounded for the
+// output: where these are split, the partial rows are fp32 too.  They cost twice as much, so sqrt(n room / 18), and one split
+// where that is small.  One split | this rule: 64 rows over 86 keys (n room 96) 14.2 | 16.0, over 184 (192) 18.4 | 17.1, over 314 (320)
+// 23.6 | 18.1; 128 rows over 150 (80) 17.1 | 18.5, 228 (128) 21.0 | 20.0; 256 over 346 (88) 25.1 | 26.2; 200 causal rows behind 150
+// (110) 25.9 | 25.7.
 //
 // Smaller head_dim: no split shorter than 6 tiles (a sliding layer's 40 tiles, step in us: 4 splits 25.7, 5 splits 24.8,
 // 6 and 7 splits 23.7, 8 splits 24.5, 10 splits 33.4).
+constexpr uint32_t kF32PartTiles = 12;
 uint32_t tiles_of_split(uint32_t ntiles, uint32_t base, uint32_t cus, uint32_t hd, bool long_splits) {
   const uint32_t room = std::max(1u, std::min(cus / std::max(1u, base), kMaxSplits));
   if (hd != 512 || long_splits) {
@@ -163,9 +169,11 @@ uint32_t tiles_of_split(uint32_t ntiles, uint32_t base, uint32_t cus, uint32_t h
     return (ntiles + s - 1) / s;
   }
   auto of = [&](uint32_t splits) { return (ntiles + splits - 1) / splits; };
-  const double s = std::sqrt((double)ntiles * room / 9.0);
+  const bool f32_parts = ntiles < kF32PartTiles;
+  if (f32_parts && ntiles * room < 108u) return ntiles;
+  const double s = std::sqrt((double)ntiles * room / (f32_parts ? 18.0 : 9.0));
   const uint32_t t = std::max(std::max(1u, (uint32_t)(ntiles / s + 0.5)), of(room));
-  const size_t split_bytes = (size_t)base * dg::kBlockM * hd * 2;
+  const size_t split_bytes = (size_t)base * dg::kBlockM * hd * (f32_parts ? 4 : 2);
   for (uint32_t few = dg::kMergeFewSplits; few >= 8u && !dg::merge_at_once(of(t), of(t) * split_bytes); few -= 8u)
     if (dg::merge_at_once(of(of(few)), of(of(few)) * split_bytes)) return of(few) > t && of(few) <= t + 3u ? of(few) : t;
   return t;
@@ -305,8 +313,8 @@ int make_plan(const dg_attn_desc* d, int cus, Plan* pl, const uint32_t* key_rang
                  span_tiles <= kWsplitMaxTiles;
   }
   const uint32_t base = d->n_kv_heads * pl->n_mtiles;
-  // workspace carve-up, with splits of `tps` key tiles
-  auto carve = [&](uint32_t tps) {
+  // workspace carve-up, with splits of `tps` key tiles; f32_parts: partial rows stay fp32 whatever the flags allow
+  auto carve = [&](uint32_t tps, bool f32_parts) {
     pl->tiles_per_split = tps;
     pl->n_splits = (ntiles + tps - 1) / tps;
     size_t off = 0;
@@ -319,7 +327,7 @@ int make_plan(const dg_attn_desc* d, int cus, Plan* pl, const uint32_t* key_rang
       off += align_up((size_t)2 * d->n_kv_heads * pl->t_all * hd * 2);
     }
     // f16 partial rows need |V| <= 65504: an f16 cache guarantees it, for a bf16 cache the caller says so
-    pl->part_half = pl->n_splits > 1 && d->out_dtype != DG_F32 && !(d->flags & DG_ATTN_F_F32_PARTIALS) &&
+    pl->part_half = pl->n_splits > 1 && !f32_parts && d->out_dtype != DG_F32 && !(d->flags & DG_ATTN_F_F32_PARTIALS) &&
                     (pl->e_dtype == DG_F16 || (d->flags & DG_ATTN_F_F16_PARTIALS));
     if (pl->n_splits > 1) {
       pl->off_part_o = off;
@@ -330,12 +338,12 @@ int make_plan(const dg_attn_desc* d, int cus, Plan* pl, const uint32_t* key_rang
     pl->total = off;
   };
   if (pl->scalar || pl->wsplit) {
-    carve(ntiles);
+    carve(ntiles, false);
   } else if (d->n_splits != 0) {
     const uint32_t splits = std::min(std::min(d->n_splits, kMaxSplits), ntiles);
-    carve((ntiles + splits - 1) / splits);
+    carve((ntiles + splits - 1) / splits, false);
   } else {
-    carve(tiles_of_split(ntiles, base, (uint32_t)cus, hd, false));
+    carve(tiles_of_split(ntiles, base, (uint32_t)cus, hd, false), hd == 512 && ntiles < kF32PartTiles);
     dg::SplitMap map;
     if (!key_range && plan_split_map(d, *pl, cus, ntiles, &map)) {
       // (sized for either, so that one workspace serves the entry points with and without a host-known prefix)
@@ -348,7 +356,7 @@ int make_plan(const dg_attn_desc* d, int cus, Plan* pl, const uint32_t* key_rang
         pl->total = both;
       }
     }
-    if (pl->total > scratch) carve(tiles_of_split(ntiles, base, (uint32_t)cus, hd, true));
+    if (pl->total > scratch) carve(tiles_of_split(ntiles, base, (uint32_t)cus, hd, true), false);
   }
   return DG_OK;
 }

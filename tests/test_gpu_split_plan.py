@@ -94,3 +94,28 @@ def test_device_prefix_with_the_scratch_of_a_split_map(gpu_ready, po):
         outs.append(out.view(torch.bfloat16).float())
     assert torch.equal(outs[1], outs[2])
     assert (outs[0] - outs[1]).abs().max() <= 2.0 ** -7 * outs[1].abs().max()
+
+
+@pytest.mark.parametrize("hd,hkv,f32_parts,out_f32", [(512, 2, False, False), (256, 8, False, False), (512, 2, True, False),
+                                                      (512, 2, True, True), (256, 8, True, False), (64, 2, True, True)])
+def test_merge_at_once_gives_the_bits_of_the_streamed_merge(gpu_ready, hd, hkv, f32_parts, out_f32):
+    """Every instance of the merge that asks for all partial rows up front, on ragged rows, flat and peaked."""
+    import torch
+    canvas, kv_len = 37, 2000
+    for n in (2, 3, 4, 5, 6, 7, 8, 9, 12, 13, 16):
+        for gain in (1.0, 0.05):
+            w = W.Workload("merge", canvas, 16, hkv, hd, kv_len, causal_rows=5, seed=n)
+            q, kv = W.generate(w)
+            qd, kd = W.device_arrays(w, q, kv)
+            qd = (qd.view(torch.bfloat16).float() * gain).to(torch.bfloat16)
+            flag = capi.DG_ATTN_F_F32_PARTIALS if f32_parts else capi.DG_ATTN_F_F16_PARTIALS
+            got = []
+            for extra in (0, capi.DG_ATTN_F_STREAMED_MERGE):
+                d = A.make_desc(canvas, 16, hkv, hd, kv_len, causal_rows=5, layout="head_major", t_cap=w.t_all, n_splits=n, flags=flag | extra |
+                                capi.DG_ATTN_F_SPLIT_OVER_WORKGROUPS, out_dtype=capi.DG_F32 if out_f32 else capi.DG_BF16)
+                out = torch.zeros(canvas, 16, hd, dtype=torch.float32 if out_f32 else torch.bfloat16, device="cuda")
+                lse = torch.zeros(canvas, 16, device="cuda")
+                A.forward(d, qd, kd, out, lse, A.alloc_workspace(d))
+                torch.cuda.synchronize()
+                got.append((out, lse))
+            assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
