@@ -425,6 +425,7 @@ __global__ void __launch_bounds__(256) topk_select_kernel(const TopkParams tp) {
     sh.n_cand = 0;
     sh.res[0] = sh.res[1] = sh.res[2] = 0;
   }
+  __syncthreads();   // (a short row's scan counts into the lists at once: a late wave 0 would reset what another has counted)
 
   uint32_t prefix = 0, pbits = 0, remaining = k, class_count = n_valid;
   int level = 0;
