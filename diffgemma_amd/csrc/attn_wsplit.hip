@@ -109,11 +109,14 @@ struct WsArgs {
   AttnParams p;
   FastDiv div_rt;        // by the number of row tiles
   FastDiv div_group;     // by the GQA group
+  FastDiv div_splits;    // by the workgroups that share a row tile's keys (AttnParams.n_splits)
   uint32_t n_rt;
   uint32_t touch;        // the key range is touched into the L2 first
 };
 
-template <int D, bool F16, int MR>
+// SHARED: several workgroups to a row tile (an instance of its own: what it takes at the start and the end is 0.4 us of a
+// launch of 7)
+template <int D, bool F16, int MR, bool SHARED>
 __global__ void __launch_bounds__(256) attn_wsplit_kernel(const WsArgs args) {
   const AttnParams p = resolve_step(args.p);
   using L = WsLay<D>;
@@ -129,12 +132,12 @@ __global__ void __launch_bounds__(256) attn_wsplit_kernel(const WsArgs args) {
   // ---- which (KV head, row tile) this workgroup owns: ids go round-robin over the 8 XCDs (each has its
   // own L2); the units, KV head first, are cut into 8 equal runs, so the row tiles of a head, which stream
   // the same keys, sit behind one L2 ----
-  const uint32_t n_units = p.hkv * args.n_rt;
+  const uint32_t n_units = p.hkv * (SHARED ? p.n_splits : 1u) * args.n_rt;
   const uint32_t per_xcd = (n_units + 7u) >> 3;
   const uint32_t unit = (blockIdx.x & 7u) * per_xcd + (blockIdx.x >> 3);
   if (unit >= n_units) return;
-  const uint32_t kvh = fast_div(unit, args.div_rt);
-  const uint32_t rt = unit - kvh * args.n_rt;
+  const uint32_t stream = fast_div(unit, args.div_rt), rt = unit - stream * args.n_rt;
+  const uint32_t kvh = SHARED ? fast_div(stream, args.div_splits) : stream, split = SHARED ? stream - kvh * p.n_splits : 0u;
 
   const uint32_t lane = threadIdx.x & 63u;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -160,9 +163,15 @@ __global__ void __launch_bounds__(256) attn_wsplit_kernel(const WsArgs args) {
     }
     if (tok_a < p.causal_rows && p.extra_lo < p.t_clip_hi) hi_max = p.t_clip_hi;
   }
-  // the key tiles these rows can see, cut into four equal runs, one per wave
-  const uint32_t mt_begin = max(lo_min / kBlockN, p.tile_first);
-  const uint32_t mt_end = max(min((hi_max + kBlockN - 1) / kBlockN, p.tile_end), mt_begin);
+  // the key tiles these rows can see (a run of them each for the workgroups that share a row tile), cut into four equal runs,
+  // one per wave
+  uint32_t mt_begin = max(lo_min / kBlockN, p.tile_first);
+  uint32_t mt_end = max(min((hi_max + kBlockN - 1) / kBlockN, p.tile_end), mt_begin);
+  if constexpr (SHARED) {
+    const uint32_t end = mt_end, per_split = fast_div(end - mt_begin + p.n_splits - 1u, args.div_splits);
+    mt_begin = min(mt_begin + split * per_split, end);
+    mt_end = min(mt_begin + per_split, end);
+  }
   const uint32_t per_run = (mt_end - mt_begin + 3u) >> 2;
   const uint32_t tb = min(mt_begin + wave * per_run, mt_end);
   const uint32_t te = min(tb + per_run, mt_end);
@@ -503,10 +512,13 @@ __global__ void __launch_bounds__(256) attn_wsplit_kernel(const WsArgs args) {
   constexpr int NU = D / 8, UPW = NU / 4;
   constexpr int OFF_T = 3 * NU * 1024, T_ROW = 4 * D + 16;   // finished rows, on their way to whole-row stores
   static_assert(OFF_T + 32 * T_ROW <= 4 * L::SLICE, "the tiles' LDS holds both");
-  const bool f32_out = p.out_dtype == DT_F32;
+  const bool f32_out = SHARED || p.out_dtype == DT_F32;
   const uint32_t cpr = f32_out ? D / 4 : D / 8;            // 16-byte chunks per row (a power of two)
   const uint32_t tok0 = fast_div(row0, args.div_group);
-  const auto out_win = wt_window((const char*)p.out + ((size_t)tok0 * p.hq + kvh * p.group) * (f32_out ? 4u * D : 2u * D));
+  // Workgroups that share a row tile leave fp32 rows relative to their (m, l), as the split kernel does, for its merge.
+  const size_t prow0 = ((size_t)split * p.hkv + kvh) * p.rows_pad + row0;
+  const auto out_win = SHARED ? wt_window(p.part_o + prow0 * D)
+                             : wt_window((const char*)p.out + ((size_t)tok0 * p.hq + kvh * p.group) * (f32_out ? 4u * D : 2u * D));
 #pragma unroll 1   // (one copy of the code: what is fetched for the first row block serves the second)
   for (uint32_t mb = 0; mb < (uint32_t)MR; ++mb) {
   const uint32_t r = row0 + 32u * mb + l32;
@@ -555,8 +567,10 @@ __global__ void __launch_bounds__(256) attn_wsplit_kernel(const WsArgs args) {
     for (int i = 0; i < 4; ++i) w[i] = li[i] > 0.f ? __builtin_amdgcn_exp2f(mi[i] - mx) : 0.f;
     const float den = (w[0] * li[0] + w[1] * li[1]) + (w[2] * li[2] + w[3] * li[3]);
     const bool den_ok = den > 0.f;
-    const float inv = den_ok ? __builtin_amdgcn_rcpf(den) : 0.f;
-    if ((p.lse || p.dbg) && wave == 0 && g2 == 0 && r < p.rows_total) {
+    const float inv = SHARED ? 1.f : den_ok ? __builtin_amdgcn_rcpf(den) : 0.f;
+    if constexpr (SHARED) {
+      if (wave == 0 && g2 == 0) wt_store8(wt_window(p.part_ml + prow0 * 2), l32 * 8u, u32x2{__float_as_uint(mx), __float_as_uint(den)});
+    } else if ((p.lse || p.dbg) && wave == 0 && g2 == 0 && r < p.rows_total) {
       const uint32_t tok = fast_div(r, args.div_group), qh = kvh * p.group + r - tok * p.group;
       if (p.lse) p.lse[(size_t)tok * p.hq + qh] = den_ok ? mx * kLn2 + __logf(den) : -INFINITY;
       if (p.dbg && !den_ok) dbg_report(p.dbg, DBG_ERR_SOFTMAX_NORM_ZERO, DBG_KERNEL_ATTENTION, (tok << 16) | qh, (tok << 16) | qh);
@@ -604,6 +618,10 @@ __global__ void __launch_bounds__(256) attn_wsplit_kernel(const WsArgs args) {
     const uint32_t rl = c / cpr, ch = c & (cpr - 1u);
     const u32x4 h = *(lds_u32x4*)((lds_char*)smem + OFF_T + rl * (uint32_t)T_ROW + ch * 16u);
     const uint32_t rr = row0 + 32u * mb + rl;
+    if constexpr (SHARED) {
+      wt_store16(out_win, (rl * cpr + ch) * 16u, h);
+      continue;
+    }
     if (rr >= p.rows_total) break;
     const uint32_t tok = fast_div(rr, args.div_group), g = rr - tok * p.group;
     if (p.dbg) {   // a NaN or infinity among the chunk's elements: an all-ones exponent carries into the top bit
@@ -620,18 +638,19 @@ __global__ void __launch_bounds__(256) attn_wsplit_kernel(const WsArgs args) {
   }
 }
 
-template <int D, bool F16, int MR>
+template <int D, bool F16, int MR, bool SHARED = false>
 hipError_t launch_rows(const AttnParams& p, hipStream_t s) {
   WsArgs a;
   a.p = p;
   a.n_rt = (p.rows_total + 32 * MR - 1) / (32 * MR);
   a.div_rt = make_fast_div(a.n_rt);
   a.div_group = make_fast_div(p.group);
+  a.div_splits = make_fast_div(p.n_splits);
   // (touches use 32-bit byte offsets: a range or ring whose rows span 4 GiB goes without)
   const uint64_t rows = p.ring_mask ? (uint64_t)p.ring_mask + 1u : (uint64_t)(p.tile_end - p.tile_first + 2u) * kBlockN;
   a.touch = p.touch_ahead && rows * 2u * (uint64_t)std::max(p.k_tok_stride, p.v_tok_stride) < (1ull << 32) ? 1u : 0u;
-  const uint32_t grid = ((p.hkv * a.n_rt + 7u) / 8u) * 8u;
-  hipLaunchKernelGGL((attn_wsplit_kernel<D, F16, MR>), dim3(grid), dim3(256), 0, s, a);
+  const uint32_t grid = ((p.hkv * p.n_splits * a.n_rt + 7u) / 8u) * 8u;
+  hipLaunchKernelGGL((attn_wsplit_kernel<D, F16, MR, SHARED>), dim3(grid), dim3(256), 0, s, a);
   return hipGetLastError();
 }
 
@@ -642,6 +661,9 @@ hipError_t launch_ws(const AttnParams& p, hipStream_t s) {
   // in us, 32 | 64 rows: 256 canvas rows = 128 workgroups of 32: 21.2 | 31.0; 901 rows = 456: 40.3 | 34.9.)
   const uint32_t cus = p.cus, r1 = (p.hkv * ((p.rows_total + 31u) / 32u) + cus - 1u) / cus;
   const uint32_t r2 = (p.hkv * ((p.rows_total + 63u) / 64u) + cus - 1u) / cus;
+  if constexpr (D == 256) {
+    if (p.n_splits > 1u) return launch_rows<D, F16, 1, true>(p, s);
+  }
   if (8u * r2 < 5u * r1) return launch_rows<D, F16, 2>(p, s);
   return launch_rows<D, F16, 1>(p, s);
 }

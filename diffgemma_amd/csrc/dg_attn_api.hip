@@ -133,6 +133,7 @@ struct Plan {
   uint32_t t_all = 0, lo_nc = 0, extra_lo = 0, win_m1 = 0xffffffffu;
   uint32_t clip_lo = 0, clip_hi = 0;   // keys that count: [clip_lo, clip_hi); the whole range unless a partial is asked for
   uint32_t cus = 256;
+  uint32_t span_tiles = 0;      // most key tiles a 32-row tile sees
   uint32_t tile_first = 0, tile_end = 0, tiles_per_split = 0, n_splits = 1;
   uint32_t e_dtype = DG_BF16;   // element type the kernels compute in (bf16 or f16)
   bool convert_q = false, gather_kv = false, q_is_bf16 = false;
@@ -177,6 +178,19 @@ uint32_t tiles_of_split(uint32_t ntiles, uint32_t base, uint32_t cus, uint32_t h
   for (uint32_t few = dg::kMergeFewSplits; few >= 8u && !dg::merge_at_once(of(t), of(t) * split_bytes); few -= 8u)
     if (dg::merge_at_once(of(of(few)), of(of(few)) * split_bytes)) return of(few) > t && of(few) <= t + 3u ? of(few) : t;
   return t;
+}
+
+// Key tiles per workgroup of the one-launch kernel: all that a 32-row tile sees, or, where a few canvas rows over most of a
+// window leave three quarters of the chip idle, a share of them, the rows merged as the split kernel's are (fp32 partial rows: in one
+// launch nothing of a row is narrower; a workgroup's run is cut over its four waves again).  A wave's tile takes 1.07 us; the
+// second launch about 4, and more with the rows.  Attention call, us, one launch | shared by 5, window 1024: behind 4000 keys 16 rows
+// 15.8 | 10.7, 32 15.8 | 11.5, 64 16.1 | 13.1, 100 16.4 | 14.9, 128 16.3 | 16.1; shorter ranges, 32 rows: 17 tiles 11.1 | 10.7, 14 10.1 |
+// 10.7; 64 rows: 24 tiles 12.7 | 12.2, 18 11.3 | 11.7; 100 rows: 29 tiles 14.8 | 13.6, 25 13.5 | 13.2, 22 12.5 | 12.8.  By 4 or 6: 0 to 0.4 slower.
+uint32_t share_of_short_range(const dg_attn_desc* d, const Plan& pl, uint32_t cus, uint32_t ntiles) {
+  const uint32_t base = d->n_kv_heads * ((pl.rows_total + 31u) / 32u);
+  if (d->head_dim != 256 || base * 9u > cus * 2u || pl.span_tiles < 17u + base / 6u) return ntiles;
+  const uint32_t s = std::min(cus / base, 5u);
+  return (ntiles + s - 1) / s;
 }
 
 // Row tiles that see different numbers of key tiles (causal rows of a global layer): split counts of their own, so that no
@@ -308,9 +322,9 @@ int make_plan(const dg_attn_desc* d, int cus, Plan* pl, const uint32_t* key_rang
       if (d->flags & DG_ATTN_F_CAUSAL_SEES_MASKED) c = pl->t_all;
       span = std::max(span, std::min(c, pl->t_all));
     }
-    const uint32_t span_tiles = std::min(ntiles, span / dg::kBlockN + 2u);
+    pl->span_tiles = std::min(ntiles, span / dg::kBlockN + 2u);
     pl->wsplit = !pl->scalar && hd <= 256 && d->n_splits == 0 && !(d->flags & DG_ATTN_F_SPLIT_OVER_WORKGROUPS) &&
-                 span_tiles <= kWsplitMaxTiles;
+                 pl->span_tiles <= kWsplitMaxTiles;
   }
   const uint32_t base = d->n_kv_heads * pl->n_mtiles;
   // workspace carve-up, with splits of `tps` key tiles; f32_parts: partial rows stay fp32 whatever the flags allow
@@ -337,7 +351,11 @@ int make_plan(const dg_attn_desc* d, int cus, Plan* pl, const uint32_t* key_rang
     }
     pl->total = off;
   };
-  if (pl->scalar || pl->wsplit) {
+  if (pl->wsplit) {
+    const uint32_t share = share_of_short_range(d, *pl, (uint32_t)cus, ntiles);
+    carve(share, true);
+    if (pl->total > scratch) carve(ntiles, true);
+  } else if (pl->scalar) {
     carve(ntiles, false);
   } else if (d->n_splits != 0) {
     const uint32_t splits = std::min(std::min(d->n_splits, kMaxSplits), ntiles);

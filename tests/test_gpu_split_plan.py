@@ -96,6 +96,43 @@ def test_device_prefix_with_the_scratch_of_a_split_map(gpu_ready, po):
     assert (outs[0] - outs[1]).abs().max() <= 2.0 ** -7 * outs[1].abs().max()
 
 
+@pytest.mark.parametrize("canvas,kv_len,causal_rows,hkv,window,ring,f16", [
+    (64, 4000, 0, 8, 1024, 2048, False), (33, 5000, 33, 8, 1024, 2048, True), (112, 3001, 40, 8, 1024, 0, False),
+    (100, 830, 0, 8, 0, 0, True), (17, 1100, 17, 4, 1024, 2048, False)])
+def test_short_range_shared_by_workgroups(gpu_ready, po, canvas, kv_len, causal_rows, hkv, window, ring, f16):
+    """A few canvas rows over most of a window: several workgroups to a row tile of the one-launch kernel, their rows merged.
+    Against the oracle (ring caches against the linear one, bit for bit); without scratch the call is one launch."""
+    import torch
+    w = dataclasses.replace(W.Workload("share", canvas, 16, hkv, 256, kv_len, causal_rows=causal_rows, window=window, seed=canvas), kv_f16=f16)
+    d = w.desc()
+    assert capi.resolved_splits(d) > 1 and capi.workspace_bytes(d) > 0
+    check_tolerances(*run_workload(po, w))
+    q, kv = W.generate(w)
+    qd, kd = W.device_arrays(w, q, kv)
+    dt = torch.int16
+    shared, one, ringed = (torch.zeros(canvas * 16 * 256, dtype=dt, device="cuda") for _ in range(3))
+    lse = torch.zeros(canvas * 16, device="cuda")
+    ws = A.alloc_workspace(d)
+    ws.fill_(255)
+    A.forward(d, qd, kd, shared, lse, ws)
+    A.forward(d, qd, kd, one, None, None)
+    assert not torch.equal(shared, one)
+    assert (shared.view(torch.bfloat16).float() - one.view(torch.bfloat16).float()).abs().max() <= 1.6e-2 * 2      # two bf16-P roundings, two stores
+    if ring:
+        planes = kd.view(dt).view(2, hkv, w.t_all, 256)
+        rd = torch.zeros(2, hkv, ring, 256, dtype=dt, device="cuda")
+        lo = max(0, w.t_all - ring)
+        rd[:, :, torch.arange(lo, w.t_all, device="cuda") % ring] = planes[:, :, lo:]
+        dr = A.make_desc(canvas, 16, hkv, 256, kv_len, causal_rows=causal_rows, window=window, kv_ring_mask=ring - 1, layout="head_major",
+                         t_cap=ring, kv_dtype=d.kv_dtype, flags=d.flags)
+        A.forward(dr, qd, rd, ringed, None, A.alloc_workspace(dr))
+        assert torch.equal(ringed, shared)
+    step = A.device_step_params(kv_len)
+    A.forward_dev(d, step, qd, kd, one, None, ws)
+    torch.cuda.synchronize()
+    assert torch.equal(one, shared)
+
+
 @pytest.mark.parametrize("hd,hkv,f32_parts,out_f32", [(512, 2, False, False), (256, 8, False, False), (512, 2, True, False),
                                                       (512, 2, True, True), (256, 8, True, False), (64, 2, True, True)])
 def test_merge_at_once_gives_the_bits_of_the_streamed_merge(gpu_ready, hd, hkv, f32_parts, out_f32):
