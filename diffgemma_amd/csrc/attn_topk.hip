@@ -741,9 +741,9 @@ __global__ void __launch_bounds__(256) topk_select_kernel(const TopkParams tp) {
 // two to four times k entries that one wave holds in registers.  Whatever tau is, the result is exact: a row whose
 // list holds fewer than k entries, or more than fit, is marked, and the general path redoes the marked rows (its
 // launches end at once where no row of the block is marked, 1.5 us each).
-// 256 rows x 16 heads over 33024 keys, layer step: 646 -> 279 us.  Launches: sampled scores 24 us (was: scores and plane, 4 x 55),
-// thresholds 16, filter 141 (0.98 PFLOP/s; the products alone, with their LDS reads and nothing else, 101), selection 30
-// and gathered P.V 55 (both: was 4 x 94).
+// 256 rows x 16 heads over 33024 keys, layer step: 646 -> 266 us.  Launches: sampled scores 19 us (was: scores and plane, 4 x 55),
+// thresholds 15, filter 124 (1.1 PFLOP/s; the products alone, with their LDS reads and nothing else, 101), selection 31
+// and gathered P.V 52 (both: was 4 x 94).
 
 // scores through an ordinary-register accumulator, query fragment in accumulation registers (256 of them hold the 64
 // query rows of a wave; a comparison cannot read that file)

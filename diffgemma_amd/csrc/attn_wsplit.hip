@@ -27,8 +27,10 @@
 // and the epilogue are written for few of them (LDS rows padded so that a tile needs one per-lane load offset instead of a
 // table, scalar address arithmetic, divisions by multiplication, accumulators stored to LDS without passing through vector
 // registers, the shares of a row exchanged in register order).
-// Measured (GPU time of producer + attention, before and after these): a sliding layer over 1279 keys 23.1 -> 21.3 us, over
-// an f16 cache 25.6 -> 22.5; 64 rows behind 22 keys 13.4 -> 9.6; 901 causal rows 50.2 -> 34.9.  Of a launch over 1279 keys
+// A few canvas rows over most of a window leave three quarters of the chip idle: there several workgroups share a row tile's
+// keys and leave fp32 rows for the split kernel's merge (SHARED; the rule with both sides measured: dg_attn_api.hip).
+// Measured (GPU time of producer + attention, before and after these): a sliding layer over 1279 keys 23.1 -> 21.0 us, over
+// an f16 cache 25.6 -> 22.4; 64 rows behind 22 keys 13.4 -> 9.5; 901 causal rows 50.2 -> 33.8; 64 rows over a window 18.8 -> 14.5.  Of a launch over 1279 keys
 // 1.5 us go before the first scores, 1.6 into the first tile (cold code), 1.07 into each later one (the compute unit's load
 // path alone takes 0.85), 2.1 into the shares of the four waves and the rows.
 // Softmax arithmetic (lazy reference max, exponent offset under which negligible weights become exact zeros,
@@ -658,7 +660,7 @@ template <int D, bool F16>
 hipError_t launch_ws(const AttnParams& p, hipStream_t s) {
   // 32 rows per workgroup while they are one round of the chip's compute units (one workgroup each: LDS); past that 64
   // rows, whose workgroups take 1.6 x as long for twice the rows, where that is fewer rounds' time.  (Sliding layer, step
-  // in us, 32 | 64 rows: 256 canvas rows = 128 workgroups of 32: 21.2 | 31.0; 901 rows = 456: 40.3 | 34.9.)
+  // in us, 32 | 64 rows: 256 canvas rows = 128 workgroups of 32: 21.0 | 31.0; 901 rows = 456: 40.3 | 33.8.)
   const uint32_t cus = p.cus, r1 = (p.hkv * ((p.rows_total + 31u) / 32u) + cus - 1u) / cus;
   const uint32_t r2 = (p.hkv * ((p.rows_total + 63u) / 64u) + cus - 1u) / cus;
   if constexpr (D == 256) {

@@ -94,12 +94,15 @@ typedef enum dg_kernel_sel {
 #define DG_ATTN_F_STREAMED_MERGE 0x20u     /* merge the split partial rows with the streaming kernel (weights
                                               first, then only the rows of splits that count) even where the
                                               library would pick the one that fetches every partial row up
-                                              front (at most 8 splits, f16 partial rows, workspace below
-                                              32 MiB).  Both give the same bits; the flag is there to compare them. */
+                                              front (at most 8 splits and partial rows below 32 MiB, or 9 to
+                                              16 of f16 rows of at most 17 MiB; not where row tiles have
+                                              split counts of their own).  Both give the same bits; the flag is there to compare them. */
 
 #define DG_ATTN_F_SPLIT_OVER_WORKGROUPS 0x80u /* head_dim <= 256 and a short key range (a sliding-window layer): the
                                               library runs one launch in which the waves of a workgroup split the
-                                              keys and merge in LDS.  This flag asks for the general kernel instead
+                                              keys and merge in LDS (several workgroups to a row tile and a merge
+                                              launch for a few canvas rows over a long window, where the workspace
+                                              holds their fp32 partial rows).  This flag asks for the general kernel instead
                                               (keys split over workgroups, partial rows in the workspace, a merge
                                               launch), as does an explicit n_splits.  Results agree to the rounding
                                               of the probabilities; the flag is there to compare the two. */
@@ -144,7 +147,8 @@ void dg_attn_desc_reference_layout(dg_attn_desc* d);
 /* Strides of two planes [Hkv][t_cap][d] (K plane, then V plane at Hkv*t_cap*d). */
 void dg_attn_desc_head_major_layout(dg_attn_desc* d, uint64_t t_cap);
 
-/* Bytes of device scratch dg_attn_forward needs for this descriptor (0 is possible). */
+/* Bytes of device scratch dg_attn_forward asks for with this descriptor (0 is possible).  With less it splits the keys less, down
+ * to splits of 6 key tiles (none at all for a short key range at head_dim <= 256); below that, DG_ERR_WORKSPACE. */
 int dg_attn_workspace_bytes(const dg_attn_desc* d, size_t* out_bytes);
 
 /* Splits the library would use for this descriptor (n_splits==0 resolved). */

@@ -131,6 +131,13 @@ def test_short_range_shared_by_workgroups(gpu_ready, po, canvas, kv_len, causal_
     A.forward_dev(d, step, qd, kd, one, None, ws)
     torch.cuda.synchronize()
     assert torch.equal(one, shared)
+    # a device prefix far below the planned one: most workgroups of a row tile have no keys
+    small = A.make_desc(canvas, 16, hkv, 256, 100, causal_rows=causal_rows, window=window, layout="head_major", t_cap=w.t_all, kv_dtype=d.kv_dtype,
+                        flags=d.flags)
+    A.forward_dev(d, A.device_step_params(100), qd, kd, one, None, ws)
+    A.forward(small, qd, kd, shared, None, A.alloc_workspace(small))
+    torch.cuda.synchronize()
+    assert (shared.view(torch.bfloat16).float() - one.view(torch.bfloat16).float()).abs().max() <= 1.6e-2 * 2
 
 
 @pytest.mark.parametrize("hd,hkv,f32_parts,out_f32", [(512, 2, False, False), (256, 8, False, False), (512, 2, True, False),
