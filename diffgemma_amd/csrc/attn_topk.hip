@@ -72,15 +72,6 @@ __global__ void __launch_bounds__(256) topk_scores_kernel(const TopkParams tp) {
 
   const uint32_t rows_total = tp.ntok * p.group;
   const uint32_t row0 = mt * kBlockM;
-  if (tp.fail_rows != nullptr) {   // only row tiles with a row that was left over (every wave looks at all of the tile's)
-    uint32_t any = 0u;
-#pragma unroll
-    for (uint32_t i = 0; i < (uint32_t)kBlockM; i += 64u) {
-      const uint32_t rf = min(row0 + i + lane, rows_total - 1u), tf = fast_div(rf, tp.div_group);
-      any |= tp.fail_rows[(size_t)(tp.tok0 + tf) * p.hq + kvh * p.group + rf - tf * p.group];
-    }
-    if (__builtin_amdgcn_ballot_w64(any != 0u) == 0ull) return;
-  }
   const uint32_t r = row0 + wave * 32u + l32;
   const bool row_ok = r < rows_total;
   const uint32_t tok_l = row_ok ? fast_div(r, tp.div_group) : 0u;           // row within this pass
@@ -749,8 +740,8 @@ __global__ void __launch_bounds__(256) topk_select_kernel(const TopkParams tp) {
 // stores only scores at or above tau, as (score, position) entries in lists, and the select kernel works on a list of
 // two to four times k entries that one wave holds in registers.  Whatever tau is, the result is exact: a row whose
 // list holds fewer than k entries, or more than fit, is marked, and the general path redoes the marked rows (its
-// launches end at once where no row of the block is marked, and so do the workgroups of a row tile without one).
-// 256 rows x 16 heads over 33024 keys, layer step: 646 -> 257 us.  Launches: sampled scores 19 us (was: scores and plane, 4 x 55),
+// launches end at once where no row of the block is marked, 1.5 us each).
+// 256 rows x 16 heads over 33024 keys, layer step: 646 -> 266 us.  Launches: sampled scores 19 us (was: scores and plane, 4 x 55),
 // thresholds 15, filter 124 (1.1 PFLOP/s; the products alone, with their LDS reads and nothing else, 101), selection 31
 // and gathered P.V 52 (both: was 4 x 94).
 

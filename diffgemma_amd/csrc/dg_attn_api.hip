@@ -733,7 +733,6 @@ namespace {
 #define DG_TOPK_PLANE_MIB 144
 #endif
 constexpr size_t kTopkPlaneBudget = (size_t)DG_TOPK_PLANE_MIB << 20;
-constexpr size_t kTopkRedoBudget = 4 * kTopkPlaneBudget;
 
 struct TopkPlan {
   uint32_t t_pad = 0, block_tok = 0;
@@ -753,9 +752,9 @@ struct TopkPlan {
 // time grows with the rounds of the chip those workgroups need.  Measured, the layer step with 16 heads, general -> filtered
 // path: 64 rows (one round) over 20k keys 99 -> 108 us, 33k 152 -> 141, 50k 297 -> 190; 128 rows (two) over 5k keys
 // 87 -> 89 us, 8k 99.5 -> 98, 12k 123 -> 107, 33k 294 -> 175; 256 rows over 3k keys 136 -> 100 us, 33k 592 -> 269.
-// That is for rows the lists hold.  A row they do not (thousands of equal scores) has its row tile scored again: the attention
-// call alone, 256 rows over 33k keys, general | filtered: one such row 700 | 437 us, one in every canvas row 955 | 635, all of
-// them 1935 | 2823; 64 rows over 33k: 232 | 357, 235 | 373, 486 | 754.  The host cannot tell.
+// That is for rows the lists hold.  A row they do not (thousands of equal scores) has its block of canvas rows scored again:
+// the attention call alone, 256 rows over 33k keys, general | filtered: one such row 706 | 462 us, one in every canvas row
+// 975 | 1300, all of them 1947 | 3120; 64 rows over 33k: 233 | 380, 235 | 384, 489 | 766.  The host cannot tell.
 constexpr uint32_t kTopkFilterMinPrefix = 2048;
 constexpr uint32_t kTopkFilterMaxK = 512;
 constexpr uint32_t kTopkFilterMinKeys[3] = {24576, 8192, 0};   // one round, two rounds, more
@@ -783,7 +782,7 @@ size_t filter_bytes(const dg_attn_desc* d, const Plan& pl, uint32_t cus, uint32_
   return tk->off_lists + align_up(std::max(segs * dg::kTopkSegAlloc * 8, sample));
 }
 
-void plan_filtered(const dg_attn_desc* d, const uint32_t* k_cfg, const Plan& pl, uint32_t cus, size_t scratch, TopkPlan* tk) {
+void plan_filtered(const dg_attn_desc* d, const uint32_t* k_cfg, const Plan& pl, uint32_t cus, TopkPlan* tk) {
   if (d->head_dim != 512 || pl.lo_nc != 0 || pl.win_m1 != 0xffffffffu || d->kv_ring_mask != 0) return;
   if (d->kv_len < kTopkFilterMinPrefix || !std::isfinite(pl.scale) || (d->flags & DG_ATTN_F_TOPK_SCORE_PLANE)) return;
   const uint64_t rows = (uint64_t)d->canvas * d->n_q_heads;
@@ -815,13 +814,6 @@ void plan_filtered(const dg_attn_desc* d, const uint32_t* k_cfg, const Plan& pl,
   const size_t per_tok = (size_t)d->n_q_heads * tk->t_pad * sizeof(float);
   size_t total = std::max(tk->total, need);
   if (tk->block_tok == d->canvas) total = std::max(total, tk->off_plane + align_up((size_t)ntok * per_tok));
-  // Left-over rows are redone in blocks of canvas rows, two launches each that mostly find nothing to do (3.5 us): as few blocks
-  // as the scratch holds planes for, the general path's own size and more.  That its plane then outgrows the memory-side cache
-  // counts for less than the launches: only row tiles with a left-over row are scored.  Attention call, us, 144 | 576 MiB:
-  // 256 rows over 33k keys 252 | 243, over 17k 149 | 145, over 41k 329 | 321; with one row left over 457 | 441, one in every
-  // canvas row 1281 | 634, all of them 3087 | 2831.
-  const size_t roomy = tk->off_plane + align_up(std::min<size_t>(ntok, kTopkRedoBudget / per_tok) * per_tok);
-  total = std::max(total, std::min(roomy, scratch));
   const size_t fit = (total - tk->off_plane) / per_tok;
   if (fit == 0) return;
   tk->total = total;
@@ -830,7 +822,7 @@ void plan_filtered(const dg_attn_desc* d, const uint32_t* k_cfg, const Plan& pl,
   tk->redo_tok = (ntok + blocks - 1) / blocks;
 }
 
-int make_topk_plan(const dg_attn_desc* d, const uint32_t* k_cfg, const Plan& pl, uint32_t cus, TopkPlan* tk, size_t scratch = SIZE_MAX) {
+int make_topk_plan(const dg_attn_desc* d, const uint32_t* k_cfg, const Plan& pl, uint32_t cus, TopkPlan* tk) {
   if (!k_cfg) return DG_ERR_NULL;
   if (pl.scalar || d->q_dtype == DG_F32 || d->kv_dtype == DG_F32) return DG_ERR_UNSUPPORTED;
   if (k_cfg[1] == 0u) {
@@ -846,7 +838,7 @@ int make_topk_plan(const dg_attn_desc* d, const uint32_t* k_cfg, const Plan& pl,
   tk->total = align_up((size_t)tk->block_tok * per_tok);
   if (tk->total / sizeof(float) >= (1ull << 32)) return DG_ERR_SHAPE;   // score rows are addressed with 32-bit offsets
   tk->general = tk->total;
-  plan_filtered(d, k_cfg, pl, cus, scratch, tk);
+  plan_filtered(d, k_cfg, pl, cus, tk);
   return DG_OK;
 }
 }  // namespace
@@ -873,7 +865,7 @@ int dg_attn_topk_forward(const dg_attn_desc* d, const uint32_t* k_cfg, const voi
   rc = make_plan(d, plan_cus(), &pl);
   if (rc != DG_OK) return rc;
   TopkPlan tk;
-  rc = make_topk_plan(d, k_cfg, pl, plan_cus(), &tk, workspace_bytes);
+  rc = make_topk_plan(d, k_cfg, pl, plan_cus(), &tk);
   if (rc != DG_OK) return rc;
   if (workspace_bytes < tk.total) tk.pass_tok = 0;
   if (!workspace || workspace_bytes < tk.general || ((uintptr_t)workspace % 16) != 0) return DG_ERR_WORKSPACE;
@@ -897,8 +889,8 @@ int dg_attn_topk_forward(const dg_attn_desc* d, const uint32_t* k_cfg, const voi
   auto mark = [&](uint32_t i) {
     if (prof) (void)hipEventRecord(g_prof.ev[2 * g_prof.used + i], s);
   };
-  // the general path over canvas rows [tok0, tok0 + ntok), or over those of them that are left over (redo)
-  auto block = [&](uint32_t tok0, uint32_t ntok, bool redo) -> hipError_t {
+  // the general path over canvas rows [tok0, tok0 + ntok)
+  auto block = [&](uint32_t tok0, uint32_t ntok, bool marks) -> hipError_t {
     tp.tok0 = tok0;
     tp.ntok = ntok;
     tp.n_mtiles = (tp.ntok * pl.group + dg::kBlockM - 1) / dg::kBlockM;
@@ -906,11 +898,10 @@ int dg_attn_topk_forward(const dg_attn_desc* d, const uint32_t* k_cfg, const voi
     // columns of the score plane, so there is nothing to merge
     const uint32_t base = d->n_kv_heads * tp.n_mtiles;
     uint32_t splits = std::max(1u, ((uint32_t)di.cus + base - 1u) / base);
-    if (redo) splits = std::max(splits, std::min(32u, ntiles / 32u));   // (left-over rows: few of the row tiles have one)
     tp.n_splits = std::max(1u, std::min(splits, ntiles / 8u));
-    if (!redo) mark(0);
+    if (marks) mark(0);
     hipError_t e = dg::launch_topk_scores(tp, d->head_dim, pl.e_dtype, s);
-    if (!redo) {
+    if (marks) {
       mark(1);
       mark(2);
     }
@@ -922,7 +913,7 @@ int dg_attn_topk_forward(const dg_attn_desc* d, const uint32_t* k_cfg, const voi
     const uint32_t ntok = std::min(step, d->canvas - tok0);
     prof = g_prof.active && 2 * (size_t)g_prof.used + 3 < g_prof.ev.size();
     if (tk.pass_tok == 0) {
-      if (block(tok0, ntok, false) != hipSuccess) return DG_ERR_LAUNCH;
+      if (block(tok0, ntok, true) != hipSuccess) return DG_ERR_LAUNCH;
     } else {
       char* const ws = (char*)workspace;
       dg::TopkParams fp = tp;
@@ -969,7 +960,7 @@ int dg_attn_topk_forward(const dg_attn_desc* d, const uint32_t* k_cfg, const voi
       for (uint32_t b = 0; b * tk.redo_tok < ntok; ++b) {
         tp.fail_block = fp.fail_block + b;
         const uint32_t at = b * tk.redo_tok;
-        if (block(tok0 + at, std::min(tk.redo_tok, ntok - at), true) != hipSuccess) return DG_ERR_LAUNCH;
+        if (block(tok0 + at, std::min(tk.redo_tok, ntok - at), false) != hipSuccess) return DG_ERR_LAUNCH;
       }
     }
     mark(3);

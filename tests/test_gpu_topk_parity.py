@@ -549,30 +549,3 @@ def test_short_rows_give_the_same_bits_every_time(gpu_ready):
     kv = rng.standard_normal((kv_len + canvas, 2, hkv, hd)).astype(np.float32)
     outs = [device_topk(canvas, hq, hkv, hd, kv_len, T.adaptive_k(), q, kv, window=17)[0] for _ in range(16)]
     assert all(np.array_equal(o, outs[0]) for o in outs)
-
-
-@pytest.mark.parametrize("canvas,kv_len", [(128, 33000), (250, 14900)])
-def test_left_over_rows_in_fewer_blocks(gpu_ready, canvas, kv_len):
-    """Left-over rows (zero queries: equal scores) are redone in as few blocks as the workspace holds: the same bits from the size
-    that is asked for, from the score plane's own, which is still taken, and from one between."""
-    import torch
-    d = A.make_desc(canvas, 16, 2, 512, kv_len, out_dtype=capi.DG_F32)
-    g = torch.Generator(device="cuda")
-    g.manual_seed(canvas)
-    q = torch.randn(canvas, 16, 512, device="cuda", generator=g).to(torch.bfloat16)
-    kv = torch.randn(kv_len + canvas, 2, 2, 512, device="cuda", generator=g).to(torch.bfloat16)
-    q[::31, 3] = 0
-    q[-1] = 0
-    full = T.workspace_bytes(d, T.adaptive_k())
-    per_row = 16 * 4 * ((kv_len + canvas + 31) // 32 * 32)
-    plane = (144 << 20) // per_row // 16 * 16 * per_row          # the general path's block of canvas rows
-    assert plane + 20 * per_row < full < (576 << 20) + (8 << 20)
-    outs = []
-    for size in (full, plane + 20 * per_row, plane):
-        ws = torch.full((size,), 255, dtype=torch.uint8, device="cuda")
-        out = torch.zeros(canvas, 16, 512, device="cuda")
-        T.forward(d, T.adaptive_k(), q, kv, out, ws)
-        T.forward(d, T.adaptive_k(), q, kv, out, ws)
-        outs.append(out)
-    torch.cuda.synchronize()
-    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
