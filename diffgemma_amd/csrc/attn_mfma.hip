@@ -333,13 +333,14 @@ __global__ void __launch_bounds__(256) attn_mfma_kernel(const MfmaArgs args) {
   lds_char* const k1 = (lds_char*)(smem + OFF_K1);
   lds_char* const v0 = (lds_char*)(smem + OFF_V0);
   lds_char* const v1 = (lds_char*)(smem + OFF_V1);
-  const uint32_t t_last = past_end_pos((te - 1u) * kBlockN, lo_min, p.t_all, p.ring_mask);
+  const uint32_t t_end = loads_end(te, p.t_all);
+  const uint32_t t_last = past_end_pos((te - 1u) * kBlockN, lo_min, t_end, p.ring_mask);
   // (in the loop only tiles behind the workgroup's first one are loaded)
   auto k_load = [&](uint32_t t0, lds_char* buf, uint32_t ln) {
-    return make_tile_load<D, false, false>(kbase, kstride_b, min(t0, t_last), 0u, p.t_all, p.ring_mask, buf, wave, ln);
+    return make_tile_load<D, false, false>(kbase, kstride_b, min(t0, t_last), 0u, t_end, p.ring_mask, buf, wave, ln);
   };
   auto v_load = [&](uint32_t t0, lds_char* buf, uint32_t ln) {
-    return make_tile_load<D, true, false>(vbase, vstride_b, min(t0, t_last), 0u, p.t_all, p.ring_mask, buf, wave, ln);
+    return make_tile_load<D, true, false>(vbase, vstride_b, min(t0, t_last), 0u, t_end, p.ring_mask, buf, wave, ln);
   };
   auto k_load_first = [&](lds_char* buf) {
     return make_tile_load<D, false, true>(kbase, kstride_b, tb * kBlockN, lo_min, p.t_all, p.ring_mask, buf, wave, lane);

@@ -227,11 +227,16 @@ __host__ __device__ __forceinline__ TileRows tile_rows(uint32_t t0, uint32_t lo,
   r.first = lo <= t0 ? 0u : lo - t0 < r.last ? lo - t0 : r.last;
   return r;
 }
-// Where loads issued for tiles behind a row tile's last one (at t_last) go, so that the tile loop need not branch around them:
-// the last tile again, its rows clamped at the end alone.  Where that tile begins before `lo` (it is then the only one), the
-// rows from `lo` on instead; a ring has memory for every slot, and 32 rows from an arbitrary slot could run past its end.
-__host__ __device__ __forceinline__ uint32_t past_end_pos(uint32_t t_last, uint32_t lo, uint32_t t_all, uint32_t ring_mask) {
-  const uint32_t see = lo < t_all ? lo : t_all - 1u;
+// End of the rows that loads in the tile loop may read, for key tiles up to `te`: the last key, or the end of the last tile (past
+// it a holder of a key range has no memory).
+__host__ __device__ __forceinline__ uint32_t loads_end(uint32_t te, uint32_t t_all) {
+  return te * (uint32_t)kBlockN < t_all ? te * (uint32_t)kBlockN : t_all;
+}
+// Where loads issued for tiles behind a row tile's last one (at t_last, its rows below t_end) go, so that the tile loop need not
+// branch around them: the last tile again, its rows clamped at the end alone.  Where that tile begins before `lo` (it is then the
+// only one), its rows from `lo` on; a ring has memory for every slot, and 32 rows from an arbitrary slot could run past its end.
+__host__ __device__ __forceinline__ uint32_t past_end_pos(uint32_t t_last, uint32_t lo, uint32_t t_end, uint32_t ring_mask) {
+  const uint32_t see = lo < t_end ? lo : t_end - 1u;
   return ring_mask == 0u && see > t_last ? see : t_last;
 }
 // whether some row of the tile may not be read

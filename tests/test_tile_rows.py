@@ -24,10 +24,12 @@ int main() {
           if (row >= t_all || (row < see && see < t0 + kBlockN)) return std::printf("t_all %u lo %u t0 %u row %u\n", t_all, lo, t0, row), 1;
           if (t0 + i >= lo && t0 + i < t_all && row != t0 + i) return std::printf("moved a visible row %u\n", t0 + i), 1;
         }
-        // loads for tiles behind t0, the last one: nothing before the first visible key where t0 is the first tile too
-        const uint32_t pos = past_end_pos(t0, lo, t_all, 0u);
-        const TileRows past = tile_rows(pos, 0u, t_all);
-        if (pos >= t_all || pos + past.last >= t_all || pos < t0 || (see < t0 + kBlockN && pos < see) || past_end_pos(t0, lo, t_all, 63u) != t0)
+        // loads for tiles behind t0, the last one: no row behind that tile or the last key, and none before the first visible
+        // key where t0 is the first tile too
+        const uint32_t end = loads_end(t0 / kBlockN + 1u, t_all), pos = past_end_pos(t0, lo, end, 0u);
+        const TileRows past = tile_rows(pos, 0u, end);
+        if (pos + past.last >= t_all || pos + past.last >= t0 + kBlockN || pos < t0 || (see < t0 + kBlockN && pos + past.first < see) ||
+            past_end_pos(t0, lo, end, 63u) != t0)
           return std::printf("t_all %u lo %u t0 %u: past the end at %u\n", t_all, lo, t0, pos), 1;
         if (clamped && !tile_is_edge(t0, lo, t_all)) return std::printf("t_all %u lo %u t0 %u: no edge tile\n", t_all, lo, t0), 1;
       }
@@ -52,3 +54,9 @@ def test_k_and_v_tiles_of_the_one_launch_kernel_share_the_rule():
     text = (build.CSRC / "attn_wsplit.hip").read_text()
     assert text.count("tile_is_edge(") == 1 and text.count("tile_rows(tile * kBlockN, lo_min, p.t_all)") == 1
     assert text.count("is_edge(tile)") == 2        # where K's loads go out and where V's do
+
+
+def test_loads_in_the_split_kernels_loop_end_with_its_last_tile():
+    """They once ended with the last key: behind a range of one tile that begins inside it, up to 31 rows past the range."""
+    text = (build.CSRC / "attn_mfma.hip").read_text()
+    assert text.count("min(t0, t_last), 0u, t_end, p.ring_mask") == 2 and text.count("min(t0, t_last)") == 2
