@@ -306,13 +306,14 @@ __global__ void __launch_bounds__(256) attn_mfma_kernel(const MfmaArgs args) {
     const char* base;   // wave-uniform
     uint32_t voff;      // per lane
   };
+  const uint32_t touch_first = tile_rows((te - 1u) * kBlockN, lo_min, p.t_all).first;
   auto touch_address = [&](uint32_t tile, uint32_t ln) -> Touch {
     const uint32_t tp = min(tile, te - 1u) * kBlockN;
     const uint32_t sh = p.n_mtiles >= 16u ? 4u : 3u;   // log2 of the number of shares
     const uint32_t share = mt & ((1u << sh) - 1u);
     const bool is_v = (share >> (sh - 1u)) != 0u;      // the upper half of the shares are V's lines
     const uint32_t li = (share & ((1u << (sh - 1u)) - 1u)) * (512u >> sh) + wave * (128u >> sh) + (ln & ((128u >> sh) - 1u));
-    const uint32_t row = min(li >> 3, p.t_all - 1u - tp);
+    const uint32_t row = touched_row(li >> 3, touch_first, tp, p.t_all);
     const int64_t stride_b = is_v ? vstride_b : kstride_b;
     const int64_t slot = (int64_t)kv_slot(p.ring_mask, tp);
     return Touch{(is_v ? vbase : kbase) + slot * stride_b, row * (uint32_t)stride_b + (li & 7u) * 128u};

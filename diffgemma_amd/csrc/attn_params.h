@@ -239,6 +239,12 @@ __host__ __device__ __forceinline__ uint32_t past_end_pos(uint32_t t_last, uint3
   const uint32_t see = lo < t_end ? lo : t_end - 1u;
   return ring_mask == 0u && see > t_last ? see : t_last;
 }
+// Row of the key tile at t0 that is touched into the L2 for row `row` of it.  Touches run from a row tile's fourth tile to its
+// last one, and with fewer tiles go to that: `first` is the first row that may be read of the last tile (0 unless it is the only one).
+__host__ __device__ __forceinline__ uint32_t touched_row(uint32_t row, uint32_t first, uint32_t t0, uint32_t t_all) {
+  const uint32_t last = t_all - 1u - t0, r = row > first ? row : first;
+  return r < last ? r : last;
+}
 // whether some row of the tile may not be read
 __host__ __device__ __forceinline__ bool tile_is_edge(uint32_t t0, uint32_t lo, uint32_t t_all) {
   return t0 < lo || t0 + (uint32_t)kBlockN > t_all;

@@ -7,6 +7,7 @@ from diffgemma_amd import build
 
 PROGRAM = r"""
 #include "attn_params.h"
+#include <algorithm>
 #include <cstdio>
 int main() {
   using namespace dg;
@@ -31,6 +32,18 @@ int main() {
         if (pos + past.last >= t_all || pos + past.last >= t0 + kBlockN || pos < t0 || (see < t0 + kBlockN && pos + past.first < see) ||
             past_end_pos(t0, lo, end, 63u) != t0)
           return std::printf("t_all %u lo %u t0 %u: past the end at %u\n", t_all, lo, t0, pos), 1;
+        // touches of a row tile whose last tile is t0 and whose first one, with `lo` in it, is up to three before
+        for (uint32_t tb = lo / kBlockN; tb <= t0 / kBlockN; ++tb) {
+          const uint32_t first = tile_rows(t0, lo, t_all).first;
+          for (uint32_t tile = tb + 3u; tile < tb + 8u; ++tile) {
+            const uint32_t at = std::min(tile * kBlockN, t0);
+            for (uint32_t i = 0; i < (uint32_t)kBlockN; ++i) {
+              const uint32_t row = at + touched_row(i, first, at, t_all);
+              if (row >= t_all || row < see || row >= t0 + kBlockN || (at + i >= see && at + i < t_all && row != at + i))
+                return std::printf("t_all %u lo %u t0 %u: touches row %u\n", t_all, lo, t0, row), 1;
+            }
+          }
+        }
         if (clamped && !tile_is_edge(t0, lo, t_all)) return std::printf("t_all %u lo %u t0 %u: no edge tile\n", t_all, lo, t0), 1;
       }
   std::puts("ok");
@@ -60,3 +73,10 @@ def test_loads_in_the_split_kernels_loop_end_with_its_last_tile():
     """They once ended with the last key: behind a range of one tile that begins inside it, up to 31 rows past the range."""
     text = (build.CSRC / "attn_mfma.hip").read_text()
     assert text.count("min(t0, t_last), 0u, t_end, p.ring_mask") == 2 and text.count("min(t0, t_last)") == 2
+
+
+def test_touches_of_the_split_kernel_begin_with_the_first_visible_key():
+    """They once began with the tile: up to 31 rows before a share of one tile that begins inside it."""
+    text = (build.CSRC / "attn_mfma.hip").read_text()
+    assert text.count("touched_row(") == 1 and "min(tile, te - 1u) * kBlockN" in text
+    assert "touch_first = tile_rows((te - 1u) * kBlockN, lo_min, p.t_all).first" in text
