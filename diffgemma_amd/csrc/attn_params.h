@@ -245,6 +245,11 @@ __host__ __device__ __forceinline__ uint32_t touched_row(uint32_t row, uint32_t 
   const uint32_t last = t_all - 1u - t0, r = row > first ? row : first;
   return r < last ? r : last;
 }
+// The one-launch kernel touches a range of keys [pos0, pos1), `per` of them to a touch: position of key `i` of touch u.
+__host__ __device__ __forceinline__ uint32_t touched_pos(uint32_t pos0, uint32_t pos1, uint32_t per, uint32_t u, uint32_t i) {
+  const uint32_t pos = pos0 + u * per + i;
+  return pos < pos1 ? pos : pos1 - 1u;
+}
 // whether some row of the tile may not be read
 __host__ __device__ __forceinline__ bool tile_is_edge(uint32_t t0, uint32_t lo, uint32_t t_all) {
   return t0 < lo || t0 + (uint32_t)kBlockN > t_all;

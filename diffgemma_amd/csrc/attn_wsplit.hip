@@ -246,7 +246,7 @@ __global__ void __launch_bounds__(256) attn_wsplit_kernel(const WsArgs args) {
     for (uint32_t t = 0; t < (uint32_t)NTOUCH; ++t) {
       const uint32_t u = min(rt * 4u + wave + t * 4u * args.n_rt, 2u * per_matrix - 1u);   // (past the end: the last one again)
       const bool is_v = u >= per_matrix;
-      const uint32_t pos = min(pos0 + (is_v ? u - per_matrix : u) * RPT + lane / LPRW, p.t_all - 1u);
+      const uint32_t pos = touched_pos(pos0, pos1, RPT, is_v ? u - per_matrix : u, lane / LPRW);
       const uint32_t first = p.ring_mask ? 0u : pos0;     // (32-bit offsets from the ring's first slot or the range's first key)
       const int64_t stride_b = is_v ? vstride_b : kstride_b;
       lds_dma_touch((is_v ? vbase : kbase) + (int64_t)first * stride_b,

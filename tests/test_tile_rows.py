@@ -9,6 +9,7 @@ PROGRAM = r"""
 #include "attn_params.h"
 #include <algorithm>
 #include <cstdio>
+#include <vector>
 int main() {
   using namespace dg;
   const uint32_t span = 3 * kBlockN + 2;
@@ -46,6 +47,19 @@ int main() {
         }
         if (clamped && !tile_is_edge(t0, lo, t_all)) return std::printf("t_all %u lo %u t0 %u: no edge tile\n", t_all, lo, t0), 1;
       }
+  // touches of the one-launch kernel: every key of the range, and no other
+  for (uint32_t per = 8; per <= 64; per *= 2)
+    for (uint32_t pos0 = 0; pos0 <= 33; pos0 += 11)
+      for (uint32_t n = 1; n <= 130; ++n) {
+        std::vector<bool> seen(n);
+        for (uint32_t u = 0; u < (n + per - 1) / per; ++u)
+          for (uint32_t i = 0; i < per; ++i) {
+            const uint32_t pos = touched_pos(pos0, pos0 + n, per, u, i);
+            if (pos < pos0 || pos >= pos0 + n) return std::printf("%u to a touch, [%u, %u): touches row %u\n", per, pos0, pos0 + n, pos), 1;
+            seen[pos - pos0] = true;
+          }
+        if (std::count(seen.begin(), seen.end(), true) != n) return std::printf("%u to a touch, %u keys: not all\n", per, n), 1;
+      }
   std::puts("ok");
   return 0;
 }
@@ -80,3 +94,10 @@ def test_touches_of_the_split_kernel_begin_with_the_first_visible_key():
     text = (build.CSRC / "attn_mfma.hip").read_text()
     assert text.count("touched_row(") == 1 and "min(tile, te - 1u) * kBlockN" in text
     assert "touch_first = tile_rows((te - 1u) * kBlockN, lo_min, p.t_all).first" in text
+
+
+def test_touches_of_the_one_launch_kernel_stay_in_its_range():
+    """They once ended with the last key, up to 63 rows behind the keys of a workgroup's range."""
+    text = (build.CSRC / "attn_wsplit.hip").read_text()
+    assert text.count("lds_dma_touch(") == 1 and text.count("touched_pos(pos0, pos1, RPT,") == 1
+    assert "pos1 = min(mt_end * kBlockN, p.t_all)" in text
