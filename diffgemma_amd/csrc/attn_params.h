@@ -107,6 +107,32 @@ __host__ __device__ __forceinline__ uint32_t fast_div(uint32_t n, FastDiv d) {
   return ((uint32_t)(((uint64_t)n * d.mul) >> 32) + n) >> d.shift;
 }
 
+// The map of the shortest length in [len, limit] that gives a KV head no more than `budget` units (and no row tile more than
+// kMapSplits); false where even `limit` gives more.  Units do not grow with the length, so it is found by bisection, and rows
+// behind a long prefix, all of which see about as many key tiles, are told by the first of them (each length in turn, with a map
+// built for each, took 140 us of host time for 1024 rows behind 32768 keys).
+template <typename Tiles>
+inline bool shortest_split_map(uint32_t n_mtiles, uint32_t len, uint32_t limit, uint32_t budget, Tiles&& tiles, SplitMap* m) {
+  if (len == 0u || len > limit || (uint64_t)n_mtiles * ((tiles(0u) + limit - 1) / limit) > budget) return false;
+  auto fits = [&](uint32_t l) {
+    const FastDiv by = make_fast_div(l);
+    uint32_t units = 0;
+    for (uint32_t mt = 0; mt < n_mtiles && units <= budget; ++mt) {
+      const uint32_t s = fast_div(tiles(mt) + l - 1, by);
+      units += s > kMapSplits ? budget + 1u : s;
+    }
+    return units <= budget;
+  };
+  if (fits(len)) limit = len;
+  else if (!fits(limit)) return false;
+  while (len < limit) {
+    const uint32_t mid = len + (limit - len) / 2u;
+    if (fits(mid)) limit = mid;
+    else len = mid + 1u;
+  }
+  return make_split_map(n_mtiles, len, tiles, m);
+}
+
 // One pass of top-k sparse attention over canvas rows [tok0, tok0 + ntok).
 constexpr int kTopkMaxK = 1024;   // most keys a row may keep
 struct TopkParams {

@@ -203,24 +203,25 @@ bool plan_split_map(const dg_attn_desc* d, const Plan& pl, int cus, uint32_t nti
   if (d->head_dim != 512 || d->causal_rows == 0 || d->window != 0 || (d->flags & DG_ATTN_F_T_LO_EXPLICIT) || !pl.part_half) return false;
   const uint32_t budget = (uint32_t)cus / d->n_kv_heads;
   if (pl.tiles_per_split >= ntiles || budget < pl.n_mtiles || ntiles >= 65536u) return false;
+  const dg::FastDiv by_group = dg::make_fast_div(pl.group);
   auto tiles = [&](uint32_t mt) -> uint32_t {   // as the kernel cuts them
-    const uint32_t a = mt * dg::kBlockM / pl.group, b = (std::min((mt + 1) * dg::kBlockM, pl.rows_total) - 1) / pl.group;
+    const uint32_t b = dg::fast_div(std::min((mt + 1) * dg::kBlockM, pl.rows_total) - 1, by_group);
     uint32_t hi = b < d->causal_rows ? std::min(pl.t_all, d->kv_len + b + 1) : pl.t_all;
-    if (a < d->causal_rows && pl.extra_lo < pl.t_all) hi = pl.t_all;
+    if (pl.extra_lo < pl.t_all && dg::fast_div(mt * dg::kBlockM, by_group) < d->causal_rows) hi = pl.t_all;
     return (hi + dg::kBlockN - 1) / dg::kBlockN;
   };
   const double s = std::sqrt((double)ntiles * budget / pl.n_mtiles / 9.0);
-  uint32_t len = std::max(1u, (uint32_t)(ntiles / std::max(1.0, s)));
-  for (; 10u * len <= 9u * pl.tiles_per_split && len + 2u <= pl.tiles_per_split; ++len)
-    if (dg::make_split_map(pl.n_mtiles, len, tiles, out) && out->units <= budget) return out->n > 1;
-  return false;
+  const uint32_t len = std::max(1u, (uint32_t)(ntiles / std::max(1.0, s))), tps = pl.tiles_per_split;
+  const uint32_t limit = tps < 3u ? 0u : std::min(tps - 2u, 9u * tps / 10u);
+  return dg::shortest_split_map(pl.n_mtiles, len, limit, budget, tiles, out) && out->n > 1;
 }
 
 // Scratch a split count takes, and the count for a call that has `scratch` bytes of it: what the rule asks for, or, where
 // that is more, splits of at least 6 tiles (a caller may hold what an earlier library asked for).
-// `on_device`: the prefix length is read when the kernels run, so every row tile has the same count.
+// `with_map`: the call may have a split map.  Not where the prefix length is read when the kernels run (every row tile then has
+// the same count), nor where the plan is not that of a dense call.
 int make_plan(const dg_attn_desc* d, int cus, Plan* pl, const uint32_t* key_range = nullptr, size_t scratch = SIZE_MAX,
-              bool on_device = false) {
+              bool with_map = true) {
   if (!d) return DG_ERR_NULL;
   pl->cus = (uint32_t)cus;
   const uint32_t hd = d->head_dim;
@@ -363,11 +364,11 @@ int make_plan(const dg_attn_desc* d, int cus, Plan* pl, const uint32_t* key_rang
   } else {
     carve(tiles_of_split(ntiles, base, (uint32_t)cus, hd, false), hd == 512 && ntiles < kF32PartTiles);
     dg::SplitMap map;
-    if (!key_range && plan_split_map(d, *pl, cus, ntiles, &map)) {
+    if (with_map && !key_range && plan_split_map(d, *pl, cus, ntiles, &map)) {
       // (sized for either, so that one workspace serves the entry points with and without a host-known prefix)
       const size_t rows = (size_t)d->n_kv_heads * map.units * dg::kBlockM, equal = pl->total;
       const size_t ml = pl->off_part_o + align_up(rows * hd * 2), both = std::max(equal, ml + align_up(rows * 8));
-      if (!on_device && both <= scratch) {
+      if (both <= scratch) {
         pl->map = map;
         pl->n_splits = map.n;
         pl->off_part_ml = ml;
@@ -442,7 +443,7 @@ int dg_attn_resolved_splits(const dg_attn_desc* d, uint32_t* out_splits) {
 int dg_attn_visible_pairs(const dg_attn_desc* d, uint64_t* pairs, double* flops) {
   if (!d) return DG_ERR_NULL;
   Plan pl;
-  const int rc = make_plan(d, plan_cus(), &pl);
+  const int rc = make_plan(d, plan_cus(), &pl, nullptr, SIZE_MAX, false);
   if (rc != DG_OK) return rc;
   uint64_t n = 0;
   for (uint32_t tok = 0; tok < d->canvas; ++tok) {
@@ -609,7 +610,7 @@ int dg_attn_forward_dev(const dg_attn_desc* d, const dg_step_params* step_dev, c
   int rc = device_info(&di);
   if (rc != DG_OK) return rc;
   Plan pl;
-  rc = make_plan(d, di.cus, &pl, nullptr, workspace ? workspace_bytes : 0, true);
+  rc = make_plan(d, di.cus, &pl, nullptr, workspace ? workspace_bytes : 0, false);
   if (rc != DG_OK) return rc;
   return forward_planned(d, pl, q, kv_base, out, lse, workspace, workspace_bytes, stream, (const uint32_t*)step_dev);
 }
@@ -653,7 +654,7 @@ inline dg_attn_desc partial_desc(const dg_attn_desc* d) {
 int dg_attn_state_bytes(const dg_attn_desc* d, size_t* out_bytes) {
   if (!d || !out_bytes) return DG_ERR_NULL;
   Plan pl;
-  const int rc = make_plan(d, plan_cus(), &pl);
+  const int rc = make_plan(d, plan_cus(), &pl, nullptr, SIZE_MAX, false);
   if (rc != DG_OK) return rc;
   *out_bytes = state_bytes_of(d);
   return DG_OK;
@@ -703,7 +704,7 @@ int dg_attn_merge(const dg_attn_desc* d, const void* const* states, uint32_t n_s
   int rc = device_info(&di);
   if (rc != DG_OK) return rc;
   Plan pl;
-  rc = make_plan(d, di.cus, &pl);
+  rc = make_plan(d, di.cus, &pl, nullptr, SIZE_MAX, false);
   if (rc != DG_OK) return rc;
   dg::StateMergeParams p;
   std::memset(&p, 0, sizeof(p));
@@ -846,7 +847,7 @@ int make_topk_plan(const dg_attn_desc* d, const uint32_t* k_cfg, const Plan& pl,
 int dg_attn_topk_workspace_bytes(const dg_attn_desc* d, const uint32_t* k_cfg, size_t* out_bytes) {
   if (!d || !out_bytes) return DG_ERR_NULL;
   Plan pl;
-  int rc = make_plan(d, plan_cus(), &pl);
+  int rc = make_plan(d, plan_cus(), &pl, nullptr, SIZE_MAX, false);
   if (rc != DG_OK) return rc;
   TopkPlan tk;
   rc = make_topk_plan(d, k_cfg, pl, plan_cus(), &tk);
@@ -862,7 +863,7 @@ int dg_attn_topk_forward(const dg_attn_desc* d, const uint32_t* k_cfg, const voi
   int rc = device_info(&di);
   if (rc != DG_OK) return rc;
   Plan pl;
-  rc = make_plan(d, plan_cus(), &pl);
+  rc = make_plan(d, plan_cus(), &pl, nullptr, SIZE_MAX, false);
   if (rc != DG_OK) return rc;
   TopkPlan tk;
   rc = make_topk_plan(d, k_cfg, pl, plan_cus(), &tk);

@@ -1,5 +1,6 @@
 """Split counts per row tile (SplitMap in csrc/attn_params.h), compiled for the host: every (row tile, split) is one unit of a
-KV head, found again from its number, and the longest share keeps the asked-for length."""
+KV head, found again from its number, the longest share keeps the asked-for length, and the shortest length is found without
+trying each."""
 import subprocess
 
 from diffgemma_amd import attention as A, build, capi
@@ -34,6 +35,27 @@ int main() {
             seen[mt] |= 1u << s;
           }
         }
+  // the shortest length: what trying every one finds, looked at a bounded number of times, once where no row tile can do with less
+  for (uint32_t n = 1; n <= 64; n += 9)
+    for (uint32_t base = 0; base <= 1100; base += base < 40 ? 8 : 353)
+      for (uint32_t per = 0; per <= 3; ++per)
+        for (uint32_t budget = n; budget <= 128; budget += 37)
+          for (uint32_t len = 1; len <= 60; len += 1 + len / 2)
+            for (uint32_t limit = 0; limit <= 520; limit += 1 + limit / 2) {
+              uint32_t calls = 0;
+              auto tiles = [&](uint32_t mt) { return ++calls, base + 1 + mt * per / 2; };
+              SplitMap want, got;
+              bool found = false;
+              for (uint32_t l = len; l <= limit && !found; ++l) found = make_split_map(n, l, tiles, &want) && want.units <= budget;
+              calls = 0;
+              if (shortest_split_map(n, len, limit, budget, tiles, &got) != found) return std::printf("n %u base %u len %u limit %u budget %u\n", n, base, len, limit, budget), 1;
+              if (calls > 1u + 12u * n || (per == 0 && limit && n * ((base + limit) / limit) > budget && calls > 1u))
+                return std::printf("n %u base %u len %u limit %u budget %u: %u calls\n", n, base, len, limit, budget, calls), 1;
+              if (!found) continue;
+              bool same = got.n == want.n && got.units == want.units;
+              for (uint32_t i = 0; i < kMapSplits; ++i) same = same && got.first[i] == want.first[i] && got.cum[i] == want.cum[i];
+              if (!same) return std::printf("n %u base %u len %u limit %u budget %u: another map\n", n, base, len, limit, budget), 1;
+            }
   std::puts("ok");
   return 0;
 }
