@@ -404,13 +404,19 @@ __global__ void __launch_bounds__(256) attn_merge_few_kernel(const MergeArgs arg
 
 template <uint32_t N>
 hipError_t launch_merge_few(const MergeArgs& a, uint32_t rows, hipStream_t s) {
-  if (!a.p.part_half) {
-    if constexpr (N > 8) return hipErrorInvalidValue;   // (not asked for)
-    else if (a.hd <= 256) hipLaunchKernelGGL((attn_merge_few_kernel<N, false, 1>), dim3((rows + 3) / 4), dim3(256), 0, s, a);
-    else hipLaunchKernelGGL((attn_merge_few_kernel<N, false, 2>), dim3((rows + 3) / 4), dim3(256), 0, s, a);
-  } else if (a.map.n) hipLaunchKernelGGL((attn_merge_few_kernel<N, true>), dim3((rows + 3) / 4), dim3(256), 0, s, a);
-  else hipLaunchKernelGGL((attn_merge_few_kernel<N, false>), dim3((rows + 3) / 4), dim3(256), 0, s, a);
-  return hipGetLastError();
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((rows + 3) / 4), dim3(256), 0, s, a);
+    return hipGetLastError();
+  };
+  if constexpr (N <= kMapSplits) {   // (what a map gives a row tile at most)
+    if (a.map.n) return launch(attn_merge_few_kernel<N, true>);
+  }
+  if constexpr (N <= 8) {
+    if (!a.p.part_half) return launch(a.hd <= 256 ? attn_merge_few_kernel<N, false, 1> : attn_merge_few_kernel<N, false, 2>);
+  } else if (a.map.n || !a.p.part_half) {
+    return hipErrorInvalidValue;   // (not asked for)
+  }
+  return launch(attn_merge_few_kernel<N, false>);
 }
 
 __device__ __forceinline__ float load_any(const void* src, uint32_t dt, size_t i) {

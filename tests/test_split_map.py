@@ -1,6 +1,7 @@
 """Split counts per row tile (SplitMap in csrc/attn_params.h), compiled for the host: every (row tile, split) is one unit of a
 KV head, found again from its number, the longest share keeps the asked-for length, and the shortest length is found without
 trying each."""
+import re
 import subprocess
 
 from diffgemma_amd import attention as A, build, capi
@@ -83,3 +84,13 @@ def test_where_a_split_map_is_planned():
         assert capi.resolved_splits(d) == 2
     row_tiles = 2 * 64 * 128
     assert capi.workspace_bytes(desc(1024, 0, 1024)) >= 2 * row_tiles * (512 * 2 + 8)      # two equal splits
+
+
+def test_every_merge_instance_can_be_reached():
+    """The merge that asks for all rows at once: one instance per split count up to 8 and every second to 16, with a map only up to
+    the splits a map gives, fp32 rows up to 8."""
+    names = subprocess.run(["nm", "-C", str(build.LIB_PATH)], stdout=subprocess.PIPE, text=True, check=True).stdout
+    built = set(re.findall(r"attn_merge_few_kernel<(\d+)u, (true|false), (\d+)u>", names))
+    few = [str(n) for n in range(2, 9)]
+    want = {(n, "false", "0") for n in few + ["10", "12", "14", "16"]} | {(n, "true", "0") for n in few}
+    assert built == want | {(n, "false", c) for n in few for c in "12"}
