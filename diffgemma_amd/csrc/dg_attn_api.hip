@@ -624,8 +624,15 @@ int dg_attn_forward_static(const dg_attn_desc* d, const void* q, const void* kv_
   int rc = device_info(&di);
   if (rc != DG_OK) return rc;
   Plan pl;
-  rc = make_plan(d, di.cus, &pl, nullptr, kStaticScratchBytes);
+  // Calls that can do without scratch do without it, whatever splitting their keys would save (64 rows over a window 16 us for
+  // 13): they never touched it, and callers may have them overlap.
+  rc = make_plan(d, di.cus, &pl, nullptr, 0);
   if (rc != DG_OK) return rc;
+  if (pl.total > 0) {
+    pl = Plan();
+    rc = make_plan(d, di.cus, &pl, nullptr, kStaticScratchBytes);
+    if (rc != DG_OK) return rc;
+  }
   if (pl.total > kStaticScratchBytes) return DG_ERR_SCRATCH_LIMIT;
   void* ptr = nullptr;
   rc = static_scratch_ptr(&ptr);

@@ -148,7 +148,9 @@ void dg_attn_desc_reference_layout(dg_attn_desc* d);
 void dg_attn_desc_head_major_layout(dg_attn_desc* d, uint64_t t_cap);
 
 /* Bytes of device scratch dg_attn_forward asks for with this descriptor (0 is possible).  With less it splits the keys less, down
- * to splits of 6 key tiles (none at all for a short key range at head_dim <= 256); below that, DG_ERR_WORKSPACE. */
+ * to splits of 6 key tiles (none at all for a short key range at head_dim <= 256, or below 12 key tiles): the result then differs by
+ * rounding, not in accuracy.  Below that, DG_ERR_WORKSPACE.  Calls that overlap need scratch of their own each, few rows over a
+ * window and short global ranges among them: given a workspace they write to it. */
 int dg_attn_workspace_bytes(const dg_attn_desc* d, size_t* out_bytes);
 
 /* Splits the library would use for this descriptor (n_splits==0 resolved). */
@@ -181,12 +183,14 @@ int dg_attn_forward_dev(const dg_attn_desc* d, const struct dg_step_params* step
  * counterpart in the reference.  The scratch dg_attn_forward takes from its workspace (split
  * partial rows, converted copies of f32 inputs) lives in DG_ATTN_STATIC_SCRATCH_BYTES of device
  * memory inside the library, held on every GPU the library runs on until the process ends; a call
- * whose dg_attn_workspace_bytes() exceeds that returns DG_ERR_SCRATCH_LIMIT and enqueues nothing.
+ * that needs more returns DG_ERR_SCRATCH_LIMIT and enqueues nothing.
  * 40 MiB covers the model's layers with f16 partial rows (global layer at any prefix: 32.3 MiB;
  * a 1024-row prefill super-chunk: 32.3 MiB), not a global layer with fp32 partial rows (64.3 MiB).
- * Same kernels, same results as dg_attn_forward, bit for bit.  The call allocates and frees
+ * A call that dg_attn_forward also takes without a workspace (short key ranges: the sliding layers, a global layer below 12 key
+ * tiles) does not touch the scratch, and its results are those of that form.  Any other has the results of dg_attn_forward
+ * with a workspace of this size.  Same kernels, bit for bit.  The call allocates and frees
  * nothing; its first call on a device looks the scratch address up (do that once outside a graph
- * capture).  All calls on one GPU share the one scratch: calls that overlap on a GPU (two
+ * capture).  All calls on one GPU share the one scratch: calls that use it and overlap on a GPU (two
  * streams, two threads) race; calls on one stream are ordered and safe. */
 #define DG_ATTN_STATIC_SCRATCH_BYTES (40u << 20)
 int dg_attn_forward_static(const dg_attn_desc* d, const void* q, const void* kv_base, void* out, float* lse,

@@ -1,7 +1,7 @@
 """dg_attn_forward_static, the entry point that allocates nothing: its split partial rows live in
 device memory inside the library instead of a caller's workspace.  It has to give what
 dg_attn_forward gives, bit for bit (same kernels), on calls that follow each other and share the
-one scratch: a larger call first, a smaller one after it."""
+one scratch: a larger call first, a smaller one after it; calls that can do without scratch leave it alone."""
 import ctypes as C
 
 import numpy as np
@@ -40,6 +40,28 @@ def test_static_scratch_entry_equals_workspace_entry_on_two_calls_in_a_row(gpu_r
         assert np.array_equal(out_a, out_b), w.name
         assert np.array_equal(lse_a.view(np.uint32), lse_b.view(np.uint32)), w.name
         assert np.isfinite(lse_a).all()
+
+
+@pytest.mark.parametrize("w", [W.Workload("few_sliding", 64, 16, 8, 256, 4000, window=1024, seed=3), W.Workload("short_global", 64, 16, 2, 512, 250, seed=4)],
+                         ids=lambda w: w.name)
+def test_static_scratch_is_left_alone_by_calls_that_can_do_without(gpu_ready, w):
+    """A few rows on a sliding layer, a short global range: dg_attn_forward splits their keys if it is given a workspace and runs
+    without one, too.  The static entry takes the second form, so that such calls, on several streams, have no memory in common."""
+    import torch
+    q, kv = W.generate(w)
+    qd, kd = W.device_arrays(w, q, kv)
+    d = w.desc()
+    assert capi.resolved_splits(d) > 1 and capi.workspace_bytes(d) > 0
+    n = w.canvas * w.n_q_heads
+    out = [torch.full((n * w.head_dim,), 0x7fc0, dtype=torch.int16, device="cuda") for _ in range(3)]
+    lse = [torch.zeros(n, dtype=torch.float32, device="cuda") for _ in range(3)]
+    A.forward(d, qd, kd, out[0], lse[0], A.alloc_workspace(d))
+    A.forward(d, qd, kd, out[1], lse[1], None)
+    capi.check(capi.load().dg_attn_forward_static(C.byref(d), qd.data_ptr(), kd.data_ptr(), out[2].data_ptr(), lse[2].data_ptr(),
+                                                  A.stream_handle()))
+    torch.cuda.synchronize()
+    assert torch.equal(out[2], out[1]) and torch.equal(lse[2], lse[1])
+    assert not torch.equal(out[2], out[0])                  # (the two forms round differently: it was not the first)
 
 
 def test_static_scratch_entry_rejects_what_does_not_fit(gpu_ready):
