@@ -323,8 +323,10 @@ __device__ __forceinline__ void dbg_report(uint32_t* dbg, uint32_t code, uint32_
 
 // Where the merge that asks for all of a row's 16-bit partial rows at once beats the one that looks at the weights first, four
 // rows at a time: up to 8 splits while they are less than 32 MiB in all; up to 16 where they are few bytes.  Attention call, us,
-// weights first | at once, flat and peaked rows (of which the first fetches a part): 64 rows over 841 keys in 9 splits 20.4 | 18.3,
-// 19.1 | 18.0, over 5064 in 16 32.2 | 29.4, 31.7 | 28.9; past 17 MiB 128 rows over 428 keys in 14 splits 20.4 | 27.1 on peaked rows.
+// weights first | at once, peaked rows (of which the first fetches a part) and flat ones: 64 rows over 841 keys in 9 splits 19.2 | 18.4,
+// 20.5 | 18.4, over 1264 in 14 20.2 | 20.6, 23.5 | 20.7, over 2064 in 13 23.4 | 23.1, 25.7 | 23.1, over 5064 in 16 30.6 | 29.7, 32.7 | 29.8; 16 rows over 3300 in
+// 15 25.3 | 22.5, 25.4 | 22.5.  With more rows peaked ones lose what flat ones gain: 96 rows in 10 splits, 15 MiB, 22.0 | 24.0, 25.3 | 24.0 (head_dim 256,
+// rows half as long, 96 rows in 14 24.7 | 22.6, 24.8 | 22.6); past 17 MiB 128 rows over 428 keys in 14 splits 20.4 | 27.1 on peaked rows.
 constexpr uint32_t kMergeFewSplits = 16;
 inline bool merge_at_once(uint32_t n_splits, size_t bytes) {
   return n_splits <= 8 ? bytes < ((size_t)32 << 20) : n_splits <= kMergeFewSplits && bytes <= ((size_t)17 << 20);

@@ -150,9 +150,15 @@ struct Plan {
 //
 // head_dim 512: a tile takes c = 1.3 to 1.6 us, and a split what its partial rows take, written and read back, about 9 c / room:
 // c n / s + 9 c s / room is least at s = sqrt(n room / 9).  The curve is flat around it; where it leads past the splits that
-// are merged at once, fewer are taken as long as that makes a share at most three tiles longer.  Attention call, us, splits
+// are merged at once, fewer are taken as long as that makes a share at most three tiles longer, or 8 in all (32 rows over 3700 keys, 29 |
+// 15 splits: peaked rows 25.0 | 24.8, flat 29.5 | 24.8; to 9 tiles, 48 rows over 4500, 29 | 16: 27.1 | 28.3, 30.3 | 28.5).  Attention call, us, splits
 // of 6 tiles and more | this rule: 64 rows (room 32) over 841 keys 21.0 | 18.3, 2064 25.9 | 23.7,
 // 5064 31.2 | 29.4; 128 rows (16) over 428 keys 21.7 | 18.6, 905 23.8 | 22.9, 2128 28.7 | 28.1; 256 rows (8) over 556 24.4 | 24.5, 1033 26.7 | 27.0.
+//
+// Once the merge has more workgroups than the chip has compute units (four rows each: past 64 rows of 16 heads), more than 8 rows at
+// once cost it what they save the shares: 8 splits where that makes a share one tile longer.  More | 8 at most: 72 rows over 1000 keys,
+// 11 splits, peaked 21.0 | 19.8, flat 21.1 | 20.1; 80 over 841, 9, 20.4 | 19.4, 20.4 | 19.5; 96 over 1264, 10, 24.0 | 23.1, 24.0 | 23.4; by
+// two tiles, 96 over 1700, 11, 24.9 | 25.2, 25.0 | 25.5; 72 over 1500, 12, 23.1 | 22.0, 23.2 | 22.3.
 //
 // Fewer than kF32PartTiles tiles were one split as long as none was shorter than 6, and its rows fp32 until they are rounded for the
 // output: where these are split, the partial rows are fp32 too.  They cost twice as much, so sqrt(n room / 18), and one split
@@ -175,8 +181,10 @@ uint32_t tiles_of_split(uint32_t ntiles, uint32_t base, uint32_t cus, uint32_t h
   const double s = std::sqrt((double)ntiles * room / (f32_parts ? 18.0 : 9.0));
   const uint32_t t = std::max(std::max(1u, (uint32_t)(ntiles / s + 0.5)), of(room));
   const size_t split_bytes = (size_t)base * dg::kBlockM * hd * (f32_parts ? 4 : 2);
-  for (uint32_t few = dg::kMergeFewSplits; few >= 8u && !dg::merge_at_once(of(t), of(t) * split_bytes); few -= 8u)
-    if (dg::merge_at_once(of(of(few)), of(of(few)) * split_bytes)) return of(few) > t && of(few) <= t + 3u ? of(few) : t;
+  auto at_once = [&](uint32_t splits) { return dg::merge_at_once(splits, splits * split_bytes); };
+  if (at_once(of(t))) return of(t) > 8u && base * (dg::kBlockM / 4) > cus && of(8) <= t + 1u ? of(8) : t;
+  for (uint32_t few = dg::kMergeFewSplits; few >= 8u; few -= 8u)
+    if (at_once(of(of(few)))) return of(few) > t && of(few) <= std::max(t + 3u, few / 2u) ? of(few) : t;
   return t;
 }
 

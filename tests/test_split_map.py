@@ -94,3 +94,11 @@ def test_every_merge_instance_can_be_reached():
     few = [str(n) for n in range(2, 9)]
     want = {(n, "false", "0") for n in few + ["10", "12", "14", "16"]} | {(n, "true", "0") for n in few}
     assert built == want | {(n, "false", c) for n in few for c in "12"}
+
+
+def test_split_counts_that_keep_the_merge_short():
+    """(rows, keys) of 16 heads over 2 -> splits: to 16 with at most a merge workgroup per compute unit, a share of up to three tiles
+    more, or 8 in all, taken for it; past that to 8 where a share gets one tile longer."""
+    splits = lambda rows, keys: capi.resolved_splits(A.make_desc(rows, 16, 2, 512, keys - rows, flags=capi.DG_ATTN_F_F16_PARTIALS))
+    assert [splits(64, 1264), splits(32, 3700), splits(32, 4064), splits(48, 4500)] == [14, 15, 16, 29]
+    assert [splits(72, 1000), splits(80, 841), splits(96, 1264), splits(96, 1700), splits(72, 1500)] == [8, 7, 8, 11, 12]
