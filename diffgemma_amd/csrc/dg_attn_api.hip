@@ -190,14 +190,24 @@ uint32_t tiles_of_split(uint32_t ntiles, uint32_t base, uint32_t cus, uint32_t h
 
 // Key tiles per workgroup of the one-launch kernel: all that a 32-row tile sees, or, where a few canvas rows over most of a
 // window leave three quarters of the chip idle, a share of them, the rows merged as the split kernel's are (fp32 partial rows: in one
-// launch nothing of a row is narrower; a workgroup's run is cut over its four waves again).  A wave's tile takes 1.07 us; the
-// second launch about 4, and more with the rows.  Attention call, us, one launch | shared by 5, window 1024: behind 4000 keys 16 rows
-// 15.8 | 10.7, 32 15.8 | 11.5, 64 16.1 | 13.1, 100 16.4 | 14.9, 128 16.3 | 16.1; shorter ranges, 32 rows: 17 tiles 11.1 | 10.7, 14 10.1 |
-// 10.7; 64 rows: 24 tiles 12.7 | 12.2, 18 11.3 | 11.7; 100 rows: 29 tiles 14.8 | 13.6, 25 13.5 | 13.2, 22 12.5 | 12.8.  By 4 or 6: 0 to 0.4 slower.
+// launch nothing of a row is narrower; a workgroup's run is cut over its four waves again).  In tiles of a wave (1.07 us; a fifth
+// more over an f16 cache, where peaked rows rescale) a number of shares costs the tiles of its longest run, and where it is not one, 2
+// for the second launch and 1 for every 55 row tiles of partial rows.  Attention call, us, in 1 | 2 | 3 | 4 | 5 shares, 16 heads over
+// 8: 16 rows over 36 tiles 15.5 in one, 10.9 in 5 (5 taken); 64 over 36 15.7 | 14.7 | 13.3 | 13.5 | 12.9 (3); 64 over 28 13.6 | 13.5 | 12.5 | 12.4 |
+// 12.5 (4); 96 over 30 14.4 | 14.2 | 13.9 | 14.1 | 15.1 (4); 112 over 28 13.6 | 14.4 | 13.6 | 14.9 (1); over an f16 cache, peaked rows and flat ones,
+// 64 over 30 18.7 | 15.7 | 14.4 | 13.3 | 13.8 and 14.7 | 13.7 | 12.9 | 12.6 | 13.1 (4).  Over 780 forms (1, 2 and 8 KV heads, 8 to 56 row tiles, 16 to 36
+// key tiles, both caches) at most 3 % behind one launch; always 5 shares, as many as fit, was up to 14 % behind.
 uint32_t share_of_short_range(const dg_attn_desc* d, const Plan& pl, uint32_t cus, uint32_t ntiles) {
   const uint32_t base = d->n_kv_heads * ((pl.rows_total + 31u) / 32u);
   if (d->head_dim != 256 || base * 9u > cus * 2u || pl.span_tiles < 17u + base / 6u) return ntiles;
-  const uint32_t s = std::min(cus / base, 5u);
+  const double row_tiles = d->n_kv_heads * (pl.rows_total / 32.0), tile = pl.e_dtype == DG_F16 ? 1.2 : 1.0;
+  auto cost = [&](uint32_t s) {
+    const uint32_t share = (pl.span_tiles + s - 1) / s;
+    return tile * ((share + 3u) / 4u) + (s > 1 ? 2.0 + s * row_tiles / 55.0 : 0.0);
+  };
+  uint32_t s = 1;
+  for (uint32_t more = 2; more <= std::min(cus / base, 5u); ++more)
+    if (cost(more) < cost(s)) s = more;
   return (ntiles + s - 1) / s;
 }
 

@@ -102,3 +102,12 @@ def test_split_counts_that_keep_the_merge_short():
     splits = lambda rows, keys: capi.resolved_splits(A.make_desc(rows, 16, 2, 512, keys - rows, flags=capi.DG_ATTN_F_F16_PARTIALS))
     assert [splits(64, 1264), splits(32, 3700), splits(32, 4064), splits(48, 4500)] == [14, 15, 16, 29]
     assert [splits(72, 1000), splits(80, 841), splits(96, 1264), splits(96, 1700), splits(72, 1500)] == [8, 7, 8, 11, 12]
+
+
+def test_shares_of_a_short_range():
+    """(rows, prefix, heads, KV heads) of a sliding layer -> workgroups to a row tile: by what their tiles, a second launch and their
+    partial rows cost; one where that is no gain, and past 112 rows of 16 heads."""
+    shares = lambda rows, kv, hq=16, hkv=8: capi.resolved_splits(A.make_desc(rows, hq, hkv, 256, kv, window=1024))
+    assert [shares(rows, 4000) for rows in (16, 48, 64, 80, 96, 112, 128, 256)] == [5, 5, 3, 3, 3, 3, 1, 1]
+    assert [shares(112, 781), shares(96, 861), shares(64, 829), shares(32, 200)] == [1, 4, 4, 1]
+    assert [shares(100, 800, 16, 2), shares(32, 800, 48, 8), shares(112, 4000, 8, 1)] == [4, 1, 3]
