@@ -153,7 +153,9 @@ void dg_attn_desc_head_major_layout(dg_attn_desc* d, uint64_t t_cap);
  * window and short global ranges among them: given a workspace they write to it. */
 int dg_attn_workspace_bytes(const dg_attn_desc* d, size_t* out_bytes);
 
-/* Splits the library would use for this descriptor (n_splits==0 resolved). */
+/* Splits dg_attn_forward uses for this descriptor (n_splits==0 resolved) with the scratch that dg_attn_workspace_bytes asks for; where
+ * row tiles have split counts of their own (causal rows of a global layer, 16-bit partial rows, a short prefix) the most of any.  The
+ * entries that read the prefix on the device take one count for all row tiles, which can be another. */
 int dg_attn_resolved_splits(const dg_attn_desc* d, uint32_t* out_splits);
 
 /* q, out: [canvas][n_q_heads][head_dim]; lse: [canvas][n_q_heads] fp32 natural-log
@@ -173,7 +175,9 @@ int dg_attn_forward(const dg_attn_desc* d, const void* q, const void* kv_base, v
  * for it (dg_attn_workspace_bytes with the same descriptor), and a device value above it is clamped to it.  A HIP
  * graph recorded with this entry stays valid while the caller advances kv_len in device memory after every committed
  * block (src/metal/step_generate/turn.rs:575-660) instead of recording again.  For every device value the result is
- * that of dg_attn_forward with kv_len set to it, bit for bit when both resolve to the same split count.  Not for the
+ * that of dg_attn_forward with kv_len set to it, up to the rounding of other splits, and bit for bit where both run the
+ * same plan: with n_splits given and the same dg_attn_resolved_splits at both prefixes, or at the planned prefix
+ * itself, unless dg_attn_forward has split counts per row tile there (see dg_attn_resolved_splits).  Not for the
  * scalar cross-check kernel or an f32 cache (DG_ERR_UNSUPPORTED). */
 int dg_attn_forward_dev(const dg_attn_desc* d, const struct dg_step_params* step_dev, const void* q, const void* kv_base,
                         void* out, float* lse, void* workspace, size_t workspace_bytes, void* stream);

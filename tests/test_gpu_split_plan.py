@@ -96,6 +96,31 @@ def test_device_prefix_with_the_scratch_of_a_split_map(gpu_ready, po):
     assert (outs[0] - outs[1]).abs().max() <= 2.0 ** -7 * outs[1].abs().max()
 
 
+@pytest.mark.parametrize("hd,hkv,splits", [(512, 2, 3), (256, 8, 2)])
+def test_device_prefix_and_an_explicit_split_count(gpu_ready, hd, hkv, splits):
+    """With n_splits given, the entry that reads the prefix on the device, planned for a longer one, gives the host entry's bits: causal
+    rows that would have split counts of their own, and a range that would be one launch."""
+    import torch
+    kv_len, planned = 300, 700
+    w = W.Workload("dev_splits", 256, 16, hkv, hd, planned, causal_rows=256, seed=7)
+    q, kv = W.generate(w)
+    qd, kd = W.device_arrays(w, q, kv)
+    mk = lambda n: A.make_desc(w.canvas, 16, hkv, hd, n, causal_rows=256, layout="head_major", t_cap=w.t_all, n_splits=splits,
+                               flags=capi.DG_ATTN_F_F16_PARTIALS)
+    host, dev = mk(kv_len), mk(planned)
+    assert capi.resolved_splits(host) == capi.resolved_splits(dev) == splits
+    outs, lses = [], []
+    for run in (lambda o, l: A.forward(host, qd, kd, o, l, A.alloc_workspace(host)),
+                lambda o, l: A.forward_dev(dev, A.device_step_params(kv_len), qd, kd, o, l, A.alloc_workspace(dev))):
+        out = torch.zeros(w.canvas * 16 * hd, dtype=torch.int16, device="cuda")
+        lse = torch.zeros(w.canvas * 16, device="cuda")
+        run(out, lse)
+        torch.cuda.synchronize()
+        outs.append(out)
+        lses.append(lse)
+    assert torch.equal(*outs) and torch.equal(*lses)
+
+
 @pytest.mark.parametrize("canvas,kv_len,causal_rows,hkv,window,ring,f16", [
     (64, 4000, 0, 8, 1024, 2048, False), (33, 5000, 33, 8, 1024, 2048, True), (112, 3001, 40, 8, 1024, 0, False),
     (100, 830, 0, 8, 0, 0, True), (17, 1100, 17, 4, 1024, 2048, False)])
