@@ -306,14 +306,14 @@ __global__ void __launch_bounds__(256) attn_mfma_kernel(const MfmaArgs args) {
     const char* base;   // wave-uniform
     uint32_t voff;      // per lane
   };
-  const uint32_t touch_first = tile_rows((te - 1u) * kBlockN, lo_min, p.t_all).first;
+  const uint32_t t_last = past_end_pos((te - 1u) * kBlockN, lo_min, p.t_all, p.ring_mask);
   auto touch_address = [&](uint32_t tile, uint32_t ln) -> Touch {
-    const uint32_t tp = min(tile, te - 1u) * kBlockN;
+    const uint32_t tp = min(tile * kBlockN, t_last);
     const uint32_t sh = p.n_mtiles >= 16u ? 4u : 3u;   // log2 of the number of shares
     const uint32_t share = mt & ((1u << sh) - 1u);
     const bool is_v = (share >> (sh - 1u)) != 0u;      // the upper half of the shares are V's lines
     const uint32_t li = (share & ((1u << (sh - 1u)) - 1u)) * (512u >> sh) + wave * (128u >> sh) + (ln & ((128u >> sh) - 1u));
-    const uint32_t row = touched_row(li >> 3, touch_first, tp, p.t_all);
+    const uint32_t row = min(li >> 3, p.t_all - 1u - tp);
     const int64_t stride_b = is_v ? vstride_b : kstride_b;
     const int64_t slot = (int64_t)kv_slot(p.ring_mask, tp);
     return Touch{(is_v ? vbase : kbase) + slot * stride_b, row * (uint32_t)stride_b + (li & 7u) * 128u};
@@ -334,14 +334,12 @@ __global__ void __launch_bounds__(256) attn_mfma_kernel(const MfmaArgs args) {
   lds_char* const k1 = (lds_char*)(smem + OFF_K1);
   lds_char* const v0 = (lds_char*)(smem + OFF_V0);
   lds_char* const v1 = (lds_char*)(smem + OFF_V1);
-  const uint32_t t_end = loads_end(te, p.t_all);
-  const uint32_t t_last = past_end_pos((te - 1u) * kBlockN, lo_min, t_end, p.ring_mask);
   // (in the loop only tiles behind the workgroup's first one are loaded)
   auto k_load = [&](uint32_t t0, lds_char* buf, uint32_t ln) {
-    return make_tile_load<D, false, false>(kbase, kstride_b, min(t0, t_last), 0u, t_end, p.ring_mask, buf, wave, ln);
+    return make_tile_load<D, false, false>(kbase, kstride_b, min(t0, t_last), 0u, p.t_all, p.ring_mask, buf, wave, ln);
   };
   auto v_load = [&](uint32_t t0, lds_char* buf, uint32_t ln) {
-    return make_tile_load<D, true, false>(vbase, vstride_b, min(t0, t_last), 0u, t_end, p.ring_mask, buf, wave, ln);
+    return make_tile_load<D, true, false>(vbase, vstride_b, min(t0, t_last), 0u, p.t_all, p.ring_mask, buf, wave, ln);
   };
   auto k_load_first = [&](lds_char* buf) {
     return make_tile_load<D, false, true>(kbase, kstride_b, tb * kBlockN, lo_min, p.t_all, p.ring_mask, buf, wave, lane);

@@ -72,7 +72,7 @@ struct AttnParams {
                               // prefix the launch was planned for
   int64_t k_tok_stride, k_head_stride, v_tok_stride, v_head_stride;  // elements
   uint32_t canvas, hq, hkv, group;
-  uint32_t kv_len, t_all;
+  uint32_t kv_len, t_all;   // (t_all: of a key range, the keys up to its end; keys_of_range)
   uint32_t causal_rows;
   uint32_t win_m1;       // window-1, or 0xffffffff when unwindowed
   uint32_t lo_nc;        // first visible key of a non-causal row
@@ -253,28 +253,22 @@ __host__ __device__ __forceinline__ TileRows tile_rows(uint32_t t0, uint32_t lo,
   r.first = lo <= t0 ? 0u : lo - t0 < r.last ? lo - t0 : r.last;
   return r;
 }
-// End of the rows that loads in the tile loop may read, for key tiles up to `te`: the last key, or the end of the last tile (past
-// it a holder of a key range has no memory).
-__host__ __device__ __forceinline__ uint32_t loads_end(uint32_t te, uint32_t t_all) {
-  return te * (uint32_t)kBlockN < t_all ? te * (uint32_t)kBlockN : t_all;
+// The number of keys a kernel is told of (AttnParams.t_all), for a launch over the key tiles [first, end): of a key range no more
+// than its tiles, so that no kernel needs another bound to stay within what a holder of that range has in memory.
+__host__ __device__ __forceinline__ uint32_t keys_of_range(uint32_t first, uint32_t end, uint32_t t_all) {
+  return end > first && end * (uint32_t)kBlockN < t_all ? end * (uint32_t)kBlockN : t_all;
 }
-// Where loads issued for tiles behind a row tile's last one (at t_last, its rows below t_end) go, so that the tile loop need not
-// branch around them: the last tile again, its rows clamped at the end alone.  Where that tile begins before `lo` (it is then the
-// only one), its rows from `lo` on; a ring has memory for every slot, and 32 rows from an arbitrary slot could run past its end.
-__host__ __device__ __forceinline__ uint32_t past_end_pos(uint32_t t_last, uint32_t lo, uint32_t t_end, uint32_t ring_mask) {
-  const uint32_t see = lo < t_end ? lo : t_end - 1u;
+// Where loads and touches issued for tiles behind a row tile's last one (at t_last) go, so that the tile loop need not branch
+// around them: the last tile again, its rows clamped at the end alone.  Where that tile begins before `lo` (it is then the only
+// one), the rows from `lo` on instead; a ring has memory for every slot, and 32 rows from an arbitrary slot could run past its end.
+__host__ __device__ __forceinline__ uint32_t past_end_pos(uint32_t t_last, uint32_t lo, uint32_t t_all, uint32_t ring_mask) {
+  const uint32_t see = lo < t_all ? lo : t_all - 1u;
   return ring_mask == 0u && see > t_last ? see : t_last;
-}
-// Row of the key tile at t0 that is touched into the L2 for row `row` of it.  Touches run from a row tile's fourth tile to its
-// last one, and with fewer tiles go to that: `first` is the first row that may be read of the last tile (0 unless it is the only one).
-__host__ __device__ __forceinline__ uint32_t touched_row(uint32_t row, uint32_t first, uint32_t t0, uint32_t t_all) {
-  const uint32_t last = t_all - 1u - t0, r = row > first ? row : first;
-  return r < last ? r : last;
 }
 // The one-launch kernel touches a range of keys [pos0, pos1), `per` of them to a touch: position of key `i` of touch u.
 __host__ __device__ __forceinline__ uint32_t touched_pos(uint32_t pos0, uint32_t pos1, uint32_t per, uint32_t u, uint32_t i) {
-  const uint32_t pos = pos0 + u * per + i;
-  return pos < pos1 ? pos : pos1 - 1u;
+  const uint32_t pos = pos0 + u * per + i, last = pos1 - 1u;
+  return pos < last ? pos : last;
 }
 // whether some row of the tile may not be read
 __host__ __device__ __forceinline__ bool tile_is_edge(uint32_t t0, uint32_t lo, uint32_t t_all) {

@@ -535,7 +535,7 @@ int fill_params(const dg_attn_desc* d, const Plan& pl, const void* q, const void
   p.hkv = d->n_kv_heads;
   p.group = pl.group;
   p.kv_len = d->kv_len;
-  p.t_all = pl.t_all;
+  p.t_all = dg::keys_of_range(pl.tile_first, pl.tile_end, pl.t_all);   // (the whole range ends with the last key)
   p.causal_rows = d->causal_rows;
   p.win_m1 = pl.win_m1;
   p.lo_nc = pl.lo_nc;

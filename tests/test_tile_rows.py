@@ -13,6 +13,14 @@ PROGRAM = r"""
 int main() {
   using namespace dg;
   const uint32_t span = 3 * kBlockN + 2;
+  // the keys a kernel is told of: those of the cache, or up to the key tile in which a range [begin, end) ends
+  for (uint32_t keys = 1; keys <= span; ++keys)
+    for (uint32_t end = 0; end <= keys; ++end)
+      for (uint32_t begin = 0; begin <= end; ++begin) {
+        const uint32_t first = begin / kBlockN, last = std::max(first, (end + kBlockN - 1) / kBlockN), told = keys_of_range(first, last, keys);
+        if (told > keys || (end > begin && (told < end || told > (end + kBlockN - 1) / kBlockN * kBlockN)) || (end == keys && told != keys))
+          return std::printf("[%u, %u) of %u: %u keys\n", begin, end, keys, told), 1;
+      }
   for (uint32_t t_all = 1; t_all <= span; ++t_all)
     for (uint32_t lo = 0; lo <= t_all + kBlockN; ++lo)
       for (uint32_t t0 = 0; t0 < t_all; t0 += kBlockN) {
@@ -26,25 +34,22 @@ int main() {
           if (row >= t_all || (row < see && see < t0 + kBlockN)) return std::printf("t_all %u lo %u t0 %u row %u\n", t_all, lo, t0, row), 1;
           if (t0 + i >= lo && t0 + i < t_all && row != t0 + i) return std::printf("moved a visible row %u\n", t0 + i), 1;
         }
-        // loads for tiles behind t0, the last one: no row behind that tile or the last key, and none before the first visible
-        // key where t0 is the first tile too
-        const uint32_t end = loads_end(t0 / kBlockN + 1u, t_all), pos = past_end_pos(t0, lo, end, 0u);
-        const TileRows past = tile_rows(pos, 0u, end);
-        if (pos + past.last >= t_all || pos + past.last >= t0 + kBlockN || pos < t0 || (see < t0 + kBlockN && pos + past.first < see) ||
-            past_end_pos(t0, lo, end, 63u) != t0)
+        // loads for tiles behind t0, the last one: nothing behind the last key, and nothing before the first visible one where t0 is
+        // the first tile too
+        const uint32_t pos = past_end_pos(t0, lo, t_all, 0u);
+        const TileRows past = tile_rows(pos, 0u, t_all);
+        if (pos + past.last >= t_all || pos < t0 || (see < t0 + kBlockN && pos + past.first < see) || past_end_pos(t0, lo, t_all, 63u) != t0)
           return std::printf("t_all %u lo %u t0 %u: past the end at %u\n", t_all, lo, t0, pos), 1;
-        // touches of a row tile whose last tile is t0 and whose first one, with `lo` in it, is up to three before
-        for (uint32_t tb = lo / kBlockN; tb <= t0 / kBlockN; ++tb) {
-          const uint32_t first = tile_rows(t0, lo, t_all).first;
+        // touches of a row tile whose last tile is t0 and whose first one, with `lo` in it, is anywhere before: from the fourth on
+        for (uint32_t tb = lo / kBlockN; tb <= t0 / kBlockN; ++tb)
           for (uint32_t tile = tb + 3u; tile < tb + 8u; ++tile) {
-            const uint32_t at = std::min(tile * kBlockN, t0);
+            const uint32_t at = std::min(tile * kBlockN, pos);
             for (uint32_t i = 0; i < (uint32_t)kBlockN; ++i) {
-              const uint32_t row = at + touched_row(i, first, at, t_all);
-              if (row >= t_all || row < see || row >= t0 + kBlockN || (at + i >= see && at + i < t_all && row != at + i))
+              const uint32_t row = at + std::min(i, t_all - 1u - at);
+              if (row >= t_all || row < see || (tile * kBlockN <= t0 && row != std::min(tile * kBlockN + i, t_all - 1u)))
                 return std::printf("t_all %u lo %u t0 %u: touches row %u\n", t_all, lo, t0, row), 1;
             }
           }
-        }
         if (clamped && !tile_is_edge(t0, lo, t_all)) return std::printf("t_all %u lo %u t0 %u: no edge tile\n", t_all, lo, t0), 1;
       }
   // touches of the one-launch kernel: every key of the range, and no other
@@ -83,17 +88,20 @@ def test_k_and_v_tiles_of_the_one_launch_kernel_share_the_rule():
     assert text.count("is_edge(tile)") == 2        # where K's loads go out and where V's do
 
 
-def test_loads_in_the_split_kernels_loop_end_with_its_last_tile():
-    """They once ended with the last key: behind a range of one tile that begins inside it, up to 31 rows past the range."""
-    text = (build.CSRC / "attn_mfma.hip").read_text()
-    assert text.count("min(t0, t_last), 0u, t_end, p.ring_mask") == 2 and text.count("min(t0, t_last)") == 2
+def test_kernels_are_told_of_the_keys_of_a_range_alone():
+    """Behind a range of one tile that begins inside it the split kernel once loaded up to 31 rows past the range: its loads ended
+    with the last key of the cache."""
+    api, text = (build.CSRC / "dg_attn_api.hip").read_text(), (build.CSRC / "attn_mfma.hip").read_text()
+    assert api.count("p.t_all = dg::keys_of_range(pl.tile_first, pl.tile_end, pl.t_all);") == api.count("  p.t_all = ") == 1
+    assert "t_last = past_end_pos((te - 1u) * kBlockN, lo_min, p.t_all, p.ring_mask)" in text
+    assert text.count("min(t0, t_last), 0u, p.t_all, p.ring_mask") == text.count("min(t0, t_last)") == 2
 
 
 def test_touches_of_the_split_kernel_begin_with_the_first_visible_key():
     """They once began with the tile: up to 31 rows before a share of one tile that begins inside it."""
     text = (build.CSRC / "attn_mfma.hip").read_text()
-    assert text.count("touched_row(") == 1 and "min(tile, te - 1u) * kBlockN" in text
-    assert "touch_first = tile_rows((te - 1u) * kBlockN, lo_min, p.t_all).first" in text
+    assert text.count("lds_dma_touch(") == 1 and text.count("tp = min(tile * kBlockN, t_last);") == 1
+    assert text.count("row = min(li >> 3, p.t_all - 1u - tp);") == 1
 
 
 def test_touches_of_the_one_launch_kernel_stay_in_its_range():
