@@ -83,7 +83,8 @@ def test_partials_match_the_oracle_and_merge_to_the_single_call(gpu_ready, po, n
 @pytest.mark.parametrize("a,b", [(1001, 1312), (1030, 1056), (1279, 1601)])
 def test_a_holder_of_a_key_range_needs_no_other_rows(gpu_ready, hkv, hd, window, a, b):
     """A buffer with the rows [a, b) alone, passed with its base shifted back by a rows, gives the whole cache's state bit for
-    bit: no row before a is read (a not on a key tile), and none past b (on a key tile, or the last key)."""
+    bit: no row before a takes part (a not on a key tile), and none past b (on a key tile, or the last key).  Loads whose values
+    nobody uses would not show here; which rows those touch is tests/test_tile_rows.py's."""
     import torch
     w = W.Workload("holder", 64, 16, hkv, hd, 1537, window=window, layout="reference", seed=a)
     q, kv = W.generate(w)
