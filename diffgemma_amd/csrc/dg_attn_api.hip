@@ -160,6 +160,10 @@ struct Plan {
 // 11 splits, peaked 21.0 | 19.8, flat 21.1 | 20.1; 80 over 841, 9, 20.4 | 19.4, 20.4 | 19.5; 96 over 1264, 10, 24.0 | 23.1, 24.0 | 23.4; by
 // two tiles, 96 over 1700, 11, 24.9 | 25.2, 25.0 | 25.5; 72 over 1500, 12, 23.1 | 22.0, 23.2 | 22.3.
 //
+// Other head counts (8 over 1 and 8, 16 over 1, 4 and 16, 32 over 4 and 8; 64 and 256 rows over 104 to 4256 keys), against the kernels and
+// counts as they were before this rule: 2 to 75 % faster; slower for flat rows in 30 splits and more alone, 64 of 8 heads over 1 over 4200
+// keys 30.1 | 31.6 (peaked 28.0 | 25.3).
+//
 // Fewer than kF32PartTiles tiles were one split as long as none was shorter than 6, and its rows fp32 until they are rounded for the
 // output: where these are split, the partial rows are fp32 too.  They cost twice as much, so sqrt(n room / 18), and one split
 // where that is small.  One split | this rule: 64 rows over 86 keys (n room 96) 14.2 | 16.0, over 184 (192) 18.4 | 17.1, over 314 (320)
