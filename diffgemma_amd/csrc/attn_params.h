@@ -146,9 +146,10 @@ struct TopkParams {
   uint32_t k_cfg[4];     // (fixed k | chunk grid, divisor, k_min, k_max)
   float scale;
   // Filtered path (launch_topk_filter): n_mtiles counts 256-row tiles there.
-  uint32_t sample_stride;   // every sample_stride-th key has its scores in the sample plane
-  uint32_t sample_n, sample_pad;
-  float* sample_plane;   // [hq][ntok][sample_pad]
+  uint32_t sample_stride;   // every sample_stride-th key is a sampled one
+  uint32_t sample_n;
+  uint32_t sample_splits;   // key-range splits of the sampled launch, at most its key tiles and kTopkSampleSplits
+  float* sample_max;     // [row of the pass][sample_splits * 32]: the largest score of each group of sampled keys
   float* tau;            // [hkv][n_mtiles * 256]: a row's threshold
   uint32_t* cand_n;      // [hkv][n_mtiles][n_splits][4 waves][kTopkSegs]: entries in a segment
   void* cand;            // the same index space, kTopkSegAlloc entries of 8 bytes each
@@ -164,8 +165,10 @@ struct TopkParams {
 constexpr uint32_t kTopkSegs = 128;         // per wave of the filter kernel and split: two blocks of 32 rows, two lanes per row
 constexpr uint32_t kTopkSegCap = 80, kTopkSegAlloc = kTopkSegCap + 16;
 constexpr uint32_t kTopkFilterRows = 256;   // stacked rows per workgroup of the filter kernel
+constexpr uint32_t kTopkSampleRows = 128;   // and of its instance for sampled keys
 constexpr uint32_t kTopkGather = 8;         // a row's list of kept keys is padded to a multiple
 constexpr uint32_t kTopkSampleMax = 8192;   // most sampled keys per row
+constexpr uint32_t kTopkSampleSplits = 128; // most splits of the sampled keys: 4096 groups, what the threshold kernel holds
 
 // Merging attention states of key-range partials (dg_attn_merge).  A state holds, per row
 // (row = canvas row * n_q_heads + query head), m and l in two planes of `rows` floats and then, from
@@ -343,9 +346,8 @@ hipError_t launch_kv_gather(const void* src, uint32_t src_dtype, void* dst, uint
                             uint32_t t_all, uint32_t head_dim, int64_t tok_stride, int64_t head_stride,
                             uint32_t ring_mask, hipStream_t s);
 
-// The filtered path over rows [tok0, tok0 + ntok): thresholds and lists (`sample`: the same rows over the sampled keys),
-// then selection out of the lists.
-hipError_t launch_topk_filter(const TopkParams& tp, const TopkParams& sample, uint32_t kv_dtype, hipStream_t s);
+// The filtered path over rows [tok0, tok0 + ntok): thresholds and lists, then selection out of the lists.
+hipError_t launch_topk_filter(const TopkParams& tp, uint32_t kv_dtype, hipStream_t s);
 hipError_t launch_topk_list_select(const TopkParams& tp, uint32_t k_most, uint32_t kv_dtype, hipStream_t s);
 hipError_t launch_topk_scores(const TopkParams& tp, uint32_t head_dim, uint32_t kv_dtype, hipStream_t s);
 hipError_t launch_topk_select(const TopkParams& tp, uint32_t head_dim, uint32_t kv_dtype, hipStream_t s);

@@ -741,8 +741,8 @@ __global__ void __launch_bounds__(256) topk_select_kernel(const TopkParams tp) {
 // two to four times k entries that one wave holds in registers.  Whatever tau is, the result is exact: a row whose
 // list holds fewer than k entries, or more than fit, is marked, and the general path redoes the marked rows (its
 // launches end at once where no row of the block is marked, 1.5 us each).
-// 256 rows x 16 heads over 33024 keys, layer step: 646 -> 266 us.  Launches: sampled scores 19 us (was: scores and plane, 4 x 55),
-// thresholds 15, filter 124 (1.1 PFLOP/s; the products alone, with their LDS reads and nothing else, 101), selection 31
+// 256 rows x 16 heads over 33024 keys, layer step: 646 -> 252 us.  Launches: sampled scores 14 us (was: scores and plane, 4 x 55),
+// thresholds 5, filter 124 (1.1 PFLOP/s; the products alone, with their LDS reads and nothing else, 101), selection 31
 // and gathered P.V 52 (both: was 4 x 94).
 
 // scores through an ordinary-register accumulator, query fragment in accumulation registers (256 of them hold the 64
@@ -766,6 +766,11 @@ __device__ __forceinline__ void mfma_filter_last(f32x16& s0, f32x16& s1, const u
   else
     asm volatile("v_mfma_f32_32x32x16_bf16 %0, %2, %3, %0\n\tv_mfma_f32_32x32x16_bf16 %1, %2, %4, %1\n\ts_nop 11"
                  : "+v"(s0), "+v"(s1) : "v"(k), "a"(q0), "a"(q1));
+}
+template <bool F16>
+__device__ __forceinline__ void mfma_filter_last(f32x16& s0, const u32x4& k, const u32x4& q0) {
+  if constexpr (F16) asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %0\n\ts_nop 11" : "+v"(s0) : "v"(k), "a"(q0));
+  else asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0\n\ts_nop 11" : "+v"(s0) : "v"(k), "a"(q0));
 }
 // Four stores of the filter kernel, each by the lanes in its mask and by lane 0.
 __device__ __forceinline__ void store4_masked(const uint64_t (&m)[4], const uint32_t (&at)[4], u32x2 e0, u32x2 e1, u32x2 e2,
@@ -800,8 +805,10 @@ __device__ __forceinline__ void wave_lds_fence() {
 }
 
 // Threshold of a row, one wave each: with `mean` = the number of sampled keys expected among the k largest, tau is about the
-// (mean + 5 sqrt(mean) + 3)-th largest sampled score, so that the k largest lie above it but for a five-sigma accident.
-// Any value near will do, so the bisection stops at the first key that leaves a count in a small range.
+// w-th largest sampled score, w = mean + 5 sqrt(mean) + 3, so that the k largest lie above it but for a five-sigma accident.
+// What there is to choose from are the largest scores of n groups of sampled keys; w keys fall into n (1 - exp(-w / n)) of them
+// (38 of 1942 keys into 37 of 512 groups).  Any value near will do, so the bisection stops at the first key that leaves a count
+// in a small range.
 template <int NV>
 __global__ void __launch_bounds__(256) topk_tau_kernel(const TopkParams tp) {
   const AttnParams& p = tp.a;
@@ -815,20 +822,18 @@ __global__ void __launch_bounds__(256) topk_tau_kernel(const TopkParams tp) {
   if (qh == 0u && tok_l % tp.fail_block_tok == 0u && lane == 0u) tp.fail_block[tok_l / tp.fail_block_tok] = 0u;
   const RowBounds rb = row_bounds(p, tok);
   const uint32_t k = row_k(tp, tok, visible_count(rb, p.t_all));
-  const float* srow = tp.sample_plane + ((size_t)qh * tp.ntok + tok_l) * tp.sample_pad;
+  const uint32_t n_groups = tp.sample_splits * kBlockN;
+  const float* srow = tp.sample_max + (size_t)rid * n_groups;
   uint32_t key[NV], top = 0u;
 #pragma unroll
-  for (int u = 0; u < NV; ++u) key[u] = __float_as_uint(srow[min(64u * u + lane, tp.sample_n - 1u)]);   // (all in flight)
+  for (int u = 0; u < NV; ++u) key[u] = __float_as_uint(srow[min(64u * u + lane, n_groups - 1u)]);   // (all in flight)
 #pragma unroll
-  for (int u = 0; u < NV; ++u) {
-    const uint32_t i = 64u * u + lane;
-    const bool in = i < tp.sample_n && key_visible(rb, i * tp.sample_stride, p.t_all);
-    key[u] = in ? score_key(__uint_as_float(key[u])) : 0u;
-  }
+  for (int u = 0; u < NV; ++u) key[u] = 64u * u + lane < n_groups ? score_key(__uint_as_float(key[u])) : 0u;
 #pragma unroll
   for (int u = 0; u < NV; ++u) top = max(top, key[u]);
   const float mean = (float)k / (float)tp.sample_stride;
-  const uint32_t want = (uint32_t)(mean + 5.f * __builtin_sqrtf(mean) + 3.f);
+  const float groups = (float)n_groups;
+  const uint32_t want = (uint32_t)(groups - groups * expf(-(mean + 5.f * __builtin_sqrtf(mean) + 3.f) / groups) + 0.5f);
   // a lower end first, from the lanes' largest keys alone: the want-th largest of those 64 has at least `want` above it
   // (one comparison a step instead of NV; `want` is below 64 at 512 keys kept)
   uint32_t lo = ~wave_max(~top), hi = wave_max(top) + 1u;      // count(>= lo) >= want, count(>= hi) < want
@@ -855,7 +860,15 @@ __global__ void __launch_bounds__(256) topk_tau_kernel(const TopkParams tp) {
 // Scores against thresholds.  256 stacked rows per workgroup, 64 per wave: with 32 (topk_scores_kernel) the four waves
 // together read the K tile from LDS as fast as the LDS can give it (128 bytes a cycle) and the matrix cores wait.
 // Splits take every n_splits-th key tile, so that keys that score high side by side spread over the segments.
-template <bool F16>
+//
+// SAMPLE: every sample_stride-th key, and instead of lists the largest score of each group of sampled keys: a register of the
+// score block is a group, of the keys it holds from one of the split's tiles to the next (n_splits tiles apart, so that a group's
+// keys are no neighbours).  The thresholds come from those (topk_tau_kernel).  256 groups a row at 256 rows over 33k keys, 4 MB
+// between the two launches; as 1942 sampled scores in a plane it was 32 MB: both launches 38 -> 21 us under the profiler (21.4 -> 15.3
+// and 16.5 -> 5.6), the layer step 257.3 -> 242.9 (replayed in a graph; 50k keys 428 -> 390, 64 rows over 50k 177 -> 165, 256 over 3k
+// 78.4 -> 76.2).  32 rows per wave: with the filter's 64 the query rows come in two trips, and the step took 241.5 - 242.1
+// where 252.4 - 252.9 was the old one, but 79.4 for 78.2 over 3k keys.
+template <bool F16, bool SAMPLE>
 __global__ void __launch_bounds__(256) topk_filter_kernel(const TopkParams tp) {
   constexpr int D = 512;
   const AttnParams& p = tp.a;
@@ -863,6 +876,7 @@ __global__ void __launch_bounds__(256) topk_filter_kernel(const TopkParams tp) {
   constexpr int NSTEP = D / 16;
   constexpr int NLD = L::NLD;
   constexpr int PF = 3, NB = PF + 1;   // K tiles in flight ahead of the one being multiplied
+  constexpr int RB = SAMPLE ? 1 : 2;   // blocks of 32 rows per wave
   __shared__ __attribute__((aligned(1024))) char smem[NB * L::K_BYTES];
 
   const uint32_t n_units = p.hkv * tp.n_splits * tp.n_mtiles;
@@ -876,26 +890,29 @@ __global__ void __launch_bounds__(256) topk_filter_kernel(const TopkParams tp) {
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t g2 = lane >> 5, l32 = lane & 31u;
   const uint32_t rows_total = tp.ntok * p.group;
-  const uint32_t row0 = mt * kTopkFilterRows + wave * 64u;
-  const uint32_t n_tiles_all = (p.t_all + kBlockN - 1u) / kBlockN;
+  const uint32_t row0 = (mt * 4u + wave) * (32u * RB);
+  const uint32_t t_end = SAMPLE ? tp.sample_n : p.t_all;
+  const uint32_t n_tiles_all = (t_end + kBlockN - 1u) / kBlockN;
   const uint32_t n_tiles = split < n_tiles_all ? fast_div(n_tiles_all - split + tp.n_splits - 1u, tp.div_splits) : 0u;
   const uint32_t seg = (((kvh * tp.n_mtiles + mt) * tp.n_splits + split) * 4u + wave) * kTopkSegs;   // this wave's first segment
-  if (n_tiles == 0u) {
-    tp.cand_n[seg + lane] = tp.cand_n[seg + 64u + lane] = 0u;
-    return;
+  if constexpr (!SAMPLE) {      // (sampled: no more splits than tiles)
+    if (n_tiles == 0u) {
+      tp.cand_n[seg + lane] = tp.cand_n[seg + 64u + lane] = 0u;
+      return;
+    }
   }
 
   const char* kbase = (const char*)p.k + (int64_t)kvh * p.k_head_stride * 2;
-  const int64_t kstride_b = p.k_tok_stride * 2;
+  const int64_t kstride_b = p.k_tok_stride * 2 * (SAMPLE ? tp.sample_stride : 1u);
   const uint32_t k_lane_off = l32 * L::K_STRIDE + g2 * 16u;
   auto tile_t0 = [&](uint32_t i) { return (split + min(i, n_tiles - 1u) * tp.n_splits) * (uint32_t)kBlockN; };
   // (past the last tile: the last one again into a buffer nobody reads, so that the wait counts stay fixed)
   auto k_desc = [&](uint32_t i) {
-    return make_tile_load<D, false, false>(kbase, kstride_b, tile_t0(i), 0u, p.t_all, 0u,
+    return make_tile_load<D, false, false>(kbase, kstride_b, tile_t0(i), 0u, t_end, 0u,
                                            (lds_char*)(smem + (i % NB) * L::K_BYTES), wave, lane);
   };
   // Query rows through the K buffers' LDS, a block of 32 at a time, into accumulation registers.
-  u32x4 qf[2][NSTEP];
+  u32x4 qf[RB][NSTEP];
   {
     static_assert(4 * 32 * kQRowLds <= NB * L::K_BYTES, "the tile buffers hold a block of every wave's query rows");
     lds_char* const qb = (lds_char*)smem + wave * (32u * kQRowLds);
@@ -923,23 +940,35 @@ __global__ void __launch_bounds__(256) topk_filter_kernel(const TopkParams tp) {
     };
     issue_q_rows(q_base, row0, rows_total, p.group, (uint32_t)(size_t)qb, lane, row_off);
     read_rows();
-    issue_q_rows(q_base, row0 + 32u, rows_total, p.group, (uint32_t)(size_t)qb, lane, row_off);
-    to_frags(std::integral_constant<int, 0>{});
-    read_rows();
+    if constexpr (RB == 2) {
+      issue_q_rows(q_base, row0 + 32u, rows_total, p.group, (uint32_t)(size_t)qb, lane, row_off);
+      to_frags(std::integral_constant<int, 0>{});
+      read_rows();
+    }
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < PF; ++i) issue_tile<D, false>(k_desc((uint32_t)i), wave, lane);
-    to_frags(std::integral_constant<int, 1>{});
+    to_frags(std::integral_constant<int, RB - 1>{});
   }
   // S = K.Q^T: the lane is a query row of the block, register e is key 8 (e >> 2) + 4 g2 + (e & 3) of the tile.  Each lane
   // keeps lists of its own, one per block, so an entry's place is the lane's count and nothing is exchanged.
-  float tau[2];
-  uint32_t lane_base[2], count[2] = {0u, 0u};
+  float tau[RB];
+  uint32_t lane_base[RB], count[RB] = {};
+  float largest[16];          // SAMPLE: of the keys a register has held
+  RowBounds rb;
+  uint32_t hi_least = 0u;
+  if constexpr (SAMPLE) {
+    rb = row_bounds(p, tp.tok0 + fast_div(min(row0 + l32, rows_total - 1u), tp.div_group));
+    hi_least = ~wave_max(~rb.hi);
 #pragma unroll
-  for (int b = 0; b < 2; ++b) {
-    const uint32_t r = row0 + 32u * b + l32;
-    tau[b] = r < rows_total ? tp.tau[(size_t)kvh * tp.n_mtiles * kTopkFilterRows + r] : INFINITY;
-    lane_base[b] = (64u * b + lane) * (kTopkSegAlloc * 8u);
+    for (int e = 0; e < 16; ++e) largest[e] = -INFINITY;
+  } else {
+#pragma unroll
+    for (int b = 0; b < RB; ++b) {
+      const uint32_t r = row0 + 32u * b + l32;
+      tau[b] = r < rows_total ? tp.tau[(size_t)kvh * tp.n_mtiles * kTopkFilterRows + r] : INFINITY;
+      lane_base[b] = (64u * b + lane) * (kTopkSegAlloc * 8u);
+    }
   }
   char* const cbase = (char*)tp.cand + (size_t)seg * (kTopkSegAlloc * 8u);
   const float scale = tp.scale;
@@ -953,9 +982,11 @@ __global__ void __launch_bounds__(256) topk_filter_kernel(const TopkParams tp) {
   uint64_t mask[4];
   uint32_t at[4];
   u32x2 entry[16];          // (score, position) of register e: positions move on by a tile step, shared by the blocks
-  auto keep = [&](auto n_c, const f32x16 (&sc)[2]) {
+  auto keep = [&](auto n_c, const f32x16 (&sc)[RB]) {
     constexpr int n0 = decltype(n_c)::value & ~3, part = decltype(n_c)::value & 3, b = n0 >> 4, e0 = n0 & 15;
-    if constexpr (part == 0) {
+    if constexpr (SAMPLE) {
+      if constexpr (b == 0) largest[e0 + part] = __builtin_fmaxf(largest[e0 + part], sc[0][e0 + part] * scale);    // (NaN: passed over)
+    } else if constexpr (part == 0) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const float v = sc[b][e0 + i] * scale;
@@ -982,12 +1013,13 @@ __global__ void __launch_bounds__(256) topk_filter_kernel(const TopkParams tp) {
 
   constexpr int CH = 8, NCHUNK = NSTEP / CH, LPC = NLD / NCHUNK;
   // tile i: its products into s, the comparison of the tile before (sp) between them
-  auto tile_step = [&](uint32_t i, f32x16 (&s)[2], const f32x16 (&sp)[2]) {
-    positions(tile_t0(i - 1u));
+  auto tile_step = [&](uint32_t i, f32x16 (&s)[RB], const f32x16 (&sp)[RB]) {
+    if constexpr (!SAMPLE) positions(tile_t0(i - 1u));
     // this wave's loads of K(i) have landed: they were issued PF tiles ago (or waited for before the loop), in front of at
     // least two tiles' worth of loads and stores, which is more than the counter can hold back
     static_assert((PF - 1) * (NLD + 32) >= 63, "operations issued behind a tile's loads");
-    wait_loads_then_barrier<63>();
+    // (SAMPLE stores nothing: exactly those loads may be outstanding)
+    wait_loads_then_barrier<SAMPLE ? (PF - 1) * NLD : 63>();
     const TileLoad tl_next = k_desc(i + PF);
     lds_char* const kb = (lds_char*)(smem + (i % NB) * L::K_BYTES);
     u32x4 fr[2][CH];
@@ -1003,8 +1035,9 @@ __global__ void __launch_bounds__(256) topk_filter_kernel(const TopkParams tp) {
       static_for<0, CH>([&](auto i_c) {
         constexpr int x = decltype(i_c)::value, st = c * CH + x;
         if constexpr (st + 1 < NSTEP) {
-          mfma_filter<F16, st == 0>(s[0], fr[c & 1][x], qf[0][st]);
-          mfma_filter<F16, st == 0>(s[1], fr[c & 1][x], qf[1][st]);
+          static_for<0, RB>([&](auto b_c) { mfma_filter<F16, st == 0>(s[decltype(b_c)::value], fr[c & 1][x], qf[decltype(b_c)::value][st]); });
+        } else if constexpr (RB == 1) {
+          mfma_filter_last<F16>(s[0], fr[c & 1][x], qf[0][st]);
         } else {
           mfma_filter_last<F16>(s[0], s[1], fr[c & 1][x], qf[0][st], qf[1][st]);
         }
@@ -1014,27 +1047,47 @@ __global__ void __launch_bounds__(256) topk_filter_kernel(const TopkParams tp) {
         __builtin_amdgcn_sched_barrier(0);
       });
     });
+    if constexpr (SAMPLE) {
+      // keys that a row does not see (behind the prefix: a few of the last tiles) and repeats of the last key do not count
+      const uint32_t t0 = tile_t0(i);
+      if ((t0 + (kBlockN - 1u)) * tp.sample_stride >= hi_least) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const uint32_t t = t0 + 8u * (e >> 2) + (e & 3) + 4u * g2;
+          if (!key_visible(rb, t * tp.sample_stride, p.t_all)) s[0][e] = __uint_as_float(0x7fc00000u);
+        }
+      }
+    }
   };
   wait_vmem_all();      // the first PF tiles
   __builtin_amdgcn_s_waitcnt(0xC07F);     // (lgkmcnt(0): or scalar loads in flight here make the compiler wait for whole chunks below)
-  f32x16 sa[2], sb[2];
+  f32x16 sa[RB], sb[RB];
 #pragma unroll
-  for (int e = 0; e < 16; ++e) sb[0][e] = sb[1][e] = __uint_as_float(0x7fc00000u);   // (in front of the first tile: NaN passes nowhere)
+  for (int e = 0; e < 16; ++e) sb[0][e] = sb[RB - 1][e] = __uint_as_float(0x7fc00000u);   // (in front of the first tile: NaN passes nowhere)
   for (uint32_t i = 0; i < n_tiles; i += 2) {
     tile_step(i, sa, sb);
     if (i + 1u < n_tiles) {
       tile_step(i + 1u, sb, sa);
     } else {
-      positions(tile_t0(i));
+      if constexpr (!SAMPLE) positions(tile_t0(i));
       static_for<0, 32>([&](auto n_c) { keep(n_c, sa); });
     }
   }
   if ((n_tiles & 1u) == 0u) {
-    positions(tile_t0(n_tiles - 1u));
+    if constexpr (!SAMPLE) positions(tile_t0(n_tiles - 1u));
     static_for<0, 32>([&](auto n_c) { keep(n_c, sb); });
   }
-  tp.cand_n[seg + lane] = count[0];
-  tp.cand_n[seg + 64u + lane] = count[1];
+  if constexpr (SAMPLE) {
+    const uint32_t r = row0 + l32;
+    float* const to = tp.sample_max + ((size_t)kvh * rows_total + r) * (tp.n_splits * kBlockN) + split * kBlockN + 16u * g2;
+    if (r < rows_total) {
+#pragma unroll
+      for (int e = 0; e < 16; e += 4) *(f32x4*)(to + e) = f32x4{largest[e], largest[e + 1], largest[e + 2], largest[e + 3]};
+    }
+  } else {
+    tp.cand_n[seg + lane] = count[0];
+    tp.cand_n[seg + 64u + lane] = count[RB - 1];
+  }
   wait_vmem_all();   // no direct-to-LDS load may outlive the workgroup's LDS
 }
 
@@ -1331,21 +1384,26 @@ hipError_t launch_by_dim(const TopkParams& tp, int stage, uint32_t head_dim, hip
 }
 
 template <bool F16>
-hipError_t launch_filter(TopkParams tp, const TopkParams& sample, hipStream_t s) {
+hipError_t launch_filter(TopkParams tp, hipStream_t s) {
   set_dividers(&tp);
-  hipError_t rc = launch_stage<512, F16>(sample, 0, s);
+  TopkParams sample = tp;
+  sample.n_splits = tp.sample_splits;
+  sample.n_mtiles = (tp.ntok * tp.a.group + kTopkSampleRows - 1u) / kTopkSampleRows;
+  set_dividers(&sample);
+  const uint32_t sample_units = tp.a.hkv * sample.n_mtiles * sample.n_splits;
+  hipLaunchKernelGGL((topk_filter_kernel<F16, true>), dim3((sample_units + 7u) / 8u * 8u), dim3(256), 0, s, sample);
+  hipError_t rc = hipGetLastError();
   if (rc != hipSuccess) return rc;
   const uint32_t rows = tp.ntok * tp.a.hq;
   const dim3 by_wave((rows + 3u) / 4u);
-  const uint32_t m = sample.a.t_all;
-  if (m <= 64u * 8u) hipLaunchKernelGGL((topk_tau_kernel<8>), by_wave, dim3(256), 0, s, tp);
-  else if (m <= 64u * 16u) hipLaunchKernelGGL((topk_tau_kernel<16>), by_wave, dim3(256), 0, s, tp);
-  else if (m <= 64u * 32u) hipLaunchKernelGGL((topk_tau_kernel<32>), by_wave, dim3(256), 0, s, tp);
-  else if (m <= 64u * 64u) hipLaunchKernelGGL((topk_tau_kernel<64>), by_wave, dim3(256), 0, s, tp);
-  else hipLaunchKernelGGL((topk_tau_kernel<128>), by_wave, dim3(256), 0, s, tp);
+  const uint32_t n_groups = tp.sample_splits * kBlockN;
+  if (n_groups <= 64u * 4u) hipLaunchKernelGGL((topk_tau_kernel<4>), by_wave, dim3(256), 0, s, tp);
+  else if (n_groups <= 64u * 8u) hipLaunchKernelGGL((topk_tau_kernel<8>), by_wave, dim3(256), 0, s, tp);
+  else if (n_groups <= 64u * 16u) hipLaunchKernelGGL((topk_tau_kernel<16>), by_wave, dim3(256), 0, s, tp);
+  else if (n_groups <= 64u * 32u) hipLaunchKernelGGL((topk_tau_kernel<32>), by_wave, dim3(256), 0, s, tp);
+  else hipLaunchKernelGGL((topk_tau_kernel<64>), by_wave, dim3(256), 0, s, tp);
   if ((rc = hipGetLastError()) != hipSuccess) return rc;
-  const uint32_t n_units = tp.a.hkv * tp.n_splits * tp.n_mtiles;
-  hipLaunchKernelGGL((topk_filter_kernel<F16>), dim3((n_units + 7u) / 8u * 8u), dim3(256), 0, s, tp);
+  hipLaunchKernelGGL((topk_filter_kernel<F16, false>), dim3((tp.a.hkv * tp.n_mtiles * tp.n_splits + 7u) / 8u * 8u), dim3(256), 0, s, tp);
   return hipGetLastError();
 }
 template <bool F16>
@@ -1364,8 +1422,8 @@ hipError_t launch_list_select(TopkParams tp, uint32_t k_most, hipStream_t s) {
 
 }  // namespace
 
-hipError_t launch_topk_filter(const TopkParams& tp, const TopkParams& sample, uint32_t kv_dtype, hipStream_t s) {
-  return kv_dtype == 1u ? launch_filter<true>(tp, sample, s) : launch_filter<false>(tp, sample, s);
+hipError_t launch_topk_filter(const TopkParams& tp, uint32_t kv_dtype, hipStream_t s) {
+  return kv_dtype == 1u ? launch_filter<true>(tp, s) : launch_filter<false>(tp, s);
 }
 hipError_t launch_topk_list_select(const TopkParams& tp, uint32_t k_most, uint32_t kv_dtype, hipStream_t s) {
   return kv_dtype == 1u ? launch_list_select<true>(tp, k_most, s) : launch_list_select<false>(tp, k_most, s);

@@ -770,7 +770,7 @@ struct TopkPlan {
   size_t general = 0;      // what the general path alone needs: with less than `total` it is taken
   // filtered path (pass_tok = 0: not taken): canvas rows per pass and, within a pass, per block of the general path
   // behind it; sampled keys; key-range splits; byte offsets in the workspace
-  uint32_t pass_tok = 0, redo_tok = 0, stride = 0, sample_n = 0, sample_pad = 0, splits = 0, k_most = 0;
+  uint32_t pass_tok = 0, redo_tok = 0, stride = 0, sample_n = 0, sample_splits = 0, splits = 0, k_most = 0;
   size_t off_block = 0, off_plane = 0, off_tau = 0, off_cand_n = 0, off_kept = 0, off_lists = 0;
   uint32_t kept_pad = 0;
 };
@@ -781,7 +781,8 @@ struct TopkPlan {
 // launches take about 75 us however small they are; the general path, a workgroup per (row, head) in the end, takes 50 and its
 // time grows with the rounds of the chip those workgroups need.  Measured, the layer step with 16 heads, general -> filtered
 // path: 64 rows (one round) over 20k keys 99 -> 108 us, 33k 152 -> 141, 50k 297 -> 190; 128 rows (two) over 5k keys
-// 87 -> 89 us, 8k 99.5 -> 98, 12k 123 -> 107, 33k 294 -> 175; 256 rows over 3k keys 136 -> 100 us, 33k 592 -> 269.
+// 87 -> 89 us, 8k 99.5 -> 98, 12k 123 -> 107, 33k 294 -> 175; 256 rows over 3k keys 136 -> 100 us, 33k 592 -> 269 (the filtered
+// path has become 4 to 12 us shorter since).
 // That is for rows the lists hold.  A row they do not (thousands of equal scores) has its block of canvas rows scored again:
 // the attention call alone, 256 rows over 33k keys, general | filtered: one such row 706 | 462 us, one in every canvas row
 // 975 | 1300, all of them 1947 | 3120; 64 rows over 33k: 233 | 380, 235 | 384, 489 | 766.  The host cannot tell.
@@ -807,8 +808,12 @@ size_t filter_bytes(const dg_attn_desc* d, const Plan& pl, uint32_t cus, uint32_
   tk->off_kept = tk->off_cand_n + align_up(segs * sizeof(uint32_t));
   tk->kept_pad = (tk->k_most + dg::kTopkGather - 1) / dg::kTopkGather * dg::kTopkGather;
   tk->off_lists = tk->off_kept + align_up((size_t)ntok * d->n_q_heads * tk->kept_pad * 8);
-  // (the lists lie where the sampled scores were)
-  const size_t sample = (size_t)d->n_q_heads * ntok * tk->sample_pad * sizeof(float);
+  // Sampled keys: a workgroup for every CU, but two key tiles each (its query rows cost as much).
+  const uint32_t sample_tiles = (tk->sample_n + dg::kBlockN - 1) / dg::kBlockN;
+  const uint32_t sample_base = d->n_kv_heads * ((ntok * pl.group + dg::kTopkSampleRows - 1) / dg::kTopkSampleRows);
+  tk->sample_splits = std::max(1u, std::min({(cus + sample_base - 1) / sample_base, sample_tiles / 2, dg::kTopkSampleSplits}));
+  // (the lists lie where the sampled keys' largest scores were)
+  const size_t sample = (size_t)ntok * d->n_q_heads * tk->sample_splits * dg::kBlockN * sizeof(float);
   return tk->off_lists + align_up(std::max(segs * dg::kTopkSegAlloc * 8, sample));
 }
 
@@ -833,7 +838,6 @@ void plan_filtered(const dg_attn_desc* d, const uint32_t* k_cfg, const Plan& pl,
   if ((uint64_t)d->k_tok_stride * 2 * tk->stride * dg::kBlockN >= (1ull << 31)) return;
   if ((uint64_t)d->v_tok_stride * 2 * pl.t_all + 1024 >= (1ull << 32)) return;      // V rows are gathered by 32-bit offsets
   tk->sample_n = (pl.t_all + tk->stride - 1) / tk->stride;
-  tk->sample_pad = (tk->sample_n + dg::kBlockN - 1) / dg::kBlockN * dg::kBlockN;
   uint32_t ntok = d->canvas;
   size_t need = filter_bytes(d, pl, cus, ntok, tk);
   while (need > kTopkPlaneBudget && ntok > 32) {
@@ -953,8 +957,8 @@ int dg_attn_topk_forward(const dg_attn_desc* d, const uint32_t* k_cfg, const voi
       fp.n_splits = tk.splits;
       fp.sample_stride = tk.stride;
       fp.sample_n = tk.sample_n;
-      fp.sample_pad = tk.sample_pad;
-      fp.sample_plane = (float*)(ws + tk.off_lists);
+      fp.sample_splits = tk.sample_splits;
+      fp.sample_max = (float*)(ws + tk.off_lists);
       fp.tau = (float*)(ws + tk.off_tau);
       fp.cand_n = (uint32_t*)(ws + tk.off_cand_n);
       fp.cand = ws + tk.off_lists;
@@ -963,25 +967,8 @@ int dg_attn_topk_forward(const dg_attn_desc* d, const uint32_t* k_cfg, const voi
       fp.fail_rows = (uint32_t*)ws;
       fp.fail_block = (uint32_t*)(ws + tk.off_block);
       fp.fail_block_tok = tk.redo_tok;
-      // the sampled keys as a cache of their own: every stride-th row of K, all of them scored
-      dg::TopkParams sp = tp;
-      sp.fail_rows = sp.fail_block = nullptr;      // (the last pass's)
-      sp.a.k_tok_stride *= tk.stride;
-      sp.a.causal_rows = 0u;
-      sp.a.t_all = tk.sample_n;
-      sp.a.t_clip_lo = 0u;
-      sp.a.t_clip_hi = sp.a.extra_lo = tk.sample_n;
-      sp.s_plane = fp.sample_plane;
-      sp.tok0 = tok0;
-      sp.ntok = ntok;
-      sp.t_pad = tk.sample_pad;
-      sp.n_mtiles = (ntok * pl.group + dg::kBlockM - 1) / dg::kBlockM;
-      sp.tile_first = 0u;
-      sp.tile_end = tk.sample_pad / dg::kBlockN;
-      const uint32_t base = d->n_kv_heads * sp.n_mtiles;
-      sp.n_splits = std::max(1u, std::min(((uint32_t)di.cus + base - 1u) / base, sp.tile_end / 2u));
       mark(0);
-      if (dg::launch_topk_filter(fp, sp, pl.e_dtype, s) != hipSuccess) return DG_ERR_LAUNCH;
+      if (dg::launch_topk_filter(fp, pl.e_dtype, s) != hipSuccess) return DG_ERR_LAUNCH;
       mark(1);
       mark(2);
       if (dg::launch_topk_list_select(fp, tk.k_most, pl.e_dtype, s) != hipSuccess) return DG_ERR_LAUNCH;

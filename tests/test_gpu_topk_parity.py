@@ -314,6 +314,28 @@ def test_sample_strides_of_very_long_rows(gpu_ready, po, t_all, stride):
         assert max_abs_diff(got, ref) <= 2e-2 and mean_abs_diff(got, ref) <= 2e-3
 
 
+@pytest.mark.parametrize("canvas,kvl,causal", [
+    (16, 2048, 0),         # one 128-row tile of stacked rows, full; 122 sampled keys in two splits, the last tile ragged
+    (17, 2159, 17),        # a second one of 8 rows; the last sampled keys behind some rows' own
+    (15, 2174, 15),        # ... and an odd number of tiles, so that one split has three
+    (48, 17 * 544, 20),    # 17 full sampled tiles before the canvas, eight splits
+    (130, 9001, 130),      # 1040 stacked rows: the last 128-row tile has 16
+])
+@pytest.mark.parametrize("kv_dtype", [capi.DG_BF16, capi.DG_F16])
+def test_thresholds_from_groups_of_sampled_keys(gpu_ready, canvas, kvl, causal, kv_dtype):
+    """Random rows are never left over (thresholds neither too high nor so low that lists overflow), whatever number of sampled
+    keys a group has; the same kept keys as through the score plane, fp32 summation error apart."""
+    hq, hkv, hd, k_cfg = 16, 2, 512, T.adaptive_k()
+    rng = np.random.default_rng(canvas + kvl)
+    rms = lambda x: x / np.sqrt(np.mean(x * x, axis=-1, keepdims=True))
+    q = rms(rng.standard_normal((canvas, hq, hd), dtype=np.float32))
+    kv = rms(rng.standard_normal((kvl + canvas, 2, hkv, hd), dtype=np.float32))
+    run = lambda flag: device_topk(canvas, hq, hkv, hd, kvl, k_cfg, q, kv, causal_rows=causal, kv_dtype=kv_dtype, flags=flag)
+    got, _, _, ws = run(capi.DG_ATTN_F_TOPK_THRESHOLD)
+    assert rows_left_over(ws, canvas * hq) == 0
+    assert max_abs_diff(got, run(capi.DG_ATTN_F_TOPK_SCORE_PLANE)[0]) < 2e-5
+
+
 @pytest.mark.parametrize("kv_dtype", [capi.DG_BF16, capi.DG_F16])
 def test_nonfinite_scores_go_the_score_planes_way(gpu_ready, kv_dtype):
     """NaN scores sort below every other (never kept while enough others are visible), an infinite score is kept and
