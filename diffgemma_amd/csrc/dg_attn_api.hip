@@ -794,11 +794,15 @@ size_t filter_bytes(const dg_attn_desc* d, const Plan& pl, uint32_t cus, uint32_
   const uint32_t n_mtiles = (ntok * pl.group + dg::kTopkFilterRows - 1) / dg::kTopkFilterRows;
   const uint32_t base = d->n_kv_heads * n_mtiles;
   const uint32_t n_tiles = (pl.t_all + dg::kBlockN - 1) / dg::kBlockN;
-  // Enough workgroups for every CU, in whole rounds of the chip, but four key tiles each; and segments that expect half
-  // of what they hold.  A row's list is about k + 5 sqrt(stride k) + 3 stride long, in two segments per split.
-  const double list = tk->k_most + 5.0 * std::sqrt((double)tk->stride * tk->k_most) + 3.0 * tk->stride;
+  // Enough workgroups for every CU, in whole rounds of the chip, but four key tiles each; and segments that hold what comes.
+  // A row's list is about stride w long, w = k / stride + 5 sqrt(k / stride) + 3 the rank of the threshold among the sampled
+  // scores, in two segments per split.  The threshold is as uncertain as w sampled keys are, 1 / sqrt(w) of the list's length:
+  // a segment that expects m entries holds m' + 4 sqrt(m') with m' = (1 + 4 / sqrt(w)) m.  (Half of what it holds, whatever w:
+  // at 64 keys kept, w = 16, 35 expected in segments of 80 left one row in 130 over: 1024 rows behind 5k keys 546 us, now 298.)
+  const double mean = (double)tk->k_most / tk->stride, w = mean + 5.0 * std::sqrt(mean) + 3.0;
+  const double root = std::sqrt(dg::kTopkSegCap + 4.0) - 2.0, most = root * root / (1.0 + 4.0 / std::sqrt(w));
   const uint32_t round = (cus + base - 1) / base;
-  const uint32_t fit = (uint32_t)(list / 2.0 / (dg::kTopkSegCap / 2)) + 1;
+  const uint32_t fit = (uint32_t)(w * tk->stride / 2.0 / most) + 1;
   tk->splits = std::min({round * ((fit + round - 1) / round), std::max(fit, n_tiles / 4), dg::kMaxSplits});
   const size_t segs = (size_t)base * tk->splits * 4 * dg::kTopkSegs;
   tk->off_block = align_up((size_t)d->canvas * d->n_q_heads * sizeof(uint32_t));

@@ -320,6 +320,7 @@ def test_sample_strides_of_very_long_rows(gpu_ready, po, t_all, stride):
     (15, 2174, 15),        # ... and an odd number of tiles, so that one split has three
     (48, 17 * 544, 20),    # 17 full sampled tiles before the canvas, eight splits
     (130, 9001, 130),      # 1040 stacked rows: the last 128-row tile has 16
+    (1024, 3000, 1024),    # few splits and keys kept: thresholds are uncertain, and the lists have to hold what that brings
 ])
 @pytest.mark.parametrize("kv_dtype", [capi.DG_BF16, capi.DG_F16])
 def test_thresholds_from_groups_of_sampled_keys(gpu_ready, canvas, kvl, causal, kv_dtype):
