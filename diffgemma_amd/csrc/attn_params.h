@@ -166,7 +166,8 @@ constexpr uint32_t kTopkSegs = 128;         // per wave of the filter kernel and
 constexpr uint32_t kTopkSegCap = 80, kTopkSegAlloc = kTopkSegCap + 16;
 constexpr uint32_t kTopkFilterRows = 256;   // stacked rows per workgroup of the filter kernel
 constexpr uint32_t kTopkSampleRows = 128;   // and of its instance for sampled keys
-constexpr uint32_t kTopkGather = 8;         // a row's list of kept keys is padded to a multiple
+constexpr uint32_t kTopkListMax = 512;      // most keys kept on the filtered path
+constexpr uint32_t kTopkListAlign = 8;      // a row's list of kept keys takes a multiple of this
 constexpr uint32_t kTopkSampleMax = 8192;   // most sampled keys per row
 constexpr uint32_t kTopkSampleSplits = 128; // most splits of the sampled keys: 4096 groups, what the threshold kernel holds
 

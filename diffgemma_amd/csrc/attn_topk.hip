@@ -741,9 +741,9 @@ __global__ void __launch_bounds__(256) topk_select_kernel(const TopkParams tp) {
 // two to four times k entries that one wave holds in registers.  Whatever tau is, the result is exact: a row whose
 // list holds fewer than k entries, or more than fit, is marked, and the general path redoes the marked rows (its
 // launches end at once where no row of the block is marked, 1.5 us each).
-// 256 rows x 16 heads over 33024 keys, layer step: 646 -> 252 us.  Launches: sampled scores 14 us (was: scores and plane, 4 x 55),
+// 256 rows x 16 heads over 33024 keys, layer step: 646 -> 250 us.  Launches: sampled scores 14 us (was: scores and plane, 4 x 55),
 // thresholds 5, filter 124 (1.1 PFLOP/s; the products alone, with their LDS reads and nothing else, 101), selection 31
-// and gathered P.V 52 (both: was 4 x 94).
+// and gathered P.V 50 (both: was 4 x 94).
 
 // scores through an ordinary-register accumulator, query fragment in accumulation registers (256 of them hold the 64
 // query rows of a wave; a comparison cannot read that file)
@@ -1277,66 +1277,83 @@ __global__ void __launch_bounds__(256, NR <= 20 ? 4 : NR == 24 ? 3 : 2) topk_lis
   }
   l = wave_sum(l);
   const float inv = l > 0.f ? 1.f / l : 0.f;
-  // the kept keys, up to a whole number of the gather's groups: the last key again, weight 0
   u32x2* const out = (u32x2*)tp.kept + (size_t)rid * tp.kept_pad;
-  const uint32_t k_up = (k + kTopkGather - 1u) / kTopkGather * kTopkGather;
-  for (uint32_t j = lane; j < k_up; j += 64u) {
-    const u32x2 v = sel[min(j, k - 1u)];
-    out[j] = u32x2{j < k ? __float_as_uint(__uint_as_float(v[0]) * inv) : 0u, v[1]};
+  for (uint32_t j = lane; j < k; j += 64u) {
+    const u32x2 v = sel[j];
+    out[j] = u32x2{__float_as_uint(__uint_as_float(v[0]) * inv), v[1]};
   }
 }
 
-// Gathered P.V of the rows the selection has listed, one wave each: a lane owns 8 consecutive d, keys in order of position.
-// A launch of its own so that its waves begin together: all waves of an XCD sweep the keys in order, and a V row
-// that four of its 512 rows want should be fetched into its L2 once.  For the same reason only four rows are loaded ahead where
-// there are waves enough.  256 rows over 33k keys: 1 row ahead 101 us, 2 rows 68, 4 rows 55 (20 TB/s out of the L2s), 8 rows 88;
-// as the tail of the selection, its waves apart by what came before, 2 rows 70 and 16 rows 110 us, half of the
-// requests missing the L2.  64 rows, a wave per SIMD: 8 rows ahead.
-template <bool F16>
-__global__ void __launch_bounds__(256) topk_gather_kernel(const TopkParams tp) {
-  constexpr int D = 512, PER = 8;
+// Gathered P.V of the rows the selection has listed.  A launch of its own so that its waves begin together: all waves of an XCD
+// sweep the keys in order, and a V row that several of its rows want should be fetched into its L2 once.
+// One wave per (row, slice of head_dim), SL slices: a slice's lanes of SL keys stand side by side and their sums meet at the end.
+// With more than 2048 rows whole rows (SL = 1), 512 rows of 256 x 16 to an XCD: bound by what the eight L2s fetch, 288 MB
+// at 33k keys where 270 are the least (each V row once into each L2 whose rows want it), and 30 us of unpacking and
+// multiplying.  Fewer loads ahead than four hide too little, more pull the sweeps apart: 1 row ahead 101 us, 2 rows 68, 4 rows 52,
+// 8 rows 88.  Up to 2048 rows there are too few waves for that, and XCDs take one slice of more rows each: 128 rows over 30k keys, layer
+// step, whole rows | halves | quarters 148.0 | 140.6 | 145.0 us, 64 rows 115.0 | 103.6 | 101.2, 64 over 50k 168.3 | 148.4 | 147.4, 16 over
+// 100k 245.0 | 207.5 | 188.8.  With 256 rows over 33k slices lose, 239.6 | 249.0 | 260.5: a slice of every row
+// lies on a part of an L2's channels, and although less is fetched (199 MB in halves), it comes slower.
+template <bool F16, uint32_t SL>
+__global__ void __launch_bounds__(256, 8) topk_gather_kernel(const TopkParams tp) {
+  constexpr uint32_t D = 512, PER = 8, LPK = 64u / SL, GU = 4;     // LPK lanes per key, GU loads in flight
+  static_assert(LPK * PER * SL == D, "a lane owns 8 consecutive d");
   const AttnParams& p = tp.a;
+  __shared__ u32x2 lists[4][kTopkListMax];
   const uint32_t lane = threadIdx.x & 63u;
-  const uint32_t n_rows = tp.ntok * p.hq;
-  const uint32_t wg = (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);   // runs of rows, one per XCD
-  const uint32_t rid = __builtin_amdgcn_readfirstlane(wg * 4u + (threadIdx.x >> 6));
-  if (rid >= n_rows) return;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t rows = tp.ntok * p.group;
-  const uint32_t kvh = fast_div(rid, tp.div_rows), rr = rid - kvh * rows;
+  const uint32_t wg = (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);   // runs of units, one per XCD
+  const uint32_t unit = wg * 4u + wave;                                           // (KV head, row, slice)
+  if (unit >= tp.ntok * p.hq * SL) return;
+  const uint32_t stream = fast_div(unit, tp.div_rows), rr = unit - stream * rows;
+  const uint32_t kvh = stream / SL, slice = stream % SL, rid = kvh * rows + rr;
   const uint32_t tok_l = fast_div(rr, tp.div_group), tok = tp.tok0 + tok_l, qh = kvh * p.group + rr - tok_l * p.group;
   if (tp.fail_rows[(size_t)tok * p.hq + qh] != 0u) return;       // (the general path's)
   const uint32_t k = row_k(tp, tok, visible_count(row_bounds(p, tok), p.t_all));
-  const u32x2* const kept = (const u32x2*)tp.kept + (size_t)rid * tp.kept_pad;
+  u32x2* const list = lists[wave];
+  {
+    const u32x2* const kept = (const u32x2*)tp.kept + (size_t)rid * tp.kept_pad;
+    for (uint32_t j = lane; j < k; j += 64u) list[j] = kept[j];
+  }
+  wave_lds_fence();
   float acc[PER];
 #pragma unroll
-  for (int i = 0; i < PER; ++i) acc[i] = 0.f;
-  const char* const vbase = (const char*)p.v + (int64_t)kvh * p.v_head_stride * 2;
-  const uint32_t lane_b = lane * 16u;
-  auto gather = [&](auto gu_c) {
-    constexpr uint32_t GU = decltype(gu_c)::value;
-    for (uint32_t j0 = 0; j0 < k; j0 += GU) {
-      float w[GU];
-      u32x4 raw[GU];
+  for (uint32_t i = 0; i < PER; ++i) acc[i] = 0.f;
+  const char* const vbase = (const char*)p.v + (int64_t)kvh * p.v_head_stride * 2 + slice * (LPK * PER * 2u);
+  const uint32_t lane_b = lane % LPK * (PER * 2u);
+  const uint32_t own = lane / LPK;
+  auto group = [&](uint32_t j0, auto tail_c) {      // keys j0 + own + SL u
+    constexpr bool TAIL = decltype(tail_c)::value;
+    float w[GU];
+    u32x4 raw[GU];
 #pragma unroll
-      for (uint32_t u = 0; u < GU; ++u) {
-        const u32x2 v = kept[j0 + u];
-        w[u] = __uint_as_float(v[0]);
-        raw[u] = *(const u32x4*)(vbase + (v[1] + lane_b));
-      }
+    for (uint32_t u = 0; u < GU; ++u) {
+      const uint32_t j = j0 + own + SL * u;
+      const u32x2 v = list[TAIL ? min(j, k - 1u) : j];
+      w[u] = __uint_as_float(v[0]);
+      raw[u] = *(const u32x4*)(vbase + (v[1] + lane_b));
+      if (TAIL && j >= k) raw[u] = u32x4{0, 0, 0, 0};
+    }
 #pragma unroll
-      for (uint32_t u = 0; u < GU; ++u) {
+    for (uint32_t u = 0; u < GU; ++u) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          acc[2 * i] = __builtin_fmaf(w[u], unpack_lo<F16>(raw[u][i]), acc[2 * i]);
-          acc[2 * i + 1] = __builtin_fmaf(w[u], unpack_hi<F16>(raw[u][i]), acc[2 * i + 1]);
-        }
+      for (int i = 0; i < 4; ++i) {
+        acc[2 * i] = __builtin_fmaf(w[u], unpack_lo<F16>(raw[u][i]), acc[2 * i]);
+        acc[2 * i + 1] = __builtin_fmaf(w[u], unpack_hi<F16>(raw[u][i]), acc[2 * i + 1]);
       }
     }
   };
-  static_assert(kTopkGather % 8 == 0, "lists are padded to whole groups");
-  if (n_rows > 2048u) gather(std::integral_constant<uint32_t, 4>{});
-  else gather(std::integral_constant<uint32_t, 8>{});
-  const size_t out_off = ((size_t)tok * p.hq + qh) * D + lane * PER;
+  uint32_t j0 = 0u;
+  for (; j0 + SL * GU <= k; j0 += SL * GU) group(j0, std::false_type{});
+  if (j0 < k) group(j0, std::true_type{});
+#pragma unroll
+  for (uint32_t i = 0; i < PER; ++i) {
+#pragma unroll
+    for (uint32_t off = LPK; off < 64u; off <<= 1) acc[i] += __shfl_xor(acc[i], (int)off, 64);
+  }
+  if (lane >= LPK) return;
+  const size_t out_off = ((size_t)tok * p.hq + qh) * D + (slice * LPK + lane) * PER;
   if (p.out_dtype == 2u) {
     float* const o = (float*)p.out + out_off;
     *(f32x4*)o = f32x4{acc[0], acc[1], acc[2], acc[3]};
@@ -1416,7 +1433,11 @@ hipError_t launch_list_select(TopkParams tp, uint32_t k_most, hipStream_t s) {
   else hipLaunchKernelGGL((topk_list_select_kernel<32>), sel, dim3(256), 0, s, tp);
   const hipError_t rc = hipGetLastError();
   if (rc != hipSuccess) return rc;
-  hipLaunchKernelGGL((topk_gather_kernel<F16>), sel, dim3(256), 0, s, tp);
+  const uint32_t n_rows = tp.ntok * tp.a.hq, slices = n_rows > 2048u ? 1u : n_rows > 1024u ? 2u : 4u;
+  const dim3 gather((n_rows * slices + 31u) / 32u * 8u);
+  if (slices == 1u) hipLaunchKernelGGL((topk_gather_kernel<F16, 1>), gather, dim3(256), 0, s, tp);
+  else if (slices == 2u) hipLaunchKernelGGL((topk_gather_kernel<F16, 2>), gather, dim3(256), 0, s, tp);
+  else hipLaunchKernelGGL((topk_gather_kernel<F16, 4>), gather, dim3(256), 0, s, tp);
   return hipGetLastError();
 }
 

@@ -787,7 +787,6 @@ struct TopkPlan {
 // the attention call alone, 256 rows over 33k keys, general | filtered: one such row 706 | 462 us, one in every canvas row
 // 975 | 1300, all of them 1947 | 3120; 64 rows over 33k: 233 | 380, 235 | 384, 489 | 766.  The host cannot tell.
 constexpr uint32_t kTopkFilterMinPrefix = 2048;
-constexpr uint32_t kTopkFilterMaxK = 512;
 constexpr uint32_t kTopkFilterMinKeys[3] = {24576, 8192, 0};   // one round, two rounds, more
 
 size_t filter_bytes(const dg_attn_desc* d, const Plan& pl, uint32_t cus, uint32_t ntok, TopkPlan* tk) {
@@ -810,7 +809,7 @@ size_t filter_bytes(const dg_attn_desc* d, const Plan& pl, uint32_t cus, uint32_
   tk->off_tau = tk->off_plane;
   tk->off_cand_n = tk->off_tau + align_up((size_t)base * dg::kTopkFilterRows * sizeof(float));
   tk->off_kept = tk->off_cand_n + align_up(segs * sizeof(uint32_t));
-  tk->kept_pad = (tk->k_most + dg::kTopkGather - 1) / dg::kTopkGather * dg::kTopkGather;
+  tk->kept_pad = (tk->k_most + dg::kTopkListAlign - 1) / dg::kTopkListAlign * dg::kTopkListAlign;
   tk->off_lists = tk->off_kept + align_up((size_t)ntok * d->n_q_heads * tk->kept_pad * 8);
   // Sampled keys: a workgroup for every CU, but two key tiles each (its query rows cost as much).
   const uint32_t sample_tiles = (tk->sample_n + dg::kBlockN - 1) / dg::kBlockN;
@@ -834,7 +833,7 @@ void plan_filtered(const dg_attn_desc* d, const uint32_t* k_cfg, const Plan& pl,
   } else {
     tk->k_most = std::max(k_cfg[0], 1u);
   }
-  if (tk->k_most == 0u || tk->k_most > kTopkFilterMaxK) return;
+  if (tk->k_most == 0u || tk->k_most > dg::kTopkListMax) return;
   // (odd: sampled rows of a head-major cache, 1 KiB each, then fall on all memory channels)
   tk->stride = std::max(17u, (pl.t_all + dg::kTopkSampleMax - 1) / dg::kTopkSampleMax | 1u);
   if (tk->stride > 21u) return;       // (17 to 21: the list of a row that keeps 512 keys still fits)

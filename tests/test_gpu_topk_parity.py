@@ -337,6 +337,27 @@ def test_thresholds_from_groups_of_sampled_keys(gpu_ready, canvas, kvl, causal, 
     assert max_abs_diff(got, run(capi.DG_ATTN_F_TOPK_SCORE_PLANE)[0]) < 2e-5
 
 
+@pytest.mark.parametrize("canvas,slices", [(64, 4), (65, 2), (128, 2), (129, 1)])
+@pytest.mark.parametrize("k", [1, 3, 4, 15, 16, 17, 33])
+def test_gather_slices(gpu_ready, canvas, slices, k):
+    """Every number of head_dim slices the gather deals out, at the edges of its groups of keys; a kept V row with an infinity
+    leaves it in its own element (nothing is multiplied by a weight of 0 to fill a group)."""
+    hq, hkv, hd, kvl = 16, 2, 512, 2100
+    rng = np.random.default_rng(canvas * 64 + k)
+    rms = lambda x: x / np.sqrt(np.mean(x * x, axis=-1, keepdims=True))
+    q = rms(rng.standard_normal((canvas, hq, hd), dtype=np.float32))
+    kv = rms(rng.standard_normal((kvl + canvas, 2, hkv, hd), dtype=np.float32))
+    kv[:, 1, :, 7 + 128 * (k % 4)] = np.inf
+    run = lambda flag: device_topk(canvas, hq, hkv, hd, kvl, (k, 0, 0, 0), q, kv, flags=flag)
+    got, _, _, ws = run(capi.DG_ATTN_F_TOPK_THRESHOLD)
+    assert rows_left_over(ws, canvas * hq) == 0
+    plane = run(capi.DG_ATTN_F_TOPK_SCORE_PLANE)[0]
+    finite = np.delete(np.arange(hd), 7 + 128 * (k % 4))
+    assert np.isfinite(got[..., finite]).all() and max_abs_diff(got[..., finite], plane[..., finite]) < 2e-5
+    # (a weight may underflow to 0: peaked rows)
+    assert (np.isposinf(got[..., 7 + 128 * (k % 4)]) | np.isnan(got[..., 7 + 128 * (k % 4)])).all()
+
+
 @pytest.mark.parametrize("kv_dtype", [capi.DG_BF16, capi.DG_F16])
 def test_nonfinite_scores_go_the_score_planes_way(gpu_ready, kv_dtype):
     """NaN scores sort below every other (never kept while enough others are visible), an infinite score is kept and
