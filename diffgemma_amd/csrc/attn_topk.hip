@@ -741,8 +741,8 @@ __global__ void __launch_bounds__(256) topk_select_kernel(const TopkParams tp) {
 // two to four times k entries that one wave holds in registers.  Whatever tau is, the result is exact: a row whose
 // list holds fewer than k entries, or more than fit, is marked, and the general path redoes the marked rows (its
 // launches end at once where no row of the block is marked, 1.5 us each).
-// 256 rows x 16 heads over 33024 keys, layer step: 646 -> 250 us.  Launches: sampled scores 14 us (was: scores and plane, 4 x 55),
-// thresholds 5, filter 124 (1.1 PFLOP/s; the products alone, with their LDS reads and nothing else, 101), selection 31
+// 256 rows x 16 heads over 33024 keys, layer step: 646 -> 230 us.  Launches: sampled scores 14 us (was: scores and plane, 4 x 55),
+// thresholds 5, filter 124 (1.1 PFLOP/s; the products alone, with their LDS reads and nothing else, 101), selection 24
 // and gathered P.V 50 (both: was 4 x 94).
 
 // scores through an ordinary-register accumulator, query fragment in accumulation registers (256 of them hold the 64
@@ -785,15 +785,28 @@ __device__ __forceinline__ void store4_masked(const uint64_t (&m)[4], const uint
       : "memory", "scc");
 }
 
+// Reductions and scans over the wave by DPP moves (through LDS, as a shuffle, each step is a round trip of its own).
+// step(x, v): x with v = the value of the lane 1, 2, 4, 8, then of the last lane of the row or half below; ends in lane 63
+template <typename T, typename F>
+__device__ __forceinline__ T wave_scan(T x, T none, F step) {
+  auto moved = [&](auto ctrl_c, auto rows_c) -> T {
+    return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, none), __builtin_bit_cast(int, x),
+                                                             decltype(ctrl_c)::value, decltype(rows_c)::value, 0xf, false));
+  };
+  x = step(x, moved(std::integral_constant<int, 0x111>{}, std::integral_constant<int, 0xf>{}));     // row_shr:1
+  x = step(x, moved(std::integral_constant<int, 0x112>{}, std::integral_constant<int, 0xf>{}));
+  x = step(x, moved(std::integral_constant<int, 0x114>{}, std::integral_constant<int, 0xf>{}));
+  x = step(x, moved(std::integral_constant<int, 0x118>{}, std::integral_constant<int, 0xf>{}));
+  x = step(x, moved(std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xa>{}));     // row_bcast:15, rows 1 and 3
+  x = step(x, moved(std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xc>{}));     // row_bcast:31, rows 2 and 3
+  return x;
+}
 __device__ __forceinline__ uint32_t wave_max(uint32_t x) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) x = max(x, (uint32_t)__shfl_xor((int)x, off, 64));
-  return (uint32_t)__builtin_amdgcn_readfirstlane((int)x);
+  return (uint32_t)__builtin_amdgcn_readlane((int)wave_scan(x, 0u, [](uint32_t a, uint32_t b) { return max(a, b); }), 63);
 }
 __device__ __forceinline__ float wave_sum(float x) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
-  return x;
+  x = wave_scan(x, 0.f, [](float a, float b) { return a + b; });
+  return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(x), 63));
 }
 __device__ __forceinline__ uint32_t rank_in(uint64_t mask) {   // set bits below this lane
   return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
@@ -1093,6 +1106,10 @@ __global__ void __launch_bounds__(256) topk_filter_kernel(const TopkParams tp) {
 
 // One wave per row: candidates from the row's segments, the k-th largest by bisection over registers (a ballot per 64
 // candidates and step; no histogram, no barrier), the kept keys in position order by ranking them in a bitmap, softmax.
+// As long as a wave's instructions, 1270 vector and 1160 scalar ones at 646 candidates for 258 kept (four waves a SIMD, in one round). The
+// last dozen steps of the bisection look at the candidates still between its ends alone, one register; only the kept ones are ranked,
+// packed once more (5 registers instead of 11); sums and scans by DPP, not through LDS: 1790 and 1260 before, without the spills,
+// 31.3 -> 26.3 us under the profiler, layer step with 256 rows over 33k keys 237.7 -> 229.8, over 3k 75.7 -> 71.1, 64 rows over 50k 147.4 -> 138.3.
 constexpr uint32_t kRankWords = 64 * 17;               // bitmap words, 17 per lane: an odd stride, no bank conflicts
 constexpr uint32_t kRankWindow = kRankWords * 32;      // positions per pass
 template <int NR>
@@ -1194,8 +1211,9 @@ __global__ void __launch_bounds__(256, NR <= 20 ? 4 : NR == 24 ? 3 : 2) topk_lis
     }
     return c;
   };
-  uint32_t lo = bot, hi = top + 1u, c_lo = n;      // count(>= lo) = c_lo >= k > count(>= hi)
-  while (hi - lo > 1u && c_lo != k) {
+  // bisection over all registers until no more than a lane's worth of candidates is between the ends, then over those alone
+  uint32_t lo = bot, hi = top + 1u, c_lo = n, c_hi = 0u;      // count(>= lo) = c_lo >= k > c_hi = count(>= hi)
+  while (hi - lo > 1u && c_lo != k && c_lo - c_hi > 64u) {
     const uint32_t mid = lo + ((hi - lo) >> 1);
     const uint32_t c = count_ge(mid);
     if (c >= k) {
@@ -1203,6 +1221,34 @@ __global__ void __launch_bounds__(256, NR <= 20 ? 4 : NR == 24 ? 3 : 2) topk_lis
       c_lo = c;
     } else {
       hi = mid;
+      c_hi = c;
+    }
+  }
+  if (hi - lo > 1u && c_lo != k) {
+    uint32_t* const few = (uint32_t*)list;
+    uint32_t at = 0u;
+#pragma unroll
+    for (int u = 0; u < NR; ++u) {
+      if ((uint32_t)u < nu) {
+        const bool own = key[u] >= lo && key[u] < hi;
+        const uint64_t m = __builtin_amdgcn_ballot_w64(own);
+        if (own) few[at + rank_in(m)] = key[u];
+        at += (uint32_t)__builtin_popcountll(m);
+      }
+    }
+    wave_lds_fence();
+    const uint32_t x = lane < at ? few[lane] : 0u;
+    wave_lds_fence();
+    while (hi - lo > 1u && c_lo != k) {
+      const uint32_t mid = lo + ((hi - lo) >> 1);
+      const uint32_t c = c_hi + (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(x >= mid && x < hi));
+      if (c >= k) {
+        lo = mid;
+        c_lo = c;
+      } else {
+        hi = mid;
+        c_hi = c;
+      }
     }
   }
   // equal scores at the threshold: the lower positions are kept, up to t_last
@@ -1222,15 +1268,35 @@ __global__ void __launch_bounds__(256, NR <= 20 ? 4 : NR == 24 ? 3 : 2) topk_lis
     }
     t_last = a - 1u;      // (position a is the last one dropped; a > 0 because at least one equal key stays)
   }
+  // ---- the kept ones, packed: fewer registers to rank ----
+  uint32_t* const bits = (uint32_t*)list;
+  uint16_t* const before = (uint16_t*)(bits + kRankWords);
+  u32x2* const sel = list + kRankWords * 6u / 8u;          // (key, position), then (weight, byte offset of the key's V row)
+  constexpr int NK = (int)(SEL + 63u) / 64;
+  uint32_t kkey[NK], kpos[NK];
+  {
+    uint32_t at = 0u;
 #pragma unroll
-  for (int u = 0; u < NR; ++u) {
-    if (key[u] < lo || (key[u] == lo && pos[u] > t_last)) pos[u] = 0xffffffffu;      // not kept: in no window below
+    for (int u = 0; u < NR; ++u) {
+      if ((uint32_t)u < nu) {
+        const bool own = key[u] > lo || (key[u] == lo && pos[u] <= t_last);
+        const uint64_t m = __builtin_amdgcn_ballot_w64(own);
+        const uint32_t to = at + rank_in(m);
+        if (own && to < SEL) sel[to] = u32x2{key[u], pos[u]};
+        at += (uint32_t)__builtin_popcountll(m);
+      }
+    }
+    wave_lds_fence();
+#pragma unroll
+    for (int u = 0; u < NK; ++u) {
+      const u32x2 v = sel[min(64u * u + lane, k - 1u)];
+      kkey[u] = v[0];
+      kpos[u] = 64u * u + lane < k ? v[1] : 0xffffffffu;      // (in no window below)
+    }
+    wave_lds_fence();
   }
 
   // ---- softmax over the kept scores (cpu.rs:95-104), and their order by position ----
-  uint32_t* const bits = (uint32_t*)list;
-  uint16_t* const before = (uint16_t*)(bits + kRankWords);
-  u32x2* const sel = list + kRankWords * 6u / 8u;          // (weight, byte offset of the key's V row)
   const uint32_t v_step = (uint32_t)p.v_tok_stride * 2u;   // (offsets stay below 2^32: the host's rule)
   const float mmax = key_score(top);
   float l = 0.f;
@@ -1240,8 +1306,8 @@ __global__ void __launch_bounds__(256, NR <= 20 ? 4 : NR == 24 ? 3 : 2) topk_lis
     for (uint32_t w = 0; w < 17u; ++w) bits[64u * w + lane] = 0u;
     wave_lds_fence();
 #pragma unroll
-    for (int u = 0; u < NR; ++u) {
-      if ((uint32_t)u < nu && pos[u] - t0 < kRankWindow) atomicOr(&bits[(pos[u] - t0) >> 5], 1u << ((pos[u] - t0) & 31u));
+    for (int u = 0; u < NK; ++u) {
+      if (kpos[u] - t0 < kRankWindow) atomicOr(&bits[(kpos[u] - t0) >> 5], 1u << ((kpos[u] - t0) & 31u));
     }
     wave_lds_fence();
     uint32_t run = 0u;
@@ -1250,26 +1316,19 @@ __global__ void __launch_bounds__(256, NR <= 20 ? 4 : NR == 24 ? 3 : 2) topk_lis
       before[17u * lane + w] = (uint16_t)run;
       run += (uint32_t)__builtin_popcount(bits[17u * lane + w]);
     }
-    uint32_t incl = run;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const uint32_t v = (uint32_t)__shfl_up((int)incl, off, 64);
-      if (lane >= (uint32_t)off) incl += v;
-    }
+    const uint32_t incl = wave_scan(run, 0u, [](uint32_t a, uint32_t b) { return a + b; });
     const uint32_t excl = incl - run;
     wave_lds_fence();
 #pragma unroll
-    for (int u = 0; u < NR; ++u) {
-      if ((uint32_t)u < nu) {
-        const bool in = pos[u] - t0 < kRankWindow;
-        const uint32_t w = in ? (pos[u] - t0) >> 5 : 0u;
-        const uint32_t base = (uint32_t)__shfl((int)excl, (int)(w / 17u), 64);
-        if (in) {
-          const uint32_t r = ranked + base + before[w] + (uint32_t)__builtin_popcount(bits[w] & ((1u << (pos[u] & 31u)) - 1u));
-          const float e = expf(key_score(key[u]) - mmax);
-          l += e;
-          if (r < SEL) sel[r] = u32x2{__float_as_uint(e), pos[u] * v_step};
-        }
+    for (int u = 0; u < NK; ++u) {
+      const bool in = kpos[u] - t0 < kRankWindow;
+      const uint32_t w = in ? (kpos[u] - t0) >> 5 : 0u;
+      const uint32_t base = (uint32_t)__shfl((int)excl, (int)(w / 17u), 64);
+      if (in) {
+        const uint32_t r = ranked + base + before[w] + (uint32_t)__builtin_popcount(bits[w] & ((1u << (kpos[u] & 31u)) - 1u));
+        const float e = expf(key_score(kkey[u]) - mmax);
+        l += e;
+        if (r < SEL) sel[r] = u32x2{__float_as_uint(e), kpos[u] * v_step};
       }
     }
     ranked += (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
