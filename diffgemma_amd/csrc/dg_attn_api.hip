@@ -778,16 +778,18 @@ struct TopkPlan {
 // Where the filtered path is taken: what its kernels are made for (head_dim 512, linear cache, every row sees all keys
 // up to its own or the last), at most 512 keys kept (what a wave holds of a row's list), prefixes long
 // enough that a pass over 1/17 of the keys tells where the k-th score lies, and calls large enough.  Its seven and more
-// launches take about 75 us however small they are; the general path, a workgroup per (row, head) in the end, takes 50 and its
-// time grows with the rounds of the chip those workgroups need.  Measured, the layer step with 16 heads, general -> filtered
-// path: 64 rows (one round) over 20k keys 99 -> 108 us, 33k 152 -> 141, 50k 297 -> 190; 128 rows (two) over 5k keys
-// 87 -> 89 us, 8k 99.5 -> 98, 12k 123 -> 107, 33k 294 -> 175; 256 rows over 3k keys 136 -> 100 us, 33k 592 -> 269 (the filtered
-// path has become 4 to 12 us shorter since).
+// launches take about 40 us however small they are; the general path, a workgroup per (row, head) in the end, takes 35 and its
+// time grows with the rounds of the chip those workgroups need (four of them at once on a compute unit).  Measured, the
+// attention call with 16 heads over a bf16 cache, general | filtered path: 16 rows (256 workgroups) over 24k keys 67.6 | 76.8 us;
+// 32 rows over 17k 66.6 | 70.7, 24k 81.7 | 77.5; 48 rows over 9k 55.0 | 62.9, 12k 75.5 | 68.0; 64 rows (a whole round) over 9k
+// 58.3 | 64.6, 12k 68.6 | 69.7, 17k 83.9 | 76.1; 96 rows over 2100 65.6 | 53.0, 6500 91.2 | 62.7; 128 rows over 2100
+// 69.7 | 55.8 (f16 71.2 | 59.7), 6500 85.6 | 64.7; 256 rows over 2100 120 | 66, 24k 450 | 172.  Over the reference's f16 cache, layer
+// step: 64 rows over 14k 77.1 | 85.6, 16k 85.7 | 88.7, 18.4k 101 | 95, 128 over 2100 73.3 | 61.8.
 // That is for rows the lists hold.  A row they do not (thousands of equal scores) has its block of canvas rows scored again:
 // the attention call alone, 256 rows over 33k keys, general | filtered: one such row 706 | 462 us, one in every canvas row
 // 975 | 1300, all of them 1947 | 3120; 64 rows over 33k: 233 | 380, 235 | 384, 489 | 766.  The host cannot tell.
 constexpr uint32_t kTopkFilterMinPrefix = 2048;
-constexpr uint32_t kTopkFilterMinKeys[3] = {24576, 8192, 0};   // one round, two rounds, more
+constexpr uint32_t kTopkFilterMinKeys[3] = {24576, 18432, 0};   // up to half a round, one round, more
 
 // Key-range splits of a launch of `base` row tiles whose workgroups take a compute unit each: between `least` and `most`, the count
 // whose rounds of the chip are shortest, in key tiles, where starting a workgroup costs `start` of them.  (One more workgroup than a
@@ -841,7 +843,7 @@ void plan_filtered(const dg_attn_desc* d, const uint32_t* k_cfg, const Plan& pl,
   if (d->head_dim != 512 || pl.lo_nc != 0 || pl.win_m1 != 0xffffffffu || d->kv_ring_mask != 0) return;
   if (d->kv_len < kTopkFilterMinPrefix || !std::isfinite(pl.scale) || (d->flags & DG_ATTN_F_TOPK_SCORE_PLANE)) return;
   const uint64_t rows = (uint64_t)d->canvas * d->n_q_heads;
-  const uint32_t min_keys = kTopkFilterMinKeys[rows <= 4ull * cus ? 0 : rows <= 8ull * cus ? 1 : 2];
+  const uint32_t min_keys = kTopkFilterMinKeys[rows <= 2ull * cus ? 0 : rows <= 4ull * cus ? 1 : 2];
   if (pl.t_all < min_keys && !(d->flags & DG_ATTN_F_TOPK_THRESHOLD)) return;
   if (k_cfg[1] != 0u) {
     const uint64_t gran = std::max(k_cfg[0], 1u);

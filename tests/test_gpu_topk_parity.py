@@ -424,6 +424,24 @@ def test_random_rows_are_not_left_over(gpu_ready):
     assert int(((left != 0) & (left != 1)).sum()) == 0 and int(left.sum()) <= 8      # (5120 rows at 1e-5 each)
 
 
+@pytest.mark.parametrize("canvas,kvl,causal,kv_dtype,lists", [
+    (64, 18432 - 65, 0, capi.DG_BF16, False), (64, 18432 - 64, 0, capi.DG_BF16, True), (33, 18432 - 33, 33, capi.DG_F16, True),
+    (32, 24576 - 33, 0, capi.DG_BF16, False), (65, 2047, 0, capi.DG_BF16, False), (65, 2048, 0, capi.DG_F16, True),
+    (101, 2048, 101, capi.DG_BF16, True), (128, 8000, 60, capi.DG_BF16, True)])
+def test_which_calls_keep_lists(gpu_ready, canvas, kvl, causal, kv_dtype, lists):
+    """Where the thresholds-and-lists path begins without being asked for, and that it gives what the score plane gives there
+    (the same kept sets: fp32 summation error)."""
+    hq, hkv, hd = 16, 2, 512
+    rng = np.random.default_rng(canvas + kvl)
+    rms = lambda x: x / np.sqrt(np.mean(x * x, axis=-1, keepdims=True))
+    q = rms(rng.standard_normal((canvas, hq, hd), dtype=np.float32))
+    kv = rms(rng.standard_normal((kvl + canvas, 2, hkv, hd), dtype=np.float32))
+    run = lambda flag: device_topk(canvas, hq, hkv, hd, kvl, T.adaptive_k(), q, kv, causal_rows=causal, kv_dtype=kv_dtype, flags=flag)
+    got, _, _, ws = run(0)
+    assert (rows_left_over(ws, canvas * hq) == 0) == lists
+    assert max_abs_diff(got, run(capi.DG_ATTN_F_TOPK_SCORE_PLANE)[0]) < 2e-5
+
+
 def test_workspace_of_the_score_plane_alone_is_enough(gpu_ready):
     """A caller with scratch for the score plane and no more gets the score plane's path, byte for byte."""
     import torch
