@@ -792,8 +792,8 @@ struct TopkPlan {
 // 69.7 | 55.8 (f16 71.2 | 59.7), 6500 85.6 | 64.7; 256 rows over 2100 120 | 66, 24k 450 | 172.  Over the reference's f16 cache, layer
 // step: 64 rows over 14k 77.1 | 85.6, 16k 85.7 | 88.7, 18.4k 101 | 95, 128 over 2100 73.3 | 61.8.
 // That is for rows the lists hold.  A row they do not (thousands of equal scores) has its block of canvas rows scored again:
-// the attention call alone, 256 rows over 33k keys, general | filtered: one such row 706 | 462 us, one in every canvas row
-// 975 | 1300, all of them 1947 | 3120; 64 rows over 33k: 233 | 380, 235 | 384, 489 | 766.  The host cannot tell.
+// the attention call alone, 256 rows over 33k keys, general | filtered: none such 621 | 234 us, one 678 | 415, one in every canvas row
+// 938 | 1248, all of them 1044 | 2020; 64 rows over 33k: 142 | 101, 210 | 327, 223 | 338, 253 | 516.  The host cannot tell.
 constexpr uint32_t kTopkFilterMinPrefix = 2048;
 constexpr uint32_t kTopkFilterMinKeys[3] = {24576, 18432, 0};   // up to half a round, one round, more
 
