@@ -232,16 +232,14 @@ bool plan_split_map(const dg_attn_desc* d, const Plan& pl, int cus, uint32_t nti
     if (pl.extra_lo < pl.t_all && dg::fast_div(mt * dg::kBlockM, by_group) < d->causal_rows) hi = pl.t_all;
     return (hi + dg::kBlockN - 1) / dg::kBlockN;
   };
-  // The shortest length in one round of the chip, down to four fifths of where partial rows cost what shorter shares save: a
-  // launch is as long as its longest share, partial rows are those of the average one.  (Down to that itself | four fifths, layer step: 1024
-  // rows behind 0 keys 46.6 | 46.0, 12 -> 11 tiles; 700 behind 0 36.2 | 34.9, 8 -> 6; 600 behind 200, no map | 6 tiles, 48.8 | 42.5;
-  // 560 behind 90 34.9 | 33.7; 512 behind 0 30.3 | 29.5; to seven tenths or half 333 behind 333 28.2 | 28.9 | 29.6.)
+  // No length below the one where the partial rows of all row tiles cost what shorter shares save.  Down to four fifths of it the
+  // longest share is shorter (layer step: 1024 rows behind 0 keys 46.4 -> 45.7 us, 12 -> 11 tiles; 700 behind 0 36.3 -> 35.1; 600 behind 200
+  // 48.2 -> 42.4), but row tiles of one share, whose rows are fp32 until the output, would be two with 16-bit partial rows (rows 352
+  // to 383 of the 1024).
   const double s = std::sqrt((double)ntiles * budget / pl.n_mtiles / 9.0);
-  const uint32_t len = std::max(1u, (uint32_t)(0.8 * ntiles / std::max(1.0, s))), tps = pl.tiles_per_split;
+  const uint32_t len = std::max(1u, (uint32_t)(ntiles / std::max(1.0, s))), tps = pl.tiles_per_split;
   const uint32_t limit = tps < 3u ? 0u : std::min(tps - 2u, 9u * tps / 10u);
-  if (!dg::shortest_split_map(pl.n_mtiles, len, limit, budget, tiles, out) || out->n <= 1) return false;
-  // (short shares that take more of the chip than equal splits do: 333 rows behind 333 keys, 84 -> 93 workgroups a KV head, 28.2 -> 28.5)
-  return tps > 6u || 50u * out->units <= 53u * pl.n_mtiles * ((ntiles + tps - 1) / tps);
+  return dg::shortest_split_map(pl.n_mtiles, len, limit, budget, tiles, out) && out->n > 1;
 }
 
 // Scratch a split count takes, and the count for a call that has `scratch` bytes of it: what the rule asks for, or, where

@@ -98,8 +98,7 @@ def test_device_prefix_with_the_scratch_of_a_split_map(gpu_ready, po):
 
 @pytest.mark.parametrize("canvas,kv_len,f16", [(512, 0, False), (600, 200, True), (560, 90, False), (350, 300, False), (333, 333, True)])
 def test_split_counts_of_short_shares(gpu_ready, po, canvas, kv_len, f16):
-    """Prompts whose shares are a few key tiles: maps (the last one: equal splits) against the oracle and against two equal
-    splits."""
+    """Prompts whose shares are a few key tiles against the oracle and against two equal splits."""
     import torch
     w = dataclasses.replace(W.Workload("short_map", canvas, 16, 2, 512, kv_len, causal_rows=canvas, seed=canvas), kv_f16=f16)
     check_tolerances(*run_workload(po, w, toks=np.unique(np.append(np.arange(0, canvas, 31), canvas - 1)).astype(np.uint32)))
@@ -114,6 +113,24 @@ def test_split_counts_of_short_shares(gpu_ready, po, canvas, kv_len, f16):
     x, y = (o.view(torch.bfloat16).float() for o in outs)
     # sums that differ by the rounding of partial rows, 2^-12 of them, can round to neighbouring bf16 values: one step, 2^-7 of the value at most
     assert float((x - y).abs().max()) <= 2.0 ** -7 * float(x.abs().max())
+
+
+@pytest.mark.parametrize("canvas,alone", [(1024, 384), (901, 320), (700, 256)])
+@pytest.mark.parametrize("f16", [False, True])
+def test_rows_of_one_share_are_fp32_until_the_output(gpu_ready, canvas, alone, f16):
+    """Behind no prefix the shares of a split map are 12, 10 and 8 key tiles long: row tiles that see no more (`alone` rows) have no
+    16-bit partial rows, the bits of a call in one split."""
+    import torch
+    w = dataclasses.replace(W.Workload("alone", canvas, 16, 2, 512, 0, causal_rows=canvas, seed=canvas), kv_f16=f16)
+    q, kv = W.generate(w)
+    qd, kd = W.device_arrays(w, q, kv)
+    outs = []
+    for desc in (w.desc(n_splits=1), w.desc()):
+        out = torch.zeros(canvas, 16 * 512, dtype=torch.int16, device="cuda")
+        A.forward(desc, qd, kd, out, None, torch.empty(max(capi.workspace_bytes(desc), 256), dtype=torch.uint8, device="cuda"))
+        outs.append(out)
+    torch.cuda.synchronize()
+    assert torch.equal(outs[0][:alone], outs[1][:alone]) and not torch.equal(*outs)
 
 
 @pytest.mark.parametrize("hd,hkv,splits", [(512, 2, 3), (256, 8, 2)])

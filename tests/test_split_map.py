@@ -86,6 +86,15 @@ def test_where_a_split_map_is_planned():
     assert capi.workspace_bytes(desc(1024, 0, 1024)) >= 2 * row_tiles * (512 * 2 + 8)      # two equal splits
 
 
+def test_shares_no_shorter_than_partial_rows_pay_for():
+    """(rows, prefix) of causal rows -> the largest split count of a row tile: a share is as long as where the partial rows of all row
+    tiles cost what shorter shares save, so that row tiles up to that length stay one share and their rows fp32 until the output."""
+    half = capi.DG_ATTN_F_F16_PARTIALS
+    for kw in ({"flags": half}, {"kv_dtype": capi.DG_F16, "flags": 0}):
+        splits = lambda rows, kv: capi.resolved_splits(A.make_desc(rows, 16, 2, 512, kv, causal_rows=rows, **kw))
+        assert [splits(*c) for c in ((1024, 0), (901, 0), (700, 0), (800, 100), (512, 0), (600, 200), (350, 300))] == [3, 3, 3, 3, 3, 3, 4]
+
+
 def test_every_merge_instance_can_be_reached():
     """The merge that asks for all rows at once: one instance per split count up to 8 and every second to 16, with a map only up to
     the splits a map gives, fp32 rows up to 8."""
