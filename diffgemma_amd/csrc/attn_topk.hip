@@ -831,8 +831,10 @@ __device__ __forceinline__ void wave_lds_fence() {
 
 // Threshold of a row, one wave each: with `mean` = the number of sampled keys expected among the k largest, tau is about the
 // w-th largest sampled score, w = mean + 5 sqrt(mean) + 3, so that the k largest lie above it but for a five-sigma accident.
-// What there is to choose from are the largest scores of n groups of sampled keys; w keys fall into n (1 - exp(-w / n)) of them
-// (38 of 1942 keys into 37 of 512 groups).  Any value near will do, so the bisection stops at the first key that leaves a count
+// What there is to choose from are the largest scores of n groups of the N sampled keys that the row sees; a group of N / n keys holds
+// one of the w largest with the chance 1 - (1 - w / N)^(N / n), so they fall into n times that many (38 of 1942 keys into 37 of 512
+// groups; as if drawn with replacement, n (1 - exp(-w / n)), 61 of 136 keys were said to fall into 39 of 64 groups, not 46: with 512 kept of
+// 2300 keys one row in 700 had a list too short).  Any value near will do, so the bisection stops at the first key that leaves a count
 // in a small range.
 template <int NV>
 __global__ void __launch_bounds__(256) topk_tau_kernel(const TopkParams tp) {
@@ -846,7 +848,8 @@ __global__ void __launch_bounds__(256) topk_tau_kernel(const TopkParams tp) {
   const uint32_t tok = tp.tok0 + tok_l;
   if (qh == 0u && tok_l % tp.fail_block_tok == 0u && lane == 0u) tp.fail_block[tok_l / tp.fail_block_tok] = 0u;
   const RowBounds rb = row_bounds(p, tok);
-  const uint32_t k = row_k(tp, tok, visible_count(rb, p.t_all));
+  const uint32_t n_valid = visible_count(rb, p.t_all);
+  const uint32_t k = row_k(tp, tok, n_valid);
   const uint32_t n_groups = tp.sample_splits * kBlockN;
   const float* srow = tp.sample_max + (size_t)rid * n_groups;
   uint32_t key[NV], top = 0u;
@@ -857,8 +860,9 @@ __global__ void __launch_bounds__(256) topk_tau_kernel(const TopkParams tp) {
 #pragma unroll
   for (int u = 0; u < NV; ++u) top = max(top, key[u]);
   const float mean = (float)k / (float)tp.sample_stride;
-  const float groups = (float)n_groups;
-  const uint32_t want = (uint32_t)(groups - groups * expf(-(mean + 5.f * __builtin_sqrtf(mean) + 3.f) / groups) + 0.5f);
+  const float groups = (float)n_groups, sampled = (float)n_valid / (float)tp.sample_stride;   // (a row of this path sees 2048 keys and more)
+  const float above = fminf((mean + 5.f * __builtin_sqrtf(mean) + 3.f) / sampled, 1.f);
+  const uint32_t want = (uint32_t)(groups - groups * expf(sampled / groups * logf(1.f - above)) + 0.5f);
   // a lower end first, from the lanes' largest keys alone: the want-th largest of those 64 has at least `want` above it
   // (one comparison a step instead of NV; `want` is below 64 at 512 keys kept)
   uint32_t lo = ~wave_max(~top), hi = wave_max(top) + 1u;      // count(>= lo) >= want, count(>= hi) < want

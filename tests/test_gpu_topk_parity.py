@@ -337,6 +337,28 @@ def test_thresholds_from_groups_of_sampled_keys(gpu_ready, canvas, kvl, causal, 
     assert max_abs_diff(got, run(capi.DG_ATTN_F_TOPK_SCORE_PLANE)[0]) < 2e-5
 
 
+@pytest.mark.parametrize("k", [64, 128, 256, 384, 512])
+@pytest.mark.parametrize("canvas,keys", [(256, 2304), (128, 2200), (512, 2700), (256, 3300), (256, 5000)])
+def test_thresholds_where_many_of_the_sampled_keys_count(gpu_ready, canvas, keys, k):
+    """Up to two sampled keys of five lie above the threshold there, and several in one group.  By the binomial distribution of the
+    groups they fall into, 5e-6 of rows at most (512 rows, 64 kept of 5000) have lists too short or too long."""
+    import torch
+    hq, hkv, hd = 16, 2, 512
+    g = torch.Generator(device="cuda")
+    g.manual_seed(keys + k)
+    q, kv = (torch.nn.functional.rms_norm(torch.randn(n, hd, device="cuda", generator=g), (hd,)).to(torch.bfloat16)
+             for n in (canvas * hq, 2 * hkv * keys))
+    runs = []
+    for flag in (capi.DG_ATTN_F_TOPK_THRESHOLD, capi.DG_ATTN_F_TOPK_SCORE_PLANE):
+        d = A.make_desc(canvas, hq, hkv, hd, keys - canvas, layout="head_major", t_cap=keys, out_dtype=capi.DG_F32, flags=flag)
+        out, ws = torch.zeros(canvas, hq, hd, device="cuda"), T.alloc_workspace(d, (k, 0, 0, 0))
+        T.forward(d, (k, 0, 0, 0), q, kv, out, ws)
+        runs.append((out, ws))
+    torch.cuda.synchronize()
+    assert rows_left_over(runs[0][1], canvas * hq) == 0
+    assert float((runs[0][0] - runs[1][0]).abs().max()) < 2e-5
+
+
 @pytest.mark.parametrize("canvas,slices", [(64, 4), (65, 2), (128, 2), (129, 1)])
 @pytest.mark.parametrize("k", [1, 3, 4, 15, 16, 17, 33])
 def test_gather_slices(gpu_ready, canvas, slices, k):
