@@ -1502,9 +1502,13 @@ template <bool F16>
 hipError_t launch_list_select(TopkParams tp, uint32_t k_most, hipStream_t s) {
   set_dividers(&tp);
   const dim3 sel((tp.ntok * tp.a.hq + 31u) / 32u * 8u);
-  if (k_most <= 160u) hipLaunchKernelGGL((topk_list_select_kernel<16>), sel, dim3(256), 0, s, tp);
-  else if (k_most <= 272u) hipLaunchKernelGGL((topk_list_select_kernel<20>), sel, dim3(256), 0, s, tp);
-  else if (k_most <= 384u) hipLaunchKernelGGL((topk_list_select_kernel<24>), sel, dim3(256), 0, s, tp);
+  // Instances by what their waves hold of a list, 1024 to 2048 candidates.  Past 139k keys every 19th or 21st is sampled and a list is
+  // longer and less certain: the next instance there.  (256 rows over 170k keys, up to 4 rows in 10^4 over: with 384 kept and two
+  // such rows 1674 -> 917 us; without one 847 -> 859 with 258 kept, 785 -> 788 with 128.)
+  const uint32_t inst = (k_most <= 160u ? 0u : k_most <= 272u ? 1u : k_most <= 384u ? 2u : 3u) + (tp.sample_stride > 17u ? 1u : 0u);
+  if (inst == 0u) hipLaunchKernelGGL((topk_list_select_kernel<16>), sel, dim3(256), 0, s, tp);
+  else if (inst == 1u) hipLaunchKernelGGL((topk_list_select_kernel<20>), sel, dim3(256), 0, s, tp);
+  else if (inst == 2u) hipLaunchKernelGGL((topk_list_select_kernel<24>), sel, dim3(256), 0, s, tp);
   else hipLaunchKernelGGL((topk_list_select_kernel<32>), sel, dim3(256), 0, s, tp);
   const hipError_t rc = hipGetLastError();
   if (rc != hipSuccess) return rc;

@@ -337,11 +337,11 @@ def test_thresholds_from_groups_of_sampled_keys(gpu_ready, canvas, kvl, causal, 
     assert max_abs_diff(got, run(capi.DG_ATTN_F_TOPK_SCORE_PLANE)[0]) < 2e-5
 
 
-@pytest.mark.parametrize("k", [64, 128, 256, 384, 512])
-@pytest.mark.parametrize("canvas,keys", [(256, 2304), (128, 2200), (512, 2700), (256, 3300), (256, 5000)])
-def test_thresholds_where_many_of_the_sampled_keys_count(gpu_ready, canvas, keys, k):
-    """Up to two sampled keys of five lie above the threshold there, and several in one group.  By the binomial distribution of the
-    groups they fall into, 5e-6 of rows at most (512 rows, 64 kept of 5000) have lists too short or too long."""
+@pytest.mark.parametrize("canvas,keys,k", [(c, t, k) for c, t in ((256, 2304), (128, 2200), (512, 2700), (256, 3300), (256, 5000))
+                                           for k in (64, 128, 256, 384, 512)] + [(256, 170000, k) for k in (160, 258, 384)])
+def test_random_rows_have_lists_that_hold_them(gpu_ready, canvas, keys, k):
+    """Where two sampled keys of five lie above the threshold, several of them in one group; and where every 21st key alone is
+    sampled.  By the binomial distribution of groups and lists 4e-6 of rows at most have a list too short or too long."""
     import torch
     hq, hkv, hd = 16, 2, 512
     g = torch.Generator(device="cuda")
