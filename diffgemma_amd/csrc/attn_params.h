@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
+
 namespace dg {
 
 enum : uint32_t { DT_BF16 = 0, DT_F16 = 1, DT_F32 = 2 };
@@ -131,6 +133,33 @@ inline bool shortest_split_map(uint32_t n_mtiles, uint32_t len, uint32_t limit, 
     else len = mid + 1u;
   }
   return make_split_map(n_mtiles, len, tiles, m);
+}
+
+// Key-range splits of a launch of `base` row tiles whose workgroups take a compute unit each: between `least` and `most`, the count
+// whose rounds of the chip are shortest, in key tiles, where starting a workgroup costs `start` of them.  (One more workgroup than a
+// whole round is a second round: with `cus` / `base` rounded up, 144 rows x 16 heads over 30k keys, 5 row tiles x 2, were 260 workgroups,
+// and the filter kernel took twice as long: layer step 226.8 -> 164.4 us, where 128 rows take 140; 224 rows 297.9 -> 216.2, 192 over 5k
+// keys 94.6 -> 75.5.)
+// Looked at: the last count of each round, and none from where full rounds without a ragged share would cost more than the best so far
+// (planning a top-k call, 256 | 1024 rows over 33k keys, with every count looked at 1.33 | 2.10 us, now 1.02 | 1.14).  `looked`: how many.
+inline uint32_t splits_in_rounds(uint32_t base, uint32_t tiles, uint32_t least, uint32_t most, uint32_t cus, uint32_t start,
+                                 uint32_t* looked = nullptr) {
+  uint32_t best = least, n = 0;
+  uint64_t best_cost = UINT64_MAX;
+  for (uint32_t s = least; s <= most; ++s) {
+    if (n != 0 && (uint64_t)base * (tiles + (uint64_t)s * start) >= best_cost * cus) break;
+    const uint64_t rounds = ((uint64_t)base * s + cus - 1) / cus;
+    s = (uint32_t)std::min<uint64_t>(most, rounds * cus / base);
+    const uint64_t cost = rounds * ((tiles + s - 1) / s + start);
+    ++n;
+    if (cost < best_cost) {
+      best_cost = cost;
+      best = s;
+    }
+  }
+  if (looked) *looked = n;
+  const uint32_t share = std::max(1u, (tiles + best - 1) / best);
+  return std::min(best, std::max(least, (tiles + share - 1) / share));      // (the fewest splits with these shares)
 }
 
 // One pass of top-k sparse attention over canvas rows [tok0, tok0 + ntok).

@@ -795,24 +795,6 @@ struct TopkPlan {
 constexpr uint32_t kTopkFilterMinPrefix = 2048;
 constexpr uint32_t kTopkFilterMinKeys[3] = {24576, 18432, 0};   // up to half a round, one round, more
 
-// Key-range splits of a launch of `base` row tiles whose workgroups take a compute unit each: between `least` and `most`, the count
-// whose rounds of the chip are shortest, in key tiles, where starting a workgroup costs `start` of them.  (One more workgroup than a
-// whole round is a second round: with `cus` / `base` rounded up, 144 rows x 16 heads over 30k keys, 5 row tiles x 2, were 260 workgroups,
-// and the filter kernel took twice as long: layer step 226.8 -> 164.4 us, where 128 rows take 140; 224 rows 297.9 -> 216.2, 192 over 5k
-// keys 94.6 -> 75.5.)
-uint32_t splits_in_rounds(uint32_t base, uint32_t tiles, uint32_t least, uint32_t most, uint32_t cus, uint32_t start) {
-  uint32_t best = least;
-  uint64_t best_cost = UINT64_MAX;
-  for (uint32_t s = least; s <= most; ++s) {
-    const uint64_t cost = (uint64_t)(((uint64_t)base * s + cus - 1) / cus) * ((tiles + s - 1) / s + start);
-    if (cost < best_cost) {
-      best_cost = cost;
-      best = s;
-    }
-  }
-  return best;
-}
-
 size_t filter_bytes(const dg_attn_desc* d, const Plan& pl, uint32_t cus, uint32_t ntok, TopkPlan* tk) {
   const uint32_t n_mtiles = (ntok * pl.group + dg::kTopkFilterRows - 1) / dg::kTopkFilterRows;
   const uint32_t base = d->n_kv_heads * n_mtiles;
@@ -825,7 +807,7 @@ size_t filter_bytes(const dg_attn_desc* d, const Plan& pl, uint32_t cus, uint32_
   const double mean = (double)tk->k_most / tk->stride, w = mean + 5.0 * std::sqrt(mean) + 3.0;
   const double root = std::sqrt(dg::kTopkSegCap + 4.0) - 2.0, most = root * root / (1.0 + 4.0 / std::sqrt(w));
   const uint32_t fit = std::min((uint32_t)(w * tk->stride / 2.0 / most) + 1, dg::kMaxSplits);
-  tk->splits = splits_in_rounds(base, n_tiles, fit, std::min(std::max(fit, n_tiles / 4), dg::kMaxSplits), cus, 3);
+  tk->splits = dg::splits_in_rounds(base, n_tiles, fit, std::min(std::max(fit, n_tiles / 4), dg::kMaxSplits), cus, 3);
   const size_t segs = (size_t)base * tk->splits * 4 * dg::kTopkSegs;
   tk->off_block = align_up((size_t)d->canvas * d->n_q_heads * sizeof(uint32_t));
   tk->off_plane = tk->off_block + align_up((size_t)ntok * sizeof(uint32_t));
@@ -837,7 +819,7 @@ size_t filter_bytes(const dg_attn_desc* d, const Plan& pl, uint32_t cus, uint32_
   // Sampled keys: two key tiles each at least.
   const uint32_t sample_tiles = (tk->sample_n + dg::kBlockN - 1) / dg::kBlockN;
   const uint32_t sample_base = d->n_kv_heads * ((ntok * pl.group + dg::kTopkSampleRows - 1) / dg::kTopkSampleRows);
-  tk->sample_splits = splits_in_rounds(sample_base, sample_tiles, 1, std::max(1u, std::min(sample_tiles / 2, dg::kTopkSampleSplits)), cus, 4);
+  tk->sample_splits = dg::splits_in_rounds(sample_base, sample_tiles, 1, std::max(1u, std::min(sample_tiles / 2, dg::kTopkSampleSplits)), cus, 4);
   // (the lists lie where the sampled keys' largest scores were)
   const size_t sample = (size_t)ntok * d->n_q_heads * tk->sample_splits * dg::kBlockN * sizeof(float);
   return tk->off_lists + align_up(std::max(segs * dg::kTopkSegAlloc * 8, sample));

@@ -63,9 +63,50 @@ int main() {
 """
 
 
+ROUNDS = r"""
+#include "attn_params.h"
+#include <cstdio>
+int main() {
+  using namespace dg;
+  double all = 0, seen = 0;
+  for (uint32_t cus : {256u, 80u})
+    for (uint32_t base = 1; base <= 700; base += base < 70 ? 1 : 37)
+      for (uint32_t tiles = 1; tiles <= 5400; tiles += 1 + tiles / 7)
+        for (uint32_t least : {1u, 6u, 14u, 16u})
+          for (uint32_t most : {least, std::max(least, std::min(tiles / 4, 64u)), std::max(least, std::min(tiles / 2, 128u))})
+            for (uint32_t start : {3u, 4u}) {
+              uint32_t want = least, looked = 0;
+              uint64_t want_cost = UINT64_MAX;
+              for (uint32_t s = least; s <= most; ++s) {
+                const uint64_t cost = ((uint64_t)base * s + cus - 1) / cus * ((tiles + s - 1) / s + start);
+                if (cost < want_cost) want_cost = cost, want = s;
+              }
+              const uint32_t got = splits_in_rounds(base, tiles, least, most, cus, start, &looked);
+              if (got != want)
+                return std::printf("base %u tiles %u least %u most %u cus %u: %u, not %u\n", base, tiles, least, most, cus, got, want), 1;
+              all += most - least + 1, seen += looked;
+            }
+  if (seen * 6 > all) return std::printf("%.0f counts looked at of %.0f\n", seen, all), 1;
+  // a canvas of many rows: as many workgroups as 32 bits hold
+  if (splits_in_rounds(1u << 24, 1000, 6, 64, 256, 3) != 6) return 1;
+  std::puts("ok");
+  return 0;
+}
+"""
+
+
 def test_units_of_a_split_map(tmp_path):
+    run_program(tmp_path, PROGRAM)
+
+
+def test_splits_in_rounds_of_the_chip(tmp_path):
+    """What working out the cost of every count finds, by looking at a sixth of them."""
+    run_program(tmp_path, ROUNDS)
+
+
+def run_program(tmp_path, program):
     src, exe = tmp_path / "map.hip", tmp_path / "map"
-    src.write_text(PROGRAM)
+    src.write_text(program)
     res = subprocess.run([build.hipcc_path(), *build.HIP_FLAGS, "-I", str(build.CSRC), str(src), "-o", str(exe)],
                          stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     assert res.returncode == 0, res.stdout[-2000:]
