@@ -199,6 +199,8 @@ constexpr uint32_t kTopkListMax = 512;      // most keys kept on the filtered pa
 constexpr uint32_t kTopkListAlign = 8;      // a row's list of kept keys takes a multiple of this
 constexpr uint32_t kTopkSampleMax = 8192;   // most sampled keys per row
 constexpr uint32_t kTopkSampleSplits = 128; // most splits of the sampled keys: 4096 groups, what the threshold kernel holds
+// head_dim slices the gather deals out, by the stacked rows of a pass (topk_gather_kernel has the times)
+inline uint32_t topk_gather_slices(uint32_t rows) { return rows > 2048u ? 1u : rows > 1024u ? 2u : 4u; }
 
 // Merging attention states of key-range partials (dg_attn_merge).  A state holds, per row
 // (row = canvas row * n_q_heads + query head), m and l in two planes of `rows` floats and then, from

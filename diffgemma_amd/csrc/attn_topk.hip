@@ -1512,7 +1512,7 @@ hipError_t launch_list_select(TopkParams tp, uint32_t k_most, hipStream_t s) {
   else hipLaunchKernelGGL((topk_list_select_kernel<32>), sel, dim3(256), 0, s, tp);
   const hipError_t rc = hipGetLastError();
   if (rc != hipSuccess) return rc;
-  const uint32_t n_rows = tp.ntok * tp.a.hq, slices = n_rows > 2048u ? 1u : n_rows > 1024u ? 2u : 4u;
+  const uint32_t n_rows = tp.ntok * tp.a.hq, slices = topk_gather_slices(n_rows);
   const dim3 gather((n_rows * slices + 31u) / 32u * 8u);
   if (slices == 1u) hipLaunchKernelGGL((topk_gather_kernel<F16, 1>), gather, dim3(256), 0, s, tp);
   else if (slices == 2u) hipLaunchKernelGGL((topk_gather_kernel<F16, 2>), gather, dim3(256), 0, s, tp);

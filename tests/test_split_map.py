@@ -1,6 +1,6 @@
 """Split counts per row tile (SplitMap in csrc/attn_params.h), compiled for the host: every (row tile, split) is one unit of a
 KV head, found again from its number, the longest share keeps the asked-for length, and the shortest length is found without
-trying each."""
+trying each.  And the split and slice counts of the same header."""
 import re
 import subprocess
 
@@ -102,6 +102,14 @@ def test_units_of_a_split_map(tmp_path):
 def test_splits_in_rounds_of_the_chip(tmp_path):
     """What working out the cost of every count finds, by looking at a sixth of them."""
     run_program(tmp_path, ROUNDS)
+
+
+def test_slices_of_the_gather(tmp_path):
+    """The slices that test_gather_slices names are those its calls get."""
+    from test_gpu_topk_parity import GATHER_SLICES
+    wrong = " || ".join(f"dg::topk_gather_slices({rows} * 16) != {n}" for rows, n in GATHER_SLICES)
+    run_program(tmp_path, '#include "attn_params.h"\n#include <cstdio>\nint main() { if (%s) return 1; std::puts("ok"); return 0; }\n' % wrong)
+    assert {n for _, n in GATHER_SLICES} == {1, 2, 4}
 
 
 def run_program(tmp_path, program):
