@@ -834,8 +834,8 @@ __device__ __forceinline__ void wave_lds_fence() {
 // What there is to choose from are the largest scores of n groups of the N sampled keys that the row sees; a group of N / n keys holds
 // one of the w largest with the chance 1 - (1 - w / N)^(N / n), so they fall into n times that many (38 of 1942 keys into 37 of 512
 // groups; as if drawn with replacement, n (1 - exp(-w / n)), 61 of 136 keys were said to fall into 39 of 64 groups, not 46: with 512 kept of
-// 2300 keys one row in 700 had a list too short).  Any value near will do, so the bisection stops at the first key that leaves a count
-// in a small range.
+// 2300 keys one row in 700 had a list too short).  Every rank more is a list 2 % longer, and twice as many lists that a wave cannot hold:
+// the bisection goes on to that very count.
 template <int NV>
 __global__ void __launch_bounds__(256) topk_tau_kernel(const TopkParams tp) {
   const AttnParams& p = tp.a;
@@ -880,7 +880,7 @@ __global__ void __launch_bounds__(256) topk_tau_kernel(const TopkParams tp) {
     for (int u = 0; u < NV; ++u) c += (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(key[u] >= mid));
     if (c >= want) lo = mid;
     else hi = mid;
-    if (c >= want && c <= want + 2u) break;
+    if (c == want) break;
   }
   // (lo = 0, a row with fewer sampled keys than wanted, is the image of NaN: nothing passes, and the row is left over)
   if (lane == 0u) tp.tau[(size_t)kvh * tp.n_mtiles * kTopkFilterRows + rr] = key_score(lo);

@@ -359,6 +359,19 @@ def test_random_rows_have_lists_that_hold_them(gpu_ready, canvas, keys, k):
     assert float((runs[0][0] - runs[1][0]).abs().max()) < 2e-5
 
 
+def test_lists_hold_the_rows_of_a_prompt(gpu_ready):
+    """1024 causal rows behind 32768 keys, 258 to 264 kept: the longest list has 1232 candidates of the 1280 a wave holds, two ranks
+    past the one that a threshold is meant to have 1296."""
+    import torch
+    w = W.Workload("topk_prompt", 1024, 16, 2, 512, 32768, causal_rows=1024, seed=41)
+    qd, kd = W.device_arrays(w, *W.generate(w))
+    d = w.desc(flags=capi.DG_ATTN_F_TOPK_THRESHOLD)
+    out, ws = torch.zeros(1024 * 16 * 512, dtype=torch.int16, device="cuda"), T.alloc_workspace(d, T.adaptive_k())
+    T.forward(d, T.adaptive_k(), qd, kd, out, ws)
+    torch.cuda.synchronize()
+    assert rows_left_over(ws, 1024 * 16) == 0
+
+
 GATHER_SLICES = [(64, 4), (65, 2), (128, 2), (129, 1)]      # canvas rows of 16 heads -> slices; test_split_map.py holds the rule to it
 
 
