@@ -753,9 +753,9 @@ __global__ void __launch_bounds__(256) topk_select_kernel(const TopkParams tp) {
 // two to four times k entries that one wave holds in registers.  Whatever tau is, the result is exact: a row whose
 // list holds fewer than k entries, or more than fit, is marked, and the general path redoes the marked rows (its
 // launches end at once where no row of the block is marked, 1.5 us each).
-// 256 rows x 16 heads over 33024 keys, layer step: 646 -> 230 us.  Launches: sampled scores 14 us (was: scores and plane, 4 x 55),
-// thresholds 5, filter 124 (1.1 PFLOP/s; the products alone, with their LDS reads and nothing else, 101), selection 24
-// and gathered P.V 50 (both: was 4 x 94).
+// 256 rows x 16 heads over 33024 keys, layer step: 646 -> 249 us.  Launches: sampled scores 15 us (was: scores and plane, 4 x 55),
+// thresholds 6, filter 126 to 133 by box (1.0 - 1.1 PFLOP/s; the products alone, with their LDS reads and nothing else, 101), selection 24
+// and gathered P.V 51 (both: was 4 x 94).
 
 // scores through an ordinary-register accumulator, query fragment in accumulation registers (256 of them hold the 64
 // query rows of a wave; a comparison cannot read that file)
@@ -882,7 +882,8 @@ __global__ void __launch_bounds__(256) topk_tau_kernel(const TopkParams tp) {
     else hi = mid;
     if (c == want) break;
   }
-  // (lo = 0, a row with fewer sampled keys than wanted, is the image of NaN: nothing passes, and the row is left over)
+  // (A row with fewer groups than wanted that hold a key other than NaN: tau is -inf, what groups without one have, every score
+  // passes, and the row is left over where its lists run over.)
   if (lane == 0u) tp.tau[(size_t)kvh * tp.n_mtiles * kTopkFilterRows + rr] = key_score(lo);
 }
 
@@ -1503,8 +1504,8 @@ hipError_t launch_list_select(TopkParams tp, uint32_t k_most, hipStream_t s) {
   set_dividers(&tp);
   const dim3 sel((tp.ntok * tp.a.hq + 31u) / 32u * 8u);
   // Instances by what their waves hold of a list, 1024 to 2048 candidates.  Past 139k keys every 19th or 21st is sampled and a list is
-  // longer and less certain: the next instance there.  (256 rows over 170k keys, up to 4 rows in 10^4 over: with 384 kept and two
-  // such rows 1674 -> 917 us; without one 847 -> 859 with 258 kept, 785 -> 788 with 128.)
+  // longer and less certain: the next instance there.  (256 rows over 170k keys, where the smaller one cannot hold 1 to 2 rows in 10^4: with
+  // 384 kept and two such rows 1674 -> 917 us; without one 847 -> 859 with 258 kept, 785 -> 788 with 128.)
   const uint32_t inst = (k_most <= 160u ? 0u : k_most <= 272u ? 1u : k_most <= 384u ? 2u : 3u) + (tp.sample_stride > 17u ? 1u : 0u);
   if (inst == 0u) hipLaunchKernelGGL((topk_list_select_kernel<16>), sel, dim3(256), 0, s, tp);
   else if (inst == 1u) hipLaunchKernelGGL((topk_list_select_kernel<20>), sel, dim3(256), 0, s, tp);

@@ -788,10 +788,14 @@ struct TopkPlan {
 // 32 rows over 17k 66.6 | 70.7, 24k 81.7 | 77.5; 48 rows over 9k 55.0 | 62.9, 12k 75.5 | 68.0; 64 rows (a whole round) over 9k
 // 58.3 | 64.6, 12k 68.6 | 69.7, 17k 83.9 | 76.1; 96 rows over 2100 65.6 | 53.0, 6500 91.2 | 62.7; 128 rows over 2100
 // 69.7 | 55.8 (f16 71.2 | 59.7), 6500 85.6 | 64.7; 256 rows over 2100 120 | 66, 24k 450 | 172.  Over the reference's f16 cache, layer
-// step: 64 rows over 14k 77.1 | 85.6, 16k 85.7 | 88.7, 18.4k 101 | 95, 128 over 2100 73.3 | 61.8.
-// That is for rows the lists hold.  A row they do not (thousands of equal scores) has its block of canvas rows scored again:
-// the attention call alone, 256 rows over 33k keys, general | filtered: none such 621 | 234 us, one 678 | 415, one in every canvas row
-// 938 | 1248, all of them 1044 | 2020; 64 rows over 33k: 142 | 101, 210 | 327, 223 | 338, 253 | 516.  The host cannot tell.
+// step: 64 rows over 14k 77.1 | 85.6, 16k 85.7 | 88.7, 18.4k 101 | 95, 128 over 2100 73.3 | 61.8.  That is with 64 to 192 keys kept (the
+// production rule); with a fixed 128, 256 and 512 the lines lie no higher: 65 rows over 2200 keys 67.0 | 55.1, 78.7 | 69.1, 100.9 | 92.5, 128 rows over
+// 2200 76.8 | 60.8, 91.1 | 76.6, 120 | 107, over 8000 101 | 72, 119 | 83, 148 | 105; 64 rows over 18.5k 81.8 | 75.1, 97.6 | 82.7, 122 | 96; 32 rows over 24.6k
+// 73.9 | 77.3, 84.0 | 81.9, 100.5 | 93.3.
+// And for rows the lists hold.  A row they do not (thousands of equal scores) has its block of canvas rows scored again:
+// the attention call alone, 256 rows over 33k keys, general | filtered: none such 603 | 228 us, one 676 | 408, one in every canvas row
+// 919 | 1229, all of them 1046 | 2031; 64 rows over 33k: 144 | 100, 224 | 334, 227 | 342, 263 | 530, over 18.5k 86 | 78, 134 | 233, 134 | 235, 168 | 355; 128 over
+// 2200 69 | 56, 77 | 107, 77 | 109, 110 | 205, over 8000 90 | 67, 107 | 158, 109 | 160, 179 | 340.  The host cannot tell.
 constexpr uint32_t kTopkFilterMinPrefix = 2048;
 constexpr uint32_t kTopkFilterMinKeys[3] = {24576, 18432, 0};   // up to half a round, one round, more
 
