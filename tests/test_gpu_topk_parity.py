@@ -459,7 +459,7 @@ def test_random_rows_are_not_left_over(gpu_ready):
     T.forward(d, k_cfg, qd, kd, torch.zeros(w.canvas * w.n_q_heads * w.head_dim, dtype=torch.int16, device="cuda"), ws)
     torch.cuda.synchronize()
     left = ws.view(torch.int32)[:w.canvas * w.n_q_heads]
-    assert int(((left != 0) & (left != 1)).sum()) == 0 and int(left.sum()) <= 8      # (5120 rows at 1e-5 each)
+    assert int(((left != 0) & (left != 1)).sum()) == 0 and int(left.sum()) == 0      # (5120 rows, 4 in 10^6 of which the lists may not hold)
 
 
 @pytest.mark.parametrize("canvas,kvl,causal,kv_dtype,lists", [
