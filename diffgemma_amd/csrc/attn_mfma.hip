@@ -106,6 +106,7 @@ struct MfmaArgs {
   FastDiv div_mtiles, div_splits, div_group;
   FastDiv div_units, div_n[kMapSplits];   // with a split map: by the units of a KV head, by 1 .. 8
   SplitMap map;
+  uint32_t rows_first;   // order of the units: rows_before_splits
 };
 
 // MAPPED: with a split map (an instance of its own: what the map takes at a workgroup's start is 0.3 us of a short call)
@@ -149,30 +150,39 @@ __global__ void __launch_bounds__(256) attn_mfma_kernel(const MfmaArgs args) {
   float* const sinv = (float*)(smem + OFF_ML);
 
   // ---- which (KV head, split, row tile) this workgroup owns ----
-  // Workgroup ids go round-robin over the 8 XCDs, each with its own L2.  The units, ordered
-  // (KV head, split) first and row tile second, are cut into 8 equal runs, one per XCD, so the
-  // row tiles that stream the same keys sit behind one L2 and every XCD has work whatever
-  // the number of (KV head, split) pairs.
+  // Workgroup ids go round-robin over the 8 XCDs, each with its own L2.  The units are cut into 8 equal runs, one per XCD.
+  // Ordered (KV head, split) first and row tile second, the row tiles that stream the same keys sit behind one L2; ordered
+  // (KV head, row tile) first, an XCD reads few query rows and holds all partial rows of a row tile (rows_before_splits).
   const SplitMap& map = args.map;
   const uint32_t n_units = p.hkv * (MAPPED ? map.units : p.n_splits * p.n_mtiles);
   const uint32_t per_xcd = (n_units + 7u) >> 3;
   const uint32_t wg = blockIdx.x;
   const uint32_t unit = (wg & 7u) * per_xcd + (wg >> 3);
   if (unit >= n_units) return;
-  uint32_t mt, kvh, split, n_splits;
+  uint32_t mt, kvh, split, n_splits, prow_tile;   // (prow_tile: with a split map, the 128 partial rows that are this workgroup's)
   FastDiv div_n = args.div_splits;
   if constexpr (MAPPED) {
     kvh = fast_div(unit, args.div_units);
     const uint32_t u = unit - kvh * map.units;
-    split = map_split_of(map, u);
-    mt = map.first[split] + u - map.cum[split];
-    n_splits = map_splits(map, mt);
+    if (args.rows_first) {
+      const MapUnit mu = map_unit_by_rows(map, args.div_n, u);
+      mt = mu.mt;
+      split = mu.split;
+      n_splits = mu.splits;
+    } else {
+      split = map_split_of(map, u);
+      mt = map.first[split] + u - map.cum[split];
+      n_splits = map_splits(map, mt);
+    }
+    prow_tile = kvh * map.units + map.cum[split] + mt - map.first[split];
     div_n = args.div_n[n_splits - 1u];
   } else {
-    const uint32_t stream = fast_div(unit, args.div_mtiles);
-    mt = unit - stream * p.n_mtiles;
-    kvh = fast_div(stream, args.div_splits);
-    split = stream - kvh * p.n_splits;
+    const uint32_t outer = fast_div(unit, args.rows_first ? args.div_splits : args.div_mtiles);
+    const uint32_t inner = unit - outer * (args.rows_first ? p.n_splits : p.n_mtiles);
+    kvh = fast_div(outer, args.rows_first ? args.div_mtiles : args.div_splits);
+    const uint32_t rest = outer - kvh * (args.rows_first ? p.n_mtiles : p.n_splits);
+    mt = args.rows_first ? rest : inner;
+    split = args.rows_first ? inner : rest;
     n_splits = p.n_splits;
   }
 
@@ -269,7 +279,7 @@ __global__ void __launch_bounds__(256) attn_mfma_kernel(const MfmaArgs args) {
   const uint32_t ntile = te - tb;
 
   // first partial row of this workgroup; partial rows and their (m, l) are written through (wt_store.h)
-  const size_t wg_prow0 = MAPPED ? (size_t)unit * kBlockM : ((size_t)split * p.hkv + kvh) * p.rows_pad + row0;
+  const size_t wg_prow0 = MAPPED ? (size_t)prow_tile * kBlockM : ((size_t)split * p.hkv + kvh) * p.rows_pad + row0;
   // No key tile to visit: the rows' share is nothing, (m, l, O) = (-inf, 0, 0).  An exit of its own, so that the epilogue
   // has one predecessor and takes O from the registers the tile loop leaves it in (with a second one the compiler moved
   // all 256 accumulation registers at the loop's exit, 512 instructions).
@@ -880,6 +890,7 @@ hipError_t launch_one(const AttnParams& p, const SplitMap& map, hipStream_t s) {
   a.div_group = make_fast_div(p.group);
   a.div_units = make_fast_div(std::max(1u, map.units));
   for (uint32_t i = 0; i < kMapSplits; ++i) a.div_n[i] = make_fast_div(i + 1u);
+  a.rows_first = rows_before_splits(p.hkv, p.n_mtiles, p.tile_end - p.tile_first) ? 1u : 0u;
   const uint32_t n_units = p.hkv * (map.n ? map.units : p.n_splits * p.n_mtiles);
   const uint32_t grid = (n_units + 7u) / 8u * 8u;
   auto launch = [&](auto kernel) {

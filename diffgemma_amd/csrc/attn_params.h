@@ -20,11 +20,13 @@ constexpr float kLn2 = 0.6931471805599453f;
 // count for all the launch is as long as the last row tile's share).  The counts do not fall with the row tile, so they
 // are given by where each begins: row tile mt has more than i splits from mt = first[i] on.  The units of a KV head are
 // ordered by split, then row tile: split i of row tile mt is unit cum[i] + mt - first[i], which also numbers its partial rows.
+// The workgroups may go by row tile, then split, instead (rows_before_splits): the row tiles of i + 1 splits begin with
+// workgroup at[i].
 constexpr uint32_t kMapSplits = 8;
 struct SplitMap {
   uint32_t n;                     // most splits of a row tile; 0: every row tile has n_splits
   uint32_t units;                 // of a KV head
-  uint32_t first[kMapSplits], cum[kMapSplits];   // past n: no row tile, no unit
+  uint32_t first[kMapSplits], cum[kMapSplits], at[kMapSplits];   // past n: no row tile, no unit
 };
 __host__ __device__ __forceinline__ uint32_t map_splits(const SplitMap& m, uint32_t mt) {
   uint32_t s = 0;
@@ -44,7 +46,7 @@ __host__ __device__ __forceinline__ uint32_t map_split_of(const SplitMap& m, uin
 template <typename Tiles>
 inline bool make_split_map(uint32_t n_mtiles, uint32_t len, Tiles&& tiles, SplitMap* m) {
   m->n = m->units = 0;
-  for (uint32_t i = 0; i < kMapSplits; ++i) m->first[i] = m->cum[i] = 0xffffffffu;
+  for (uint32_t i = 0; i < kMapSplits; ++i) m->first[i] = m->cum[i] = m->at[i] = 0xffffffffu;
   for (uint32_t mt = 0; mt < n_mtiles; ++mt) {
     const uint32_t s = (tiles(mt) + len - 1) / len;
     if (s > kMapSplits) return false;
@@ -53,6 +55,7 @@ inline bool make_split_map(uint32_t n_mtiles, uint32_t len, Tiles&& tiles, Split
   for (uint32_t i = 0; i < m->n; ++i) {
     m->cum[i] = m->units;
     m->units += n_mtiles - m->first[i];
+    m->at[i] = i == 0 ? 0u : m->at[i - 1] + i * (m->first[i] - m->first[i - 1]);
   }
   return true;
 }
@@ -109,6 +112,18 @@ __host__ __device__ __forceinline__ uint32_t fast_div(uint32_t n, FastDiv d) {
   return ((uint32_t)(((uint64_t)n * d.mul) >> 32) + n) >> d.shift;
 }
 
+// Workgroup u of a KV head in the order by row tile, then split; by[i] divides by i + 1.
+struct MapUnit {
+  uint32_t mt, split, splits;
+};
+__host__ __device__ __forceinline__ MapUnit map_unit_by_rows(const SplitMap& m, const FastDiv* by, uint32_t u) {
+  uint32_t i = 0;
+#pragma unroll
+  for (uint32_t j = 1; j < kMapSplits; ++j) i = u >= m.at[j] ? j : i;
+  const uint32_t v = u - m.at[i], tiles = fast_div(v, by[i]);
+  return MapUnit{m.first[i] + tiles, v - tiles * (i + 1u), i + 1u};
+}
+
 // The map of the shortest length in [len, limit] that gives a KV head no more than `budget` units (and no row tile more than
 // kMapSplits); false where even `limit` gives more.  Units do not grow with the length, so it is found by bisection, and rows
 // behind a long prefix, all of which see about as many key tiles, are told by the first of them (each length in turn, with a map
@@ -160,6 +175,21 @@ inline uint32_t splits_in_rounds(uint32_t base, uint32_t tiles, uint32_t least, 
   if (looked) *looked = n;
   const uint32_t share = std::max(1u, (tiles + best - 1) / best);
   return std::min(best, std::max(least, (tiles + share - 1) / share));      // (the fewest splits with these shares)
+}
+
+// In which order the split kernel's workgroups take their units.  Each of the 8 XCDs gets a run of them and reads what its run
+// needs through an L2 of its own: by split, then row tile, a share of the keys and all query rows of a KV head; by row tile, then
+// split, its own query rows alone, which no workgroup can begin without, and all keys.  And a row tile's partial rows are then
+// written on one XCD: see merge_on_xcd.  Attention call, 16 heads over 2, us, splits first | rows first, with the keys in a cache | from
+// HBM: 64 rows over 1564 keys 22.1 | 20.8, 22.1 | 19.3, 2564 24.6 | 22.3, 25.9 | 26.0, layer step over 6064 34.3 | 36.5; 128 rows over 905 26.0 |
+// 23.0 (step), 23.0 | 19.8, 2628 27.7 | 27.0, 29.0 | 28.5, 5128 35.5 | 35.1, 37.7 | 37.4; 256 rows over 556 29.4 | 26.0 (step), 24.0 | 21.4, 3256 42.4 |
+// 41.2 (step), 40.5 | 40.3, 6256 61.1 | 60.3 (step), 59.2 | 60.3, 16256 120.8 | 121.5 (step); 512 rows over 1512 43.0 | 39.8 (step), 40.5 | 37.9, 4512
+// 78.7 | 77.2 (HBM), 8512 129.2 | 130.5 (HBM); 1024 causal rows behind 0 46.6 | 46.1 (step), 3000 123.5 | 121.8 (HBM), 8000 240.9 | 238.3, 243.3 | 244.3,
+// 32768 849 | 847, 860 | 868; 700 behind 700 48.9 | 47.1 (step).  Row tiles that do not come in eights end in the middle of an XCD's
+// run: 72 rows over 972 keys 19.2 | 18.1, over 1672 22.7 | 23.1; 96 over 1696 24.4 | 21.7, 2496 26.1 | 25.4; 200 over 2600 33.2 | 32.3; the few
+// of 8 to 48 rows gain 4 % or lose 1 (32 over 432 keys 14.9 | 14.2, 40 over 440 14.8 | 15.0).
+inline bool rows_before_splits(uint32_t hkv, uint32_t n_mtiles, uint32_t key_tiles) {
+  return key_tiles <= std::min((hkv * n_mtiles % 8u == 0u ? 20u : 10u) * n_mtiles, 72u + 2u * n_mtiles);
 }
 
 // One pass of top-k sparse attention over canvas rows [tok0, tok0 + ntok).
@@ -361,6 +391,16 @@ inline bool merge_at_once(uint32_t n_splits, size_t bytes) {
   return n_splits <= 8 ? bytes < ((size_t)32 << 20) : n_splits <= kMergeFewSplits && bytes <= ((size_t)17 << 20);
 }
 
+// Whether the merge that asks for all rows at once takes a row on the XCD that wrote its partial rows (their splits on one XCD):
+// where these, `part_bytes` in all, and the keys an XCD has read since, `head_bytes` for each KV head, are still in its L2 of 4 MiB
+// when they are wanted.  Rows that another XCD has read are also slower to write the next time.  Layer step, 16 heads over 2, us, rows
+// in turn over the XCDs | where they were written: 256 rows over 556 keys (3.2 MiB) 29.4 | 26.0, 1033 (5.1) 29.6 | 28.2, 1756 (7.5)
+// 32.8 | 32.5; 128 rows over 905 (4.1) 26.0 | 23.0; 64 rows over 1564 (4.7) 23.3 | 22.0; call alone, 64 over 2564 (7) 22.3 | 22.5, over 4064 26.0 |
+// 26.3; 64 rows over a window of 8 KV heads x 256 (1.6) 15.3 | 14.7 (step).
+inline bool merge_on_xcd(uint32_t hkv, size_t head_bytes, size_t part_bytes) {
+  return head_bytes * std::max(1u, hkv / 8u) + part_bytes / 8 <= ((size_t)6 << 20);
+}
+
 // host-side launchers (defined next to their kernels)
 hipError_t launch_attn_scalar(const AttnParams& p, uint32_t head_dim, uint32_t kv_dtype, hipStream_t s);
 // (map: row tiles with split counts of their own, head_dim 512; n = 0 for none. It stands behind AttnParams in the
@@ -368,7 +408,8 @@ hipError_t launch_attn_scalar(const AttnParams& p, uint32_t head_dim, uint32_t k
 // line of the arguments, and a call with 64 canvas rows on a sliding layer took 9.77 us for 9.52.)
 hipError_t launch_attn_mfma(const AttnParams& p, const SplitMap& map, uint32_t head_dim, uint32_t kv_dtype, hipStream_t s);
 hipError_t launch_attn_wsplit(const AttnParams& p, uint32_t head_dim, uint32_t kv_dtype, hipStream_t s);
-hipError_t launch_attn_merge(const AttnParams& p, const SplitMap& map, uint32_t head_dim, bool streamed, hipStream_t s);
+// (shared_tiles: the partial rows are the one-launch kernel's, whose workgroups go by split, then row tile)
+hipError_t launch_attn_merge(const AttnParams& p, const SplitMap& map, uint32_t head_dim, bool streamed, bool shared_tiles, hipStream_t s);
 hipError_t launch_state_merge(const StateMergeParams& p, hipStream_t s);
 // l[row] = 1 where m[row] is finite, else 0: completes a state whose rows are already normalised
 hipError_t launch_state_unit_l(float* m_plane, float* l_plane, uint32_t rows, hipStream_t s);

@@ -611,7 +611,8 @@ int forward_planned(const dg_attn_desc* d, const Plan& pl, const void* q, const 
     (void)hipEventRecord(g_prof.ev[2 * g_prof.used + 1], s);
     ++g_prof.used;
   }
-  if (pl.n_splits > 1 && dg::launch_attn_merge(p, pl.map, hd, (d->flags & DG_ATTN_F_STREAMED_MERGE) != 0, s) != hipSuccess) return DG_ERR_LAUNCH;
+  if (pl.n_splits > 1 && dg::launch_attn_merge(p, pl.map, hd, (d->flags & DG_ATTN_F_STREAMED_MERGE) != 0, pl.wsplit, s) != hipSuccess)
+    return DG_ERR_LAUNCH;
   return DG_OK;
 }
 }  // namespace

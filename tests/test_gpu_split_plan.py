@@ -225,3 +225,27 @@ def test_merge_at_once_gives_the_bits_of_the_streamed_merge(gpu_ready, hd, hkv, 
                 torch.cuda.synchronize()
                 got.append((out, lse))
             assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+
+
+@pytest.mark.parametrize("canvas,kv_len,hq,hkv,hd,causal_rows", [
+    (1, 300, 16, 2, 512, 0), (64, 2496, 16, 2, 512, 0), (64, 2497, 16, 2, 512, 0), (72, 1528, 16, 2, 512, 30), (72, 1529, 16, 2, 512, 0),
+    (37, 500, 8, 8, 512, 37), (65, 700, 9, 3, 512, 0), (37, 3500, 16, 16, 256, 0), (250, 3000, 16, 2, 512, 0), (64, 4000, 16, 8, 256, 0)])
+def test_units_by_row_tile_and_rows_merged_where_they_were_written(gpu_ready, po, canvas, kv_len, hq, hkv, hd, causal_rows):
+    """Either order of the workgroups, with row tiles that are cut by an XCD's run and rows that do not fill one, against the oracle; and
+    the merge that takes rows on the XCD that wrote them gives the bits of the one that takes them in turn."""
+    import torch
+    w = W.Workload("order", canvas, hq, hkv, hd, kv_len, causal_rows=causal_rows, window=1024 if hkv == 8 and hd == 256 else 0, seed=canvas)
+    d = w.desc()
+    assert capi.resolved_splits(d) > 1
+    check_tolerances(*run_workload(po, w, toks=np.unique(np.linspace(0, canvas - 1, 12).round().astype(np.uint32))))
+    q, kv = W.generate(w)
+    qd, kd = W.device_arrays(w, q, kv)
+    got = []
+    for flags in (d.flags, d.flags | capi.DG_ATTN_F_STREAMED_MERGE):
+        d.flags = flags
+        out = torch.zeros(canvas * hq * hd, dtype=torch.int16, device="cuda")
+        lse = torch.zeros(canvas * hq, device="cuda")
+        A.forward(d, qd, kd, out, lse, A.alloc_workspace(d))
+        torch.cuda.synchronize()
+        got.append((out, lse))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])

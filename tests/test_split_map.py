@@ -95,6 +95,41 @@ int main() {
 """
 
 
+BY_ROWS = r"""
+#include "attn_params.h"
+#include <cstdio>
+int main() {
+  using namespace dg;
+  FastDiv by[kMapSplits];
+  for (uint32_t i = 0; i < kMapSplits; ++i) by[i] = make_fast_div(i + 1);
+  for (uint32_t n = 1; n <= 70; n += n < 6 ? 1 : 13)
+    for (uint32_t len = 1; len <= 20; ++len)
+      for (uint32_t base = 0; base <= 40; base += 8)
+        for (uint32_t per = 0; per <= 3; ++per) {
+          SplitMap m;
+          if (!make_split_map(n, len, [&](uint32_t mt) { return base + 1 + mt * per / 2; }, &m)) continue;
+          uint32_t u = 0;
+          for (uint32_t mt = 0; mt < n; ++mt)
+            for (uint32_t s = 0; s < map_splits(m, mt); ++s, ++u) {
+              const MapUnit got = map_unit_by_rows(m, by, u);
+              if (got.mt != mt || got.split != s || got.splits != map_splits(m, mt)) return std::printf("n %u len %u unit %u\n", n, len, u), 1;
+            }
+          if (u != m.units) return std::printf("units %u %u\n", u, m.units), 1;
+        }
+  // both sides of each line: 20 or 10 key tiles to a row tile, and where many row tiles see more than a few thousand keys
+  if (!rows_before_splits(2, 4, 80) || rows_before_splits(2, 4, 81) || !rows_before_splits(2, 5, 50) || rows_before_splits(2, 5, 51)) return 2;
+  if (!rows_before_splits(2, 16, 104) || rows_before_splits(2, 16, 105) || !rows_before_splits(8, 1, 20) || rows_before_splits(1, 1, 11)) return 3;
+  std::puts("ok");
+  return 0;
+}
+"""
+
+
+def test_units_by_row_tile(tmp_path):
+    """A split map's workgroups in the order by row tile, then split: every unit once, and the lines of the rule that takes it."""
+    run_program(tmp_path, BY_ROWS)
+
+
 def test_units_of_a_split_map(tmp_path):
     run_program(tmp_path, PROGRAM)
 
