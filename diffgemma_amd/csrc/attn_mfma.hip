@@ -307,7 +307,8 @@ __global__ void __launch_bounds__(256) attn_mfma_kernel(const MfmaArgs args) {
   const char* vbase = (const char*)p.v + (int64_t)kvh * p.v_head_stride * 2;
   const int64_t kstride_b = p.k_tok_stride * 2, vstride_b = p.v_tok_stride * 2;
   // Touch this workgroup's share of key tile `tile` of the split (the last tile instead of one past it).
-  // The row tiles of a (KV head, split) pair stream the same keys behind one L2, so they share the
+  // The row tiles of a (KV head, split) pair stream the same keys behind one L2 (with the units by row tile: behind a few of
+  // them, and a line touched for another L2 waits in the memory-side cache), so they share the
   // work: a tile is 256 lines of K and 256 of V (a row is 1 KiB = 8 lines); with 16 row tiles or more,
   // row tile mt takes the sixteenth (mt mod 16) of them, 8 lines per wave in one instruction (the
   // other lanes repeat them); with fewer, an eighth.  Every workgroup touching whole tiles cost more
