@@ -258,9 +258,9 @@ __global__ void __launch_bounds__(256) attn_merge_kernel(const AttnParams p, con
 // then i + 4, ..., and the rows are added in the same order with the same cut, so both kernels give the same bits.
 struct MergeArgs {
   AttnParams p;
-  FastDiv div_rows, div_group;   // by the rows of a KV head and by the GQA group
+  FastDiv div_span, div_group;   // by the rows counted for a KV head and by the GQA group
   uint32_t hd;
-  uint32_t xcd_run;   // workgroups of each XCD, which then take a run of the rows (merge_on_xcd); 0: rows in turn
+  MergeRuns rows;   // in runs, one for each XCD, or in turn
   SplitMap map;
 };
 // MAPPED: row tiles have split counts of their own (a split map), at most N; rows of one split are in the output already.
@@ -271,10 +271,9 @@ __global__ void __launch_bounds__(256) attn_merge_few_kernel(const MergeArgs arg
   const AttnParams& p = args.p;
   const uint32_t hd = args.hd;
   const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
-  const uint32_t wg = args.xcd_run ? (blockIdx.x & 7u) * args.xcd_run + (blockIdx.x >> 3) : blockIdx.x;
-  const uint32_t gr = wg * 4 + wave;  // global stacked row over all KV heads
-  if (gr >= p.hkv * p.rows_total) return;
-  const uint32_t kvh = fast_div(gr, args.div_rows), r = gr - kvh * p.rows_total;
+  const uint32_t gr = merge_row(blockIdx.x, wave, args.rows.run);
+  const uint32_t kvh = fast_div(gr, args.div_span), r = gr - kvh * args.rows.span;
+  if (kvh >= p.hkv || r >= p.rows_total) return;
   const uint32_t tok = fast_div(r, args.div_group), qh = kvh * p.group + r - tok * p.group;
   const bool live = lane < hd / 8;
   const uint32_t d8 = live ? lane : 0u;
@@ -407,7 +406,7 @@ __global__ void __launch_bounds__(256) attn_merge_few_kernel(const MergeArgs arg
 template <uint32_t N>
 hipError_t launch_merge_few(const MergeArgs& a, uint32_t rows, hipStream_t s) {
   auto launch = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, dim3(a.xcd_run ? 8u * a.xcd_run : (rows + 3) / 4), dim3(256), 0, s, a);
+    hipLaunchKernelGGL(kernel, dim3(a.rows.run ? 8u * a.rows.run : (rows + 3) / 4), dim3(256), 0, s, a);
     return hipGetLastError();
   };
   if constexpr (N <= kMapSplits) {   // (what a map gives a row tile at most)
@@ -657,19 +656,15 @@ hipError_t launch_state_merge(const StateMergeParams& p, hipStream_t s) {
 
 hipError_t launch_attn_merge(const AttnParams& p, const SplitMap& map, uint32_t head_dim, bool streamed, bool shared_tiles, hipStream_t s) {
   const uint32_t rows = p.hkv * p.rows_total;
-  // not many splits, not many bytes: the variant that asks for every partial row up front
-  const size_t part_bytes = (size_t)p.n_splits * p.hkv * p.rows_pad * head_dim * (p.part_half ? 2 : 4);
-  if (map.n || (!streamed && (p.part_half || p.n_splits <= 8) && head_dim % 8 == 0 && head_dim <= 512 && merge_at_once(p.n_splits, part_bytes))) {
+  const MergePlan plan = plan_merge(p, map, head_dim, streamed, shared_tiles);
+  if (plan.at_once) {
     MergeArgs a;
     a.p = p;
-    a.div_rows = make_fast_div(p.rows_total);
+    a.rows = plan.rows;
+    a.div_span = make_fast_div(plan.rows.span);
     a.div_group = make_fast_div(p.group);
     a.hd = head_dim;
     a.map = map;
-    // (with a split map the rows without a merge would leave some XCDs idle: 1024 causal rows behind 0 keys 46.1 -> 51.5 us)
-    const uint32_t key_tiles = p.tile_end - p.tile_first;
-    const bool one_xcd = map.n == 0 && (p.hkv % 8 == 0 || (!shared_tiles && rows_before_splits(p.hkv, p.n_mtiles, key_tiles)));
-    a.xcd_run = one_xcd && merge_on_xcd(p.hkv, (size_t)key_tiles * kBlockN * head_dim * 4, part_bytes) ? ((rows + 3) / 4 + 7) / 8 : 0u;
     switch (map.n ? map.n : p.n_splits) {
       case 2: return launch_merge_few<2>(a, rows, s);
       case 3: return launch_merge_few<3>(a, rows, s);

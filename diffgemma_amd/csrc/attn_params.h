@@ -402,6 +402,47 @@ inline bool merge_on_xcd(uint32_t hkv, size_t head_bytes, size_t part_bytes) {
   return head_bytes * std::max(1u, hkv / 8u) + part_bytes / 8 <= ((size_t)6 << 20);
 }
 
+// Rows of the merge that asks for all at once, four to a workgroup.  In turn: run = 0, span the rows of a KV head.  In runs, one of
+// `run` workgroups for each XCD, that follow the split kernel's run of units there (one 8th of them, by row tile, then split), so they are
+// counted with the padding of the last row tile; with KV heads in eights an XCD has whole heads in either order and in the one-launch
+// kernel, and only the last workgroup of a head is padded.  A row tile that the end of a run cuts is merged by both sides in the
+// share each wrote.  (Rows counted without the padding drift from the tiles: with 49 rows, 16 heads over 2, XCD 3 wrote the
+// tile of rows 384 to 391 and merged rows 294 to 391.)
+struct MergeRuns {
+  uint32_t span, run;
+};
+inline MergeRuns merge_runs(uint32_t hkv, uint32_t rows_total, uint32_t n_mtiles, uint32_t n_splits) {
+  if (hkv % 8u == 0u) {
+    const uint32_t wgs = (rows_total + 3u) / 4u;
+    return MergeRuns{wgs * 4u, hkv / 8u * wgs};
+  }
+  const uint32_t units = (hkv * n_mtiles * n_splits + 7u) / 8u;
+  return MergeRuns{n_mtiles * (uint32_t)kBlockM, (units * (uint32_t)(kBlockM / 4) + n_splits - 1u) / n_splits};
+}
+// row of a wave, counted over KV heads of `span` rows each
+__host__ __device__ __forceinline__ uint32_t merge_row(uint32_t block, uint32_t wave, uint32_t run) {
+  return (run ? (block & 7u) * run + (block >> 3) : block) * 4u + wave;
+}
+
+// How the partial rows of a call are merged: by the kernel that asks for all of a row's at once or the one that looks at
+// the weights first; and by the first in runs or in turn.  (shared_tiles: the partial rows are the one-launch kernel's, whose workgroups go by
+// split, then row tile.  With a split map the rows without a merge would leave some XCDs idle: 1024 causal rows behind 0 keys
+// 46.1 -> 51.5 us.)
+struct MergePlan {
+  bool at_once;
+  MergeRuns rows;
+};
+inline MergePlan plan_merge(const AttnParams& p, const SplitMap& map, uint32_t head_dim, bool streamed, bool shared_tiles) {
+  const uint32_t key_tiles = p.tile_end - p.tile_first;
+  const size_t part_bytes = (size_t)p.n_splits * p.hkv * p.rows_pad * head_dim * (p.part_half ? 2 : 4);
+  const bool at_once = map.n || (!streamed && (p.part_half || p.n_splits <= 8) && head_dim % 8 == 0 && head_dim <= 512 &&
+                                 merge_at_once(p.n_splits, part_bytes));
+  const bool one_xcd = map.n == 0 && (p.hkv % 8 == 0 || (!shared_tiles && rows_before_splits(p.hkv, p.n_mtiles, key_tiles)));
+  if (at_once && one_xcd && merge_on_xcd(p.hkv, (size_t)key_tiles * kBlockN * head_dim * 4, part_bytes))
+    return MergePlan{true, merge_runs(p.hkv, p.rows_total, p.n_mtiles, p.n_splits)};
+  return MergePlan{at_once, MergeRuns{p.rows_total, 0u}};
+}
+
 // host-side launchers (defined next to their kernels)
 hipError_t launch_attn_scalar(const AttnParams& p, uint32_t head_dim, uint32_t kv_dtype, hipStream_t s);
 // (map: row tiles with split counts of their own, head_dim 512; n = 0 for none. It stands behind AttnParams in the
@@ -409,7 +450,7 @@ hipError_t launch_attn_scalar(const AttnParams& p, uint32_t head_dim, uint32_t k
 // line of the arguments, and a call with 64 canvas rows on a sliding layer took 9.77 us for 9.52.)
 hipError_t launch_attn_mfma(const AttnParams& p, const SplitMap& map, uint32_t head_dim, uint32_t kv_dtype, hipStream_t s);
 hipError_t launch_attn_wsplit(const AttnParams& p, uint32_t head_dim, uint32_t kv_dtype, hipStream_t s);
-// (shared_tiles: the partial rows are the one-launch kernel's, whose workgroups go by split, then row tile)
+// (shared_tiles: see plan_merge)
 hipError_t launch_attn_merge(const AttnParams& p, const SplitMap& map, uint32_t head_dim, bool streamed, bool shared_tiles, hipStream_t s);
 hipError_t launch_state_merge(const StateMergeParams& p, hipStream_t s);
 // l[row] = 1 where m[row] is finite, else 0: completes a state whose rows are already normalised

@@ -130,6 +130,60 @@ def test_units_by_row_tile(tmp_path):
     run_program(tmp_path, BY_ROWS)
 
 
+MERGE_RUNS = r"""
+#include "attn_params.h"
+#include <cstdio>
+#include <vector>
+using namespace dg;
+int main() {
+  const uint32_t heads[] = {1, 2, 3, 4, 5, 8, 12, 16}, rows[] = {1, 8, 74, 127, 128, 129, 333, 392, 512, 576, 768, 1600, 2048, 4095};
+  for (uint32_t hkv : heads)
+    for (uint32_t rt : rows)
+      for (uint32_t S = 2; S <= kMergeFewSplits; ++S) {
+        const uint32_t mt = (rt + kBlockM - 1) / kBlockM, T = hkv * mt, per = (T * S + 7) / 8;
+        // which XCD writes split s of row tile t of a KV head: whole heads in either order, else by row tile, then split
+        auto wrote = [&](uint32_t h, uint32_t t, uint32_t s) { return ((h * mt + t) * S + s) / per; };
+        const MergeRuns r = merge_runs(hkv, rt, mt, S);
+        std::vector<uint32_t> seen(hkv * rt, 0);
+        const FastDiv by = make_fast_div(r.span);
+        uint64_t own = 0;
+        for (uint32_t b = 0; b < 8 * r.run; ++b)
+          for (uint32_t w = 0; w < 4; ++w) {
+            const uint32_t n = merge_row(b, w, r.run), h = fast_div(n, by), row = n - h * r.span;
+            if (h >= hkv || row >= rt) continue;
+            ++seen[h * rt + row];
+            uint32_t here = 0;
+            for (uint32_t s = 0; s < S; ++s) here += wrote(h, row / kBlockM, s) == b % 8 ? 1 : 0;
+            own += here;
+            const bool whole = hkv % 8 == 0 || (T % 8 == 0 && T * S % 8 == 0);
+            if (whole && here != S) return std::printf("%u heads, %u rows, %u splits: row %u of head %u\n", hkv, rt, S, row, h), 1;
+          }
+        for (uint32_t n : seen)
+          if (n != 1) return std::printf("%u heads, %u rows, %u splits: a row %u times\n", hkv, rt, S, n), 2;
+        // row tiles cut by the end of a run: half of what is merged was written there at the least
+        if (T >= 8 && own * 2 < (uint64_t)hkv * rt * S) return std::printf("%u heads, %u rows, %u splits: %g\n", hkv, rt, S, (double)own / (hkv * rt * S)), 3;
+        // in turn: every row once
+        std::fill(seen.begin(), seen.end(), 0u);
+        for (uint32_t b = 0; b < (hkv * rt + 3) / 4; ++b)
+          for (uint32_t w = 0; w < 4; ++w) {
+            const uint32_t n = merge_row(b, w, 0), h = fast_div(n, make_fast_div(rt));
+            if (h < hkv) ++seen[n];
+          }
+        for (uint32_t n : seen)
+          if (n != 1) return 4;
+      }
+  std::puts("ok");
+  return 0;
+}
+"""
+
+
+def test_rows_are_merged_where_they_were_written(tmp_path):
+    """The merge's runs of rows, one for each XCD, against the split kernel's runs of units: every row once, on the XCD that wrote its
+    partial rows where no row tile is cut by the end of a run, and on one that wrote most of them otherwise."""
+    run_program(tmp_path, MERGE_RUNS)
+
+
 def test_units_of_a_split_map(tmp_path):
     run_program(tmp_path, PROGRAM)
 
