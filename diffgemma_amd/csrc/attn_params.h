@@ -391,15 +391,18 @@ inline bool merge_at_once(uint32_t n_splits, size_t bytes) {
   return n_splits <= 8 ? bytes < ((size_t)32 << 20) : n_splits <= kMergeFewSplits && bytes <= ((size_t)17 << 20);
 }
 
-// Whether the merge that asks for all rows at once takes a row on the XCD that wrote its partial rows (their splits on one XCD):
-// where these, `part_bytes` in all, and the keys an XCD has read since, `head_bytes` for each KV head, are still in its L2 of 4 MiB
-// when they are wanted.  (Reading there and writing rows of which no other L2 holds a copy are not told apart: under the profiler, 256 rows
-// over 556 keys, the attention kernel took 17.4 us for 19.4 and the merge what it took.)  Layer step, 16 heads over 2, us, rows
-// in turn over the XCDs | where they were written: 256 rows over 556 keys (3.2 MiB) 29.4 | 26.0, 1033 (5.1) 29.6 | 28.2, 1756 (7.5)
-// 32.8 | 32.5; 128 rows over 905 (4.1) 26.0 | 23.0; 64 rows over 1564 (4.7) 23.3 | 22.0; call alone, 64 over 2564 (7) 22.3 | 22.5, over 4064 26.0 |
-// 26.3; 64 rows over a window of 8 KV heads x 256 (1.6) 15.3 | 14.7 (step).
+// Whether the merge that asks for all rows at once takes a row on the XCD that wrote its partial rows (merge_runs): where these,
+// `part_bytes` in all, and the keys that an XCD has read, `head_bytes` for each of its KV heads, are no more than 6 MiB.  An XCD's L2 is 4,
+// and not all of it is wanted again; the line is a fit to the times, not worked out.  (Reading there and writing rows of which no other L2
+// holds a copy are not told apart: under the profiler, 256 rows over 556 keys, rows in turn | in runs, the attention kernel took
+// 20.0 | 17.4 us and the merge 6.0 | 5.8.)  Layer step, 16 heads over 2, us, units by row tile and rows in turn | in runs: 256 rows over 356 keys 26.8 |
+// 25.0, 556 (3.2 MiB) 29.4 | 26.0, 1033 (5.1) 29.6 | 28.2, 1756 (7.5) 32.8 | 32.5; 128 rows over 905 (4.1) 26.0 | 23.0; 64 rows over 841 20.7 | 19.3,
+// 1564 (4.7) 23.3 | 22.0; 512 over 612 33.3 | 32.7, f16 36.6 | 32.3; call alone, 64 over 2564 (7) 22.3 | 22.5, over 4064 26.0 | 26.3.  Other heads,
+// call alone: 8 over 8, 256 rows over 556 20.2 | 18.1, over 1256 24.1 | 21.8; 32 over 8, 64 rows over 1064 24.1 | 21.2; 16 over 1, 64 rows
+// over 1064 19.8 | 17.2; the one-launch kernel's shared row tiles, 64 rows over a window of 8 KV heads x 256 (1.6), 15.3 | 14.7 (step).
+// Heads are rounded up: 12 KV heads are one and a half to an XCD, and it reads the keys of two.
 inline bool merge_on_xcd(uint32_t hkv, size_t head_bytes, size_t part_bytes) {
-  return head_bytes * std::max(1u, hkv / 8u) + part_bytes / 8 <= ((size_t)6 << 20);
+  return head_bytes * ((hkv + 7u) / 8u) + part_bytes / 8 <= ((size_t)6 << 20);
 }
 
 // Rows of the merge that asks for all at once, four to a workgroup.  In turn: run = 0, span the rows of a KV head.  In runs, one of

@@ -184,6 +184,15 @@ def test_rows_are_merged_where_they_were_written(tmp_path):
     run_program(tmp_path, MERGE_RUNS)
 
 
+def test_keys_an_xcd_reads_before_the_merge(tmp_path):
+    """KV heads of an XCD, rounded up, times their keys, and an eighth of the partial rows, against 6 MiB."""
+    mib = 1 << 20
+    wrong = " || ".join(f"dg::merge_on_xcd({hkv}, {head}, {part}) != {str(yes).lower()}" for hkv, head, part, yes in (
+        (1, 6 * mib, 0, True), (2, 5 * mib, 8 * mib, True), (2, 5 * mib, 8 * mib + 8, False), (8, 6 * mib, 0, True), (8, 6 * mib + 1, 0, False),
+        (12, 3 * mib, 0, True), (12, 3 * mib + 1, 0, False), (16, 3 * mib, 0, True), (17, 2 * mib, 0, True), (17, 3 * mib, 0, False)))
+    run_program(tmp_path, '#include "attn_params.h"\n#include <cstdio>\nint main() { if (%s) return 1; std::puts("ok"); return 0; }\n' % wrong)
+
+
 def test_units_of_a_split_map(tmp_path):
     run_program(tmp_path, PROGRAM)
 
