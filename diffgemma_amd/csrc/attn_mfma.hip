@@ -106,7 +106,7 @@ struct MfmaArgs {
   FastDiv div_mtiles, div_splits, div_group;
   FastDiv div_units, div_n[kMapSplits];   // with a split map: by the units of a KV head, by 1 .. 8
   SplitMap map;
-  uint32_t rows_first;   // order of the units: rows_before_splits
+  uint32_t rows_first;   // order of the units: units_by_row_tile
 };
 
 // MAPPED: with a split map (an instance of its own: what the map takes at a workgroup's start is 0.3 us of a short call)
@@ -891,7 +891,7 @@ hipError_t launch_one(const AttnParams& p, const SplitMap& map, hipStream_t s) {
   a.div_group = make_fast_div(p.group);
   a.div_units = make_fast_div(std::max(1u, map.units));
   for (uint32_t i = 0; i < kMapSplits; ++i) a.div_n[i] = make_fast_div(i + 1u);
-  a.rows_first = rows_before_splits(p.hkv, p.n_mtiles, p.tile_end - p.tile_first) ? 1u : 0u;
+  a.rows_first = units_by_row_tile(p, map) ? 1u : 0u;
   const uint32_t n_units = p.hkv * (map.n ? map.units : p.n_splits * p.n_mtiles);
   const uint32_t grid = (n_units + 7u) / 8u * 8u;
   auto launch = [&](auto kernel) {

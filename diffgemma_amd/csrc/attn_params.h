@@ -20,7 +20,7 @@ constexpr float kLn2 = 0.6931471805599453f;
 // count for all the launch is as long as the last row tile's share).  The counts do not fall with the row tile, so they
 // are given by where each begins: row tile mt has more than i splits from mt = first[i] on.  The units of a KV head are
 // ordered by split, then row tile: split i of row tile mt is unit cum[i] + mt - first[i], which also numbers its partial rows.
-// The workgroups may go by row tile, then split, instead (rows_before_splits): the row tiles of i + 1 splits begin with
+// The workgroups may go by row tile, then split, instead (units_by_row_tile): the row tiles of i + 1 splits begin with
 // workgroup at[i].
 constexpr uint32_t kMapSplits = 8;
 struct SplitMap {
@@ -190,6 +190,16 @@ inline uint32_t splits_in_rounds(uint32_t base, uint32_t tiles, uint32_t least, 
 // of 8 to 48 rows gain 4 % or lose 1 (32 over 432 keys 14.9 | 14.2, 40 over 440 14.8 | 15.0).
 inline bool rows_before_splits(uint32_t hkv, uint32_t n_mtiles, uint32_t key_tiles) {
   return key_tiles <= std::min((hkv * n_mtiles % 8u == 0u ? 20u : 10u) * n_mtiles, 72u + 2u * n_mtiles);
+}
+// Whether a call takes that order.  With fewer than eight row tiles the splits of one are on several XCDs in either order; taken there
+// where every XCD has a run of the same length out of one row tile (4 row tiles: 32 rows over 432 keys in 14 splits 14.9 -> 14.2; 8
+// heads over 1, 64 rows over 364 keys 14.4 -> 13.8), and not where the ends of runs cut them (6 row tiles, 40 rows over 440 keys in 7 splits
+// 14.8 -> 15.0; 4, 32 rows over 92 keys in 3 splits 15.1 -> 15.3, over 532 in 9 14.65 -> 14.64; turned away with them: 2, 16 rows over 316
+// keys in 5 splits, 18.9 either way, f16 19.3 -> 18.9).
+inline bool units_by_row_tile(const AttnParams& p, const SplitMap& map) {
+  const uint32_t tiles = p.hkv * p.n_mtiles;
+  if (tiles < 8u && (map.n || 8u % tiles != 0u || tiles * p.n_splits % 8u != 0u)) return false;
+  return rows_before_splits(p.hkv, p.n_mtiles, p.tile_end - p.tile_first);
 }
 
 // One pass of top-k sparse attention over canvas rows [tok0, tok0 + ntok).
@@ -440,7 +450,7 @@ inline MergePlan plan_merge(const AttnParams& p, const SplitMap& map, uint32_t h
   const size_t part_bytes = (size_t)p.n_splits * p.hkv * p.rows_pad * head_dim * (p.part_half ? 2 : 4);
   const bool at_once = map.n || (!streamed && (p.part_half || p.n_splits <= 8) && head_dim % 8 == 0 && head_dim <= 512 &&
                                  merge_at_once(p.n_splits, part_bytes));
-  const bool one_xcd = map.n == 0 && (p.hkv % 8 == 0 || (!shared_tiles && rows_before_splits(p.hkv, p.n_mtiles, key_tiles)));
+  const bool one_xcd = map.n == 0 && (p.hkv % 8 == 0 || (!shared_tiles && units_by_row_tile(p, map)));
   if (at_once && one_xcd && merge_on_xcd(p.hkv, (size_t)key_tiles * kBlockN * head_dim * 4, part_bytes))
     return MergePlan{true, merge_runs(p.hkv, p.rows_total, p.n_mtiles, p.n_splits)};
   return MergePlan{at_once, MergeRuns{p.rows_total, 0u}};
