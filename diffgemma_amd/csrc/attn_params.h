@@ -196,10 +196,14 @@ inline bool rows_before_splits(uint32_t hkv, uint32_t n_mtiles, uint32_t key_til
 // heads over 1, 64 rows over 364 keys 14.4 -> 13.8), and not where the ends of runs cut them (6 row tiles, 40 rows over 440 keys in 7 splits
 // 14.8 -> 15.0; 4, 32 rows over 92 keys in 3 splits 15.1 -> 15.3, over 532 in 9 14.65 -> 14.64; turned away with them: 2, 16 rows over 316
 // keys in 5 splits, 18.9 either way, f16 19.3 -> 18.9).
+// With rows from HBM the gain ends sooner: 256 peaked rows over 3256 keys, 102 tiles, of an f16 cache 54.1 -> 54.7 (bf16 40.5 -> 40.3), and
+// the line there leaves that form out and 128 rows over 2628 (83 tiles, 29.0 -> 28.5) and 1024 causal ones behind 3000 (126, 123.5 -> 121.8) in.
 inline bool units_by_row_tile(const AttnParams& p, const SplitMap& map) {
   const uint32_t tiles = p.hkv * p.n_mtiles;
   if (tiles < 8u && (map.n || 8u % tiles != 0u || tiles * p.n_splits % 8u != 0u)) return false;
-  return rows_before_splits(p.hkv, p.n_mtiles, p.tile_end - p.tile_first);
+  const uint32_t key_tiles = p.tile_end - p.tile_first;
+  if (p.touch_ahead && key_tiles > 72u + 3u * p.n_mtiles / 2u) return false;
+  return rows_before_splits(p.hkv, p.n_mtiles, key_tiles);
 }
 
 // One pass of top-k sparse attention over canvas rows [tok0, tok0 + ntok).

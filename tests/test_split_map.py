@@ -135,12 +135,13 @@ BY_ROWS_CALLS = r"""
 #include <cstdio>
 using namespace dg;
 int main() {
-  struct Call { uint32_t hkv, n_mtiles, n_splits, key_tiles, map_n; bool by_rows; };
+  struct Call { uint32_t hkv, n_mtiles, n_splits, key_tiles, map_n; bool by_rows; uint32_t from_hbm; };
   const Call calls[] = {
 %s  };
   for (const Call& c : calls) {
     AttnParams p = {};
     p.hkv = c.hkv, p.n_mtiles = c.n_mtiles, p.n_splits = c.n_splits, p.tile_first = 3, p.tile_end = 3 + c.key_tiles;
+    p.touch_ahead = c.from_hbm;
     SplitMap map = {};
     map.n = c.map_n;
     if (units_by_row_tile(p, map) != c.by_rows)
@@ -154,11 +155,15 @@ int main() {
 
 def test_calls_whose_units_go_by_row_tile(tmp_path):
     """(KV heads, row tiles of a KV head, splits, key tiles, a map's splits): with fewer than eight row tiles only where every XCD has an equal
-    run out of one of them; from eight on by the number of key tiles alone."""
+    run out of one of them; from eight on by the number of key tiles, fewer where the rows come from HBM."""
     calls = [((2, 2, 14, 14, 0), True), ((2, 3, 7, 14, 0), False), ((2, 2, 3, 3, 0), False), ((2, 2, 9, 17, 0), False), ((2, 1, 4, 4, 0), True),
              ((2, 3, 8, 14, 0), False), ((2, 2, 4, 14, 4), False), ((1, 4, 12, 12, 0), True), ((1, 7, 8, 12, 0), False), ((1, 8, 5, 12, 0), True),
              ((2, 4, 7, 14, 0), True), ((2, 5, 7, 14, 0), True), ((2, 16, 6, 33, 0), True), ((2, 16, 8, 105, 0), False), ((2, 44, 4, 44, 4), True)]
-    rows = "".join("    {%d, %d, %d, %d, %d, %s},\n" % (*c, str(yes).lower()) for c, yes in calls)
+    cold = [((2, 16, 8, 96, 0), True), ((2, 16, 8, 97, 0), False), ((2, 16, 8, 102, 0), False), ((2, 8, 12, 83, 0), True), ((2, 64, 2, 126, 2), True),
+            ((2, 4, 7, 14, 0), True), ((2, 4, 14, 78, 0), True), ((2, 4, 14, 79, 0), False)]
+    calls += [((2, 16, 8, 104, 0), True), ((2, 4, 14, 80, 0), True)]
+    rows = "".join("    {%d, %d, %d, %d, %d, %s, %d},\n" % (*c, str(yes).lower(), hbm)
+                   for hbm, forms in ((0, calls), (1, cold)) for c, yes in forms)
     run_program(tmp_path, BY_ROWS_CALLS % rows)
 
 
