@@ -891,7 +891,7 @@ hipError_t launch_one(const AttnParams& p, const SplitMap& map, hipStream_t s) {
   a.div_group = make_fast_div(p.group);
   a.div_units = make_fast_div(std::max(1u, map.units));
   for (uint32_t i = 0; i < kMapSplits; ++i) a.div_n[i] = make_fast_div(i + 1u);
-  a.rows_first = units_by_row_tile(p, map) ? 1u : 0u;
+  a.rows_first = units_by_row_tile(p, map, D) ? 1u : 0u;
   const uint32_t n_units = p.hkv * (map.n ? map.units : p.n_splits * p.n_mtiles);
   const uint32_t grid = (n_units + 7u) / 8u * 8u;
   auto launch = [&](auto kernel) {

@@ -198,7 +198,10 @@ inline bool rows_before_splits(uint32_t hkv, uint32_t n_mtiles, uint32_t key_til
 // keys in 5 splits, 18.9 either way, f16 19.3 -> 18.9).
 // With rows from HBM the gain ends sooner: 256 peaked rows over 3256 keys, 102 tiles, of an f16 cache 54.1 -> 54.7 (bf16 40.5 -> 40.3), and
 // the line there leaves that form out and 128 rows over 2628 (83 tiles, 29.0 -> 28.5) and 1024 causal ones behind 3000 (126, 123.5 -> 121.8) in.
-inline bool units_by_row_tile(const AttnParams& p, const SplitMap& map) {
+// With KV heads in eights an XCD has whole heads in either order: nothing to gain (8 over 8, 256 rows over 556 keys 20.2 | 20.2, 1256 24.1 |
+// 24.1; 32 over 8, 64 rows over 364 17.8 | 17.8).  head_dim 256: 256 rows over 3256 keys 32.9 | 29.3; below it there are no times.
+inline bool units_by_row_tile(const AttnParams& p, const SplitMap& map, uint32_t head_dim) {
+  if (head_dim < 256u || p.hkv % 8u == 0u) return false;
   const uint32_t tiles = p.hkv * p.n_mtiles;
   if (tiles < 8u && (map.n || 8u % tiles != 0u || tiles * p.n_splits % 8u != 0u)) return false;
   const uint32_t key_tiles = p.tile_end - p.tile_first;
@@ -407,7 +410,7 @@ inline bool merge_at_once(uint32_t n_splits, size_t bytes) {
 
 // Whether the merge that asks for all rows at once takes a row on the XCD that wrote its partial rows (merge_runs): where these,
 // `part_bytes` in all, and the keys that an XCD has read, `head_bytes` for each of its KV heads, are no more than 6 MiB.  An XCD's L2 is 4,
-// and not all of it is wanted again; the line is a fit to the times, not worked out.  (Reading there and writing rows of which no other L2
+// and not all of it is wanted again; the line is a fit to times at head_dim 512 and 256, not worked out.  (Reading there and writing rows of which no other L2
 // holds a copy are not told apart: under the profiler, 256 rows over 556 keys, rows in turn | in runs, the attention kernel took
 // 20.0 | 17.4 us and the merge 6.0 | 5.8.)  Layer step, 16 heads over 2, us, units by row tile and rows in turn | in runs: 256 rows over 356 keys 26.8 |
 // 25.0, 556 (3.2 MiB) 29.4 | 26.0, 1033 (5.1) 29.6 | 28.2, 1756 (7.5) 32.8 | 32.5; 128 rows over 905 (4.1) 26.0 | 23.0; 64 rows over 841 20.7 | 19.3,
@@ -454,7 +457,7 @@ inline MergePlan plan_merge(const AttnParams& p, const SplitMap& map, uint32_t h
   const size_t part_bytes = (size_t)p.n_splits * p.hkv * p.rows_pad * head_dim * (p.part_half ? 2 : 4);
   const bool at_once = map.n || (!streamed && (p.part_half || p.n_splits <= 8) && head_dim % 8 == 0 && head_dim <= 512 &&
                                  merge_at_once(p.n_splits, part_bytes));
-  const bool one_xcd = map.n == 0 && (p.hkv % 8 == 0 || (!shared_tiles && units_by_row_tile(p, map)));
+  const bool one_xcd = map.n == 0 && head_dim >= 256 && (p.hkv % 8 == 0 || (!shared_tiles && units_by_row_tile(p, map, head_dim)));
   if (at_once && one_xcd && merge_on_xcd(p.hkv, (size_t)key_tiles * kBlockN * head_dim * 4, part_bytes))
     return MergePlan{true, merge_runs(p.hkv, p.rows_total, p.n_mtiles, p.n_splits)};
   return MergePlan{at_once, MergeRuns{p.rows_total, 0u}};

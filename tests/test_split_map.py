@@ -135,7 +135,7 @@ BY_ROWS_CALLS = r"""
 #include <cstdio>
 using namespace dg;
 int main() {
-  struct Call { uint32_t hkv, n_mtiles, n_splits, key_tiles, map_n; bool by_rows; uint32_t from_hbm; };
+  struct Call { uint32_t hkv, n_mtiles, n_splits, key_tiles, map_n; bool by_rows; uint32_t from_hbm, hd; };
   const Call calls[] = {
 %s  };
   for (const Call& c : calls) {
@@ -144,8 +144,22 @@ int main() {
     p.touch_ahead = c.from_hbm;
     SplitMap map = {};
     map.n = c.map_n;
-    if (units_by_row_tile(p, map) != c.by_rows)
+    if (units_by_row_tile(p, map, c.hd) != c.by_rows)
       return std::printf("%%u KV heads, %%u row tiles, %%u splits, %%u key tiles\\n", c.hkv, c.n_mtiles, c.n_splits, c.key_tiles), 1;
+  }
+  // merged in runs: the same, or KV heads in eights, from head_dim 256 on
+  AttnParams p = {};
+  p.hkv = 8, p.n_mtiles = 1, p.rows_total = 74, p.rows_pad = 128, p.n_splits = 3, p.part_half = 1, p.tile_end = 9;
+  for (uint32_t hd = 32; hd <= 512; hd *= 2)
+    for (uint32_t shared = 0; shared < 2; ++shared) {
+      const MergePlan m = plan_merge(p, SplitMap{}, hd, false, shared != 0);
+      if (!m.at_once || m.rows.run != (hd >= 256 ? 19u : 0u) || m.rows.span != (hd >= 256 ? 76u : 74u)) return std::printf("head_dim %%u\n", hd), 1;
+      if (plan_merge(p, SplitMap{}, hd, true, shared != 0).at_once) return 1;
+    }
+  p.hkv = 2, p.n_mtiles = 4, p.rows_total = 392, p.rows_pad = 512;
+  for (uint32_t shared = 0; shared < 2; ++shared) {
+    const MergePlan m = plan_merge(p, SplitMap{}, 512, false, shared != 0);
+    if (!m.at_once || m.rows.run != (shared ? 0u : 32u) || m.rows.span != (shared ? 392u : 512u)) return 1;
   }
   std::puts("ok");
   return 0;
@@ -155,15 +169,16 @@ int main() {
 
 def test_calls_whose_units_go_by_row_tile(tmp_path):
     """(KV heads, row tiles of a KV head, splits, key tiles, a map's splits): with fewer than eight row tiles only where every XCD has an equal
-    run out of one of them; from eight on by the number of key tiles, fewer where the rows come from HBM."""
+    run out of one of them; from eight on by the number of key tiles, fewer where the rows come from HBM; not
+    with KV heads in eights, nor below head_dim 256."""
     calls = [((2, 2, 14, 14, 0), True), ((2, 3, 7, 14, 0), False), ((2, 2, 3, 3, 0), False), ((2, 2, 9, 17, 0), False), ((2, 1, 4, 4, 0), True),
              ((2, 3, 8, 14, 0), False), ((2, 2, 4, 14, 4), False), ((1, 4, 12, 12, 0), True), ((1, 7, 8, 12, 0), False), ((1, 8, 5, 12, 0), True),
              ((2, 4, 7, 14, 0), True), ((2, 5, 7, 14, 0), True), ((2, 16, 6, 33, 0), True), ((2, 16, 8, 105, 0), False), ((2, 44, 4, 44, 4), True)]
     cold = [((2, 16, 8, 96, 0), True), ((2, 16, 8, 97, 0), False), ((2, 16, 8, 102, 0), False), ((2, 8, 12, 83, 0), True), ((2, 64, 2, 126, 2), True),
             ((2, 4, 7, 14, 0), True), ((2, 4, 14, 78, 0), True), ((2, 4, 14, 79, 0), False)]
-    calls += [((2, 16, 8, 104, 0), True), ((2, 4, 14, 80, 0), True)]
-    rows = "".join("    {%d, %d, %d, %d, %d, %s, %d},\n" % (*c, str(yes).lower(), hbm)
-                   for hbm, forms in ((0, calls), (1, cold)) for c, yes in forms)
+    calls += [((2, 16, 8, 104, 0), True), ((2, 4, 14, 80, 0), True), ((8, 1, 6, 12, 0), False), ((16, 2, 6, 12, 0), False), ((12, 2, 6, 12, 0), True)]
+    rows = "".join("    {%d, %d, %d, %d, %d, %s, %d, %d},\n" % (*c, str(yes and hd >= 256).lower(), hbm, hd)
+                   for hd in (32, 128, 256, 512) for hbm, forms in ((0, calls), (1, cold)) for c, yes in forms)
     run_program(tmp_path, BY_ROWS_CALLS % rows)
 
 
