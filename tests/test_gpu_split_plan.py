@@ -52,15 +52,24 @@ def test_smaller_scratch_takes_fewer_splits(gpu_ready):
         A.forward(d, qd, kd, outs[0], None, torch.empty(least - 256, dtype=torch.uint8, device="cuda"))
 
 
-@pytest.mark.parametrize("canvas,kv_len,causal_rows,f16,sees_masked", [
-    (1024, 0, 1024, False, False), (1024, 300, 1024, True, False), (901, 0, 901, False, False), (700, 700, 700, True, False),
-    (1000, 5, 1000, False, True), (800, 0, 500, False, False)])
+# (canvas, prefix, causal rows, f16 cache, sees masked) of calls with a split map, and the order of its units (test_split_map.py holds it to
+# the rules)
+MAP_FORMS = [
+    (1024, 0, 1024, False, False, "by row tile"), (1024, 300, 1024, True, False, "by row tile"), (901, 0, 901, False, False, "by row tile"),
+    (700, 700, 700, True, False, "by row tile"), (1000, 5, 1000, False, True, "by row tile"), (800, 0, 500, False, False, "by row tile"),
+    (700, 5060, 700, False, False, "by split"), (520, 4000, 520, True, False, "by split")]
+
+
+def map_workload(canvas, kv_len, causal_rows, f16, sees_masked):
+    return dataclasses.replace(W.Workload("map", canvas, 16, 2, 512, kv_len, causal_rows=causal_rows, sees_masked=sees_masked, seed=canvas), kv_f16=f16)
+
+
+@pytest.mark.parametrize("canvas,kv_len,causal_rows,f16,sees_masked", [f[:5] for f in MAP_FORMS])
 def test_split_counts_per_row_tile(gpu_ready, po, canvas, kv_len, causal_rows, f16, sees_masked):
-    """Causal rows behind a short prefix: row tiles of one split go straight to the output, the others are merged by counts of
-    their own.  Rows at the edges of row tiles against the oracle; the same bits on every run."""
+    """Causal rows with a split map: row tiles of one split go straight to the output, the others are merged by counts of their own,
+    with the units in either order.  Rows at the edges of row tiles against the oracle; the same bits on every run."""
     import torch
-    w = dataclasses.replace(W.Workload("map", canvas, 16, 2, 512, kv_len, causal_rows=causal_rows, sees_masked=sees_masked, seed=canvas),
-                            kv_f16=f16)
+    w = map_workload(canvas, kv_len, causal_rows, f16, sees_masked)
     toks = np.unique(np.concatenate([np.arange(0, canvas, 61), np.arange(15, canvas, 160), np.arange(16, canvas, 160),
                                      [causal_rows - 1, min(causal_rows, canvas - 1), canvas - 1]])).astype(np.uint32)
     check_tolerances(*run_workload(po, w, toks=toks))
@@ -227,17 +236,37 @@ def test_merge_at_once_gives_the_bits_of_the_streamed_merge(gpu_ready, hd, hkv, 
             assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
 
 
-@pytest.mark.parametrize("canvas,kv_len,hq,hkv,hd,causal_rows", [
-    (1, 300, 16, 2, 512, 0), (64, 2496, 16, 2, 512, 0), (64, 2497, 16, 2, 512, 0), (72, 1528, 16, 2, 512, 30), (72, 1529, 16, 2, 512, 0),
-    (37, 500, 8, 8, 512, 37), (65, 700, 9, 3, 512, 0), (37, 3500, 16, 16, 256, 0), (250, 3000, 16, 2, 512, 0), (64, 4000, 16, 8, 256, 0)])
+# (canvas, prefix, heads, KV heads, head_dim, causal rows), and the order of the units, how the rows are merged and the partial rows' type
+# (test_split_map.py holds them to the rules)
+ORDER_FORMS = [
+    (1, 300, 16, 2, 512, 0, "by split, in turn, f32"), (16, 100, 16, 2, 512, 0, "by row tile, in runs, f32"),
+    (32, 400, 16, 2, 512, 0, "by row tile, in runs, f16"), (40, 400, 16, 2, 512, 0, "by split, in turn, f16"),
+    (64, 120, 16, 2, 512, 0, "by row tile, in runs, f32"), (49, 700, 16, 2, 512, 30, "by row tile, in runs, f16"),
+    (64, 2496, 16, 2, 512, 0, "by row tile, in turn, f16"), (64, 2497, 16, 2, 512, 0, "by split, in turn, f16"),
+    (72, 1528, 16, 2, 512, 30, "by row tile, in runs, f16"), (72, 1529, 16, 2, 512, 0, "by split, in turn, f16"),
+    (200, 400, 16, 2, 512, 0, "by row tile, in runs, f16"), (250, 900, 16, 2, 512, 0, "by row tile, in runs, f16"),
+    (37, 500, 8, 8, 512, 37, "by split, in runs, f16"), (65, 700, 9, 3, 512, 0, "by split, in turn, f16"),
+    (140, 700, 9, 3, 512, 0, "by row tile, in runs, f16"), (64, 300, 16, 1, 512, 0, "by row tile, in runs, f16"),
+    (37, 3500, 16, 16, 256, 0, "by split, in turn, f16"), (64, 2100, 16, 2, 256, 0, "by row tile, in runs, f16"),
+    (64, 2100, 16, 2, 128, 0, "by split, in turn, f16"), (64, 4000, 16, 8, 256, 0, "shared, in runs, f32")]
+
+
+def order_workload(canvas, kv_len, hq, hkv, hd, causal_rows):
+    return W.Workload("order", canvas, hq, hkv, hd, kv_len, causal_rows=causal_rows, window=1024 if hkv == 8 and hd == 256 else 0, seed=canvas)
+
+
+ORDER_FLAGS = capi.DG_ATTN_F_KV_CACHED      # (the order also depends on where the rows come from)
+
+
+@pytest.mark.parametrize("canvas,kv_len,hq,hkv,hd,causal_rows", [f[:6] for f in ORDER_FORMS])
 def test_units_by_row_tile_and_rows_merged_where_they_were_written(gpu_ready, po, canvas, kv_len, hq, hkv, hd, causal_rows):
     """Either order of the workgroups, with row tiles that are cut by an XCD's run and rows that do not fill one, against the oracle; and
-    the merge that takes rows on the XCD that wrote them gives the bits of the one that takes them in turn."""
+    the merge that asks for all rows at once, its rows in turn or in runs, gives the bits of the one that looks at the weights first."""
     import torch
-    w = W.Workload("order", canvas, hq, hkv, hd, kv_len, causal_rows=causal_rows, window=1024 if hkv == 8 and hd == 256 else 0, seed=canvas)
-    d = w.desc()
+    w = order_workload(canvas, kv_len, hq, hkv, hd, causal_rows)
+    d = w.desc(flags=ORDER_FLAGS)
     assert capi.resolved_splits(d) > 1
-    check_tolerances(*run_workload(po, w, toks=np.unique(np.linspace(0, canvas - 1, 12).round().astype(np.uint32))))
+    check_tolerances(*run_workload(po, w, flags=ORDER_FLAGS, toks=np.unique(np.linspace(0, canvas - 1, 12).round().astype(np.uint32))))
     q, kv = W.generate(w)
     qd, kd = W.device_arrays(w, q, kv)
     got = []

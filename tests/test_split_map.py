@@ -1,6 +1,6 @@
 """Split counts per row tile (SplitMap in csrc/attn_params.h), compiled for the host: every (row tile, split) is one unit of a
 KV head, found again from its number, the longest share keeps the asked-for length, and the shortest length is found without
-trying each.  And the split and slice counts of the same header."""
+trying each.  And the other rules of the same header: split and slice counts, the order of units, how rows are merged."""
 import re
 import subprocess
 
@@ -182,6 +182,42 @@ def test_calls_whose_units_go_by_row_tile(tmp_path):
     run_program(tmp_path, BY_ROWS_CALLS % rows)
 
 
+PATHS = r"""
+#include "dg_attn_api.hip"
+#include <cstdio>
+#include <string>
+int main() {
+  const struct { unsigned char desc[sizeof(dg_attn_desc)]; const char* path; } calls[] = {
+%s  };
+  for (const auto& c : calls) {
+    dg_attn_desc d;
+    std::memcpy(&d, c.desc, sizeof(d));
+    Plan pl;
+    if (make_plan(&d, 256, &pl) != DG_OK) return 1;
+    dg::AttnParams p = {};
+    p.hkv = d.n_kv_heads, p.n_mtiles = pl.n_mtiles, p.n_splits = pl.n_splits, p.rows_total = pl.rows_total, p.rows_pad = pl.rows_pad;
+    p.tile_first = pl.tile_first, p.tile_end = pl.tile_end, p.part_half = pl.part_half;
+    const dg::MergePlan m = dg::plan_merge(p, pl.map, d.head_dim, false, pl.wsplit);
+    const std::string path = std::string(pl.wsplit ? "shared" : dg::units_by_row_tile(p, pl.map, d.head_dim) ? "by row tile" : "by split") +
+                             (pl.map.n ? ", map" : !m.at_once ? ", streamed" : m.rows.run ? ", in runs" : ", in turn") + (pl.part_half ? ", f16" : ", f32");
+    if (path != c.path) return std::printf("%%u rows behind %%u: %%s, not %%s\n", d.canvas, d.kv_len, path.c_str(), c.path), 1;
+  }
+  std::puts("ok");
+  return 0;
+}
+"""
+
+
+def test_paths_of_the_order_tests(tmp_path):
+    """The order of the units, the merge and the partial rows' type that the GPU tests' calls are named for are those they get."""
+    from test_gpu_split_plan import MAP_FORMS, ORDER_FLAGS, ORDER_FORMS, map_workload, order_workload
+    calls = [(order_workload(*f[:6]).desc(flags=ORDER_FLAGS), f[6]) for f in ORDER_FORMS]
+    calls += [(map_workload(*f[:5]).desc(), f[5] + ", map, f16") for f in MAP_FORMS]
+    rows = "".join('    {{%s}, "%s"},\n' % (",".join(map(str, bytes(d))), path) for d, path in calls)
+    run_program(tmp_path, PATHS % rows, "-I", str(build.CSRC.parent.parent / "include"),
+                "-L", str(build.LIB_PATH.parent), "-l:" + build.LIB_NAME, "-Wl,-rpath," + str(build.LIB_PATH.parent))
+
+
 MERGE_RUNS = r"""
 #include "attn_params.h"
 #include <cstdio>
@@ -262,10 +298,10 @@ def test_slices_of_the_gather(tmp_path):
     assert {n for _, n in GATHER_SLICES} == {1, 2, 4}
 
 
-def run_program(tmp_path, program):
+def run_program(tmp_path, program, *more):
     src, exe = tmp_path / "map.hip", tmp_path / "map"
     src.write_text(program)
-    res = subprocess.run([build.hipcc_path(), *build.HIP_FLAGS, "-I", str(build.CSRC), str(src), "-o", str(exe)],
+    res = subprocess.run([build.hipcc_path(), *build.HIP_FLAGS, "-I", str(build.CSRC), str(src), *more, "-o", str(exe)],
                          stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     assert res.returncode == 0, res.stdout[-2000:]
     res = subprocess.run([str(exe)], stdout=subprocess.PIPE, text=True)
