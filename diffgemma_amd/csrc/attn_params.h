@@ -180,14 +180,17 @@ inline uint32_t splits_in_rounds(uint32_t base, uint32_t tiles, uint32_t least, 
 // In which order the split kernel's workgroups take their units.  Each of the 8 XCDs gets a run of them and reads what its run
 // needs through an L2 of its own: by split, then row tile, a share of the keys and all query rows of a KV head; by row tile, then
 // split, its own query rows alone, which no workgroup can begin without, and all keys.  And a row tile's partial rows are then
-// written on one XCD: see merge_on_xcd.  Attention call, 16 heads over 2, us, splits first | rows first, with the keys in a cache | from
-// HBM: 64 rows over 1564 keys 22.1 | 20.8, 22.1 | 19.3, 2564 24.6 | 22.3, 25.9 | 26.0, layer step over 6064 34.3 | 36.5; 128 rows over 905 26.0 |
-// 23.0 (step), 23.0 | 19.8, 2628 27.7 | 27.0, 29.0 | 28.5, 5128 35.5 | 35.1, 37.7 | 37.4; 256 rows over 556 29.4 | 26.0 (step), 24.0 | 21.4, 3256 42.4 |
-// 41.2 (step), 40.5 | 40.3, 6256 61.1 | 60.3 (step), 59.2 | 60.3, 16256 120.8 | 121.5 (step); 512 rows over 1512 43.0 | 39.8 (step), 40.5 | 37.9, 4512
-// 78.7 | 77.2 (HBM), 8512 129.2 | 130.5 (HBM); 1024 causal rows behind 0 46.6 | 46.1 (step), 3000 123.5 | 121.8 (HBM), 8000 240.9 | 238.3, 243.3 | 244.3,
-// 32768 849 | 847, 860 | 868; 700 behind 700 48.9 | 47.1 (step).  Row tiles that do not come in eights end in the middle of an XCD's
-// run: 72 rows over 972 keys 19.2 | 18.1, over 1672 22.7 | 23.1; 96 over 1696 24.4 | 21.7, 2496 26.1 | 25.4; 200 over 2600 33.2 | 32.3; the few
-// of 8 to 48 rows gain 4 % or lose 1 (32 over 432 keys 14.9 | 14.2, 40 over 440 14.8 | 15.0).
+// written on one XCD, where the merge may take them up again (merge_on_xcd, whose gain is another and is not in these figures unless said).
+// 16 heads over 2, us, splits first | rows first, rows merged in turn, keys in a cache.  Layer step: 64 rows over 841 keys 21.0 | 20.7, 1564
+// 24.8 | 23.3, 3064 28.8 | 26.5, 6064 34.3 | 36.5; 128 rows over 905 26.1 | 26.0, 1628 29.6 | 27.4, 3128 32.4 | 31.9; 256 rows over 556 30.3 | 29.4, 1033
+// 29.8 | 29.6, 1756 33.5 | 32.8, 3256 42.4 | 41.2, 6256 61.1 | 60.3, 24256 172.9 | 173.4; 512 rows over 612 33.4 | 33.3 (f16 33.8 | 36.6, and 32.3 merged in
+// runs), 1289 43.0 | 39.8, 3512 69.9 | 67.5; 1024 causal rows behind 0 46.6 | 46.1, 300 57.2 | 55.4, 1000 78.4 | 75.7; 700 behind 700 48.9 | 47.1.
+// Attention call: 64 rows over 2564 24.6 | 22.3, 4064 26.8 | 26.0; 128 over 2628 27.7 | 27.0, 5128 35.5 | 35.1; 1024 behind 8000 240.9 | 238.3,
+// 32768 849 | 847.  Call with keys from HBM (rows merged in runs where merge_on_xcd says so, the first alone): 64 rows over 1564 22.1 | 19.3, 2564 25.9 |
+// 26.0; 128 over 2628 29.0 | 28.5, 5128 37.7 | 37.4; 256 over 3256 40.5 | 40.3, 6256 59.2 | 60.3; 512 over 4512 78.7 | 77.2, 8512 129.2 | 130.5; 1024
+// behind 3000 123.5 | 121.8, 8000 243.3 | 244.3, 32768 860 | 868.  The line lies where calls from HBM stop to gain; it turns away cached
+// ones that do (64 rows over 3064, 6064 being a loss).  Row tiles that do not come in eights end in the middle of an XCD's run (call, merged in runs where that is
+// taken): 72 rows over 972 keys 19.2 | 18.1, over 1672 22.7 | 23.1; 96 over 1696 24.4 | 21.7, 2496 26.1 | 25.4; 200 over 2600 33.2 | 32.3.
 inline bool rows_before_splits(uint32_t hkv, uint32_t n_mtiles, uint32_t key_tiles) {
   return key_tiles <= std::min((hkv * n_mtiles % 8u == 0u ? 20u : 10u) * n_mtiles, 72u + 2u * n_mtiles);
 }
@@ -466,7 +469,7 @@ inline MergePlan plan_merge(const AttnParams& p, const SplitMap& map, uint32_t h
 // host-side launchers (defined next to their kernels)
 hipError_t launch_attn_scalar(const AttnParams& p, uint32_t head_dim, uint32_t kv_dtype, hipStream_t s);
 // (map: row tiles with split counts of their own, head_dim 512; n = 0 for none. It stands behind AttnParams in the
-// arguments of these two and not inside it: its 72 bytes pushed what the one-launch kernel reads first to a further
+// arguments of these two and not inside it: its bytes, then 72 and now 104, pushed what the one-launch kernel reads first to a further
 // line of the arguments, and a call with 64 canvas rows on a sliding layer took 9.77 us for 9.52.)
 hipError_t launch_attn_mfma(const AttnParams& p, const SplitMap& map, uint32_t head_dim, uint32_t kv_dtype, hipStream_t s);
 hipError_t launch_attn_wsplit(const AttnParams& p, uint32_t head_dim, uint32_t kv_dtype, hipStream_t s);
